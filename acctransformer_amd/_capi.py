@@ -82,6 +82,8 @@ def load():
     lib.acct_fa_bwd_dkdv.restype = ctypes.c_int
     lib.acct_fa_fwd_workspace_bytes.argtypes = [P]
     lib.acct_fa_fwd_workspace_bytes.restype = ctypes.c_size_t
+    lib.acct_fa_fwd_split_workspace_bytes.argtypes = [P]
+    lib.acct_fa_fwd_split_workspace_bytes.restype = ctypes.c_size_t
     lib.acct_fa_drop_bits_bytes.argtypes = [P]
     lib.acct_fa_drop_bits_bytes.restype = ctypes.c_size_t
     lib.acct_fa_mask_bits_bytes.argtypes = [P]
@@ -244,7 +246,7 @@ def fa_fwd(p, q):
     if not any(p.o_stride):
         p.o_stride = _bhs_strides(o)
     lse = torch.empty((p.B, p.N, p.Sq), dtype=torch.float32, device=q.device)
-    nws = lib.acct_fa_fwd_workspace_bytes(ctypes.byref(p))
+    nws = lib.acct_fa_fwd_split_workspace_bytes(ctypes.byref(p))
     ws = _workspace(nws, q.device)
     with torch.cuda.device(q.device):
         _check(lib.acct_fa_fwd(ctypes.byref(p), _ptr(o), _ptr(lse), _ptr(ws), nws, _stream(q)))

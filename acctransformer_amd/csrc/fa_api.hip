@@ -260,6 +260,11 @@ size_t dropcol_bytes(const acct_fa_params* p) {
   return align_up((size_t)p->B * p->N * (size_t)((p->Sq + 127) / 128) * (size_t)p->Sk * 16, 256);
 }
 
+acct::FwdPlan plan_forward(const acct_fa_params* p, bool can_split, int n_cu) {
+  return acct::fwd_plan(p->B, p->N, p->Sq, p->Sk, p->D, p->alibi || dropout_on(p), p->mask_kind == ACCT_MASK_CAUSAL || p->next_block_num == 0,
+                        can_split, n_cu);
+}
+
 // Pre-passes over the attention mask: block classes of a dense mask (all three kernels) and the mask packed by
 // key column (dK/dV kernel; also for the compact tile).  They run into `own` (a workspace region of
 // flag_bytes + colbit_bytes) or, when the caller lends a mask_bits buffer, once into that buffer: the call that
@@ -297,6 +302,13 @@ int acct_build_is_complete(void) { return acct::launch_variants_complete() ? 1 :
 size_t acct_fa_fwd_workspace_bytes(const acct_fa_params* p) {
   if (!p || p->B <= 0 || p->N <= 0 || p->Sq <= 0 || p->Sk <= 0) return 0;
   return (p->mask_bits ? 0 : flag_bytes(p)) + (p->drop_bits ? 0 : droprow_bytes(p));
+}
+
+size_t acct_fa_fwd_split_workspace_bytes(const acct_fa_params* p) {
+  if (!p || p->B <= 0 || p->N <= 0 || p->Sq <= 0 || p->Sk <= 0 || p->D <= 0) return 0;
+  const size_t part = plan_forward(p, true, 256).part_bytes;
+  const size_t need = acct_fa_fwd_workspace_bytes(p);
+  return part ? align_up(need, 256) + part : need;
 }
 
 size_t acct_fa_mask_bits_bytes(const acct_fa_params* p) {
@@ -355,10 +367,13 @@ int acct_fa_fwd(const acct_fa_params* p, void* O, float* LSE, void* workspace, s
       if (e != hipSuccess) return fail(ACCT_E_LAUNCH, "dropout bitmap kernel: %s", hipGetErrorString(e));
     }
   }
-  // 8 waves x 32 query rows (two waves per SIMD overlap MFMA and softmax work) once that still
-  // fills the chip, else 4 waves x 32 rows for more workgroups
-  int qg = ((long long)p->B * p->N * ((p->Sq + 255) / 256) >= n_cu) ? 3 : 1;
-  hipError_t e = acct::launch_fwd(a, p->dtype, p->D, qg, st);
+  acct::FwdPlan plan = plan_forward(p, true, n_cu);
+  const size_t part_at = align_up(need, 256);
+  if (plan.kv_split > 1 && (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < part_at + plan.part_bytes))
+    plan = plan_forward(p, false, n_cu);              // no room for the slices' sums
+  a.kv_split = plan.kv_split;
+  if (plan.kv_split > 1) a.fwd_part = (float*)((char*)workspace + part_at);
+  hipError_t e = p->dtype == ACCT_F16 ? acct::launch_fwd_elem<acct::f16>(a, p->D, plan.kg, st) : acct::launch_fwd_elem<acct::bf16>(a, p->D, plan.kg, st);
   if (e != hipSuccess) return fail(ACCT_E_LAUNCH, "forward kernel: %s", hipGetErrorString(e));
   return ACCT_OK;
 }
@@ -433,7 +448,7 @@ static int bwd_impl(const acct_fa_params* p, const void* O, const void* dO, cons
       a.dkdv_part = (float*)((char*)workspace + part_at);
     }
   }
-  hipError_t e = acct::launch_bwd(a, p->dtype, p->D, stages, st);
+  hipError_t e = p->dtype == ACCT_F16 ? acct::launch_bwd_elem<acct::f16>(a, p->D, stages, st) : acct::launch_bwd_elem<acct::bf16>(a, p->D, stages, st);
   if (e != hipSuccess) return fail(ACCT_E_LAUNCH, "backward kernels: %s", hipGetErrorString(e));
   if (p->grad_f32) {
     e = cast_rows_to_f32(a.dq, (float*)out_f32[0], p->dtype, p->B, p->N, p->Sq, p->D, a.q_sb, a.q_sh, a.q_ss, st);

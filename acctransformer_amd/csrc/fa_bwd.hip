@@ -18,6 +18,10 @@
 #include "fa_common.hpp"
 #include "fa_launch.hpp"
 
+#ifndef ACCT_ELEM
+#error "compiled once per element type: -DACCT_ELEM=f16 and -DACCT_ELEM=bf16"
+#endif
+
 #include <type_traits>
 
 namespace acct {
@@ -1142,36 +1146,21 @@ static hipError_t launch_bwd_d(const FaArgs& a, int stages, hipStream_t st) {
   return launch_bwd_t<T, D, false, false>(a, stages, st);
 }
 
-bool fwd_variants_complete();
-#ifdef ACCT_DEV_BUILD
-bool launch_variants_complete() { return false; }
-#else
-bool launch_variants_complete() { return fwd_variants_complete(); }
-#endif
-
-hipError_t launch_bwd(const FaArgs& a, int dtype, int Dr, int stages, hipStream_t st) {
+template <typename T>
+hipError_t launch_bwd_elem(const FaArgs& a, int Dr, int stages, hipStream_t st) {
   const int D = head_dim_class(Dr);
+  if (D == 128) return launch_bwd_d<T, 128>(a, stages, st);
 #ifdef ACCT_DEV_BUILD
-  if (dtype != 0 || D != 128) return hipErrorNotSupported;
-  return launch_bwd_d<f16, 128>(a, stages, st);
+  return hipErrorNotSupported;
 #else
-  if (dtype == 0) {
-    if (D == 128) return launch_bwd_d<f16, 128>(a, stages, st);
-    if (D == 64) return launch_bwd_d<f16, 64>(a, stages, st);
-    if (D == 80) return launch_bwd_d<f16, 80>(a, stages, st);
-    if (D == 40) return launch_bwd_d<f16, 40, 1>(a, stages, st);
-    if (D == 160) return launch_bwd_d<f16, 160, 1>(a, stages, st);
-    if (D == 256) return launch_bwd_d<f16, 256, 1>(a, stages, st);
-  } else {
-    if (D == 128) return launch_bwd_d<bf16, 128>(a, stages, st);
-    if (D == 64) return launch_bwd_d<bf16, 64>(a, stages, st);
-    if (D == 80) return launch_bwd_d<bf16, 80>(a, stages, st);
-    if (D == 40) return launch_bwd_d<bf16, 40, 1>(a, stages, st);
-    if (D == 160) return launch_bwd_d<bf16, 160, 1>(a, stages, st);
-    if (D == 256) return launch_bwd_d<bf16, 256, 1>(a, stages, st);
-  }
+  if (D == 64) return launch_bwd_d<T, 64>(a, stages, st);
+  if (D == 80) return launch_bwd_d<T, 80>(a, stages, st);
+  if (D == 40) return launch_bwd_d<T, 40, 1>(a, stages, st);
+  if (D == 160) return launch_bwd_d<T, 160, 1>(a, stages, st);
+  if (D == 256) return launch_bwd_d<T, 256, 1>(a, stages, st);
   return hipErrorInvalidValue;
 #endif
 }
+template hipError_t launch_bwd_elem<ACCT_ELEM>(const FaArgs& a, int Dr, int stages, hipStream_t st);
 
 }  // namespace acct

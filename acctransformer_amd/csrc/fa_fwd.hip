@@ -16,31 +16,52 @@
 #include "fa_common.hpp"
 #include "fa_launch.hpp"
 
+#ifndef ACCT_ELEM
+#error "compiled once per element type: -DACCT_ELEM=f16 and -DACCT_ELEM=bf16"
+#endif
+
 namespace acct {
 
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2>
+// LDS of the key-group merge: behind the output staging of the RG row groups, one slot per wave of the key groups
+// 1 .. KG - 1 (accumulators as they sit in the registers, then running max and sum)
+template <int D, int RG> constexpr int fwd_merge_at() { return RG * 32 * (SwzCfg<D>::DB * 64 + 16); }
+template <int D> constexpr int fwd_merge_slot() { return SwzCfg<D>::DB * 4096 + 512; }
+
+// KG > 1 (small grids): the waves of a workgroup form NW / KG row groups times KG key groups.  A wave then works on
+// its key group's share of every tile only, with softmax statistics of its own, and the key groups of a row group
+// are merged through LDS before the epilogue -- KG times as many workgroups for the same rows, every wave busy.
+template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2, int KG = 1>
 ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   static_assert(KT == 2 || KT == 4, "key tiles are 64 or 128 rows (with a bias, 128 rows take the key-only form of it only)");
+  static_assert(KG == 1 || (QG == 1 && KT % KG == 0 && NW % KG == 0), "key groups own whole 32-key chunks");
   constexpr int BN = 32 * KT;                       // key rows per tile
+  constexpr int KTW = KT / KG, WN = 32 * KTW;       // 32-key chunks and keys of a tile that one wave works on
+  constexpr int RG = NW / KG;                       // row groups
   constexpr int FRING = 4, VRING = 3;   // fragment reads in flight ahead of their MFMA (K row-major / V transposed)
   constexpr int TPB = 128 / BN;                     // tiles per 128-column block
   using E = Elem<T>;
   using V8 = typename E::V8;
   using C = SwzCfg<D>;
-  constexpr int BM = 32 * QG * NW;
+  constexpr int BM = 32 * QG * RG;
   constexpr int TILEB = BN * C::PITCH;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   ACCT_LDS char* smem = (ACCT_LDS char*)smem_raw;   // [2 buffers][K tile | V tile]; reused by the epilogue
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: everything derived from it stays in scalar registers
-  const int BH = a.B * a.N;
+  const int rg = KG > 1 ? wave % RG : wave, kg = KG > 1 ? wave / RG : 0;
+  const int BH = a.B * a.N, n_wg = BH * a.n_tiles;
+  int wg = blockIdx.x, slice = 0;                           // kv_split > 1: the grid holds every query tile once per key slice
+  if (a.kv_split > 1) {
+    slice = wg / n_wg;
+    wg -= slice * n_wg;
+  }
   int bh, rank;
-  wg_map(blockIdx.x, BH, a.n_tiles, bh, rank);
+  wg_map(wg, BH, a.n_tiles, bh, rank);
   const int qt = a.n_tiles - 1 - rank;                      // heaviest (latest) causal tiles first
   const int b = bh / a.N, h = bh % a.N;
   const int q0 = qt * BM;
-  const int wq0 = q0 + wave * 32 * QG;                      // first query row of this wave
+  const int wq0 = q0 + rg * 32 * QG;                        // first query row of this wave
   const int q_end = min(q0 + BM, a.Sq);                     // one past the last valid row of the block
   const int wq_end = min(wq0 + 32 * QG, a.Sq);
 
@@ -77,6 +98,11 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       };
       trim_dead_tiles(j_lo, j_hi, lane, dead);
     }
+  }
+  if (a.kv_split > 1) {                                     // this workgroup's slice of the tiles it sees
+    const int n = max(j_hi - j_lo + 1, 0), lo = j_lo;
+    j_lo = lo + (int)((int64_t)n * slice / a.kv_split);
+    j_hi = lo + (int)((int64_t)n * (slice + 1) / a.kv_split) - 1;
   }
   const int wkv_limit = a.row_prefix ? (wq0 / a.row_prefix + 1) * a.row_prefix : 0x7fffffff;   // keys past it are absent
 
@@ -115,7 +141,8 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   float m[QG], lsum[QG];
 #pragma unroll
   for (int gq = 0; gq < QG; gq++) {
-    m[gq] = -INFINITY;
+    // (finite: the first keys a key group or a key slice sees may all be hidden from a row, and -inf - -inf is NaN)
+    m[gq] = -1e30f;
     lsum[gq] = 0.f;
 #pragma unroll
     for (int db = 0; db < C::DB; db++)
@@ -172,10 +199,11 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   // what this wave does with tile j (tiles must be asked for in ascending order)
   auto classify = [&](int j) -> uint32_t {
     const uint32_t fl_cur = flwin.get(j / TPB, lane);
-    const int kv0 = j * BN, kvb = j / TPB;
+    const int kv0 = j * BN + kg * WN, kvb = j / TPB;
     bool act = (kvb - a.next_blk <= wqb) && (wqb <= kvb + a.prev_blk) && (wq0 < a.Sq);
     if (causal) act = act && (kv0 <= wq_end - 1);
     act = act && (kv0 < wkv_limit);
+    if (KG > 1) act = act && (kv0 < a.Sk);
     bool apply_mask = false;
     bool diag = causal;                                     // keys after the query are hidden, by index compare
     uint32_t tail = 0;
@@ -199,16 +227,16 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     else tile_dma<T, D, BN, NW>(base, ss, j * BN, a.Sk, dst, cpr);   // ragged last tile: clamped rows
   };
   // S^T = K Q^T : s[gq][c] is the 32(kv) x 32(q) tile of kv chunk c
-  auto gemm_s = [&](const ACCT_LDS char* kbuf, int j, f32x16 (&s)[QG][KT]) {
+  auto gemm_s = [&](const ACCT_LDS char* kbuf, int j, f32x16 (&s)[QG][KTW]) {
     if (BIAS && acc_bias) {
       // element (c, r) belongs to key 32 c + 8 (r/4) + 4 g + r%4 of the tile, whatever the lane's row
 #pragma unroll
       for (int gq = 0; gq < QG; gq++)
 #pragma unroll
-        for (int c = 0; c < KT; c++)
+        for (int c = 0; c < KTW; c++)
 #pragma unroll
           for (int r4 = 0; r4 < 4; r4++) {
-            const typename E::V4 bv = bias_tile_read<T>(bias_lds + gq * 4096 + (j & 1) * 256, 0, 4 * c + r4, g);
+            const typename E::V4 bv = bias_tile_read<T>(bias_lds + gq * 4096 + (j & 1) * 256, 0, 4 * (kg * KTW + c) + r4, g);
 #pragma unroll
             for (int e = 0; e < 4; e++) s[gq][c][4 * r4 + e] = (float)bv[e] * a.inv_scale;
           }
@@ -216,14 +244,14 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
 #pragma unroll
       for (int gq = 0; gq < QG; gq++)
 #pragma unroll
-        for (int c = 0; c < KT; c++)
+        for (int c = 0; c < KTW; c++)
 #pragma unroll
           for (int r = 0; r < 16; r++) s[gq][c][r] = 0.f;
     }
     // K fragments travel through a ring of FRING register sets: FRING reads are in flight ahead of the
     // MFMA that consumes the oldest one, so that a wave covers the LDS latency (well over one MFMA) by
     // itself.  The scheduling barriers keep the compiler from folding the ring back into read-wait-MFMA.
-    constexpr int NF = KT * C::KS;
+    constexpr int NF = KTW * C::KS;
     constexpr int RING = FRING < NF ? FRING : NF;
     V8 ring[RING];
     auto kread = [&](int i) { return lds_read_frag<T>(kbuf + koff(i % C::KS) + (i / C::KS) * 32 * C::PITCH); };
@@ -241,8 +269,8 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     __builtin_amdgcn_sched_barrier(0);
   };
   // O^T += V^T P^T, the transposed V fragments through a ring as well
-  auto gemm_pv = [&](const ACCT_LDS char* vbuf, const V8 (&pf)[QG][KT][2]) {
-    constexpr int NT = 2 * KT * C::DB;
+  auto gemm_pv = [&](const ACCT_LDS char* vbuf, const V8 (&pf)[QG][KTW][2]) {
+    constexpr int NT = 2 * KTW * C::DB;
     constexpr int RING = VRING < NT ? VRING : NT;
     auto tread = [&](int i) {
       const int db = i % C::DB, ch = i / C::DB;               // ch = 2 c + hh: rows 16 ch .. of the tile
@@ -263,24 +291,25 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     __builtin_amdgcn_sched_barrier(0);
   };
   // online softmax of the scores of tile j -> P^T fragments; `buf` = parity of the tile's staging buffers
-  auto softmax = [&](int j, int buf, uint32_t info, f32x16 (&s)[QG][KT], V8 (&pf)[QG][KT][2]) {
-    const int kv0 = j * BN;
+  auto softmax = [&](int j, int buf, uint32_t info, f32x16 (&s)[QG][KTW], V8 (&pf)[QG][KTW][2]) {
+    const int kv0 = j * BN + kg * WN;
     const bool apply_mask = MASKT && (info & kApply), diag = info & kDiag;
     const int tail = MASKT ? (int)((info >> kTailShift) & 0xffu) : 0;
     const int last_key = tail ? min(a.Sk, (j / TPB) * 128 + tail) - 1 : a.Sk - 1;     // last key that exists and is not behind a key tail
     // element (gq, c, r): q = wq0 + 32 gq + l32 ; kv = kv0 + 32 c + 8 (r/4) + 4 g + r%4
-    const bool edge = apply_mask || (diag && (kv0 + BN - 1 > wq0)) || (kv0 + BN - 1 > last_key);
+    const bool edge = apply_mask || (diag && (kv0 + WN - 1 > wq0)) || (kv0 + WN - 1 > last_key);
 #pragma unroll
     for (int gq = 0; gq < QG; gq++) {
       const int qrow = wq0 + 32 * gq + l32;
       const int qrow_c = min(qrow, a.Sq - 1);            // clamped for side-input addressing
       if (BIAS && !acc_bias) {
         if (bias_staged) {
-          typename E::V4 bv[2][4];
+          constexpr int KB = KT == 2 ? KTW : 1;                // (this path is that of the 64-key tiles)
+          typename E::V4 bv[KB][4];
 #pragma unroll
-          for (int c = 0; c < 2; c++)
+          for (int c = 0; c < KB; c++)
 #pragma unroll
-            for (int r4 = 0; r4 < 4; r4++) bv[c][r4] = bias_tile_read<T>(bias_lds + gq * 4096, row_bias ? 0 : l32, 4 * c + r4, g);
+            for (int r4 = 0; r4 < 4; r4++) bv[c][r4] = bias_tile_read<T>(bias_lds + gq * 4096, row_bias ? 0 : l32, 4 * (kg * KTW + c) + r4, g);
           if (gq == QG - 1) {
             // the tile is in registers: its LDS region can take the next tile, which has the rest of
             // this step to land (the end-of-step wait covers it)
@@ -288,7 +317,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
             if (j < j_hi) stage_bias(j + 1);
           }
 #pragma unroll
-          for (int c = 0; c < 2; c++)
+          for (int c = 0; c < KB; c++)
 #pragma unroll
             for (int r4 = 0; r4 < 4; r4++)
 #pragma unroll
@@ -296,7 +325,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
                 s[gq][c][4 * r4 + e] = __builtin_fmaf(s[gq][c][4 * r4 + e], a.scale, (float)bv[c][r4][e]);
         } else {
 #pragma unroll
-          for (int c = 0; c < 2; c++)
+          for (int c = 0; c < KTW; c++)
 #pragma unroll
             for (int r4 = 0; r4 < 4; r4++) {
               const int kv = kv0 + 32 * c + 8 * r4 + 4 * g;
@@ -311,7 +340,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       if (edge) {
         if (apply_mask) {
 #pragma unroll
-          for (int c = 0; c < KT; c++)
+          for (int c = 0; c < KTW; c++)
 #pragma unroll
             for (int r4 = 0; r4 < 4; r4++) {
               const int kv = kv0 + 32 * c + 8 * r4 + 4 * g;
@@ -332,7 +361,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
           // (compare and select through VCC: see select_if_gt)
           const float ninf = -INFINITY;
 #pragma unroll
-          for (int c = 0; c < KT; c++) {
+          for (int c = 0; c < KTW; c++) {
             const int visc = vis - 32 * c;
 #pragma unroll
             for (int r = 0; r < 16; r++) s[gq][c][r] = select_if_gt(s[gq][c][r], 8 * (r >> 2) + (r & 3), visc, ninf);
@@ -342,7 +371,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       // ---- online softmax for query row qrow ----
       float mx = s[gq][0][0];
 #pragma unroll
-      for (int c = 0; c < KT; c++)
+      for (int c = 0; c < KTW; c++)
 #pragma unroll
         for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[gq][c][r]);
       mx = pair_max(mx);
@@ -356,9 +385,9 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       const float mc = m_new * cmul;
       m[gq] = m_new;
       float rs = 0.f;
-      float p[KT][16];
+      float p[KTW][16];
 #pragma unroll
-      for (int c = 0; c < KT; c++)
+      for (int c = 0; c < KTW; c++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           p[c][r] = fast_exp2(__builtin_fmaf(s[gq][c][r], cmul, -mc));
@@ -368,8 +397,8 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       if (DROP) {
         // keep bits of this row and tile: word c covers keys kv0 + 32c .. +31
 #pragma unroll
-        for (int c = 0; c < KT; c++) {
-          const uint32_t w = DropStage::word(drop_lds + buf * DropStage::BYTES, 32 * gq + l32, c) >> (4 * g);
+        for (int c = 0; c < KTW; c++) {
+          const uint32_t w = DropStage::word(drop_lds + buf * DropStage::BYTES, 32 * gq + l32, kg * KTW + c) >> (4 * g);
 #pragma unroll
           for (int r = 0; r < 16; r++) {
             const int32_t sel = __builtin_amdgcn_sbfe((int)w, 8 * (r >> 2) + (r & 3), 1);   // keep ? ~0 : 0
@@ -378,7 +407,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
         }
       }
 #pragma unroll
-      for (int c = 0; c < KT; c++)
+      for (int c = 0; c < KTW; c++)
 #pragma unroll
         for (int hh = 0; hh < 2; hh++) {
           typename E::V2 t0 = E::cvt2(p[c][8 * hh + 0], p[c][8 * hh + 1]);
@@ -419,11 +448,11 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       }
       const uint32_t info = classify(j);
       if (info & kAct) {
-        f32x16 s[QG][KT];
-        V8 pf[QG][KT][2];
-        gemm_s(kbuf, j, s);
+        f32x16 s[QG][KTW];
+        V8 pf[QG][KTW][2];
+        gemm_s(kbuf + kg * (WN * C::PITCH), j, s);
         softmax(j, buf, info, s, pf);
-        gemm_pv(vbuf, pf);
+        gemm_pv(vbuf + kg * (WN * C::PITCH), pf);
       } else if (BIAS && bias_staged && !acc_bias && j < j_hi && wq0 < a.Sq) {
         stage_bias(j + 1);                                  // nothing to read in this step: the region is free
       }
@@ -432,13 +461,80 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     }
   }
 
+  // ---- key groups: the waves of group 0 take in the sums of the others ----
+  if constexpr (KG > 1) {
+    ACCT_LDS char* mg = smem + fwd_merge_at<D, RG>();
+    if (kg > 0) {
+      ACCT_LDS char* slot = mg + ((kg - 1) * RG + rg) * fwd_merge_slot<D>();
+#pragma unroll
+      for (int db = 0; db < C::DB; db++)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+          const f32x4 v = {o[0][db][4 * r4], o[0][db][4 * r4 + 1], o[0][db][4 * r4 + 2], o[0][db][4 * r4 + 3]};
+          *reinterpret_cast<ACCT_LDS f32x4*>(slot + (4 * db + r4) * 1024 + lane * 16) = v;
+        }
+      const f32x2 ml = {m[0], lsum[0]};
+      *reinterpret_cast<ACCT_LDS f32x2*>(slot + C::DB * 4096 + lane * 8) = ml;
+    }
+    __syncthreads();
+    if (kg > 0) return;
+    f32x2 ml[KG - 1];
+    float mm = m[0];
+#pragma unroll
+    for (int k = 0; k < KG - 1; k++) {
+      ml[k] = *reinterpret_cast<const ACCT_LDS f32x2*>(mg + (k * RG + rg) * fwd_merge_slot<D>() + C::DB * 4096 + lane * 8);
+      mm = fmaxf(mm, ml[k][0]);
+    }
+    const float w0 = fast_exp2((m[0] - mm) * cmul);
+    m[0] = mm;
+    lsum[0] *= w0;
+#pragma unroll
+    for (int db = 0; db < C::DB; db++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) o[0][db][r] *= w0;
+#pragma unroll
+    for (int k = 0; k < KG - 1; k++) {
+      const ACCT_LDS char* slot = mg + (k * RG + rg) * fwd_merge_slot<D>();
+      const float w = fast_exp2((ml[k][0] - mm) * cmul);
+      lsum[0] = __builtin_fmaf(ml[k][1], w, lsum[0]);
+#pragma unroll
+      for (int db = 0; db < C::DB; db++)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+          const f32x4 v = *reinterpret_cast<const ACCT_LDS f32x4*>(slot + (4 * db + r4) * 1024 + lane * 16);
+#pragma unroll
+          for (int e = 0; e < 4; e++) o[0][db][4 * r4 + e] = __builtin_fmaf(v[e], w, o[0][db][4 * r4 + e]);
+        }
+    }
+  }
+  // ---- key slices: sums and statistics go to the workspace, fa_fwd_combine_kernel adds the slices up ----
+  if (a.kv_split > 1) {
+    if (wq0 >= a.Sq) return;
+    const int64_t idx = ((int64_t)slice * n_wg + wg) * RG + rg, n_idx = (int64_t)a.kv_split * n_wg * RG;
+#pragma unroll
+    for (int gq = 0; gq < QG; gq++) {
+      float* part = a.fwd_part + (idx * QG + gq) * (C::DB * 1024) + lane * 4;
+#pragma unroll
+      for (int db = 0; db < C::DB; db++)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+          const f32x4 v = {o[gq][db][4 * r4], o[gq][db][4 * r4 + 1], o[gq][db][4 * r4 + 2], o[gq][db][4 * r4 + 3]};
+          *reinterpret_cast<f32x4*>(part + (4 * db + r4) * 256) = v;
+        }
+      const float l = pair_sum(lsum[gq]);
+      const f32x2 ml = {m[gq], l};
+      if (g == 0) *reinterpret_cast<f32x2*>(a.fwd_part + n_idx * QG * (C::DB * 1024) + ((idx * QG + gq) * 32 + l32) * 2) = ml;
+    }
+    return;
+  }
+
   // ---- epilogue: O = O^T / l, LSE = m + ln l.  Each wave transposes its rows through its own
   // LDS region (pitch 2D+16 keeps the 8-byte writes of 16 rows on distinct banks) so that the
   // global stores are whole rows. ----
   T* op = (T*)a.o + b * a.o_sb + h * a.o_sh;
   const float mnat = scaled ? 1.0f : a.scale;
   constexpr int OPITCH = C::DB * 64 + 16;
-  ACCT_LDS char* obuf = smem + wave * (32 * OPITCH);
+  ACCT_LDS char* obuf = smem + rg * (32 * OPITCH);
 #pragma unroll
   for (int gq = 0; gq < QG; gq++) {
     const int row = wq0 + 32 * gq + l32;
@@ -475,13 +571,16 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
 // rows see nothing but the causal pattern in a dense mask (block classes: clean before the diagonal, the
 // causal diagonal, skipped after it) runs the code of the variant without side inputs, by index compare.
 // A causal mask given as a tensor then costs one look at the class table per workgroup.
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2>
+template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2, int KG = 1>
 __global__ void __launch_bounds__(64 * NW) fa_fwd_kernel(const FaArgs a) {
   if constexpr (MASKT && !BIAS && !DROP) {
     if (a.mask_kind == kMaskDense) {
-      constexpr int BM = 32 * QG * NW;
+      constexpr int BM = 32 * QG * NW / KG;
+      const int BH = a.B * a.N;
+      int wg = blockIdx.x;
+      if (a.kv_split > 1) wg -= (wg / (BH * a.n_tiles)) * (BH * a.n_tiles);
       int bh, rank;
-      wg_map(blockIdx.x, a.B * a.N, a.n_tiles, bh, rank);
+      wg_map(wg, BH, a.n_tiles, bh, rank);
       const int q0 = (a.n_tiles - 1 - rank) * BM, q_end = min(q0 + BM, a.Sq);
       const int qb_lo = q0 / 128, qb_hi = (q_end - 1) / 128;
       const int kvb_lo = max(0, qb_lo - a.prev_blk), kvb_hi = min(a.Tc - 1, qb_hi + a.next_blk);
@@ -489,102 +588,181 @@ __global__ void __launch_bounds__(64 * NW) fa_fwd_kernel(const FaArgs a) {
       if (dense_lines_are_causal(fl, 1, a.Tc, qb_lo, qb_hi - qb_lo + 1, kvb_lo, kvb_hi, false, a, threadIdx.x & 63)) {
         FaArgs c = a;
         c.mask_kind = kMaskCausal;
-        fa_fwd_body<T, D, QG, NW, false, false, false, KT>(c);
+        fa_fwd_body<T, D, QG, NW, false, false, false, KT, KG>(c);
         return;
       }
     }
   }
-  fa_fwd_body<T, D, QG, NW, BIAS, DROP, MASKT, KT>(a);
+  fa_fwd_body<T, D, QG, NW, BIAS, DROP, MASKT, KT, KG>(a);
 }
 
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, int KT>
+// Second half of a forward launch whose key range was cut into a.kv_split slices: O = sum_s w_s O_s / sum_s w_s l_s
+// with w_s = exp2((m_s - max m) cmul), LSE from the same sums.  One workgroup per 32 query rows and 8 output columns
+// (the 1 KB a wave of the first half stored with one instruction), so that a single head's rows still spread over
+// the chip; its four waves take every fourth slice, eight loads in flight, and meet in LDS.
+template <typename T>
+__global__ void __launch_bounds__(256) fa_fwd_combine_kernel(const FaArgs a, int rgs, int dbs, float cmul, float mnat, float omul) {
+  __shared__ float red[3][6][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5;
+  const int BH = a.B * a.N, n_wg = BH * a.n_tiles;
+  const int dr = blockIdx.x % (4 * dbs), idx0 = blockIdx.x / (4 * dbs);     // dr = 4 db + r4
+  const int rg = idx0 % rgs;
+  int bh, rank;
+  wg_map(idx0 / rgs, BH, a.n_tiles, bh, rank);
+  const int wq0 = ((a.n_tiles - 1 - rank) * rgs + rg) * 32, row = wq0 + l32;
+  if (wq0 >= a.Sq) return;
+  const int64_t step = (int64_t)n_wg * rgs;
+  const float* part = a.fwd_part + (int64_t)idx0 * (dbs * 1024) + dr * 256 + lane * 4;
+  const float* stat = a.fwd_part + a.kv_split * step * (dbs * 1024) + ((int64_t)idx0 * 32 + l32) * 2;
+  float m = -1e30f, l = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  constexpr int U = 8;
+  for (int s0 = wave; s0 < a.kv_split; s0 += 4 * U) {
+    f32x4 v[U];
+    f32x2 ml[U];
+    float mb = m;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int s = min(s0 + 4 * u, a.kv_split - 1);                        // (a repeated slice gets weight 0 below)
+      v[u] = *reinterpret_cast<const f32x4*>(part + s * step * (dbs * 1024));
+      ml[u] = *reinterpret_cast<const f32x2*>(stat + s * step * 64);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) mb = fmaxf(mb, ml[u][0]);
+    const float al = fast_exp2((m - mb) * cmul);
+    m = mb;
+    l *= al;
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[e] *= al;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const float w = s0 + 4 * u < a.kv_split ? fast_exp2((ml[u][0] - m) * cmul) : 0.f;
+      l = __builtin_fmaf(ml[u][1], w, l);
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[e] = __builtin_fmaf(v[u][e], w, o[e]);
+    }
+  }
+  if (wave > 0) {
+    float (*slot)[64] = red[wave - 1];
+    slot[0][lane] = m;
+    slot[1][lane] = l;
+#pragma unroll
+    for (int e = 0; e < 4; e++) slot[2 + e][lane] = o[e];
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  float mm = m;
+#pragma unroll
+  for (int k = 0; k < 3; k++) mm = fmaxf(mm, red[k][0][lane]);
+  const float w0 = fast_exp2((m - mm) * cmul);
+  l *= w0;
+#pragma unroll
+  for (int e = 0; e < 4; e++) o[e] *= w0;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const float w = fast_exp2((red[k][0][lane] - mm) * cmul);
+    l = __builtin_fmaf(red[k][1][lane], w, l);
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[e] = __builtin_fmaf(red[k][2 + e][lane], w, o[e]);
+  }
+  if (row >= a.Sq) return;
+  const int b = bh / a.N, h = bh % a.N, d = 8 * dr + 4 * g;
+  const float inv = l > 0.f ? omul / l : 0.f;
+  if (d < a.hd) {
+    const typename Elem<T>::V2 t0 = Elem<T>::cvt2(o[0] * inv, o[1] * inv), t1 = Elem<T>::cvt2(o[2] * inv, o[3] * inv);
+    const typename Elem<T>::V4 ov = {t0[0], t0[1], t1[0], t1[1]};
+    *reinterpret_cast<typename Elem<T>::V4*>((T*)a.o + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_ss + d) = ov;
+  }
+  if (dr == 0 && g == 0) a.lse[(int64_t)bh * a.Sq + row] = l > 0.f ? mm * mnat + __logf(l) : -INFINITY;
+}
+
+template <typename T, int D, int NW, bool BIAS, bool DROP, int KT, int KG>
 static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   using C = SwzCfg<D>;
-  constexpr int BM = 32 * QG * NW;
+  constexpr int QG = 1, RG = NW / KG, BM = 32 * QG * RG;
   a.n_tiles = (a.Sq + BM - 1) / BM;
   const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
   constexpr size_t biasb = BIAS ? (KT == 4 ? 512 : QG * 4096) : 0;     // per wave, as in the kernel
-  const size_t tiles = 4 * 32 * KT * (size_t)C::PITCH + NW * biasb + (size_t)NW * 2 * DropRowStage<DROP, QG, KT>::BYTES, stage = (size_t)NW * 32 * (C::DB * 64 + 16);
-  static_assert(4 * 32 * KT * (size_t)C::PITCH + NW * biasb + (size_t)NW * 2 * DropRowStage<DROP, QG, KT>::BYTES <= 160 * 1024, "the workgroup's LDS must fit the CU's 160 KB");
-  const size_t smem = tiles > stage ? tiles : stage;
-  auto kern = mask_t ? fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, true, KT> : fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, BIAS || DROP, KT>;
+  constexpr size_t tiles = 4 * 32 * KT * (size_t)C::PITCH + NW * biasb + (size_t)NW * 2 * DropRowStage<DROP, QG, KT>::BYTES,
+                   stage = KG > 1 ? fwd_merge_at<D, RG>() + (size_t)(KG - 1) * RG * fwd_merge_slot<D>() : (size_t)NW * 32 * (C::DB * 64 + 16);
+  constexpr size_t smem = tiles > stage ? tiles : stage;
+  static_assert(smem <= 160 * 1024, "the workgroup's LDS must fit the CU's 160 KB");
+  auto kern = mask_t ? fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, true, KT, KG> : fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, BIAS || DROP, KT, KG>;
   hipError_t e = allow_dynamic_lds((const void*)kern, smem);
   if (e != hipSuccess) return e;
   const long long nblk = (long long)a.n_tiles * a.B * a.N;
-  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(64 * NW), smem, st, a);
-  return hipGetLastError();
+  hipLaunchKernelGGL(kern, dim3((unsigned)(nblk * (a.kv_split > 1 ? a.kv_split : 1))), dim3(64 * NW), smem, st, a);
+  e = hipGetLastError();
+  if (e == hipSuccess && a.kv_split > 1) {
+    // a full bias is added in natural units, everything else in units of q.k (see the kernel)
+    const bool acc_bias = BIAS && a.al_sq == 0 && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh) & 7)) == 0;
+    const bool scaled = BIAS && !acc_bias;
+    hipLaunchKernelGGL(fa_fwd_combine_kernel<T>, dim3((unsigned)(nblk * RG * 4 * C::DB)), dim3(256), 0, st, a, RG, (int)C::DB,
+                       scaled ? kLog2e : a.scale_log2e, scaled ? 1.0f : a.scale, DROP ? a.inv_keep : 1.0f);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP>
+template <typename T, int D, int NW, int KG, bool BIAS, bool DROP>
 static hipError_t launch_fwd_t(const FaArgs& a, hipStream_t st) {
-  // K/V stream in tiles of 128 keys where registers and LDS allow (8 waves x 32 rows, D <= 128): twice the
+  // K/V stream in tiles of 128 keys where registers and LDS allow (8 waves, D <= 128): twice the
   // matrix work between two barriers, -2 % (causal) to -6 % (full).  A bias tile per wave does not fit beside
   // them; a key-only bias that the DMA can stage (the kernel's own test, repeated here) is a 256-byte row and does.
-  constexpr bool BIG = QG == 1 && NW == 8 && D <= 128;
+  constexpr bool BIG = NW == 8 && D <= 128;
   if constexpr (BIG && BIAS) {
     const bool row_staged = a.al_sq == 0 && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh) & 7)) == 0;
-    return row_staged ? launch_fwd_kt<T, D, QG, NW, BIAS, DROP, 4>(a, st) : launch_fwd_kt<T, D, QG, NW, BIAS, DROP, 2>(a, st);
+    return row_staged ? launch_fwd_kt<T, D, NW, BIAS, DROP, 4, KG>(a, st) : launch_fwd_kt<T, D, NW, BIAS, DROP, 2, KG>(a, st);
   } else {
-    return launch_fwd_kt<T, D, QG, NW, BIAS, DROP, BIG ? 4 : 2>(a, st);
+    return launch_fwd_kt<T, D, NW, BIAS, DROP, BIG ? 4 : 2, KG>(a, st);
   }
 }
 
 // SIDE: 2 = bias and dropout variants, 1 = the dropout variant only (head dims 40, 160, 256)
-template <typename T, int D, int QG, int NW, int SIDE = 2>
+template <typename T, int D, int NW, int KG, int SIDE>
 static hipError_t launch_fwd_q(const FaArgs& a, hipStream_t st) {
   const bool bias = a.alibi != nullptr, drop = a.droprow != nullptr || a.dropcol != nullptr;
 #ifndef ACCT_DEV_BUILD
   if constexpr (SIDE == 2) {
-    if (bias) return drop ? launch_fwd_t<T, D, QG, NW, true, true>(a, st) : launch_fwd_t<T, D, QG, NW, true, false>(a, st);
+    if (bias) return drop ? launch_fwd_t<T, D, NW, KG, true, true>(a, st) : launch_fwd_t<T, D, NW, KG, true, false>(a, st);
   }
   if constexpr (SIDE >= 1) {
-    if (drop && !bias) return launch_fwd_t<T, D, QG, NW, false, true>(a, st);
+    if (drop && !bias) return launch_fwd_t<T, D, NW, KG, false, true>(a, st);
   }
 #endif
   if (bias || drop) return hipErrorNotSupported;       // (development build: plain variants only)
-  return launch_fwd_t<T, D, QG, NW, false, false>(a, st);
+  return launch_fwd_t<T, D, NW, KG, false, false>(a, st);
 }
 
-// variant: 1 = 4 waves x 32 rows, 3 = 8 waves x 32 rows
-template <typename T, int D>
-static hipError_t launch_fwd_d(const FaArgs& a, int variant, hipStream_t st) {
-  return variant == 3 ? launch_fwd_q<T, D, 1, 8>(a, st) : launch_fwd_q<T, D, 1, 4>(a, st);
-}
-// head dims 40 and 160: no bias variants
-template <typename T, int D>
-static hipError_t launch_fwd_plain(const FaArgs& a, int variant, hipStream_t st) {
-  return variant == 3 ? launch_fwd_q<T, D, 1, 8, 1>(a, st) : launch_fwd_q<T, D, 1, 4, 1>(a, st);
-}
-
-#ifdef ACCT_DEV_BUILD
-bool fwd_variants_complete() { return false; }
-#else
-bool fwd_variants_complete() { return true; }
-#endif
-
-hipError_t launch_fwd(const FaArgs& a, int dtype, int Dr, int qg, hipStream_t st) {
-  const int D = head_dim_class(Dr);
-#ifdef ACCT_DEV_BUILD
-  if (dtype != 0 || D != 128) return hipErrorNotSupported;
-  return launch_fwd_d<f16, 128>(a, qg, st);
-#else
-  if (dtype == 0) {
-    if (D == 128) return launch_fwd_d<f16, 128>(a, qg, st);
-    if (D == 64) return launch_fwd_d<f16, 64>(a, qg, st);
-    if (D == 80) return launch_fwd_d<f16, 80>(a, qg, st);
-    if (D == 40) return launch_fwd_plain<f16, 40>(a, qg, st);
-    if (D == 160) return launch_fwd_plain<f16, 160>(a, qg, st);
-    if (D == 256) return launch_fwd_q<f16, 256, 1, 4, 1>(a, st);     // one wave per SIMD: 128 accumulator registers
+// Head dim 256 leaves registers for one wave per SIMD only: 4 waves, no key groups.  Four key groups (64 query rows
+// per workgroup) are built without bias and dropout and for 128-key tiles.
+template <typename T, int D, int SIDE = 2>
+static hipError_t launch_fwd_d(const FaArgs& a, int kg, hipStream_t st) {
+  if constexpr (D > 160) {
+    return launch_fwd_q<T, D, 4, 1, SIDE>(a, st);
   } else {
-    if (D == 128) return launch_fwd_d<bf16, 128>(a, qg, st);
-    if (D == 64) return launch_fwd_d<bf16, 64>(a, qg, st);
-    if (D == 80) return launch_fwd_d<bf16, 80>(a, qg, st);
-    if (D == 40) return launch_fwd_plain<bf16, 40>(a, qg, st);
-    if (D == 160) return launch_fwd_plain<bf16, 160>(a, qg, st);
-    if (D == 256) return launch_fwd_q<bf16, 256, 1, 4, 1>(a, st);
+    if constexpr (D <= 128) {
+      if (kg == 4) return launch_fwd_q<T, D, 8, 4, 0>(a, st);
+    }
+    return kg == 1 ? launch_fwd_q<T, D, 8, 1, SIDE>(a, st) : launch_fwd_q<T, D, 8, 2, SIDE>(a, st);
   }
+}
+
+template <typename T>
+hipError_t launch_fwd_elem(const FaArgs& a, int Dr, int kg, hipStream_t st) {
+  const int D = head_dim_class(Dr);
+  if (D == 128) return launch_fwd_d<T, 128>(a, kg, st);
+#ifdef ACCT_DEV_BUILD
+  return hipErrorNotSupported;
+#else
+  if (D == 64) return launch_fwd_d<T, 64>(a, kg, st);
+  if (D == 80) return launch_fwd_d<T, 80>(a, kg, st);
+  if (D == 40) return launch_fwd_d<T, 40, 1>(a, kg, st);
+  if (D == 160) return launch_fwd_d<T, 160, 1>(a, kg, st);
+  if (D == 256) return launch_fwd_d<T, 256, 1>(a, kg, st);
   return hipErrorInvalidValue;
 #endif
 }
+template hipError_t launch_fwd_elem<ACCT_ELEM>(const FaArgs& a, int Dr, int kg, hipStream_t st);
 
 }  // namespace acct

@@ -94,4 +94,46 @@ ACCT_HD DkdvSplit dkdv_split(int B, int N, int Sq, int Sk, int D, int n_cu = 256
   return {(int)s, (size_t)s * (size_t)n_wg * 8 * ngk * db * 1024 * sizeof(float)};
 }
 
+// How the forward kernel cuts its work.  kg: key groups of the workgroup (fa_fwd.hip; 256 / kg query rows per
+// workgroup).  kv_split: slices of the key range on workgroups of their own, which a second kernel adds up (1: none).
+//
+// A workgroup of kg = 4 steps through its key tiles 2.2 times as fast as one of kg = 1 (1.22 against 2.68 us per 128
+// keys at head dim 128, each alone on its CU) but does a quarter of the work, so kg > 1 pays only where its larger
+// number of workgroups still runs in one round: B1 N16 S1024 D64 (64 / 128 / 256 workgroups) 20.2 / 14.5 / 11.7 us
+// for kg 1 / 2 / 4, N20 (80 / 160 / 320) 20.3 / 14.8 / 16.6, N40 (160 / 320 / 640) 20.9 / 21.8 / 24.3.  Below the
+// causal diagonal (`tri`) half of the workgroups are light and one and a quarter (kg 4) or, over long rows, two
+// (kg 2) times the CUs still pay: N24 S2048 D128 (192 / 384 / 768) 50.1 / 36.3 / 51.0, but N96 S512 18.3 / 20.0 / 28.3.
+//
+// The slices cost a second launch and the slices' sums written and read (about 6.5 us, and 3 TB/s); they are
+// taken where the estimate below says that the shorter walk saves more: 1 head, 256 queries x 131072 keys
+// 1253 -> 37 us; 8 heads, 512 x 8192 80 -> 33; not for 4 heads, 2048 x 2048 causal (24.8 against 28.9).
+struct FwdPlan { int kg, kv_split; size_t part_bytes; };
+ACCT_HD size_t fwd_part_bytes(int B, int N, int Sq, int D, int kg, int split) {
+  const int dc = head_dim_class(D), rows = dc > 160 ? 128 : 256 / kg;
+  const long long groups = (long long)B * N * ((Sq + rows - 1) / rows) * (rows / 32);     // of 32 query rows
+  return split > 1 ? (size_t)split * (size_t)groups * ((dc + 31) / 32 * 1024 + 64) * sizeof(float) : 0;
+}
+// `side`: a bias or dropout (not built for kg = 4); `tri`: key blocks after the query's block are left out;
+// `can_split`: there is room for the slices' sums
+ACCT_HD FwdPlan fwd_plan(int B, int N, int Sq, int Sk, int D, bool side, bool tri, bool can_split, int n_cu = 256) {
+  const int dc = head_dim_class(D);
+  const long long bh = (long long)B * N, n1 = bh * ((Sq + 255) / 256), n2 = bh * ((Sq + 127) / 128), n4 = bh * ((Sq + 63) / 64);
+  int kg = 1;
+  if (dc <= 128 && !side && n4 <= (tri ? n_cu + n_cu / 4 : n_cu)) kg = 4;
+  else if (dc <= 160 && (n2 <= n_cu || (tri && n1 < n_cu && Sk >= 1024))) kg = 2;
+  // slices: microseconds of a workgroup's walk against those of a slice's, plus the second launch and the traffic
+  const int kg_s = dc > 160 ? 1 : 2;
+  const long long n_s = kg_s == 2 ? n2 : bh * ((Sq + 127) / 128);
+  const int seen = tri ? (Sq < Sk ? Sq : Sk) : Sk, tiles = (seen + 127) / 128;
+  const double per_tile = 0.5 + 0.72 / 128 * dc;                       // kg = 4; 1.3 and 2.2 times that for kg = 2 and 1
+  double best = per_tile * (kg == 4 ? 1.0 : kg == 2 ? 1.3 : 2.2) * tiles;
+  int split = 1;
+  for (int s = 2; can_split && s <= tiles && s <= 256 && s * n_s <= n_cu; s *= 2) {
+    const double t = per_tile * (kg_s == 2 ? 1.3 : 2.2) * ((tiles + s - 1) / s) + 6.5 + 2e6 / 3e12 * (double)fwd_part_bytes(B, N, Sq, D, kg_s, s);
+    if (t < best) { best = t; split = s; }
+  }
+  if (split > 1) kg = kg_s;
+  return {kg, split, fwd_part_bytes(B, N, Sq, D, kg, split)};
+}
+
 }  // namespace acct

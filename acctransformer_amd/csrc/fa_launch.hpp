@@ -22,20 +22,25 @@ inline hipError_t allow_dynamic_lds(const void* kern, size_t bytes) {
   return e;
 }
 
-// forward: variant 3 = 8 waves x 32 query rows, 1 = 4 waves x 32 rows; the bias / dropout
-// variants are picked from a.alibi / a.droprow
-hipError_t launch_fwd(const FaArgs& a, int dtype, int D, int qg, hipStream_t st);
+// forward: kg = key groups of the workgroup (FwdPlan, fa_index_math.hpp); the bias / dropout variants are picked from
+// a.alibi / a.droprow, the key-range split from a.kv_split / a.fwd_part
+template <typename T> hipError_t launch_fwd_elem(const FaArgs& a, int D, int kg, hipStream_t st);
 
 // backward: delta pre-pass, dK/dV kernel (kv-tile owner) and dQ kernel (q-tile owner)
 enum : int { kStageDq = 1, kStageDkDv = 2 };
-hipError_t launch_bwd(const FaArgs& a, int dtype, int D, int stages, hipStream_t st);
+template <typename T> hipError_t launch_bwd_elem(const FaArgs& a, int D, int stages, hipStream_t st);
 
 // the dQ kernel with 64 query rows per wave (fa_bwd_dq64.hip): head dim 128, no side inputs, aligned lengths
 bool dq64_applicable(const FaArgs& a);
 hipError_t launch_bwd_dq64(FaArgs a, int dtype, hipStream_t st);
 
-// false when the kernel translation units were compiled with a reduced variant set (ACCT_DEV_BUILD)
-bool launch_variants_complete();
+// false when the kernel translation units were compiled with a reduced variant set (ACCT_DEV_BUILD: head dim 128
+// without side inputs)
+#ifdef ACCT_DEV_BUILD
+constexpr bool launch_variants_complete() { return false; }
+#else
+constexpr bool launch_variants_complete() { return true; }
+#endif
 
 // classify the 128x128 blocks of a dense mask into clean / apply / skip / causal diagonal and, with `colbits`
 // non-null, pack its 'apply' blocks into per-key-column bitmaps [MB, Tr, Sk, 4 x u32] (one launch for aligned masks)

@@ -159,6 +159,11 @@ typedef struct acct_fa_params {
 int acct_fa_fwd(const acct_fa_params* p, void* O, float* LSE,
                 void* workspace, size_t workspace_bytes, void* stream);
 size_t acct_fa_fwd_workspace_bytes(const acct_fa_params* p);
+/* The same plus, where few query rows meet many keys (a launch that would leave most of the chip idle), room for a
+ * launch that cuts the key range into slices on workgroups of their own and adds the slices' sums in a second kernel
+ * (fixed order: deterministic).  A call with a workspace of this size makes use of it; with a smaller one that holds
+ * acct_fa_fwd_workspace_bytes it runs the unsplit launch.  The two differ in the last bits of O and LSE. */
+size_t acct_fa_fwd_split_workspace_bytes(const acct_fa_params* p);
 /* Size of the optional drop_bits buffer (0 without dropout): keep bits by query row for the forward and dQ
  * kernels, then by key column for the dK/dV kernel, a quarter of a byte per score in total. */
 size_t acct_fa_drop_bits_bytes(const acct_fa_params* p);
