@@ -228,6 +228,8 @@ acct::FaArgs make_args(const acct_fa_params* p) {
   // the kernels know one dense and one tile kind; the element size travels beside it
   a.mask_kind = mask_is_dense(p) ? (int)acct::kMaskDense : (mask_is_tile(p) ? (int)acct::kMaskTile : p->mask_kind);
   a.row_prefix = p->row_block_prefix;
+  // (a shared buffer of keep bits belongs to one attn_mask and band where there is a dense mask, else to any call)
+  a.drop_visible = !p->drop_bits || mask_is_dense(p);
   return a;
 }
 
@@ -279,14 +281,12 @@ int mask_prepass(acct::FaArgs& a, const acct_fa_params* p, uint8_t* own, bool wa
   const bool cols = p->mask_bits ? true : want_cols;
   if (mask_is_dense(p)) {
     a.blkflags = flags;
-    // (only the one-launch pre-pass writes the key tails; which path runs follows from the arguments alone, so every
-    // call of a step that shares a mask_bits buffer decides alike)
-    a.blktail = acct::mask_prepass_is_fused(a) ? flags + class_count(p) : nullptr;
+    a.blktail = flags + class_count(p);
   }
   if (cols) a.colbits = cbits;
   if (filled) return ACCT_OK;
   hipError_t e = mask_is_dense(p) ? acct::launch_mask_blocks(a, flags, cols ? cbits : nullptr, p->mask_stride_b ? p->B : 1, st)
-                                  : (cols ? acct::launch_mask_colbits(a, flags, cbits, 1, st) : hipSuccess);
+                                  : (cols ? acct::launch_mask_tilebits(a, cbits, st) : hipSuccess);
   if (e != hipSuccess) return fail(ACCT_E_LAUNCH, "mask pre-pass kernel: %s", hipGetErrorString(e));
   return ACCT_OK;
 }

@@ -158,8 +158,6 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
   const int mb = a.mask_sb ? b : 0;
   const uint8_t* maskp = a.mask ? a.mask + (a.mask_kind == kMaskDense ? (int64_t)mb * a.mask_sb * a.mask_es : 0) : nullptr;
   const T* alibip = BIAS ? (const T*)a.alibi + b * a.al_sb + h * a.al_sh : nullptr;
-  const bool mask_vec = a.mask_kind == kMaskDense ? ((((uintptr_t)a.mask / a.mask_es) | (uintptr_t)a.Sk | (uintptr_t)a.mask_sb) & 3) == 0
-                                                  : ((uintptr_t)a.mask & (4 * a.mask_es - 1)) == 0;
   const bool alibi_vec = BIAS && (((uintptr_t)a.alibi & 7) | ((a.al_sb | a.al_sh | a.al_sq) & 3)) == 0;
 
   TileDma<T, D, 64, NW> kdma, vdma;
@@ -341,8 +339,8 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
                 for (int r4 = 0; r4 < 4; r4++) {
                   const int kv = kv0 + 32 * c + 8 * r4 + 4 * g;
                   uint32_t mbits;
-                  if (a.mask_kind == kMaskDense) mbits = load_mask4(maskp + (int64_t)qrow_c * a.Sk * a.mask_es, kv, a.Sk, mask_vec, a.mask_es);
-                  else mbits = load_mask4(maskp + (qrow_c & 127) * 128 * a.mask_es, kv & 127, 128, mask_vec, a.mask_es);
+                  if (a.mask_kind == kMaskDense) mbits = load_mask4(maskp + (int64_t)qrow_c * a.Sk * a.mask_es, kv, a.Sk, a.mask_es);
+                  else mbits = load_mask4(maskp + (qrow_c & 127) * 128 * a.mask_es, kv & 127, 128, a.mask_es);
 #pragma unroll
                   for (int e = 0; e < 4; e++)
                     if ((mbits >> (8 * e)) & 0xffu) x[4 * r4 + e] += kMaskFill * kLog2e;

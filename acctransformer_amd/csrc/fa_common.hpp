@@ -90,7 +90,8 @@ ACCT_DEV void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, 
 #pragma unroll
   for (int r = 0; r < 10; r++) {
     const uint64_t p0 = (uint64_t)0xD2511F53u * c0, p1 = (uint64_t)0xCD9E8D57u * c2;
-    const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0, n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+    // (one three-input instruction each)
+    const uint32_t n0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c1, k0, 0x96), n2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c3, k1, 0x96);
     c1 = (uint32_t)p1;
     c3 = (uint32_t)p0;
     c0 = n0;
@@ -139,6 +140,7 @@ struct FaArgs {
   int n_tiles;                         // tiles along the owner dimension
   int kv_split;                        // forward kernel: slices of the key range, each on workgroups of its own (1 = no split)
   int q_split;                         // dK/dV kernel: slices of the query range, each on workgroups of its own (1 = no split)
+  int drop_visible;                    // keep bits: != 0 when those of key blocks outside the band (or past the causal / prefix limit) may be left out
   int droprow_w;                       // 32-bit words per row of droprow: 2 * ceil(Sk / 64)
   uint32_t philox_k0, philox_k1;       // counter-based dropout: key, call offset and keep threshold (byte < thr keeps)
   uint32_t philox_offset, philox_thr;
@@ -335,9 +337,17 @@ ACCT_DEV bool dense_lines_are_causal(const uint8_t* tbl, int64_t stride, int64_t
   return __all(ok);
 }
 
+// a V from an address that is a multiple of ALIGN bytes only (global memory takes loads of any width there)
+template <typename V, int ALIGN>
+ACCT_DEV V load_any(const uint8_t* p) {
+  V v;
+  __builtin_memcpy(&v, __builtin_assume_aligned(p, ALIGN), sizeof(V));
+  return v;
+}
+
 // four consecutive mask / dropout bytes starting at column kv of a row
-ACCT_DEV uint32_t load_u8x4(const uint8_t* row, int kv, int limit, bool vec_ok) {
-  if (vec_ok && kv + 4 <= limit) return *reinterpret_cast<const uint32_t*>(row + kv);
+ACCT_DEV uint32_t load_u8x4(const uint8_t* row, int kv, int limit) {
+  if (kv + 4 <= limit) return load_any<uint32_t, 1>(row + kv);
   uint32_t r = 0;
 #pragma unroll
   for (int e = 0; e < 4; e++)
@@ -351,12 +361,12 @@ template <int ES> ACCT_DEV bool elem_nonzero(const uint8_t* p, int64_t idx) {
   return (reinterpret_cast<const uint16_t*>(p)[idx] & 0x7fffu) != 0;
 }
 // the same four consecutive elements for a mask of `es`-byte elements, as four "nonzero" bytes (row = first byte of the row)
-ACCT_DEV uint32_t load_mask4(const uint8_t* row, int kv, int limit, bool vec_ok, int es) {
-  if (es == 1) return load_u8x4(row, kv, limit, vec_ok);
+ACCT_DEV uint32_t load_mask4(const uint8_t* row, int kv, int limit, int es) {
+  if (es == 1) return load_u8x4(row, kv, limit);
   const uint16_t* r16 = reinterpret_cast<const uint16_t*>(row);
   uint32_t r = 0;
-  if (vec_ok && kv + 4 <= limit) {
-    const u32x2 t = *reinterpret_cast<const u32x2*>(r16 + kv);
+  if (kv + 4 <= limit) {
+    const u32x2 t = load_any<u32x2, 2>(row + 2 * (int64_t)kv);
 #pragma unroll
     for (int e = 0; e < 4; e++)
       if ((t[e >> 1] >> (16 * (e & 1))) & 0x7fffu) r |= 1u << (8 * e);

@@ -16,14 +16,13 @@
 
 namespace acct {
 
-constexpr uint8_t kBlkAllMasked = 255;  // provisional: resolved to skip or apply below
-
-// Fast path (Sk and the mask pointers 16-byte aligned): ONE launch that leaves the block classes and, for the
-// dK/dV kernel, the column bitmaps of the mixed blocks (every launch costs a few microseconds of a step that
-// takes a few hundred).  One workgroup of 256 threads per (mask batch, q block, key block) inside the band, so
-// that the work spreads over the chip whatever the shape (a [1, 2048, 2048] mask has 16 row blocks but 256
-// blocks).  Thread t owns 64 consecutive elements of row t % 128 (half t / 128 of the block's 128 columns),
-// four or eight 16-byte loads, as a 64-bit "nonzero" mask.
+// ONE launch leaves the block classes and, for the dK/dV kernel, the column bitmaps of the mixed blocks (every
+// launch costs a few microseconds of a step that takes a few hundred).  One workgroup of 256 threads per (mask
+// batch, q block, key block) inside the band, so that the work spreads over the chip whatever the shape (a
+// [1, 2048, 2048] mask has 16 row blocks but 256 blocks).  Thread t owns 64 consecutive elements of row t % 128
+// (half t / 128 of the block's 128 columns), four or eight 16-byte loads at whatever alignment the rows have (a
+// sequence length that is no multiple of 16 shifts every row; such loads touch one cache line more, no more
+// instructions), as a 64-bit "nonzero" mask.
 //
 // A wholly masked block may be skipped only if every row of its q block sees an unmasked key somewhere (see the
 // top of the file).  A workgroup cannot see the other blocks of its row block's band, so it checks a sufficient
@@ -54,11 +53,12 @@ __global__ void __launch_bounds__(256) fa_mask_prepass_kernel(const FaArgs a, ui
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int kv = kb * 128 + c0 + 16 * i;
-      if (kv < a.Sk) {                                  // Sk % 16 == 0: a piece is entirely inside or outside
-        uint32_t bits = 0;                              // bit e: element e of these 16 is nonzero
+      if (kv >= a.Sk) continue;
+      uint32_t bits = 0;                                // bit e: element e of these 16 is nonzero
+      if (kv + 16 <= a.Sk) {
 #pragma unroll
         for (int h = 0; h < ES; h++) {
-          const u32x4 v = *reinterpret_cast<const u32x4*>(mrow + (int64_t)kv * ES + 16 * h);
+          const u32x4 v = load_any<u32x4, ES>(mrow + (int64_t)kv * ES + 16 * h);
 #pragma unroll
           for (int w = 0; w < 4; w++) {
             if (ES == 1) {
@@ -70,9 +70,12 @@ __global__ void __launch_bounds__(256) fa_mask_prepass_kernel(const FaArgs a, ui
             }
           }
         }
-        nz |= (unsigned long long)bits << (16 * i);
         valid |= 0xffffull << (16 * i);
+      } else {                                          // the row ends inside this piece
+        for (int e = 0; e < a.Sk - kv; e++) bits |= (elem_nonzero<ES>(mrow, kv + e) ? 1u : 0u) << e;
+        valid |= ((1ull << (a.Sk - kv)) - 1ull) << (16 * i);
       }
+      nz |= (unsigned long long)bits << (16 * i);
     }
   };
   unsigned long long nz, valid;
@@ -140,73 +143,8 @@ __global__ void __launch_bounds__(256) fa_mask_prepass_kernel(const FaArgs a, ui
   }
 }
 
-// Generic path (any alignment): one workgroup per (mask batch, q block); thread t scans 64 columns of row t/2
-template <int ES>
-__global__ void __launch_bounds__(256) fa_mask_blocks_kernel(const FaArgs a, uint8_t* flags) {
-  const int qb = blockIdx.x % a.Tr, mb = blockIdx.x / a.Tr;
-  const int tid = threadIdx.x, row = qb * 128 + (tid >> 1), c0 = (tid & 1) * 64;
-  const uint8_t* mrow = a.mask + ((int64_t)mb * a.mask_sb + (int64_t)min(row, a.Sq - 1) * a.Sk) * ES;
-  const bool vec_ok = ((((uintptr_t)a.mask / ES) | (uintptr_t)a.Sk | (uintptr_t)a.mask_sb) & 3) == 0;
-  uint8_t* frow = flags + ((int64_t)mb * a.Tr + qb) * a.Tc;
-  int lo = max(0, qb - a.prev_blk), hi = min(a.Tc - 1, qb + a.next_blk);
-  if (a.row_prefix) hi = min(hi, ((qb * 128 / a.row_prefix + 1) * a.row_prefix - 1) / 128);
-  for (int kvb = tid; kvb < a.Tc; kvb += 256)
-    if (kvb < lo || kvb > hi) frow[kvb] = kBlkClean;
-  bool row_unmasked = false;
-  bool tri_bad = false;
-  for (int kvb = lo; kvb <= hi; kvb++) {
-    bool any_m = false, any_u = false;
-    if (row < a.Sq) {
-#pragma unroll 4
-      for (int c = 0; c < 64; c += 4) {
-        const int kv = kvb * 128 + c0 + c;
-        if (kv >= a.Sk) break;
-        const int n = min(4, a.Sk - kv);
-        const uint32_t bits = load_mask4(mrow, kv, a.Sk, vec_ok, ES);
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-          if (e < n) {
-            const bool masked = ((bits >> (8 * e)) & 0xffu) != 0;
-            if (masked) any_m = true; else any_u = true;
-            if (kvb == qb) tri_bad |= masked != (c0 + c + e > (tid >> 1));
-          }
-      }
-    }
-    row_unmasked |= any_u;
-    const int blk_m = __syncthreads_or(any_m), blk_u = __syncthreads_or(any_u);
-    if (tid == 0) frow[kvb] = !blk_m ? kBlkClean : (!blk_u ? kBlkAllMasked : kBlkApply);
-  }
-  row_unmasked |= (bool)__shfl_xor((int)row_unmasked, 1);
-  const int rows_ok = __syncthreads_and(row >= a.Sq || row_unmasked);
-  // (the barrier above also orders thread 0's provisional writes before the reads below)
-  const int not_tri = __syncthreads_or(tri_bad);
-  for (int kvb = lo + tid; kvb <= hi; kvb += 256) {
-    if (frow[kvb] == kBlkAllMasked) frow[kvb] = rows_ok ? kBlkSkip : kBlkApply;
-    else if (kvb == qb && frow[kvb] == kBlkApply && !not_tri) frow[kvb] = kBlkTriu;
-  }
-}
-
-// Column bitmaps of the mixed ('apply') blocks for the dK/dV kernel, whose lanes own key columns: the 128
-// rows of a block packed into 128 bits per key column, so that the kernel reads one 32-bit word per lane
-// and 32-row chunk instead of 16 single bytes.  One thread per key column and word (32 rows): the loads
-// of a thread are independent, and 512 threads keep enough of them in flight.
-template <int ES>
-__global__ void __launch_bounds__(512) fa_mask_colbits_kernel(const FaArgs a, const uint8_t* flags, uint32_t* out) {
-  const int kvb = blockIdx.x % a.Tc, qb = (blockIdx.x / a.Tc) % a.Tr, mb = blockIdx.x / (a.Tc * a.Tr);
-  if (flags[((int64_t)mb * a.Tr + qb) * a.Tc + kvb] != kBlkApply) return;
-  const int kv = kvb * 128 + (threadIdx.x & 127), i = threadIdx.x >> 7;
-  if (kv >= a.Sk) return;
-  const uint8_t* col = a.mask + ((int64_t)mb * a.mask_sb + kv) * ES;
-  uint32_t w = 0u;
-#pragma unroll
-  for (int r = 0; r < 32; r++) {
-    const int row = qb * 128 + 32 * i + r;
-    if (row < a.Sq && elem_nonzero<ES>(col, (int64_t)row * a.Sk)) w |= 1u << r;
-  }
-  out[(((int64_t)mb * a.Tr + qb) * a.Sk + kv) * 4 + i] = w;
-}
-
-// the same for the compact 128x128 tile that is applied on diagonal blocks: out[key][4]
+// The compact 128x128 tile that is applied on diagonal blocks, packed by key column for the dK/dV kernel, whose lanes
+// own key columns: out[key][4], bit r of the 128-bit entry = tile[r][key]
 template <int ES>
 __global__ void __launch_bounds__(128) fa_mask_tilebits_kernel(const uint8_t* tile, uint32_t* out) {
   uint32_t w[4] = {0u, 0u, 0u, 0u};
@@ -219,231 +157,245 @@ __global__ void __launch_bounds__(128) fa_mask_tilebits_kernel(const uint8_t* ti
   *reinterpret_cast<u32x4*>(out + threadIdx.x * 4) = v;
 }
 
-hipError_t launch_mask_colbits(const FaArgs& a, const uint8_t* flags, uint32_t* out, int MB, hipStream_t st) {
-  if (a.mask_kind == kMaskTile) {
-    if (a.mask_es == 2) hipLaunchKernelGGL(fa_mask_tilebits_kernel<2>, dim3(1), dim3(128), 0, st, a.mask, out);
-    else hipLaunchKernelGGL(fa_mask_tilebits_kernel<1>, dim3(1), dim3(128), 0, st, a.mask, out);
-    return hipGetLastError();
-  }
-  const dim3 grid((unsigned)(MB * a.Tr * a.Tc));
-  if (a.mask_es == 2) hipLaunchKernelGGL(fa_mask_colbits_kernel<2>, grid, dim3(512), 0, st, a, flags, out);
-  else hipLaunchKernelGGL(fa_mask_colbits_kernel<1>, grid, dim3(512), 0, st, a, flags, out);
+hipError_t launch_mask_tilebits(const FaArgs& a, uint32_t* out, hipStream_t st) {
+  if (a.mask_es == 2) hipLaunchKernelGGL(fa_mask_tilebits_kernel<2>, dim3(1), dim3(128), 0, st, a.mask, out);
+  else hipLaunchKernelGGL(fa_mask_tilebits_kernel<1>, dim3(1), dim3(128), 0, st, a.mask, out);
   return hipGetLastError();
 }
 
-// Column entries of the dropout bitmaps, written whole.  The four waves of a workgroup each hold, per lane and for
-// sixteen keys, the 32-bit word of their 32 rows; a key's 16-byte entry is the four waves' words.  Written straight
-// from the waves every entry would be four 4-byte stores from four places; instead the words cross LDS and every
-// thread stores complete entries, consecutive threads consecutive entries.  cw[e]: bit r = row r of the wave's 32;
-// key_of(lane, e): the key of a lane's e-th word.  (One spare entry after every sixteen keeps the word stores of a
-// wave on different banks.)  `flags`: the class row of the attention mask for these query rows, or null: entries of
-// key blocks classed 'skip' are never read and are not written.
-template <typename KeyOf>
-ACCT_DEV void store_col_entries(uint32_t* s_cw, const uint32_t (&cw)[16], int wave, int lane, int key0, int Sk, uint32_t* out,
-                                const uint8_t* flags, KeyOf key_of) {
-#pragma unroll
-  for (int e = 0; e < 16; e++) {
-    const int k = key_of(lane, e);                       // 0 .. 1023 within the span
-    s_cw[(k + (k >> 4)) * 4 + wave] = cw[e];
+// Key blocks whose keep bits no attention kernel reads: those that the attention mask's pre-pass classed 'skip', and
+// those that the band, the causal index compare or the row prefix leaves out for every row of the q block.  (Only
+// with `drop_visible`: a buffer of keep bits that the caller shares between calls without a dense mask holds them all.)
+// `flags`: the class row of the q block, or null.
+ACCT_DEV bool keep_bits_unread(const FaArgs& a, const uint8_t* flags, int qb, int kvb) {
+  if (flags && flags[kvb] == kBlkSkip) return true;
+  if (!a.drop_visible) return false;
+  return kvb - a.next_blk > qb || qb > kvb + a.prev_blk || (a.mask_kind == kMaskCausal && kvb > qb) ||
+         (a.row_prefix && kvb * 128 >= (qb * 128 / a.row_prefix + 1) * a.row_prefix);
+}
+
+// Both dropout pre-passes below work in units of ONE WAVE per (batch*head, 128 query rows, 128 keys), a block that is
+// either left out as a whole or needed; a workgroup's four waves take neighbouring key blocks.  A lane holds the keep
+// bits of a piece of the block, puts its bits of every row and its words of every key column into a wave-private LDS
+// image of the block's two outputs, and the wave stores the image: whole 16-byte column entries, consecutive lanes
+// consecutive entries, and 16-byte row pieces.  (Written straight from the lanes, an entry would be four or eight
+// stores.)  One spare 16-byte entry after every sixteen keeps the lanes' pieces on different banks.
+constexpr int kKeepImage = 128 + 8;                      // 16-byte entries of one output of a block
+struct KeepBlock {
+  int kvb, qb, bh, lane;
+  ACCT_LDS char* row;                                    // [row][16 bytes]: bit k = keep[row][128 kvb + k]
+  ACCT_LDS char* col;                                    // [key][16 bytes]: bit r = keep[128 qb + r][key]
+  static ACCT_DEV int at(int i) { return (i + (i >> 4)) * 16; }
+  // false: nothing to do for this wave
+  ACCT_DEV bool init(const FaArgs& a, ACCT_LDS char* lds) {
+    const int wave = threadIdx.x >> 6, nspan = (a.Tc + 3) / 4, blk = blockIdx.x;
+    lane = threadIdx.x & 63;
+    kvb = __builtin_amdgcn_readfirstlane(4 * (blk % nspan) + wave);
+    qb = (blk / nspan) % a.Tr;
+    bh = blk / (nspan * a.Tr);
+    row = lds + wave * (2 * kKeepImage * 16);
+    col = row + kKeepImage * 16;
+    if (kvb >= a.Tc) return false;
+    return !keep_bits_unread(a, a.blkflags ? a.blkflags + ((int64_t)(a.mask_sb ? bh / a.N : 0) * a.Tr + qb) * a.Tc : nullptr, qb, kvb);
   }
-  __syncthreads();
+  ACCT_DEV void store(const FaArgs& a, uint32_t* rowbits, uint32_t* colbits) const {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (a wave's LDS operations complete in order: its lanes see each other's)
 #pragma unroll
-  for (int m = 0; m < 4; m++) {
-    const int k = threadIdx.x + 256 * m;
-    if (key0 + k < Sk && !(flags && flags[(key0 + k) >> 7] == kBlkSkip))
-      *reinterpret_cast<u32x4*>(out + (int64_t)(key0 + k) * 4) = *reinterpret_cast<const u32x4*>(s_cw + (k + (k >> 4)) * 4);
+    for (int m = 0; m < 2; m++) {
+      const int i = lane + 64 * m, r = qb * 128 + i, key = kvb * 128 + i;
+      if (rowbits && r < a.Sq) {
+        const u32x4 w = *reinterpret_cast<const ACCT_LDS u32x4*>(row + at(i));
+        // (an even number of words per row: 8-byte pieces, the second half of the last block may lie past the row)
+        uint32_t* out = rowbits + ((int64_t)bh * a.Sq + r) * a.droprow_w + 4 * kvb;
+        const u32x2 w0 = {w[0], w[1]}, w1 = {w[2], w[3]};
+        *reinterpret_cast<u32x2*>(out) = w0;
+        if (4 * kvb + 2 < a.droprow_w) *reinterpret_cast<u32x2*>(out + 2) = w1;
+      }
+      if (colbits && key < a.Sk)
+        *reinterpret_cast<u32x4*>(colbits + (((int64_t)bh * a.Tr + qb) * a.Sk + key) * 4) = *reinterpret_cast<const ACCT_LDS u32x4*>(col + at(i));
+    }
   }
+};
+
+// 8 x 8 bit transposes of all four bytes of x[0..7] at once: bit k of byte b of x[j] <-> bit j of byte b of x[k]
+ACCT_DEV void transpose_bytes8(uint32_t (&x)[8]) {
+  uint32_t mask = 0x0f0f0f0fu;
+#pragma unroll
+  for (int sft = 4; sft >= 1; sft >>= 1) {
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      if (k & sft) continue;
+      const uint32_t t = ((x[k] >> sft) ^ x[k + sft]) & mask;
+      x[k + sft] ^= t;
+      x[k] ^= t << sft;
+    }
+    mask ^= mask << (sft >> 1);
+  }
+}
+// the column words of sixteen keys x sixteen rows: x[j] holds rows j (low half) and j + 8 (high half), bit = key;
+// afterwards keys j and j + 8, bit = row
+ACCT_DEV void transpose_16x16(uint32_t (&x)[8]) {
+#pragma unroll
+  for (int j = 0; j < 8; j++) x[j] = __builtin_amdgcn_perm(x[j], x[j], 0x03010200u);   // the off-diagonal bytes change places
+  transpose_bytes8(x);
 }
 
 // Dropout mask (uint8 {0,1}, or the reference's {0, 1/keep_prob} in the I/O dtype; nonzero = keep) packed into keep bits, by query row for the kernels whose lanes own
-// query rows (forward, dQ) and by key column for the dK/dV kernel.  One workgroup of four waves per (batch*head,
-// 128 query rows, 1024 keys), one wave per 32 rows -- enough waves to keep the memory system busy --: per row every lane loads the 16 bytes of keys 16*lane .. +15 (a kilobyte per wave
-// instruction keeps enough bytes in flight) and turns them into 16 bits; lane pairs form the 32-bit row words.
+// query rows (forward, dQ) and by key column for the dK/dV kernel.
 //   rowbits [B*N*Sq, 2*ceil(Sk/64)] 32-bit: bit k of word w = keep[row][32w + k];
 //   colbits [B*N, Tr, Sk, 4] 32-bit: bit r of the 128-bit entry = keep[128*qb + r][key].
+// Bound by the mask bytes it reads.  A wave's load instruction reads the block's 128 or 256 bytes of eight or four
+// rows, sixteen such loads in flight, at any alignment (a key count that is no multiple of 16 shifts every row).
+// Blocks whose bits no kernel reads are not loaded.  Before, a wave walked 32 rows of 1024 keys: hidden blocks then
+// left lanes idle but saved no instruction, and those bound it.  B4 N8 S4096 causal, 2-byte mask (half of 1.07 GB
+// is needed): 274.7 -> 185.1 us = 3.7 TB/s read and written.
 template <int ES>
 __global__ void __launch_bounds__(256) fa_drop_bits_kernel(const FaArgs a, uint32_t* rowbits, uint32_t* colbits) {
-  __shared__ __attribute__((aligned(16))) uint32_t s_cw[(1024 + 64) * 4];
-  // A lane's sixteen keys of the span come from ES 16-byte loads of 16 / ES keys each; load h of the wave reads one
-  // contiguous kilobyte: keys 16*lane + e for bytes, keys 512 h + 8*lane + e for 2-byte elements.
-  constexpr int NH = ES, KH = 16 / ES;
-  const int nspan = (a.Sk + 1023) / 1024;
-  const int i = threadIdx.x >> 6;                       // which 32 rows of the 128-row block: word i of the column entries
-  const int blk = blockIdx.x;
-  const int span = blk % nspan, qb = (blk / nspan) % a.Tr, bh = blk / (nspan * a.Tr);
-  const int lane = threadIdx.x & 63;
-  const bool aligned = (((uintptr_t)a.drop | (uintptr_t)a.Sk) & 15) == 0;     // (16 elements: aligned 16-byte loads)
-  // Keys in a block that the attention mask's pre-pass classed 'skip' are never visited by the attention kernels:
-  // their keep bits are not read, so their mask bytes are not loaded either (this pass is bound by the bytes it
-  // reads; a padded batch skips a third to a half of them).
-  const uint8_t* flags = a.blkflags ? a.blkflags + ((int64_t)(a.mask_sb ? bh / a.N : 0) * a.Tr + qb) * a.Tc : nullptr;
-  int kv[NH];                                           // first key of each load
-  bool vec[NH], dead[NH];
-  const uint8_t* p[NH];
+  __shared__ __attribute__((aligned(16))) char s_img[4 * 2 * kKeepImage * 16];
+  KeepBlock kb;
+  if (!kb.init(a, (ACCT_LDS char*)s_img)) return;
+  constexpr int KH = 16 / ES, LPR = 128 / KH, NR = 2 * LPR;   // keys per load; lanes per row; rows of a lane (16 for bytes, 32 for 2-byte elements)
+  const int c = kb.lane % LPR, R = kb.lane / LPR;
+  const int row0 = kb.qb * 128 + NR * R, kv = kb.kvb * 128 + KH * c;
+  const int nrow = min(NR, a.Sq - row0);
+  const uint8_t* p = a.drop + (((int64_t)kb.bh * a.Sq + row0) * a.Sk + kv) * ES;
+  uint32_t cw[8];                                        // bytes: rows j, j + 8 in the halves; 2-byte: rows j, j + 8, j + 16, j + 24 in the bytes
 #pragma unroll
-  for (int h = 0; h < NH; h++) {
-    kv[h] = span * 1024 + (ES == 1 ? 16 * lane : 512 * h + 8 * lane);
-    vec[h] = aligned && kv[h] + KH <= a.Sk;
-    dead[h] = kv[h] >= a.Sk || (flags && flags[kv[h] / 128] == kBlkSkip);
-    p[h] = a.drop + (((int64_t)bh * a.Sq + qb * 128 + 32 * i) * a.Sk + min(kv[h], max(a.Sk - KH, 0))) * ES;
-  }
-  // row words: 32 keys are two lanes' bits for bytes, four lanes' for 2-byte elements (whose second load fills
-  // the words sixteen further on)
-  constexpr int LPW = 32 / KH;                          // lanes per word
-  const int widx = 32 * span + lane / LPW;
-  const bool writer = rowbits && lane % LPW == 0;
-  uint32_t* rowout = rowbits + ((int64_t)bh * a.Sq + qb * 128 + 32 * i) * a.droprow_w + widx;
-  const int nrow = min(128, a.Sq - qb * 128);
-  // cw[j]: the keep bits (bit e = this lane's key e) of rows j (low half) and j + 16 (high half) of the wave's 32
-  uint32_t cw[16];
+  for (int j = 0; j < 8; j++) cw[j] = 0u;
+  auto take = [&](int j, uint32_t nz) {                  // nz: bit e = key e of this lane is kept in its row j
+    ACCT_LDS char* out = kb.row + KeepBlock::at(NR * R + j);
+    if (ES == 1) {
+      *reinterpret_cast<ACCT_LDS uint16_t*>(out + 2 * c) = (uint16_t)nz;
+      cw[j & 7] |= nz << (16 * (j >> 3));
+    } else {
+      *reinterpret_cast<ACCT_LDS uint8_t*>(out + c) = (uint8_t)nz;
+      cw[j & 7] |= nz << (8 * (j >> 3));
+    }
+  };
+  auto pack = [&](const u32x4& v) {
+    uint32_t nz = 0;
 #pragma unroll
-  for (int e = 0; e < 16; e++) cw[e] = 0u;
-  for (int rh = 0; rh < 2; rh++) {
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-      const int rr = 32 * i + 16 * rh + j;
-      uint32_t nz = 0;                                  // bit KH*h + e: key e of this lane's load h is kept
-#pragma unroll
-      for (int h = 0; h < NH; h++) {
-        if (rr < nrow && !dead[h]) {
-          if (vec[h]) {
-            const u32x4 v = *reinterpret_cast<const u32x4*>(p[h]);
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-              if (ES == 1) {
-                // bit 8e: byte e is nonzero (no carry leaves a byte); then the four bits side by side
-                const uint32_t y = ((((v[w] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | v[w]) >> 7) & 0x01010101u;
-                nz |= ((y | (y >> 7) | (y >> 14) | (y >> 21)) & 0xfu) << (4 * w);
-              } else {
-                // 2-byte floating-point elements: nonzero apart from the sign bit
-                const uint32_t m = v[w] & 0x7fff7fffu;
-                const uint32_t y = (((m + 0x7fff7fffu) | m) >> 15) & 0x00010001u;
-                nz |= ((y | (y >> 15)) & 3u) << (KH * h + 2 * w);
-              }
-            }
-          } else {
-            const uint8_t* q = a.drop + ((int64_t)bh * a.Sq + qb * 128 + rr) * a.Sk * ES;
-#pragma unroll
-            for (int e = 0; e < KH; e++)
-              if (kv[h] + e < a.Sk && elem_nonzero<ES>(q, kv[h] + e)) nz |= 1u << (KH * h + e);
-          }
-        }
-        p[h] += (int64_t)a.Sk * ES;                     // per-lane pointers walk down the rows
+    for (int w = 0; w < 4; w++) {
+      if (ES == 1) {
+        // bit 7 of byte e: nonzero (no carry leaves a byte); the dot product with 1 2 4 8 (16 32 64 128) gathers the bits
+        const uint32_t y = (((v[w] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | v[w]) & 0x80808080u;
+        nz += __builtin_amdgcn_udot4(y, w & 1 ? 0x80402010u : 0x08040201u, 0u, false) << (8 * (w >> 1));
+      } else {
+        // 2-byte floating-point elements: nonzero apart from the sign bit
+        const uint32_t y = ((v[w] & 0x7fff7fffu) + 0x7fff7fffu) & 0x80008000u;
+        nz |= (y >> (15 - 2 * w)) | (y >> (30 - 2 * w));
       }
-      cw[j] |= nz << (16 * rh);
+    }
+    return ES == 1 ? nz >> 7 : nz & 0xffu;
+  };
+  if (kb.qb * 128 + 128 <= a.Sq && kb.kvb * 128 + 128 <= a.Sk) {   // (wave-uniform: no lane tests anything)
 #pragma unroll
-      for (int h = 0; h < NH; h++) {
-        uint32_t x = ((nz >> (KH * h)) & ((1u << KH) - 1u)) << (KH * (lane % LPW));
-        x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);                   // lane ^ 1
-        if (LPW == 4) x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true);     // lane ^ 2
-        if (writer && rr < nrow && !dead[h] && widx + 16 * h < a.droprow_w) rowout[16 * h] = x;   // (words of hidden key blocks are never read)
+    for (int r0 = 0; r0 < NR; r0 += 16) {
+      u32x4 v[16];
+#pragma unroll
+      for (int j = 0; j < 16; j++) {
+        v[j] = load_any<u32x4, ES>(p);
+        p += (int64_t)a.Sk * ES;
       }
-      rowout += a.droprow_w;
+#pragma unroll
+      for (int j = 0; j < 16; j++) take(r0 + j, pack(v[j]));
+    }
+  } else {
+    const bool whole = kv + KH <= a.Sk;
+#pragma unroll
+    for (int j = 0; j < NR; j++) {
+      uint32_t nz = 0;
+      if (j < nrow) {
+        if (whole) nz = pack(load_any<u32x4, ES>(p));
+        else                                             // the row ends inside (or before) this lane's piece
+          for (int e = 0; e < a.Sk - kv; e++) nz |= (elem_nonzero<ES>(p, e) ? 1u : 0u) << e;
+      }
+      take(j, nz);
+      p += (int64_t)a.Sk * ES;
     }
   }
-  // The column words are the transpose of that 32 x 16 bit matrix: two 16 x 16 transposes side by side in the
-  // sixteen registers (sub-blocks of 8, 4, 2, 1 swapped across the diagonal), after which bit r of cw[e] is the
-  // keep bit of row r and key e.  (Shifting every key's bit into sixteen words row by row cost five times as many
-  // instructions; this pass is bound by them, not by memory, once lanes of hidden key blocks load nothing.)
-  {
-    uint32_t mask = 0x00ff00ffu;
+  if (ES == 1) transpose_16x16(cw);
+  else transpose_bytes8(cw);
 #pragma unroll
-    for (int sft = 8; sft >= 1; sft >>= 1) {
-#pragma unroll
-      for (int k = 0; k < 16; k++) {
-        if (k & sft) continue;
-        const uint32_t t = ((cw[k] >> sft) ^ cw[k + sft]) & mask;
-        cw[k + sft] ^= t;
-        cw[k] ^= t << sft;
-      }
-      mask ^= mask << (sft >> 1);
-    }
+  for (int t = 0; t < KH; t++) {
+    ACCT_LDS char* out = kb.col + KeepBlock::at(KH * c + t);
+    if (ES == 1) *reinterpret_cast<ACCT_LDS uint16_t*>(out + 2 * R) = (uint16_t)(cw[t & 7] >> (16 * (t >> 3)));
+    else *reinterpret_cast<ACCT_LDS uint32_t*>(out + 4 * R) = cw[t & 7];
   }
-  if (colbits)
-    store_col_entries(s_cw, cw, i, lane, span * 1024, a.Sk, colbits + ((int64_t)bh * a.Tr + qb) * a.Sk * 4, flags,
-                      [](int l, int e) { return ES == 1 ? 16 * l + e : 512 * (e >> 3) + 8 * l + (e & 7); });
+  kb.store(a, rowbits, colbits);
 }
 
 // The same bitmaps for counter-based dropout: nothing is read, the keep decisions come from Philox4x32-10.
 // One call yields the 16 bytes of one (query row, 32-key group M, half g): keys 32M + 8u + 4g + e for
 // u = 0..3, e = 0..3 -- the keys one lane of the attention kernels owns in a 32-key group, so a kernel
-// could also draw them in place.  One workgroup of four waves per (batch*head, 128 query rows, 1024 keys), one
-// wave per 32 rows; lane 2L + g owns
-// (M = 32*span + L, g), the lane pair forms the 32-bit row word of group M.
+// could also draw them in place.
+// Bound by vector instructions: the ten rounds' twenty 32 x 32 -> 64-bit products, a quarter-rate instruction each,
+// are more than half of them.  Lane 8R + 2M + g draws rows 16R .. +15 of (M, g).  The sixteen byte comparisons of a
+// call are done on whole words, four dot products gather their outcomes into sixteen adjacent bits, and the column
+// words come from a bit-matrix transpose in registers.
+// Padded batch B16 N16 S1024, 69 % of the blocks visible: 73.6 -> 48.0 us (a wave that walked 32 rows of all keys
+// drew the hidden ones too, and compared and shifted key by key).
 __global__ void __launch_bounds__(256) fa_drop_philox_kernel(const FaArgs a, uint32_t* rowbits, uint32_t* colbits) {
-  __shared__ __attribute__((aligned(16))) uint32_t s_cw[(1024 + 64) * 4];
-  const int nspan = (a.Sk + 1023) / 1024;
-  const int i = threadIdx.x >> 6;                       // which 32 rows of the 128-row block: word i of the column entries
-  const int blk = blockIdx.x;
-  const int span = blk % nspan, qb = (blk / nspan) % a.Tr, bh = blk / (nspan * a.Tr);
-  const int lane = threadIdx.x & 63, g = lane & 1;
-  const int grp = 32 * span + (lane >> 1);              // 32-key group = word index within the row
-  const bool writer = rowbits && g == 0 && grp < a.droprow_w;
-  uint32_t* rowout = rowbits + ((int64_t)bh * a.Sq + qb * 128 + 32 * i) * a.droprow_w + grp;
-  const int nrow = min(128, a.Sq - qb * 128);
-  uint32_t cw[16];                                      // per key: the word of these 32 rows, most significant bit first
-  {
+  __shared__ __attribute__((aligned(16))) char s_img[4 * 2 * kKeepImage * 16];
+  KeepBlock kb;
+  if (!kb.init(a, (ACCT_LDS char*)s_img)) return;
+  const int g = kb.lane & 1, M = (kb.lane >> 1) & 3, R = kb.lane >> 3;
+  const int row0 = kb.qb * 128 + 16 * R;
+  // byte < thr on four bytes at once: with bit 7 set aside the difference stays inside its byte, and its bit 7 joins
+  // the two sevenths bits: not (x & z) for thr >= 128, not (x | z) below -- the majority with a constant.
+  const uint32_t thr7 = (a.philox_thr & 0x7fu) * 0x01010101u, low = a.philox_thr & 0x80u ? 0u : ~0u;
+  const uint32_t all = a.philox_thr >= 256u ? 0x80808080u : 0u;
+  uint32_t cw[8];                                       // rows j (low half) and j + 8 (high half), bit 4u + e
 #pragma unroll
-    for (int t = 0; t < 16; t++) cw[t] = 0u;
-#pragma unroll 2
-    for (int r = 0; r < 32; r++) {
-      const int rr = 32 * i + r;
-      uint32_t v[4];
-      philox4x32_10((uint32_t)(qb * 128 + rr), (uint32_t)(2 * grp + g), (uint32_t)bh, a.philox_offset, a.philox_k0, a.philox_k1, v);
-      uint32_t bits = 0;
+  for (int j = 0; j < 8; j++) cw[j] = 0u;
 #pragma unroll
-      for (int t = 0; t < 16; t++) {                    // t = 4u + e
-        const uint32_t keep = ((v[t >> 2] >> (8 * (t & 3))) & 0xffu) < a.philox_thr ? 1u : 0u;
-        bits |= keep << (8 * (t >> 2) + (t & 3));
-        cw[t] = (cw[t] << 1) | (rr < nrow ? keep : 0u);
-      }
-      uint32_t x = bits << (4 * g);
-      x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);    // lane ^ 1
-      if (writer && rr < nrow) *rowout = x;
-      rowout += a.droprow_w;
+  for (int r = 0; r < 16; r++) {
+    const int row = row0 + r;
+    uint32_t v[4];
+    philox4x32_10((uint32_t)row, (uint32_t)(2 * (4 * kb.kvb + M) + g), (uint32_t)kb.bh, a.philox_offset, a.philox_k0, a.philox_k1, v);
+    uint32_t y[4];                                      // bit 7 of byte e: kept
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const uint32_t z = (v[u] | 0x80808080u) - thr7;
+      y[u] = (~((v[u] & z) | ((v[u] | z) & low)) & 0x80808080u) | all;
     }
+    // byte weights 1 2 4 8 and 16 32 64 128: 128 times the eight bits of two words
+    const uint32_t b01 = __builtin_amdgcn_udot4(y[1], 0x80402010u, __builtin_amdgcn_udot4(y[0], 0x08040201u, 0u, false), false);
+    const uint32_t b23 = __builtin_amdgcn_udot4(y[3], 0x80402010u, __builtin_amdgcn_udot4(y[2], 0x08040201u, 0u, false), false);
+    uint32_t bits = (b01 >> 7) | (b23 << 1);
+    uint32_t x = (bits | (bits << 8)) & 0x00ff00ffu;    // nibble u to byte u
+    x = ((x | (x << 4)) & 0x0f0f0f0fu) << (4 * g);
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);    // lane ^ 1: the other half
+    if (g == 0) *reinterpret_cast<ACCT_LDS uint32_t*>(kb.row + KeepBlock::at(16 * R + r) + 4 * M) = x;
+    if (row >= a.Sq) bits = 0;
+    cw[r & 7] |= bits << (16 * (r >> 3));
   }
-  if (colbits) {
+  transpose_16x16(cw);
 #pragma unroll
-    for (int t = 0; t < 16; t++) cw[t] = __builtin_bitreverse32(cw[t]);
-    store_col_entries(s_cw, cw, i, lane, span * 1024, a.Sk, colbits + ((int64_t)bh * a.Tr + qb) * a.Sk * 4, nullptr,
-                      [](int l, int t) { return 32 * (l >> 1) + 8 * (t >> 2) + 4 * (l & 1) + (t & 3); });
-  }
+  for (int t = 0; t < 16; t++)
+    *reinterpret_cast<ACCT_LDS uint16_t*>(kb.col + KeepBlock::at(32 * M + 8 * (t >> 2) + 4 * g + (t & 3)) + 2 * R) = (uint16_t)(cw[t & 7] >> (16 * (t >> 3)));
+  kb.store(a, rowbits, colbits);
 }
 
 hipError_t launch_drop_philox(const FaArgs& a, uint32_t* rowbits, uint32_t* colbits, hipStream_t st) {
-  const long long nblk = (long long)a.B * a.N * a.Tr * ((a.Sk + 1023) / 1024);
+  const long long nblk = (long long)a.B * a.N * a.Tr * ((a.Tc + 3) / 4);
   hipLaunchKernelGGL(fa_drop_philox_kernel, dim3((unsigned)nblk), dim3(256), 0, st, a, rowbits, colbits);
   return hipGetLastError();
 }
 
 hipError_t launch_drop_bits(const FaArgs& a, uint32_t* rowbits, uint32_t* colbits, hipStream_t st) {
-  const long long nblk = (long long)a.B * a.N * a.Tr * ((a.Sk + 1023) / 1024);
+  const long long nblk = (long long)a.B * a.N * a.Tr * ((a.Tc + 3) / 4);
   if (a.drop_es == 2) hipLaunchKernelGGL(fa_drop_bits_kernel<2>, dim3((unsigned)nblk), dim3(256), 0, st, a, rowbits, colbits);
   else hipLaunchKernelGGL(fa_drop_bits_kernel<1>, dim3((unsigned)nblk), dim3(256), 0, st, a, rowbits, colbits);
   return hipGetLastError();
 }
 
-// true when launch_mask_blocks takes the fast path, which also writes the column bitmaps
-bool mask_prepass_is_fused(const FaArgs& a) {
-  // every 16-element piece of a row is 16-byte aligned and entirely inside or outside the row
-  return (((uintptr_t)a.mask | (uintptr_t)a.Sk | (uintptr_t)a.mask_sb) & 15) == 0;
-}
-
 hipError_t launch_mask_blocks(const FaArgs& a, uint8_t* flags, uint32_t* colbits, int MB, hipStream_t st) {
-  if (mask_prepass_is_fused(a)) {
-    const dim3 grid((unsigned)((long long)MB * a.Tr * a.Tc));
-    uint8_t* tails = flags + (size_t)MB * a.Tr * a.Tc;  // (the key-tail table follows the classes)
-    if (a.mask_es == 2) hipLaunchKernelGGL(fa_mask_prepass_kernel<2>, grid, dim3(256), 0, st, a, flags, tails, colbits);
-    else hipLaunchKernelGGL(fa_mask_prepass_kernel<1>, grid, dim3(256), 0, st, a, flags, tails, colbits);
-    return hipGetLastError();
-  }
-  const dim3 grid((unsigned)(MB * a.Tr));
-  if (a.mask_es == 2) hipLaunchKernelGGL(fa_mask_blocks_kernel<2>, grid, dim3(256), 0, st, a, flags);
-  else hipLaunchKernelGGL(fa_mask_blocks_kernel<1>, grid, dim3(256), 0, st, a, flags);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !colbits) return e;
-  return launch_mask_colbits(a, flags, colbits, MB, st);
+  const dim3 grid((unsigned)((long long)MB * a.Tr * a.Tc));
+  uint8_t* tails = flags + (size_t)MB * a.Tr * a.Tc;    // (the key-tail table follows the classes)
+  if (a.mask_es == 2) hipLaunchKernelGGL(fa_mask_prepass_kernel<2>, grid, dim3(256), 0, st, a, flags, tails, colbits);
+  else hipLaunchKernelGGL(fa_mask_prepass_kernel<1>, grid, dim3(256), 0, st, a, flags, tails, colbits);
+  return hipGetLastError();
 }
 
 }  // namespace acct

@@ -122,8 +122,9 @@ typedef struct acct_fa_params {
      into that buffer and a call with drop_bits_filled != 0 reads what an earlier call left there.  The
      caller sets drop_bits_filled after the first call returns; the bits depend on drop_mask or on
      (drop_seed, drop_offset, keep_prob) and on B, N, Sq, Sk; with a dense attn_mask the bits of the 128x128
-     blocks that the mask hides completely are left out (no kernel reads them), so the buffer belongs to the
-     calls of one step on one attn_mask. */
+     blocks that the mask hides completely, or that lie outside the band (prev_block_num, next_block_num,
+     row_block_prefix), are left out (no kernel reads them), so the buffer belongs to the calls of one step on
+     one attn_mask and one band. */
   void*    drop_bits;
   int32_t  drop_bits_filled;
   int32_t  drop_mask_kind;       /* ACCT_DROP_* (field added in version 104; 0 = the uint8 form) */
