@@ -33,10 +33,12 @@ from __future__ import annotations
 import weakref
 
 import torch
+from torch.autograd import forward_ad
 
 from acctransformer_amd import _capi
 
 TILING_BLOCK_SIZE = 128                       # constants.py:19 of the reference ops
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 _STRATEGIES = ("sparse", "wukong")            # tiling_strategy/sparse_tiling.py, wukong_tiling.py
 
 
@@ -124,7 +126,7 @@ def _attach_mask_bits(p, mask_tensor, device):
     from an earlier call, or a fresh one that `_mask_bits_done(p)` marks as filled once a call has run."""
     if p.mask_kind not in (_capi.MASK_DENSE_U8, _capi.MASK_DENSE_F16, _capi.MASK_TILE_U8, _capi.MASK_TILE_F16):
         return
-    stream = torch.cuda.current_stream(device).cuda_stream
+    stream = _capi._stream(device)
     sig = (p.mask_kind, p.B, p.Sq, p.Sk, p.prev_block_num, p.next_block_num, p.row_block_prefix, stream,
            mask_tensor.data_ptr())
     key = id(mask_tensor)
@@ -207,6 +209,20 @@ def _rows_contiguous(t):
     return t if t.stride(-1) == 1 else t.contiguous()
 
 
+def _nothing_to_record(*tensors):
+    """No gradient, tangent, transform or trace can want to know of this call: plain tensors, none of which asks for a
+    gradient in this mode, outside vmap / jvp / grad transforms, forward-mode levels and compilation.  The forward then
+    runs without an autograd function around it, whose bookkeeping costs a small call half of its host time."""
+    if (torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0 or torch.compiler.is_compiling()
+            or torch._C._get_tracing_state() is not None):
+        return False
+    record = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in _PLAIN or (record and t.requires_grad):
+            return False
+    return True
+
+
 class _FlashAttentionFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, attn_mask, dropout_mask, alibi_mask, prev_block_num, next_block_num, scale, keep_prob,
@@ -224,11 +240,14 @@ class _FlashAttentionFn(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.params = p
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)              # (no tensor of zeros for lse, which has no gradient)
         return o, lse
 
     @staticmethod
     def backward(ctx, do, _dlse):
         q, k, v, o, lse = ctx.saved_tensors
+        if do is None:
+            do = torch.zeros_like(o)
         dq, dk, dv = _capi.fa_bwd(ctx.params, q, k, v, o, do, lse)
         return dq, dk, dv, None, None, None, None, None, None, None, None
 
@@ -263,6 +282,13 @@ def get_flash_attention(prev_block_num=65536, next_block_num=65536, tiling_stgy_
     _check_strategy(tiling_stgy_name)
 
     def fa_forward(query, key, value, attn_mask=None, dropout_mask=None, alibi_mask=None):
+        if _nothing_to_record(query, key, value):
+            q, k, v = _rows_contiguous(query), _rows_contiguous(key), _rows_contiguous(value)
+            p = _build_params(q, k, v, attn_mask, dropout_mask, alibi_mask, prev_block_num, next_block_num, scale, keep_prob,
+                              row_block_prefix)
+            out = _capi.fa_fwd(p, q)
+            _mask_bits_done(p)
+            return out
         return _FlashAttentionFn.apply(query, key, value, attn_mask, dropout_mask, alibi_mask,
                                        prev_block_num, next_block_num, scale, keep_prob, row_block_prefix)
 
