@@ -262,9 +262,17 @@ size_t dropcol_bytes(const acct_fa_params* p) {
   return align_up((size_t)p->B * p->N * (size_t)((p->Sq + 127) / 128) * (size_t)p->Sk * 16, 256);
 }
 
+// key blocks after the query's block are left out, row by row (a row prefix of a few large blocks leaves out less, and in
+// steps: 4 row blocks, 16 heads, S3584, D64 59.8 us with 224 forward workgroups, 61.0 with 448)
+bool is_tri(const acct_fa_params* p) {
+  return (p->mask_kind == ACCT_MASK_CAUSAL || p->next_block_num == 0) && 8 * (int64_t)p->row_block_prefix <= p->Sq;
+}
+
 acct::FwdPlan plan_forward(const acct_fa_params* p, bool can_split, int n_cu) {
-  return acct::fwd_plan(p->B, p->N, p->Sq, p->Sk, p->D, p->alibi || dropout_on(p), p->mask_kind == ACCT_MASK_CAUSAL || p->next_block_num == 0,
-                        can_split, n_cu);
+  return acct::fwd_plan(p->B, p->N, p->Sq, p->Sk, p->D, p->alibi || dropout_on(p), is_tri(p), can_split, n_cu);
+}
+acct::DkdvPlan plan_dkdv(const acct_fa_params* p, size_t room, int n_cu) {
+  return acct::dkdv_plan(p->B, p->N, p->Sq, p->Sk, p->D, is_tri(p), room, n_cu);
 }
 
 // Pre-passes over the attention mask: block classes of a dense mask (all three kernels) and the mask packed by
@@ -332,7 +340,7 @@ size_t acct_fa_bwd_workspace_bytes(const acct_fa_params* p) {
   if (p->Sk <= 0 || p->D <= 0) return 0;
   // plus room for the per-slice sums of a dK/dV launch that splits the query range (few heads, short key
   // sequence); a caller that passes less gets the unsplit launch
-  return align_up(bwd_min_workspace_bytes(p), 256) + acct::dkdv_split(p->B, p->N, p->Sq, p->Sk, p->D).part_bytes;
+  return align_up(bwd_min_workspace_bytes(p), 256) + plan_dkdv(p, SIZE_MAX, 256).part_bytes;
 }
 
 int acct_fa_fwd(const acct_fa_params* p, void* O, float* LSE, void* workspace, size_t workspace_bytes, void* stream) {
@@ -439,14 +447,13 @@ static int bwd_impl(const acct_fa_params* p, const void* O, const void* dO, cons
     a.dk = tmp + grad_tmp_bytes(p, 0);
     a.dv = tmp + grad_tmp_bytes(p, 0) + grad_tmp_bytes(p, 1);
   }
-  a.q_split = 1;
-  if (want_dkdv) {
-    const acct::DkdvSplit sp = acct::dkdv_split(p->B, p->N, p->Sq, p->Sk, p->D, n_cu);
+  a.dq_kg = acct::dq_key_groups(p->B, p->N, p->Sq, p->Sk, p->D, is_tri(p), n_cu);
+  {
     const size_t part_at = align_up(need, 256);
-    if (sp.q_split > 1 && workspace_bytes >= part_at + sp.part_bytes) {
-      a.q_split = sp.q_split;
-      a.dkdv_part = (float*)((char*)workspace + part_at);
-    }
+    const acct::DkdvPlan plan = plan_dkdv(p, workspace_bytes > part_at ? workspace_bytes - part_at : 0, n_cu);
+    a.dkdv_ngk = plan.ngk;
+    a.q_split = plan.q_split;
+    if (plan.q_split > 1) a.dkdv_part = (float*)((char*)workspace + part_at);
   }
   hipError_t e = p->dtype == ACCT_F16 ? acct::launch_bwd_elem<acct::f16>(a, p->D, stages, st) : acct::launch_bwd_elem<acct::bf16>(a, p->D, stages, st);
   if (e != hipSuccess) return fail(ACCT_E_LAUNCH, "backward kernels: %s", hipGetErrorString(e));

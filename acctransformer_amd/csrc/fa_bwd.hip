@@ -36,27 +36,35 @@ ACCT_DEV typename Elem<T>::V8 pack8(const float* x) {
 // ============================================================================
 // dQ kernel (and delta): query-tile owner, structure of the forward kernel
 // ============================================================================
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT>
+//
+// KG = 2 (grids that leave CUs idle): the waves form NW / 2 row groups times two key groups, one 32-key chunk of every
+// tile each; the key groups' sums meet in LDS before the epilogue -- twice as many workgroups for the same rows.
+template <int D, int RG> constexpr int dq_merge_at() { return RG * 32 * (SwzCfg<D>::DB * 64 + 16); }   // behind the epilogue's staging
+template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KG = 1>
 ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
+  static_assert(KG == 1 || (KG == 2 && QG == 1 && NW % 2 == 0), "two key groups of one 32-key chunk each");
+  constexpr int CW = 2 / KG, WN = 32 * CW;                // 32-key chunks and keys of a tile that one wave works on
+  constexpr int RG = NW / KG;                             // row groups
   using E = Elem<T>;
   using V8 = typename E::V8;
   using C = SwzCfg<D>;
-  constexpr int BM = 32 * QG * NW;
+  constexpr int BM = 32 * QG * RG;
   constexpr int TILEB = 64 * C::PITCH;
   constexpr int FRING = 4, TRING = 3;                     // fragment reads in flight ahead of their MFMA (row-major / transposed)
-  constexpr bool RINGS = !(BIAS || DROP);                 // (the side-input variants have no registers for the rings)   // fragment reads in flight ahead of their MFMA (row-major / transposed)
+  constexpr bool RINGS = !(BIAS || DROP);                 // (the side-input variants have no registers for the rings)
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   ACCT_LDS char* smem = (ACCT_LDS char*)smem_raw;   // [2 buffers][K tile | V tile]; reused by the epilogue
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: everything derived from it stays in scalar registers
+  const int rg = KG > 1 ? wave % RG : wave, kg = KG > 1 ? wave / RG : 0;
   const int BH = a.B * a.N;
   int bh, rank;
   wg_map(blockIdx.x, BH, a.n_tiles, bh, rank);
   const int qt = a.n_tiles - 1 - rank;
   const int b = bh / a.N, h = bh % a.N;
   const int q0 = qt * BM;
-  const int wq0 = q0 + wave * 32 * QG;
+  const int wq0 = q0 + rg * 32 * QG;
   const int q_end = min(q0 + BM, a.Sq);
   const int wq_end = min(wq0 + 32 * QG, a.Sq);
 
@@ -126,7 +134,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
     if (row < a.Sq) {
       // (minus p_shift: the recomputed probabilities carry a factor 2^p_shift, see FaArgs)
       lq[gq] = a.lse[(int64_t)bh * a.Sq + row] * kLog2e - a.p_shift;
-      if (g == 0) {
+      if (g == 0 && kg == 0) {
         a.delta[(int64_t)bh * a.Sq + row] = dl[gq];
         a.nlse[(int64_t)bh * a.Sq + row] = -lq[gq];        // p_shift - LSE*log2(e): the exp2 offset the dK/dV kernel adds
       }
@@ -207,11 +215,12 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
         }
         DropStage::issue(a, bh, wq0, j + 1, lane, drop_lds + (buf ^ 1) * DropStage::BYTES);
       }
-      const int kv0 = j * 64;
+      const int kv0 = j * 64 + kg * WN;                     // this wave's first key of the tile
       const int kvb = j >> 1;
       bool act = (kvb - a.next_blk <= wqb) && (wqb <= kvb + a.prev_blk) && (wq0 < a.Sq);
       if (causal) act = act && (kv0 <= wq_end - 1);
       act = act && (kv0 < wkv_limit);
+      if (KG > 1) act = act && (kv0 < a.Sk);
       bool apply_mask = false;
       bool diag = causal;                                   // keys after the query are hidden, by index compare
       int last_key = a.Sk - 1;                              // last key that exists and is not behind a key tail
@@ -231,11 +240,14 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
       } else if (MASKT && a.mask_kind == kMaskTile) {
         apply_mask = wqb == kvb;
       }
-      const bool edge = apply_mask || (diag && (kv0 + 63 > wq0)) || (kv0 + 63 > last_key);
+      const bool edge = apply_mask || (diag && (kv0 + WN - 1 > wq0)) || (kv0 + WN - 1 > last_key);
       if (act) {
-        V8 dsf[QG][2][2];
+        const ACCT_LDS char* kw = kbuf + kg * (WN * C::PITCH);  // this wave's keys of the tile
+        const ACCT_LDS char* vw = vbuf + kg * (WN * C::PITCH);
+        V8 dsf[QG][CW][2];
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
+        for (int c = 0; c < CW; c++) {
+          const int ct = kg * CW + c;                           // chunk within the tile
           f32x16 s[QG], dp[QG];
 #pragma unroll
           for (int gq = 0; gq < QG; gq++) {
@@ -244,7 +256,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
               // q.k): nothing per score afterwards, no bias registers alive next to the scores
               typename E::V4 bv[4];
 #pragma unroll
-              for (int r4 = 0; r4 < 4; r4++) bv[r4] = bias_tile_read<T>(bias_lds + gq * 4096, row_bias ? 0 : l32, 4 * c + r4, g);
+              for (int r4 = 0; r4 < 4; r4++) bv[r4] = bias_tile_read<T>(bias_lds + gq * 4096, row_bias ? 0 : l32, 4 * ct + r4, g);
 #pragma unroll
               for (int r = 0; r < 16; r++) s[gq][r] = (float)bv[r >> 2][r & 3] * a.inv_scale;
             } else {
@@ -259,7 +271,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
             // flight ahead of the MFMA that consumes the oldest); S and dP MFMAs alternate.  The scheduling
             // barriers keep the compiler from folding the ring back into read-wait-MFMA.
             constexpr int NF = 2 * C::KS;
-            auto faddr = [&](int i) { return ((i & 1) ? vbuf : kbuf) + koff(i >> 1) + c * 32 * C::PITCH; };
+            auto faddr = [&](int i) { return ((i & 1) ? vw : kw) + koff(i >> 1) + c * 32 * C::PITCH; };
             V8 ring[FRING];
 #pragma unroll
             for (int i = 0; i < FRING; i++) ring[i] = lds_read_frag<T>(faddr(i));
@@ -278,9 +290,9 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
           } else {
             V8 kf[C::KS], vf[C::KS];
 #pragma unroll
-            for (int t = 0; t < C::KS; t++) kf[t] = lds_read_frag<T>(kbuf + koff(t) + c * 32 * C::PITCH);
+            for (int t = 0; t < C::KS; t++) kf[t] = lds_read_frag<T>(kw + koff(t) + c * 32 * C::PITCH);
 #pragma unroll
-            for (int t = 0; t < C::KS; t++) vf[t] = lds_read_frag<T>(vbuf + koff(t) + c * 32 * C::PITCH);
+            for (int t = 0; t < C::KS; t++) vf[t] = lds_read_frag<T>(vw + koff(t) + c * 32 * C::PITCH);
 #pragma unroll
             for (int t = 0; t < C::KS; t++)
 #pragma unroll
@@ -290,8 +302,8 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
 #pragma unroll
               for (int gq = 0; gq < QG; gq++) dp[gq] = E::mfma(vf[t], dof[gq][t], dp[gq]);
           }
-          if (BIAS && bias_staged && c == 1) {
-            // the whole bias tile has been read and the reads consumed: its LDS region can take the next
+          if (BIAS && bias_staged && c == CW - 1) {
+            // this wave's part of the bias tile has been read and the reads consumed: its LDS region can take the next
             // tile, which has the rest of this step to land (the end-of-step wait covers it)
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (j < j_hi) stage_bias(j + 1);
@@ -346,7 +358,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
                     if ((mbits >> (8 * e)) & 0xffu) x[4 * r4 + e] += kMaskFill * kLog2e;
                 }
               }
-              if ((diag && (kv0 + 63 > wq0)) || (kv0 + 63 > last_key)) {
+              if ((diag && (kv0 + WN - 1 > wq0)) || (kv0 + WN - 1 > last_key)) {
                 // keys after the query (causal), past Sk or behind a key tail: P is exactly 0
                 int vis = last_key - kv0 - 32 * c - 4 * g;
                 if (diag) vis = min(vis, qrow - kv0 - 32 * c - 4 * g);
@@ -355,7 +367,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
                   if (8 * (r >> 2) + (r & 3) > vis) x[r] = -INFINITY;
               }
               uint32_t dw = 0xffffffffu;                        // keep bits of this row: keys kv0 + 32c .. +31
-              if (DROP) dw = DropStage::word(drop_lds + buf * DropStage::BYTES, 32 * gq + l32, c) >> (4 * g);
+              if (DROP) dw = DropStage::word(drop_lds + buf * DropStage::BYTES, 32 * gq + l32, ct) >> (4 * g);
 #pragma unroll
               for (int r = 0; r < 16; r++) {
                 const float p = fast_exp2(x[r]);
@@ -375,10 +387,10 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
         }
         // ---- dQ^T += K^T dS^T : transposed K fragments through a ring of TRING register sets ----
         if constexpr (RINGS) {
-          constexpr int NT = 4 * C::DB;
+          constexpr int NT = 2 * CW * C::DB;
           auto tread = [&](int i) {
             const int db = i % C::DB, ch = i / C::DB;           // ch = 2 c + hh: rows 16 ch .. of the tile
-            const ACCT_LDS char* kaddr = kbuf + toff[db] + 16 * ch * C::PITCH;
+            const ACCT_LDS char* kaddr = kw + toff[db] + 16 * ch * C::PITCH;
             return join_tr<T>(lds_read_tr(kaddr), lds_read_tr(kaddr + C::tr_hi(db)));
           };
           V8 ring[TRING];
@@ -395,12 +407,12 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
           __builtin_amdgcn_sched_barrier(0);
         } else {
 #pragma unroll
-          for (int c = 0; c < 2; c++)
+          for (int c = 0; c < CW; c++)
 #pragma unroll
             for (int hh = 0; hh < 2; hh++)
 #pragma unroll
               for (int db = 0; db < C::DB; db++) {
-                const ACCT_LDS char* kaddr = kbuf + toff[db] + (32 * c + 16 * hh) * C::PITCH;
+                const ACCT_LDS char* kaddr = kw + toff[db] + (32 * c + 16 * hh) * C::PITCH;
                 const V8 ktf = join_tr<T>(lds_read_tr(kaddr), lds_read_tr(kaddr + C::tr_hi(db)));
 #pragma unroll
                 for (int gq = 0; gq < QG; gq++) acc[gq][db] = E::mfma(ktf, dsf[gq][c][hh], acc[gq][db]);
@@ -414,11 +426,35 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
     }
   }
 
+  // ---- key groups: the waves of group 0 take in the sums of the others ----
+  if constexpr (KG > 1) {
+    ACCT_LDS char* slot = smem + dq_merge_at<D, RG>() + rg * (C::DB * 4096) + lane * 16;
+    if (kg > 0) {
+#pragma unroll
+      for (int db = 0; db < C::DB; db++)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+          const f32x4 v = {acc[0][db][4 * r4], acc[0][db][4 * r4 + 1], acc[0][db][4 * r4 + 2], acc[0][db][4 * r4 + 3]};
+          *reinterpret_cast<ACCT_LDS f32x4*>(slot + (4 * db + r4) * 1024) = v;
+        }
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int db = 0; db < C::DB; db++)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; r4++) {
+        const f32x4 v = *reinterpret_cast<const ACCT_LDS f32x4*>(slot + (4 * db + r4) * 1024);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[0][db][4 * r4 + e] += v[e];
+      }
+  }
+
   // ---- epilogue: dQ = scale * dQ^T, transposed through the wave's own LDS region ----
   const float dq_scale = a.scale * a.p_unshift;
   T* dqp = (T*)a.dq + b * a.q_sb + h * a.q_sh;
   constexpr int OPITCH = C::DB * 64 + 16;
-  ACCT_LDS char* obuf = smem + wave * (32 * OPITCH);
+  ACCT_LDS char* obuf = smem + rg * (32 * OPITCH);
 #pragma unroll
   for (int gq = 0; gq < QG; gq++) {
 #pragma unroll
@@ -448,11 +484,11 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
 // The variant that knows mask tensors but neither a bias nor dropout carries a second body: a workgroup whose
 // rows see nothing but the causal pattern in a dense mask (block classes: clean before the diagonal, the
 // causal diagonal, skipped after it) runs the code of the variant without side inputs, by index compare.
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT>
+template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KG>
 __global__ void __launch_bounds__(64 * NW) fa_bwd_dq_kernel(const FaArgs a) {
   if constexpr (MASKT && !BIAS && !DROP) {
     if (a.mask_kind == kMaskDense) {
-      constexpr int BM = 32 * QG * NW;
+      constexpr int BM = 32 * QG * NW / KG;
       int bh, rank;
       wg_map(blockIdx.x, a.B * a.N, a.n_tiles, bh, rank);
       const int q0 = (a.n_tiles - 1 - rank) * BM, q_end = min(q0 + BM, a.Sq);
@@ -462,12 +498,12 @@ __global__ void __launch_bounds__(64 * NW) fa_bwd_dq_kernel(const FaArgs a) {
       if (dense_lines_are_causal(fl, 1, a.Tc, qb_lo, qb_hi - qb_lo + 1, kvb_lo, kvb_hi, false, a, threadIdx.x & 63)) {
         FaArgs c = a;
         c.mask_kind = kMaskCausal;
-        fa_bwd_dq_body<T, D, QG, NW, false, false, false>(c);
+        fa_bwd_dq_body<T, D, QG, NW, false, false, false, KG>(c);
         return;
       }
     }
   }
-  fa_bwd_dq_body<T, D, QG, NW, BIAS, DROP, MASKT>(a);
+  fa_bwd_dq_body<T, D, QG, NW, BIAS, DROP, MASKT, KG>(a);
 }
 
 // Epilogue of the dK/dV kernel: dV (V role) or dK (K role) of a wave's key rows, scaled, converted and transposed
@@ -510,42 +546,48 @@ ACCT_DEV void dkdv_store_rows(const f32x16 (&acc)[NGK][SwzCfg<D>::DB], const FaA
 }
 
 // Second half of a dK/dV launch whose query range was cut into a.q_split slices (few heads and a short key
-// sequence would otherwise leave most of the chip idle): one workgroup per key tile, the same wave and lane
-// roles as the dK/dV kernel; every lane adds up its accumulators over the slices in ascending order (a fixed
-// order: the result does not depend on which slice finished first) and stores the rows.
-template <typename T, int D, int NGK>
-__global__ void __launch_bounds__(512) fa_bwd_dkdv_reduce_kernel(const FaArgs a, float drop_scale) {
-  using C = SwzCfg<D>;
-  constexpr int NW = 8, WK = 32 * NGK, BNK = 4 * WK;
-  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  ACCT_LDS char* smem = (ACCT_LDS char*)smem_raw;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const bool krole = wave >= 4;
-  const int BH = a.B * a.N, n_wg = BH * a.n_tiles, wg = blockIdx.x;
+// sequence would otherwise leave most of the chip idle).  Every wave adds up one 32 x 32 tile of dK or dV over the
+// slices, four loads in flight, in ascending order (a fixed order: the result does not depend on which slice finished
+// first); the tile sits in the workspace as the registers of the wave that made it.
+template <typename T>
+__global__ void __launch_bounds__(256) fa_bwd_dkdv_reduce_kernel(const FaArgs a, float drop_scale, int ngk, int dbs) {
+  using E = Elem<T>;
+  const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+  const int BH = a.B * a.N, n_wg = BH * a.n_tiles;
+  const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);           // ((workgroup * 8 + wave) * ngk + key group) * dbs + d block
+  if (tile >= n_wg * 8 * ngk * dbs) return;
+  const int db = tile % dbs, gk = (tile / dbs) % ngk, wave = (tile / (dbs * ngk)) & 7, wg = tile / (dbs * ngk * 8);
   int bh, kt;
   wg_map(wg, BH, a.n_tiles, bh, kt);
-  const int b = bh / a.N, h = bh % a.N;
-  const int wk0 = kt * BNK + (wave & 3) * WK;
-  f32x16 acc[NGK][C::DB];
+  const bool krole = wave >= 4;
+  const int key = (kt * 4 + (wave & 3)) * 32 * ngk + 32 * gk + l32;
+  const int64_t step = (int64_t)n_wg * 8 * ngk * dbs << 10;
+  const float* part = a.dkdv_part + ((int64_t)tile << 10) + lane * 16;
+  f32x16 acc;
 #pragma unroll
-  for (int gk = 0; gk < NGK; gk++)
+  for (int r = 0; r < 16; r++) acc[r] = 0.f;
+  for (int s0 = 0; s0 < a.q_split; s0 += 4) {
+    f32x16 v[4];
 #pragma unroll
-    for (int db = 0; db < C::DB; db++)
+    for (int u = 0; u < 4; u++) v[u] = *reinterpret_cast<const f32x16*>(part + min(s0 + u, a.q_split - 1) * step);
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[gk][db][r] = 0.f;
-  for (int slice = 0; slice < a.q_split; slice++) {
-    const float* part = a.dkdv_part + ((((int64_t)slice * n_wg + wg) * NW + wave) * (NGK * C::DB) << 10) + lane * 16;
+    for (int u = 0; u < 4; u++)
+      if (s0 + u < a.q_split)
 #pragma unroll
-    for (int gk = 0; gk < NGK; gk++)
-#pragma unroll
-      for (int db = 0; db < C::DB; db++) {
-        const f32x16 v = *reinterpret_cast<const f32x16*>(part + ((gk * C::DB + db) << 10));
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[gk][db][r] += v[r];
-      }
+        for (int r = 0; r < 16; r++) acc[r] += v[u][r];
   }
+  if (key >= a.Sk) return;
+  const int b = bh / a.N, h = bh % a.N;
   const float oscale = (krole ? a.scale : drop_scale) * a.p_unshift;
-  dkdv_store_rows<T, D, NGK>(acc, a, b, h, wk0, krole, oscale, smem);
+  T* out = krole ? (T*)a.dk + b * a.k_sb + h * a.k_sh + key * a.k_ss : (T*)a.dv + b * a.v_sb + h * a.v_sh + key * a.v_ss;
+#pragma unroll
+  for (int r4 = 0; r4 < 4; r4++) {
+    const int d = 32 * db + 8 * r4 + 4 * g;
+    if (d >= a.hd) continue;
+    const typename E::V2 t0 = E::cvt2(acc[4 * r4 + 0] * oscale, acc[4 * r4 + 1] * oscale), t1 = E::cvt2(acc[4 * r4 + 2] * oscale, acc[4 * r4 + 3] * oscale);
+    const typename E::V4 ov = {t0[0], t0[1], t1[0], t1[1]};
+    *reinterpret_cast<typename E::V4*>(out + d) = ov;
+  }
 }
 
 // ============================================================================
@@ -561,16 +603,15 @@ __global__ void __launch_bounds__(512) fa_bwd_dkdv_reduce_kernel(const FaArgs a,
 constexpr int kPark = 6;        // stationary fragments parked in LDS per wave (D = 128)
 constexpr int kParkHot = 4;     // the variant without side inputs has registers for two more fragments
 // stationary fragments parked in LDS per wave: the bias variants give one up for the bias tiles' LDS
-template <int D, bool BIAS, bool MASKT>
-constexpr int dkdv_park() { return D == 128 ? (BIAS ? kPark - 1 : (MASKT ? kPark : kParkHot)) : 0; }
-// key groups of 32 rows per wave: head dims above 128 leave registers for the accumulators of one only
-template <int D> constexpr int dkdv_groups() { return D > 128 ? 1 : 2; }
+template <int D, bool BIAS, bool MASKT, int NGK>
+constexpr int dkdv_park() { return D == 128 && NGK == 2 ? (BIAS ? kPark - 1 : (MASKT ? kPark : kParkHot)) : 0; }
 
 // MASKT = false compiles the mask-tensor handling out (no mask, or the causal mask by index compare):
 // the hot variant must not carry that code's register pressure.
-template <typename T, int D, bool BIAS, bool DROP, bool MASKT, int NGK = 2>
+// NGK: key groups of 32 rows per wave.  One where head dims above 128 leave registers for the accumulators of one only,
+// and in grids that two would leave half empty (DkdvPlan).
+template <typename T, int D, bool BIAS, bool DROP, bool MASKT, int NGK>
 ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
-  static_assert(NGK == 2 || (NGK == 1 && !BIAS), "one key group per wave: no bias variants");
   using E = Elem<T>;
   using V8 = typename E::V8;
   using C = SwzCfg<D>;
@@ -646,7 +687,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
   // lane holds key row 32 gk + l32, d = 16t + 8g ..
   // The last PARK k-steps of the second key group live in a wave-private LDS slab instead of
   // registers (16 VGPRs at D = 128): that is what lets two waves share a SIMD without spilling.
-  constexpr int PARK = dkdv_park<D, BIAS, MASKT>();
+  constexpr int PARK = dkdv_park<D, BIAS, MASKT, NGK>();
   V8 bf[NGK][C::KS];
   ACCT_LDS char* park = pexch + 8 * PXB + wave * (PARK * 1024) + lane * 16;
   // bias tile (32 query rows x the pair's 64 keys) of the V-role wave, staged one chunk ahead by DMA
@@ -1048,7 +1089,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
 
 // (two bodies in the variant that knows mask tensors only, as in the dQ kernel: a workgroup whose key blocks
 // see nothing but the causal pattern runs the code of the variant without side inputs)
-template <typename T, int D, bool BIAS, bool DROP, bool MASKT, int NGK = 2>
+template <typename T, int D, bool BIAS, bool DROP, bool MASKT, int NGK>
 __global__ void __launch_bounds__(512) fa_bwd_dkdv_kernel(const FaArgs a) {
   if constexpr (MASKT && !BIAS && !DROP) {
     if (a.mask_kind == kMaskDense) {
@@ -1074,56 +1115,74 @@ __global__ void __launch_bounds__(512) fa_bwd_dkdv_kernel(const FaArgs a) {
 }
 
 // ---- launchers ----------------------------------------------------------------
+template <typename T, int D, bool BIAS, bool DROP, int KG>
+static hipError_t launch_bwd_dq(FaArgs a, hipStream_t st) {
+  constexpr int QG = 1, NW = D > 128 ? 4 : 8;            // (wide head dims: one wave per SIMD has the registers)
+  constexpr int RG = NW / KG, BM = 32 * QG * RG;
+  using CS = SwzCfg<D>;
+  constexpr size_t tiles = 4 * 64 * (size_t)CS::PITCH + (BIAS ? (size_t)NW * QG * 4096 : 0) + (size_t)NW * 2 * DropRowStage<DROP, QG, 2>::BYTES,
+                   stage = dq_merge_at<D, RG>() + (KG > 1 ? (size_t)RG * CS::DB * 4096 : 0);
+  constexpr size_t smem = tiles > stage ? tiles : stage;
+  static_assert(smem <= 160 * 1024, "the workgroup's LDS must fit the CU's 160 KB");
+  a.n_tiles = (a.Sq + BM - 1) / BM;
+  const bool mask_q = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
+  auto kern = mask_q ? fa_bwd_dq_kernel<T, D, QG, NW, BIAS, DROP, true, KG> : fa_bwd_dq_kernel<T, D, QG, NW, BIAS, DROP, BIAS || DROP, KG>;
+  const hipError_t e = allow_dynamic_lds((const void*)kern, smem);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((long long)a.n_tiles * a.B * a.N)), dim3(64 * NW), smem, st, a);
+  return hipGetLastError();
+}
+
+template <typename T, int D, bool BIAS, bool DROP, int NGK>
+static hipError_t launch_bwd_dkdv(FaArgs a, hipStream_t st) {
+  using CS = SwzCfg<D>;
+  constexpr size_t stageb = 2 * 64 * (size_t)CS::PITCH + 512 + (DROP ? 2048 : 0);
+  constexpr size_t loopb = 2 * stageb + 8 * 2048 * NGK + 8 * (size_t)dkdv_park<D, BIAS, true, NGK>() * 1024 + (BIAS ? 4 * 4096 : 0),
+                   epib = (size_t)8 * 32 * (CS::DB * 64 + 16);
+  constexpr size_t smem = loopb > epib ? loopb : epib;
+  static_assert(smem <= 160 * 1024, "the workgroup's LDS must fit the CU's 160 KB");
+  a.n_tiles = (a.Sk + 128 * NGK - 1) / (128 * NGK);
+  const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
+  auto kern = mask_t ? fa_bwd_dkdv_kernel<T, D, BIAS, DROP, true, NGK> : fa_bwd_dkdv_kernel<T, D, BIAS, DROP, BIAS || DROP, NGK>;
+  hipError_t e = allow_dynamic_lds((const void*)kern, smem);
+  if (e != hipSuccess) return e;
+  const long long n_wg = (long long)a.n_tiles * a.B * a.N;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(n_wg * (a.q_split > 1 ? a.q_split : 1))), dim3(512), smem, st, a);
+  e = hipGetLastError();
+  if (e == hipSuccess && a.q_split > 1) {
+    const long long waves = n_wg * 8 * NGK * CS::DB;
+    hipLaunchKernelGGL(fa_bwd_dkdv_reduce_kernel<T>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, a, DROP ? a.inv_keep : 1.0f, NGK, (int)CS::DB);
+    e = hipGetLastError();
+  }
+  return e;
+}
+
 template <typename T, int D, bool BIAS, bool DROP>
 static hipError_t launch_bwd_t(FaArgs a, int stages, hipStream_t st) {
   hipError_t e = hipSuccess;
-  bool dq_done = false;
-  if constexpr (D == 128 && !BIAS && !DROP) {
-    // head dim 128 without side inputs on aligned lengths: the kernel with 64 query rows per wave
-    if ((stages & kStageDq) && dq64_applicable(a)) {
-      e = launch_bwd_dq64(a, std::is_same<T, bf16>::value ? 1 : 0, st);
-      if (e != hipSuccess) return e;
-      dq_done = true;
+  if (stages & kStageDq) {
+    bool done = false;
+    if constexpr (D <= 128) {
+      if (a.dq_kg == 2) {
+        e = launch_bwd_dq<T, D, BIAS, DROP, 2>(a, st);
+        done = true;
+      }
     }
-  }
-  if ((stages & kStageDq) && !dq_done) {
-    constexpr int QG = 1, NW = D > 128 ? 4 : 8;          // (wide head dims: one wave per SIMD has the registers)
-    constexpr int BM = 32 * QG * NW;
-    using CS = SwzCfg<D>;
-    constexpr size_t tiles = 4 * 64 * (size_t)CS::PITCH + (BIAS ? (size_t)NW * QG * 4096 : 0) + (size_t)NW * 2 * DropRowStage<DROP, QG, 2>::BYTES, stage = (size_t)NW * 32 * (CS::DB * 64 + 16);
-    const size_t smem = tiles > stage ? tiles : stage;
-    a.n_tiles = (a.Sq + BM - 1) / BM;
-    const bool mask_q = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
-    auto kern = mask_q ? fa_bwd_dq_kernel<T, D, QG, NW, BIAS, DROP, true> : fa_bwd_dq_kernel<T, D, QG, NW, BIAS, DROP, BIAS || DROP>;
-    e = allow_dynamic_lds((const void*)kern, smem);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((long long)a.n_tiles * a.B * a.N)), dim3(64 * NW), smem, st, a);
-    e = hipGetLastError();
+    if constexpr (D == 128 && !BIAS && !DROP) {
+      // head dim 128 without side inputs on aligned lengths: the kernel with 64 query rows per wave
+      if (!done && dq64_applicable(a)) {
+        e = launch_bwd_dq64(a, std::is_same<T, bf16>::value ? 1 : 0, st);
+        done = true;
+      }
+    }
+    if (!done) e = launch_bwd_dq<T, D, BIAS, DROP, 1>(a, st);
     if (e != hipSuccess) return e;
   }
   if (stages & kStageDkDv) {
-    using CS = SwzCfg<D>;
-    constexpr int NGK = dkdv_groups<D>();
-    constexpr size_t stageb = 2 * 64 * (size_t)CS::PITCH + 512 + (DROP ? 2048 : 0);
-    constexpr size_t loopb = 2 * stageb + 8 * 2048 * NGK + 8 * (size_t)dkdv_park<D, BIAS, true>() * 1024 + (BIAS ? 4 * 4096 : 0),
-                     epib = (size_t)8 * 32 * (CS::DB * 64 + 16);
-    static_assert(loopb <= 160 * 1024 && epib <= 160 * 1024, "the workgroup's LDS must fit the CU's 160 KB");
-    const size_t smem2 = loopb > epib ? loopb : epib;
-    a.n_tiles = (a.Sk + 128 * NGK - 1) / (128 * NGK);
-    const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
-    auto kern = mask_t ? fa_bwd_dkdv_kernel<T, D, BIAS, DROP, true, NGK> : fa_bwd_dkdv_kernel<T, D, BIAS, DROP, BIAS || DROP, NGK>;
-    e = allow_dynamic_lds((const void*)kern, smem2);
-    if (e != hipSuccess) return e;
-    const long long n_wg = (long long)a.n_tiles * a.B * a.N;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(n_wg * (a.q_split > 1 ? a.q_split : 1))), dim3(512), smem2, st, a);
-    e = hipGetLastError();
-    if (e == hipSuccess && a.q_split > 1) {
-      auto red = fa_bwd_dkdv_reduce_kernel<T, D, NGK>;
-      e = allow_dynamic_lds((const void*)red, epib);
-      if (e != hipSuccess) return e;
-      hipLaunchKernelGGL(red, dim3((unsigned)n_wg), dim3(512), epib, st, a, DROP ? a.inv_keep : 1.0f);
-      e = hipGetLastError();
+    if constexpr (D <= 128) {
+      if (a.dkdv_ngk == 2) return launch_bwd_dkdv<T, D, BIAS, DROP, 2>(a, st);
     }
+    return launch_bwd_dkdv<T, D, BIAS, DROP, 1>(a, st);
   }
   return e;
 }

@@ -139,6 +139,8 @@ struct FaArgs {
   int row_prefix;                      // >0: row i sees keys j < (i/row_prefix + 1)*row_prefix only (multiple of 128)
   int n_tiles;                         // tiles along the owner dimension
   int kv_split;                        // forward kernel: slices of the key range, each on workgroups of its own (1 = no split)
+  int dq_kg;                           // dQ kernel: key groups of the workgroup (dq_key_groups, fa_index_math.hpp)
+  int dkdv_ngk;                        // dK/dV kernel: 32-key groups per wave (DkdvPlan, fa_index_math.hpp)
   int q_split;                         // dK/dV kernel: slices of the query range, each on workgroups of its own (1 = no split)
   int drop_visible;                    // keep bits: != 0 when those of key blocks outside the band (or past the causal / prefix limit) may be left out
   int droprow_w;                       // 32-bit words per row of droprow: 2 * ceil(Sk / 64)

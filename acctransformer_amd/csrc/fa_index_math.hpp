@@ -76,22 +76,69 @@ ACCT_HD int head_dim_class(int D) {
   return D <= 64 ? 64 : (D <= 128 ? 128 : 256);
 }
 
-// The dK/dV kernel gives every workgroup 256 keys (128 above head dim 128) of one head and all query rows.  With
-// few heads and a short key sequence (cross attention on 77 keys) that is a handful of workgroups for 256 CUs:
-// the query range is then cut into q_split slices that run side by side, and a second kernel adds their sums.
+// With few heads and a short key sequence (cross attention on 77 keys) the dK/dV kernel's key tiles are a handful of
+// workgroups for 256 CUs: the query range is then cut into q_split slices that run side by side, and a second kernel
+// adds their sums.  The split of a launch whose waves own two key groups (256 keys per workgroup, 128 above head dim
+// 128): as many slices as fill the CUs, at least 512 query rows each.
 // Returns q_split (1 = no split) and the bytes of workspace the slices' sums take.
 // `n_cu`: compute units of the device that runs the launch; the workspace-size query passes the 256 of a whole
 // MI355X, which is also the upper bound of what a partition of it asks for.
 struct DkdvSplit { int q_split; size_t part_bytes; };
+ACCT_HD size_t dkdv_part_bytes(int B, int N, int Sk, int D, int ngk, int split) {
+  const int db = (head_dim_class(D) + 31) / 32;
+  const long long n_wg = (long long)B * N * ((Sk + 128 * ngk - 1) / (128 * ngk));
+  return split > 1 ? (size_t)split * (size_t)n_wg * 8 * ngk * db * 1024 * sizeof(float) : 0;
+}
 ACCT_HD DkdvSplit dkdv_split(int B, int N, int Sq, int Sk, int D, int n_cu = 256) {
-  const int dc = head_dim_class(D), ngk = dc > 128 ? 1 : 2, db = (dc + 31) / 32;
+  const int ngk = head_dim_class(D) > 128 ? 1 : 2;
   const long long n_wg = (long long)B * N * ((Sk + 128 * ngk - 1) / (128 * ngk));
   const long long tiles64 = (Sq + 63) / 64;
   long long s = (n_cu > 256 ? 256 : n_cu) / n_wg;
   if (tiles64 / 8 < s) s = tiles64 / 8;              // a slice keeps at least 512 query rows
   if (s > 16) s = 16;
   if (s < 2) return {1, 0};
-  return {(int)s, (size_t)s * (size_t)n_wg * 8 * ngk * db * 1024 * sizeof(float)};
+  return {(int)s, dkdv_part_bytes(B, N, Sk, D, ngk, (int)s)};
+}
+
+// How the dK/dV kernel cuts its work: ngk 32-key groups per wave (4 * 32 * ngk keys per workgroup) and q_split slices
+// of the query range.  One key group per wave does half the work of two in 0.65 of the time (every Q / dO fragment
+// read from LDS feeds one MFMA instead of two), or in 0.53 where the head dim lets several workgroups share a CU, so
+// it pays where its finer units fill the last round better.  The estimate below prices the candidates in microseconds:
+// steps of 32 query rows, rounds of workgroups, and for slices the second launch and the sums written and read.
+// Measured, two groups / one group (us): 96 heads, 1000 x 1000, D64 93.6 / 74.4; 24, 3000 x 3000, D64 250 / 196;
+// 16, 4096 x 4096, D64 (256 and 512 workgroups: no round to save) 158 / 173; 144, 285 x 285, D128 47.5 / 33.8;
+// 80, 2000 x 2000, D128 378 / 394; causal: 64, 2048 x 2048, D128 154 / 177; 24, 2424 x 2424, D128 165 / 120.
+// With slices, before / now: 32 heads, 1024 x 77, D80 44.2 (two groups, 2 slices) / 26.1 (one group, 4); 40, 1611 x 77,
+// D160 43.7 (6) / 39.4 (4).
+struct DkdvPlan { int ngk, q_split; size_t part_bytes; };
+ACCT_HD double dkdv_estimate(int B, int N, int Sq, int Sk, int D, bool tri, int ngk, int split, int n_cu) {
+  const int dc = head_dim_class(D);
+  const double n = (double)B * N * ((Sk + 128 * ngk - 1) / (128 * ngk)) * split;
+  const int steps = 2 * (((Sq + 63) / 64 + split - 1) / split);
+  double walk = steps * (0.62 + 0.0037 * dc) * (ngk == 2 ? 1 / 0.65 : 1.0);
+  if (ngk == 1 && dc <= 64 && n > n_cu) walk *= 0.53 / 0.65;
+  // below the causal diagonal half of the workgroups' steps are absent, the heaviest start first
+  double rounds = (double)(((long long)n + n_cu - 1) / n_cu);
+  if (tri) rounds = 0.5 * n / n_cu + 0.3 < 1.0 ? 1.0 : 0.5 * n / n_cu + 0.3;
+  return 8.0 + walk * rounds + (split > 1 ? 6.5 + 2e6 / 6e12 * (double)dkdv_part_bytes(B, N, Sk, D, ngk, split) : 0.0);
+}
+// `room`: bytes of workspace there are for the slices' sums; `tri`: key blocks after the query's block are left out
+ACCT_HD DkdvPlan dkdv_plan(int B, int N, int Sq, int Sk, int D, bool tri, size_t room, int n_cu = 256) {
+  const bool wide = head_dim_class(D) > 128;           // (one key group per wave is all the registers hold)
+  DkdvPlan best = {wide ? 1 : 2, 1, 0};
+  double t_best = dkdv_estimate(B, N, Sq, Sk, D, tri, best.ngk, 1, n_cu);
+  const DkdvSplit two = dkdv_split(B, N, Sq, Sk, D, n_cu);
+  if (!wide && two.q_split > 1 && two.part_bytes <= room) {
+    const double t = dkdv_estimate(B, N, Sq, Sk, D, tri, 2, two.q_split, n_cu);
+    if (t < t_best) { t_best = t; best = {2, two.q_split, two.part_bytes}; }
+  }
+  const double n1 = (double)B * N * ((Sk + 127) / 128);
+  for (int s = 1; s <= 16 && s <= (Sq + 63) / 64 && (s == 1 || n1 * s <= (tri ? 2.0 : 1.0) * n_cu); s *= 2) {
+    const size_t bytes = dkdv_part_bytes(B, N, Sk, D, 1, s);
+    const double t = dkdv_estimate(B, N, Sq, Sk, D, tri, 1, s, n_cu);
+    if (bytes <= room && t < (s > 1 ? 0.95 : 1.0) * t_best) { t_best = t; best = {1, s, bytes}; }
+  }
+  return best;
 }
 
 // How the forward kernel cuts its work.  kg: key groups of the workgroup (fa_fwd.hip; 256 / kg query rows per
@@ -113,6 +160,13 @@ ACCT_HD size_t fwd_part_bytes(int B, int N, int Sq, int D, int kg, int split) {
   const long long groups = (long long)B * N * ((Sq + rows - 1) / rows) * (rows / 32);     // of 32 query rows
   return split > 1 ? (size_t)split * (size_t)groups * ((dc + 31) / 32 * 1024 + 64) * sizeof(float) : 0;
 }
+// A launch that fills the chip more than once still ends in a round that may be nearly empty.  Workgroups of half the
+// rows take `half` of the time of a whole one; true when their rounds add up to less.  Forward, kg 1 / 2 (us): 96 heads,
+// 1000 x 1000, D64 (384 / 768 workgroups) 42.5 / 37.0; 24, 3000 x 3000, D64 (288 / 576) 109.5 / 86.6; 144, 285 x 285, D128
+// (288 / 432) 25.3 / 22.6; but 96, 1000 x 1000, D128 (2 and 3 rounds of 0.7) 64.5 / 67.9; 16, 4096 x 4096, D64 (256 / 512) 80 / 84.
+ACCT_HD bool half_workgroups_pay(long long n1, long long n2, int n_cu, double half) {
+  return (double)((n2 + n_cu - 1) / n_cu) * half < 0.97 * (double)((n1 + n_cu - 1) / n_cu);
+}
 // `side`: a bias or dropout (not built for kg = 4); `tri`: key blocks after the query's block are left out;
 // `can_split`: there is room for the slices' sums
 ACCT_HD FwdPlan fwd_plan(int B, int N, int Sq, int Sk, int D, bool side, bool tri, bool can_split, int n_cu = 256) {
@@ -121,6 +175,7 @@ ACCT_HD FwdPlan fwd_plan(int B, int N, int Sq, int Sk, int D, bool side, bool tr
   int kg = 1;
   if (dc <= 128 && !side && n4 <= (tri ? n_cu + n_cu / 4 : n_cu)) kg = 4;
   else if (dc <= 160 && (n2 <= n_cu || (tri && n1 < n_cu && Sk >= 1024))) kg = 2;
+  else if (dc <= 128 && !tri && half_workgroups_pay(n1, n2, n_cu, dc <= 64 ? 0.55 : 0.7)) kg = 2;
   // slices: microseconds of a workgroup's walk against those of a slice's, plus the second launch and the traffic
   const int kg_s = dc > 160 ? 1 : 2;
   const long long n_s = kg_s == 2 ? n2 : bh * ((Sq + 127) / 128);
@@ -134,6 +189,17 @@ ACCT_HD FwdPlan fwd_plan(int B, int N, int Sq, int Sk, int D, bool side, bool tr
   }
   if (split > 1) kg = kg_s;
   return {kg, split, fwd_part_bytes(B, N, Sq, D, kg, split)};
+}
+
+// Key groups of the dQ kernel (fa_bwd.hip): 2 where 256-row workgroups would leave CUs idle.  A workgroup of half the
+// rows takes 0.6 to 0.75 of the time, so it pays in one round only: 8 heads, S3728, D128 causal 175 -> 112 us; 16 heads,
+// 1024 x 1024, D128 with dropout 47.9 -> 33.4; 24 heads, S2424, D128 causal 116 -> 90; but 80 heads, 2000 x 2000 272 / 277
+// and 16 heads, 4096 x 4096, D64 107 / 124.
+ACCT_HD int dq_key_groups(int B, int N, int Sq, int Sk, int D, bool tri, int n_cu = 256) {
+  const int dc = head_dim_class(D);
+  if (dc > 128) return 1;
+  const long long bh = (long long)B * N, n1 = bh * ((Sq + 255) / 256), n2 = bh * ((Sq + 127) / 128);
+  return n2 <= n_cu || (tri && n1 < n_cu && Sk >= 1024) ? 2 : 1;
 }
 
 }  // namespace acct
