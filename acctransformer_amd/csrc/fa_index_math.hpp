@@ -154,6 +154,9 @@ ACCT_HD DkdvPlan dkdv_plan(int B, int N, int Sq, int Sk, int D, bool tri, size_t
 // The slices cost a second launch and the slices' sums written and read (about 6.5 us, and 3 TB/s); they are
 // taken where the estimate below says that the shorter walk saves more: 1 head, 256 queries x 131072 keys
 // 1253 -> 37 us; 8 heads, 512 x 8192 80 -> 33; not for 4 heads, 2048 x 2048 causal (24.8 against 28.9).
+// Their number is a power of two or as many as the CUs hold, whichever walks least; powers of two alone leave up to
+// half of the CUs idle.  With / without the latter: 3 heads, 300 x 60000, D128 (28 / 16 slices) 54.2 / 75.0 us; 5 heads,
+// 400 x 60000, D64 (12 / 8) 67.6 / 88.1; 40 heads, 1 x 8000, D64 (6 / 4) 24.1 / 29.7; 7 heads, 500 x 20000 (9 / 8) 57.8 / 58.2.
 struct FwdPlan { int kg, kv_split; size_t part_bytes; };
 ACCT_HD size_t fwd_part_bytes(int B, int N, int Sq, int D, int kg, int split) {
   const int dc = head_dim_class(D), rows = dc > 160 ? 128 : 256 / kg;
@@ -183,9 +186,13 @@ ACCT_HD FwdPlan fwd_plan(int B, int N, int Sq, int Sk, int D, bool side, bool tr
   const double per_tile = 0.5 + 0.72 / 128 * dc;                       // kg = 4; 1.3 and 2.2 times that for kg = 2 and 1
   double best = per_tile * (kg == 4 ? 1.0 : kg == 2 ? 1.3 : 2.2) * tiles;
   int split = 1;
-  for (int s = 2; can_split && s <= tiles && s <= 256 && s * n_s <= n_cu; s *= 2) {
-    const double t = per_tile * (kg_s == 2 ? 1.3 : 2.2) * ((tiles + s - 1) / s) + 6.5 + 2e6 / 3e12 * (double)fwd_part_bytes(B, N, Sq, D, kg_s, s);
+  const long long fit = n_cu / n_s < 256 ? n_cu / n_s : 256;
+  const int most = fit < tiles ? (int)fit : tiles;
+  for (int i = 2; can_split && most >= 2; i *= 2) {                    // 2, 4, 8 ... and as many as there are CUs for
+    const int cut = i < most ? i : most, walk = (tiles + cut - 1) / cut, s = (tiles + walk - 1) / walk;
+    const double t = per_tile * (kg_s == 2 ? 1.3 : 2.2) * walk + 6.5 + 2e6 / 3e12 * (double)fwd_part_bytes(B, N, Sq, D, kg_s, s);
     if (t < best) { best = t; split = s; }
+    if (i >= most) break;
   }
   if (split > 1) kg = kg_s;
   return {kg, split, fwd_part_bytes(B, N, Sq, D, kg, split)};

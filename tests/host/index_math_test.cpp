@@ -3,6 +3,7 @@
 // prints one line per failed check and exits with the number of failures.
 // Test tier modelled on the reference's helper-level unit tests
 // (tests/train/flash_attention/ut/test_split_core_strategy.py, test_tensor_transformat.py).
+#include <cstdint>
 #include <cstdio>
 #include <set>
 #include <vector>
@@ -154,6 +155,34 @@ static void test_dkdv_split() {
   CHECK(dkdv_split(4, 16, 2048, 2048, 128).q_split == 1, "the benchmark shape splits");
 }
 
+// key slices of the forward kernel: any number that fits one round of workgroups, none of them empty, room as stated;
+// query slices of the dK/dV kernel: no more room than there is
+static void test_slice_plans() {
+  for (int BH : {1, 3, 5, 7, 24, 40, 56, 200})
+    for (int Sq : {1, 65, 300, 513, 1611, 4096})
+      for (int Sk : {1, 77, 130, 1000, 8197, 131072})
+        for (int D : {40, 64, 80, 128, 160, 256})
+          for (int n_cu : {32, 256})
+            for (bool tri : {false, true}) {
+              const FwdPlan f = fwd_plan(1, BH, Sq, Sk, D, false, tri, true, n_cu);
+              const int rows = head_dim_class(D) > 160 ? 128 : 256 / f.kg, tiles = ((tri && Sq < Sk ? Sq : Sk) + 127) / 128;
+              CHECK(f.part_bytes == fwd_part_bytes(1, BH, Sq, D, f.kg, f.kv_split), "part_bytes");
+              if (f.kv_split > 1) {
+                const int walk = (tiles + f.kv_split - 1) / f.kv_split;
+                CHECK((long long)f.kv_split * BH * ((Sq + rows - 1) / rows) <= n_cu, "%d slices do not fit", f.kv_split);
+                CHECK((f.kv_split - 1) * walk < tiles, "an empty slice: %d of %d tiles", f.kv_split, tiles);
+              }
+              CHECK(fwd_plan(1, BH, Sq, Sk, D, false, tri, false, n_cu).kv_split == 1, "a split without room");
+              for (size_t room : {(size_t)0, (size_t)1 << 22, SIZE_MAX}) {
+                const DkdvPlan p = dkdv_plan(1, BH, Sq, Sk, D, tri, room, n_cu);
+                CHECK(p.part_bytes <= room && p.part_bytes == dkdv_part_bytes(1, BH, Sk, D, p.ngk, p.q_split), "part_bytes");
+                CHECK(p.q_split == 1 || (long long)p.q_split * BH * ((Sk + 128 * p.ngk - 1) / (128 * p.ngk)) <= (tri ? 2 : 1) * n_cu,
+                      "%d slices do not fit", p.q_split);
+              }
+            }
+  CHECK(fwd_plan(1, 3, 300, 60000, 128, false, false, true).kv_split == 28, "9 workgroups, 256 CUs");
+}
+
 static void test_div_small() {
   for (int n = 1; n <= 32; n++)
     for (int idx = 0; idx < 1024; idx++) CHECK(div_small(idx, recip16(n)) == idx / n, "div_small(%d, %d)", idx, n);
@@ -169,6 +198,7 @@ int main() {
   test_tr_hi<256>();
   test_head_dim_class();
   test_dkdv_split();
+  test_slice_plans();
   test_div_small();
   if (failures) printf("%d checks failed\n", failures);
   else printf("index math: all checks passed\n");
