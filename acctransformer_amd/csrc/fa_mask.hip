@@ -187,8 +187,8 @@ struct KeepBlock {
   ACCT_LDS char* col;                                    // [key][16 bytes]: bit r = keep[128 qb + r][key]
   static ACCT_DEV int at(int i) { return (i + (i >> 4)) * 16; }
   // false: nothing to do for this wave
-  ACCT_DEV bool init(const FaArgs& a, ACCT_LDS char* lds) {
-    const int wave = threadIdx.x >> 6, nspan = (a.Tc + 3) / 4, blk = blockIdx.x;
+  ACCT_DEV bool init(const FaArgs& a, ACCT_LDS char* lds, int blk) {
+    const int wave = threadIdx.x >> 6, nspan = (a.Tc + 3) / 4;
     lane = threadIdx.x & 63;
     kvb = __builtin_amdgcn_readfirstlane(4 * (blk % nspan) + wave);
     qb = (blk / nspan) % a.Tr;
@@ -240,6 +240,15 @@ ACCT_DEV void transpose_16x16(uint32_t (&x)[8]) {
   transpose_bytes8(x);
 }
 
+// workgroup id -> block span: the ids that one XCD gets (id % 8) take consecutive spans
+ACCT_DEV int xcd_span(int id, int n) {
+  const int per = n / 8, rem = n % 8, xcd = id & 7;
+  return xcd * per + min(xcd, rem) + (id >> 3);
+}
+// sixteen bytes at any address that nothing reads again
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+ACCT_DEV u32x4 load_once(const uint8_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p)); }
+
 // Dropout mask (uint8 {0,1}, or the reference's {0, 1/keep_prob} in the I/O dtype; nonzero = keep) packed into keep bits, by query row for the kernels whose lanes own
 // query rows (forward, dQ) and by key column for the dK/dV kernel.
 //   rowbits [B*N*Sq, 2*ceil(Sk/64)] 32-bit: bit k of word w = keep[row][32w + k];
@@ -247,13 +256,17 @@ ACCT_DEV void transpose_16x16(uint32_t (&x)[8]) {
 // Bound by the mask bytes it reads.  A wave's load instruction reads the block's 128 or 256 bytes of eight or four
 // rows, sixteen such loads in flight, at any alignment (a key count that is no multiple of 16 shifts every row).
 // Blocks whose bits no kernel reads are not loaded.  Before, a wave walked 32 rows of 1024 keys: hidden blocks then
-// left lanes idle but saved no instruction, and those bound it.  B4 N8 S4096 causal, 2-byte mask (half of 1.07 GB
-// is needed): 274.7 -> 185.1 us = 3.7 TB/s read and written.
+// left lanes idle but saved no instruction, and those bound it: B4 N8 S4096 causal, 2-byte mask (half of 1.07 GB
+// is needed) 274.7 -> 185.1 us.  Neighbouring blocks share the lines of the row words and of each mask row's pages:
+// each XCD takes one contiguous eighth of them, and the mask, read once, does not displace anything in the caches:
+// 155.5 us with the first alone, 175.1 with the second alone, 142.3 = 4.2 TB/s with both; S3001, 3 x 8 heads 83.9 ->
+// 82.0, S1024 12.6 -> 11.8.  (The Philox kernel below reads nothing, and an eighth of its blocks each evens out less
+// well: 46.5 -> 48.8 on a padded batch, so it takes them in order.)
 template <int ES>
 __global__ void __launch_bounds__(256) fa_drop_bits_kernel(const FaArgs a, uint32_t* rowbits, uint32_t* colbits) {
   __shared__ __attribute__((aligned(16))) char s_img[4 * 2 * kKeepImage * 16];
   KeepBlock kb;
-  if (!kb.init(a, (ACCT_LDS char*)s_img)) return;
+  if (!kb.init(a, (ACCT_LDS char*)s_img, xcd_span(blockIdx.x, gridDim.x))) return;
   constexpr int KH = 16 / ES, LPR = 128 / KH, NR = 2 * LPR;   // keys per load; lanes per row; rows of a lane (16 for bytes, 32 for 2-byte elements)
   const int c = kb.lane % LPR, R = kb.lane / LPR;
   const int row0 = kb.qb * 128 + NR * R, kv = kb.kvb * 128 + KH * c;
@@ -294,7 +307,7 @@ __global__ void __launch_bounds__(256) fa_drop_bits_kernel(const FaArgs a, uint3
       u32x4 v[16];
 #pragma unroll
       for (int j = 0; j < 16; j++) {
-        v[j] = load_any<u32x4, ES>(p);
+        v[j] = load_once(p);
         p += (int64_t)a.Sk * ES;
       }
 #pragma unroll
@@ -338,7 +351,7 @@ __global__ void __launch_bounds__(256) fa_drop_bits_kernel(const FaArgs a, uint3
 __global__ void __launch_bounds__(256) fa_drop_philox_kernel(const FaArgs a, uint32_t* rowbits, uint32_t* colbits) {
   __shared__ __attribute__((aligned(16))) char s_img[4 * 2 * kKeepImage * 16];
   KeepBlock kb;
-  if (!kb.init(a, (ACCT_LDS char*)s_img)) return;
+  if (!kb.init(a, (ACCT_LDS char*)s_img, blockIdx.x)) return;
   const int g = kb.lane & 1, M = (kb.lane >> 1) & 3, R = kb.lane >> 3;
   const int row0 = kb.qb * 128 + 16 * R;
   // byte < thr on four bytes at once: with bit 7 set aside the difference stays inside its byte, and its bit 7 joins
