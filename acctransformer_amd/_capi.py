@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+from operator import index
 
 import torch
 
@@ -144,6 +145,10 @@ def make_params(q, k, v, *, scale, keep_prob=1.0, prev_block_num=BLOCK_UNBOUNDED
     to [B,N,Sq,Sk].  With drop_seed (and no drop_mask) and
     keep_prob < 1 the library draws the keep mask itself from
     (drop_seed, drop_offset), identically in forward and backward."""
+    # (plain numbers from here on: the key of a kept block and the block itself hold the values of this call, whatever
+    # object they come in -- a 0-d tensor hashes by its identity and may be changed in place between calls)
+    scale, keep_prob, mask_kind, row_block_prefix = float(scale), float(keep_prob), index(mask_kind), int(row_block_prefix)
+    prev_block_num, next_block_num = int(min(prev_block_num, BLOCK_UNBOUNDED)), int(min(next_block_num, BLOCK_UNBOUNDED))
     key = None
     if o_like is None:
         key = (q.shape, q.stride(), q.dtype, k.shape, k.stride(), k.dtype, v.shape, v.stride(), v.dtype, scale, keep_prob, prev_block_num,
@@ -184,10 +189,10 @@ def make_params(q, k, v, *, scale, keep_prob=1.0, prev_block_num=BLOCK_UNBOUNDED
     p = AcctFaParams()
     p.dtype = dt
     p.B, p.N, p.Sq, p.Sk, p.D = B, N, Sq, Sk, D
-    p.scale, p.keep_prob = float(scale), float(keep_prob)
-    p.prev_block_num, p.next_block_num = int(min(prev_block_num, BLOCK_UNBOUNDED)), int(min(next_block_num, BLOCK_UNBOUNDED))
+    p.scale, p.keep_prob = scale, keep_prob
+    p.prev_block_num, p.next_block_num = prev_block_num, next_block_num
     p.mask_kind = mask_kind
-    p.row_block_prefix = int(row_block_prefix)
+    p.row_block_prefix = row_block_prefix
     p.q_stride, p.k_stride, p.v_stride = _bhs_strides(q), _bhs_strides(k), _bhs_strides(v)
     if o_like is not None:
         p.o_stride = _bhs_strides(o_like)

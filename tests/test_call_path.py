@@ -1,5 +1,6 @@
 """The host path of a call: parameter blocks that are kept between calls, and the forward that runs without an autograd
 function where nothing is recorded."""
+import numpy as np
 import pytest
 import torch
 from torch.autograd import forward_ad
@@ -55,6 +56,19 @@ def test_kept_parameter_blocks_equal_fresh_ones():
         _block(t(), t()[:, :, :8], t(), scale=0.1)
     with pytest.raises(ValueError):
         _block(t(), t()[:, :, :8], t(), scale=0.1)
+
+
+@pytest.mark.parametrize("name, first, second", [("scale", 0.125, 0.25), ("keep_prob", 0.5, 0.75), ("prev_block_num", 3, 5),
+                                                 ("next_block_num", 3, 5), ("row_block_prefix", 128, 256)])
+def test_numbers_in_tensors_and_arrays(name, first, second):
+    """A number may come as a 0-d tensor or array; one that is changed in place between two calls counts as it is."""
+    q, k, v = (torch.randn(1, 1, 64, 64).half() for _ in range(3))
+    for x in (torch.tensor(first), np.array(first)):
+        kw = dict(dict(scale=0.1), **{name: x})
+        assert _block(q, k, v, **kw)[0][name] == first
+        x.fill_(second) if isinstance(x, torch.Tensor) else x.fill(second)
+        assert _block(q, k, v, **kw)[0][name] == second
+        assert _block(q, k, v, **dict(kw, **{name: first}))[0][name] == first
 
 
 @pytest.mark.gpu
