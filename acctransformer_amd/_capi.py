@@ -17,6 +17,7 @@ _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), _LIB_NAME)
 
 ACCT_F16, ACCT_BF16 = 0, 1
 MASK_NONE, MASK_DENSE_U8, MASK_DENSE_F16, MASK_TILE_U8, MASK_CAUSAL, MASK_TILE_F16 = 0, 1, 2, 3, 4, 5
+_TENSOR_MASKS = (MASK_DENSE_U8, MASK_TILE_U8, MASK_DENSE_F16, MASK_TILE_F16)      # the kinds that read a tensor
 DROP_U8, DROP_F16 = 0, 1
 BLOCK_UNBOUNDED = 65536
 
@@ -158,7 +159,7 @@ def make_params(q, k, v, *, scale, keep_prob=1.0, prev_block_num=BLOCK_UNBOUNDED
             p = AcctFaParams.from_buffer_copy(block)
             p.q, p.k, p.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
             keep = [q, k, v]
-            if p.attn_mask:
+            if mask_kind in _TENSOR_MASKS:
                 p.attn_mask = attn_mask.data_ptr()
                 keep.append(attn_mask)
             if drop_mask is not None:
@@ -198,7 +199,7 @@ def make_params(q, k, v, *, scale, keep_prob=1.0, prev_block_num=BLOCK_UNBOUNDED
         p.o_stride = _bhs_strides(o_like)
     p.q, p.k, p.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
     keep = [q, k, v]
-    if mask_kind in (MASK_DENSE_U8, MASK_TILE_U8, MASK_DENSE_F16, MASK_TILE_F16):
+    if mask_kind in _TENSOR_MASKS:
         want = torch.uint8 if mask_kind in (MASK_DENSE_U8, MASK_TILE_U8) else q.dtype
         if attn_mask is None or attn_mask.dtype != want or not attn_mask.is_contiguous():
             raise TypeError(f"attn_mask must be a contiguous {want} tensor for mask_kind {mask_kind}")

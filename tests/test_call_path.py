@@ -71,6 +71,22 @@ def test_numbers_in_tensors_and_arrays(name, first, second):
         assert _block(q, k, v, **dict(kw, **{name: first}))[0][name] == first
 
 
+def test_blocks_of_tensors_without_memory():
+    """A call on meta tensors has no addresses; a later one of the same shapes hands over its own."""
+    shapes = [(1, 2, 64, 64)] * 3
+    kw = dict(scale=0.1, mask_kind=_capi.MASK_DENSE_U8, keep_prob=0.5)
+    _capi._blocks.clear()
+    for device in ("meta", "cpu"):
+        q, k, v = (torch.zeros(s, dtype=torch.float16, device=device) for s in shapes)
+        mask = torch.zeros(1, 64, 64, dtype=torch.uint8, device=device)
+        drop = torch.ones(1, 2, 64, 64, dtype=torch.uint8, device=device)
+        alibi = torch.zeros(1, 2, 1, 64, dtype=torch.float16, device=device)
+        got, p = _block(q, k, v, attn_mask=mask, drop_mask=drop, alibi=alibi, **kw)
+    assert (got["q"], got["k"], got["v"]) == (q.data_ptr(), k.data_ptr(), v.data_ptr())
+    assert (got["attn_mask"], got["drop_mask"], got["alibi"]) == (mask.data_ptr(), drop.data_ptr(), alibi.data_ptr())
+    assert len(p._keepalive) == 6
+
+
 @pytest.mark.gpu
 def test_forward_with_and_without_recording():
     q, k, v = (torch.randn(1, 2, 96, 64, device=DEV).half() for _ in range(3))
