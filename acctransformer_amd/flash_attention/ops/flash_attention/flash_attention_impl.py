@@ -210,15 +210,19 @@ def _rows_contiguous(t):
 
 
 def _nothing_to_record(*tensors):
-    """No gradient, tangent, transform or trace can want to know of this call: plain tensors, none of which asks for a
-    gradient in this mode, outside vmap / jvp / grad transforms, forward-mode levels and compilation.  The forward then
-    runs without an autograd function around it, whose bookkeeping costs a small call half of its host time."""
+    """No gradient, tangent, transform or trace can want to know of this call: plain tensors, none of which -- side inputs
+    included -- asks for a gradient in this mode, outside vmap / jvp / grad transforms, forward-mode levels and
+    compilation.  The forward then runs without an autograd function around it, whose bookkeeping costs a small call
+    half of its host time."""
     if (torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0 or torch.compiler.is_compiling()
             or torch._C._get_tracing_state() is not None):
         return False
     record = torch.is_grad_enabled()
     for t in tensors:
-        if type(t) not in _PLAIN or (record and t.requires_grad):
+        if type(t) in _PLAIN:
+            if record and t.requires_grad:
+                return False
+        elif t is not None and not _is_seed_pair(t):
             return False
     return True
 
@@ -282,7 +286,7 @@ def get_flash_attention(prev_block_num=65536, next_block_num=65536, tiling_stgy_
     _check_strategy(tiling_stgy_name)
 
     def fa_forward(query, key, value, attn_mask=None, dropout_mask=None, alibi_mask=None):
-        if _nothing_to_record(query, key, value):
+        if _nothing_to_record(query, key, value, attn_mask, dropout_mask, alibi_mask):
             q, k, v = _rows_contiguous(query), _rows_contiguous(key), _rows_contiguous(value)
             p = _build_params(q, k, v, attn_mask, dropout_mask, alibi_mask, prev_block_num, next_block_num, scale, keep_prob,
                               row_block_prefix)

@@ -87,6 +87,27 @@ def test_blocks_of_tensors_without_memory():
     assert len(p._keepalive) == 6
 
 
+@pytest.mark.parametrize("side", ["query", "attn_mask", "dropout_mask", "alibi_mask", None])
+def test_a_side_input_that_asks_for_a_gradient_is_recorded(side, monkeypatch):
+    """The output belongs to the graph as soon as any input asks for a gradient; masks and biases then get none."""
+    monkeypatch.setattr(_capi, "fa_fwd", lambda p, q: (torch.zeros_like(q), torch.zeros(q.shape[:3])))
+    monkeypatch.setattr(_capi, "fa_bwd", lambda p, q, k, v, o, do, lse: tuple(torch.zeros_like(t) for t in (q, k, v)))
+    monkeypatch.setattr(_capi, "attach_drop_bits", lambda p, device: None)
+    inputs = dict(query=torch.randn(1, 2, 64, 64).half(), key=torch.randn(1, 2, 64, 64).half(), value=torch.randn(1, 2, 64, 64).half(),
+                  attn_mask=torch.zeros(1, 64, 64).half(), dropout_mask=torch.ones(1, 2, 64, 64).half(), alibi_mask=torch.zeros(1, 2, 1, 64).half())
+    if side:
+        inputs[side].requires_grad_(True)
+    op = get_flash_attention(scale=0.125, keep_prob=0.9)
+    o, lse = op(**inputs)
+    assert o.requires_grad == (side is not None) and not lse.requires_grad
+    if side:
+        o.sum().backward()
+        assert (inputs[side].grad is not None) == (side == "query")
+    with torch.no_grad():
+        assert not op(**inputs)[0].requires_grad
+    assert op(**dict(inputs, dropout_mask=(3, 4), **({side: inputs[side].detach()} if side and side != "dropout_mask" else {})))[0].grad_fn is None
+
+
 @pytest.mark.gpu
 def test_forward_with_and_without_recording():
     q, k, v = (torch.randn(1, 2, 96, 64, device=DEV).half() for _ in range(3))
