@@ -166,6 +166,10 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   const int mb = a.mask_sb ? b : 0;
   const uint8_t* maskp = a.mask ? a.mask + (a.mask_kind == kMaskDense ? (int64_t)mb * a.mask_sb * a.mask_es : 0) : nullptr;
   const T* alibip = BIAS ? (const T*)a.alibi + b * a.al_sb + h * a.al_sh : nullptr;
+  // (named here and not compared where it is used: with this value among what the softmax lambda captures the compiler
+  // allocates the head dim 256 kernel with 758 moves between the two register files instead of 826, and the mask and
+  // dropout variants likewise: 32 heads, 3000 x 3000 358 -> 350 us)
+  const bool mask_dense = a.mask_kind == kMaskDense;
   const bool alibi_vec = BIAS && (((uintptr_t)a.alibi & 7) | ((a.al_sb | a.al_sh | a.al_sq) & 3)) == 0;
 
   TileDma<T, D, BN, NW> kdma, vdma;
@@ -343,7 +347,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
             for (int r4 = 0; r4 < 4; r4++) {
               const int kv = kv0 + 32 * c + 8 * r4 + 4 * g;
               uint32_t mbits;
-              if (a.mask_kind == kMaskDense) mbits = load_mask4(maskp + (int64_t)qrow_c * a.Sk * a.mask_es, kv, a.Sk, a.mask_es);
+              if (mask_dense) mbits = load_mask4(maskp + (int64_t)qrow_c * a.Sk * a.mask_es, kv, a.Sk, a.mask_es);
               else mbits = load_mask4(maskp + (qrow_c & 127) * 128 * a.mask_es, kv & 127, 128, a.mask_es);
 #pragma unroll
               for (int e = 0; e < 4; e++)
