@@ -625,7 +625,7 @@ __global__ void __launch_bounds__(256) fa_fwd_combine_kernel(const FaArgs a, int
     float mb = m;
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int s = min(s0 + 4 * u, a.kv_split - 1);                        // (a repeated slice gets weight 0 below)
+      const int s = min(s0 + 4 * u, a.kv_split - 1);                        // (a repeated slice is left out below)
       v[u] = *reinterpret_cast<const f32x4*>(part + s * step * (dbs * 1024));
       ml[u] = *reinterpret_cast<const f32x2*>(stat + s * step * 64);
     }
@@ -638,7 +638,8 @@ __global__ void __launch_bounds__(256) fa_fwd_combine_kernel(const FaArgs a, int
     for (int e = 0; e < 4; e++) o[e] *= al;
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const float w = s0 + 4 * u < a.kv_split ? fast_exp2((ml[u][0] - m) * cmul) : 0.f;
+      if (s0 + 4 * u >= a.kv_split) break;                                  // (weight 0 would turn an infinity of V into NaN)
+      const float w = fast_exp2((ml[u][0] - m) * cmul);
       l = __builtin_fmaf(ml[u][1], w, l);
 #pragma unroll
       for (int e = 0; e < 4; e++) o[e] = __builtin_fmaf(v[u][e], w, o[e]);

@@ -67,3 +67,21 @@ def test_forward_of_small_grids(Sq, Sk, D, side, splits):
         ok, ratio, mx = orc.tolerance_gate(O, o.float().cpu().numpy(), atol=2e-3, rtol=1e-3)
         assert ok, f"workspace {size}: worst ratio {ratio:.3f}, max |d| {mx:.3e}"
         assert np.max(np.abs(L - lse.cpu().numpy())) < 1e-4 * max(1.0, np.abs(L).max() / 10), f"LSE, workspace {size}"
+
+
+@pytest.mark.parametrize("Sq, Sk, D", [(64, 8192, 40), (1, 3072, 128), (129, 4608, 256)])
+def test_infinite_values_stay_infinite(Sq, Sk, D):
+    """An infinity of V belongs to its output column only, whichever slice of the keys holds it.  (Whole key tiles: a tile
+    that the keys end in repeats the last row of V with probability 0.)"""
+    g = torch.Generator().manual_seed(Sk)
+    q, k, v = (torch.randn(1, 2, S, D, generator=g).half() for S in (Sq, Sk, Sk))
+    v[:, :, Sk - 1, 5], v[:, :, Sk // 2, 6], v[:, :, 0, 7] = float("inf"), float("-inf"), float("inf")
+    qd = q.to(DEV)
+    p = _capi.make_params(qd, k.to(DEV), v.to(DEV), scale=D ** -0.5)
+    lib = _capi.load()
+    for size in (lib.acct_fa_fwd_workspace_bytes(ctypes.byref(p)), lib.acct_fa_fwd_split_workspace_bytes(ctypes.byref(p))):
+        o = _forward(p, qd, size)[0].cpu()
+        assert (o[..., 5] == float("inf")).all() and (o[..., 6] == float("-inf")).all() and (o[..., 7] == float("inf")).all(), f"workspace {size}"
+        finite = torch.ones(D, dtype=torch.bool)
+        finite[5:8] = False
+        assert torch.isfinite(o[..., finite]).all()
