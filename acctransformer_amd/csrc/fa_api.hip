@@ -264,15 +264,23 @@ size_t dropcol_bytes(const acct_fa_params* p) {
 
 // key blocks after the query's block are left out, row by row (a row prefix of a few large blocks leaves out less, and in
 // steps: 4 row blocks, 16 heads, S3584, D64 59.8 us with 224 forward workgroups, 61.0 with 448)
-bool is_tri(const acct_fa_params* p) {
+// (not a band that leaves out the blocks far before the query's too: its workgroups are equally long.  32 heads, S2048, D128,
+// 8 blocks back: backward 130.7 us as equal workgroups, 143.6 as a triangle)
+bool ends_at_query(const acct_fa_params* p) {
   return (p->mask_kind == ACCT_MASK_CAUSAL || p->next_block_num == 0) && 8 * (int64_t)p->row_block_prefix <= p->Sq;
+}
+// (not a band that leaves out the blocks far before the query's too: its workgroups are equally long.  32 heads, S2048, D128,
+// 8 blocks back: backward 130.7 us as equal workgroups, 143.6 as a triangle)
+bool is_tri(const acct_fa_params* p) {
+  return ends_at_query(p) && 4 * (int64_t)p->prev_block_num >= 3 * (((int64_t)p->Sq + 127) / 128);
 }
 
 acct::FwdPlan plan_forward(const acct_fa_params* p, bool can_split, int n_cu) {
-  return acct::fwd_plan(p->B, p->N, p->Sq, p->Sk, p->D, p->alibi || dropout_on(p), is_tri(p), can_split, n_cu);
+  const int row_keys = acct::visible_row_keys(p->Sq, p->Sk, p->prev_block_num, p->next_block_num, p->row_block_prefix);
+  return acct::fwd_plan(p->B, p->N, p->Sq, p->Sk, p->D, p->alibi || dropout_on(p), is_tri(p), can_split, n_cu, row_keys, ends_at_query(p));
 }
 acct::DkdvPlan plan_dkdv(const acct_fa_params* p, size_t room, int n_cu) {
-  return acct::dkdv_plan(p->B, p->N, p->Sq, p->Sk, p->D, is_tri(p), room, n_cu);
+  return acct::dkdv_plan(p->B, p->N, p->Sq, p->Sk, p->D, is_tri(p), room, n_cu, p->prev_block_num, p->mask_kind == ACCT_MASK_CAUSAL ? 0 : p->next_block_num);
 }
 
 // Pre-passes over the attention mask: block classes of a dense mask (all three kernels) and the mask packed by

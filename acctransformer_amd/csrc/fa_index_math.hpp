@@ -110,35 +110,65 @@ ACCT_HD DkdvSplit dkdv_split(int B, int N, int Sq, int Sk, int D, int n_cu = 256
 // 80, 2000 x 2000, D128 378 / 394; causal: 64, 2048 x 2048, D128 154 / 177; 24, 2424 x 2424, D128 165 / 120.
 // With slices, before / now: 32 heads, 1024 x 77, D80 44.2 (two groups, 2 slices) / 26.1 (one group, 4); 40, 1611 x 77,
 // D160 43.7 (6) / 39.4 (4).
+//
+// A band lets 128 keys see only `blocks` of the 128-row blocks (`share` of that on average; all of them in the
+// `whole` part of the sequence, less at its ends), so 128 * ngk keys are walked by blocks + ngk - 1 of them and finer units
+// pass fewer rows that their keys do not see.  Backward of a launch with two groups / one group: 64 heads, S4096, D64, one
+// block back 144.5 / 117.8 us; 32, S2048, D128, eight back 128.6 / 143.6; 48, S1500, D80 (288 and 576 workgroups, of which
+// 168 and 336 are whole), five back 78.9 / 86.4; 24, S2048, D128 (192 and 384), four back 81.6 / 89.1.
+struct RowBand { bool on; int blocks; double share, whole; };
+ACCT_HD RowBand row_band(int Sq, int prev_blk, int next_blk) {
+  const int T = (Sq + 127) / 128, p = prev_blk < T ? prev_blk : T - 1, q = next_blk < T ? next_blk : T - 1;
+  const double all = (double)T * (1 + p + q);
+  return {p + q + 1 < T, 1 + p + q, (all - 0.5 * p * (p + 1.0) - 0.5 * q * (q + 1.0)) / all, (double)(T - p - q) / T};
+}
 struct DkdvPlan { int ngk, q_split; size_t part_bytes; };
-ACCT_HD double dkdv_estimate(int B, int N, int Sq, int Sk, int D, bool tri, int ngk, int split, int n_cu) {
+ACCT_HD double dkdv_estimate(int B, int N, int Sq, int Sk, int D, bool tri, int ngk, int split, int n_cu, int prev_blk, int next_blk) {
   const int dc = head_dim_class(D);
   const double n = (double)B * N * ((Sk + 128 * ngk - 1) / (128 * ngk)) * split;
-  const int steps = 2 * (((Sq + 63) / 64 + split - 1) / split);
+  const RowBand band = row_band(Sq, prev_blk, next_blk);
+  int steps = 2 * (((Sq + 63) / 64 + split - 1) / split);
+  if (band.on && band.blocks + ngk - 1 < steps / 4) steps = 4 * (band.blocks + ngk - 1);
   double walk = steps * (0.62 + 0.0037 * dc) * (ngk == 2 ? 1 / 0.65 : 1.0);
   if (ngk == 1 && dc <= 64 && n > n_cu) walk *= 0.53 / 0.65;
-  // below the causal diagonal half of the workgroups' steps are absent, the heaviest start first
   double rounds = (double)(((long long)n + n_cu - 1) / n_cu);
-  if (tri) rounds = 0.5 * n / n_cu + 0.3 < 1.0 ? 1.0 : 0.5 * n / n_cu + 0.3;
+  if (tri) {   // below the causal diagonal half of the workgroups' steps are absent, the heaviest start first
+    rounds = 0.5 * n / n_cu + 0.3 < 1.0 ? 1.0 : 0.5 * n / n_cu + 0.3;
+  } else if (band.on) {   // the workgroups at the ends of the band are shorter than the rest
+    const double whole = (double)(((long long)(band.whole * n) + n_cu - 1) / n_cu), r = band.share * n / n_cu + 0.3;
+    rounds = r < whole ? whole : r < rounds ? r : rounds;
+  }
   return 8.0 + walk * rounds + (split > 1 ? 6.5 + 2e6 / 6e12 * (double)dkdv_part_bytes(B, N, Sk, D, ngk, split) : 0.0);
 }
-// `room`: bytes of workspace there are for the slices' sums; `tri`: key blocks after the query's block are left out
-ACCT_HD DkdvPlan dkdv_plan(int B, int N, int Sq, int Sk, int D, bool tri, size_t room, int n_cu = 256) {
+// `room`: bytes of workspace there are for the slices' sums; `tri`: key blocks after the query's block are left out;
+// `prev_blk`, `next_blk`: the band
+ACCT_HD DkdvPlan dkdv_plan(int B, int N, int Sq, int Sk, int D, bool tri, size_t room, int n_cu = 256, int prev_blk = 65536, int next_blk = 65536) {
   const bool wide = head_dim_class(D) > 128;           // (one key group per wave is all the registers hold)
   DkdvPlan best = {wide ? 1 : 2, 1, 0};
-  double t_best = dkdv_estimate(B, N, Sq, Sk, D, tri, best.ngk, 1, n_cu);
+  double t_best = dkdv_estimate(B, N, Sq, Sk, D, tri, best.ngk, 1, n_cu, prev_blk, next_blk);
   const DkdvSplit two = dkdv_split(B, N, Sq, Sk, D, n_cu);
   if (!wide && two.q_split > 1 && two.part_bytes <= room) {
-    const double t = dkdv_estimate(B, N, Sq, Sk, D, tri, 2, two.q_split, n_cu);
+    const double t = dkdv_estimate(B, N, Sq, Sk, D, tri, 2, two.q_split, n_cu, prev_blk, next_blk);
     if (t < t_best) { t_best = t; best = {2, two.q_split, two.part_bytes}; }
   }
   const double n1 = (double)B * N * ((Sk + 127) / 128);
+  const bool banded = row_band(Sq, prev_blk, next_blk).on;
   for (int s = 1; s <= 16 && s <= (Sq + 63) / 64 && (s == 1 || n1 * s <= (tri ? 2.0 : 1.0) * n_cu); s *= 2) {
     const size_t bytes = dkdv_part_bytes(B, N, Sk, D, 1, s);
-    const double t = dkdv_estimate(B, N, Sq, Sk, D, tri, 1, s, n_cu);
-    if (bytes <= room && t < (s > 1 ? 0.95 : 1.0) * t_best) { t_best = t; best = {1, s, bytes}; }
+    const double t = dkdv_estimate(B, N, Sq, Sk, D, tri, 1, s, n_cu, prev_blk, next_blk);
+    if (bytes <= room && t < (banded ? 0.9 : s > 1 ? 0.95 : 1.0) * t_best) { t_best = t; best = {1, s, bytes}; }
   }
   return best;
+}
+
+// Keys that the 128-row block with the longest walk sees: the band (blocks qb - prev_blk .. qb + next_blk) and the row
+// prefix, whose last group sees the most, bound it; the caller's Sk bounds it as well.
+ACCT_HD int visible_row_keys(int Sq, int Sk, int prev_blk, int next_blk, int row_prefix) {
+  const long long qb_last = (Sq - 1) / 128, kb_last = (Sk - 1) / 128;
+  const long long before = prev_blk < qb_last ? prev_blk : qb_last, after = next_blk < kb_last ? next_blk : kb_last;
+  long long keys = (before + 1 + after) * 128;
+  if (row_prefix > 0 && ((long long)(Sq - 1) / row_prefix + 1) * row_prefix < keys) keys = ((long long)(Sq - 1) / row_prefix + 1) * row_prefix;
+  return keys < Sk ? (int)keys : Sk;
 }
 
 // How the forward kernel cuts its work.  kg: key groups of the workgroup (fa_fwd.hip; 256 / kg query rows per
@@ -171,18 +201,23 @@ ACCT_HD bool half_workgroups_pay(long long n1, long long n2, int n_cu, double ha
   return (double)((n2 + n_cu - 1) / n_cu) * half < 0.97 * (double)((n1 + n_cu - 1) / n_cu);
 }
 // `side`: a bias or dropout (not built for kg = 4); `tri`: key blocks after the query's block are left out;
-// `can_split`: there is room for the slices' sums
-ACCT_HD FwdPlan fwd_plan(int B, int N, int Sq, int Sk, int D, bool side, bool tri, bool can_split, int n_cu = 256) {
+// `can_split`: there is room for the slices' sums; `row_keys`: keys that the widest row block sees (visible_row_keys) --
+// what the slices are cut from; `one_sided`: a band that ends at the query's block, where the workgroups at one end are
+// short and whole rounds do not count (48 heads, S1500, D64, five blocks back 19.6 us for kg 1, 22.6 for kg 2)
+ACCT_HD FwdPlan fwd_plan(int B, int N, int Sq, int Sk, int D, bool side, bool tri, bool can_split, int n_cu = 256, int row_keys = 0x7fffffff,
+                         bool one_sided = false) {
   const int dc = head_dim_class(D);
   const long long bh = (long long)B * N, n1 = bh * ((Sq + 255) / 256), n2 = bh * ((Sq + 127) / 128), n4 = bh * ((Sq + 63) / 64);
   int kg = 1;
   if (dc <= 128 && !side && n4 <= (tri ? n_cu + n_cu / 4 : n_cu)) kg = 4;
   else if (dc <= 160 && (n2 <= n_cu || (tri && n1 < n_cu && Sk >= 1024))) kg = 2;
-  else if (dc <= 128 && !tri && half_workgroups_pay(n1, n2, n_cu, dc <= 64 ? 0.55 : 0.7)) kg = 2;
+  else if (dc <= 128 && !tri && !one_sided && half_workgroups_pay(n1, n2, n_cu, dc <= 64 ? 0.55 : 0.7)) kg = 2;
   // slices: microseconds of a workgroup's walk against those of a slice's, plus the second launch and the traffic
   const int kg_s = dc > 160 ? 1 : 2;
   const long long n_s = kg_s == 2 ? n2 : bh * ((Sq + 127) / 128);
-  const int seen = tri ? (Sq < Sk ? Sq : Sk) : Sk, tiles = (seen + 127) / 128;
+  int seen = tri && Sq < Sk ? Sq : Sk;
+  if (row_keys < seen) seen = row_keys;
+  const int tiles = (seen + 127) / 128;
   const double per_tile = 0.5 + 0.72 / 128 * dc;                       // kg = 4; 1.3 and 2.2 times that for kg = 2 and 1
   double best = per_tile * (kg == 4 ? 1.0 : kg == 2 ? 1.3 : 2.2) * tiles;
   int split = 1;

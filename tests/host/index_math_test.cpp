@@ -183,6 +183,40 @@ static void test_slice_plans() {
   CHECK(fwd_plan(1, 3, 300, 60000, 128, false, false, true).kv_split == 28, "9 workgroups, 256 CUs");
 }
 
+// the longest walk of a 128-row block, counted key block by key block
+static void test_visible_row_keys() {
+  for (int Sq : {1, 128, 129, 1000, 8192})
+    for (int Sk : {1, 77, 128, 1000, 8192, 8200})
+      for (int prev : {0, 1, 3, 65536})
+        for (int next : {0, 1, 5, 65536, 0x7fffffff})
+          for (int prefix : {0, 128, 1024, 4096}) {
+            int most = 0;
+            for (int qb = 0; qb < (Sq + 127) / 128; qb++) {
+              int lo = Sk, hi = 0;
+              for (int j = 0; j < Sk; j++) {
+                if (j / 128 > (long long)qb + next || qb > (long long)j / 128 + prev) continue;
+                if (prefix && j >= (qb * 128 / prefix + 1) * prefix) continue;
+                if (j < lo) lo = j;
+                hi = j + 1;
+              }
+              if (hi - lo > most) most = hi - lo;
+            }
+            const int keys = visible_row_keys(Sq, Sk, prev, next, prefix);
+            CHECK(keys >= most && keys <= Sk, "Sq %d Sk %d band %d/%d prefix %d: %d keys, %d visible", Sq, Sk, prev, next, prefix, keys, most);
+            if (!prefix && prev == 65536 && next == 65536) CHECK(keys == Sk, "no band");
+          }
+  CHECK(visible_row_keys(8192, 8192, 1, 1, 0) == 384 && visible_row_keys(8192, 8192, 2, 0, 0) == 384, "three key blocks");
+  CHECK(visible_row_keys(1000, 9000, 65536, 65536, 512) == 1024, "two groups of rows");
+  // the dK/dV units of a band: as few as fill the CUs where the band is wide, finer ones where it is narrow
+  CHECK(dkdv_plan(2, 16, 2048, 2048, 128, false, SIZE_MAX, 256, 8, 0).ngk == 2, "256 workgroups of a wide band");
+  CHECK(dkdv_plan(3, 16, 1500, 1500, 80, false, SIZE_MAX, 256, 5, 0).ngk == 2, "288 workgroups, those at the end shorter");
+  CHECK(dkdv_plan(4, 16, 4096, 4096, 64, false, SIZE_MAX, 256, 1, 0).ngk == 1, "a narrow band");
+  // a band of three key blocks is one launch, whatever the length; a wide one is cut, by what its rows see
+  CHECK(fwd_plan(1, 1, 8192, 8192, 64, false, false, true, 256, visible_row_keys(8192, 8192, 1, 1, 0)).kv_split == 1, "a narrow band is cut");
+  CHECK(fwd_plan(1, 1, 256, 131072, 128, false, false, true, 256, visible_row_keys(256, 131072, 0, 2, 0)).kv_split == 1, "few keys are cut");
+  CHECK(fwd_plan(1, 1, 256, 131072, 128, false, false, true, 256, visible_row_keys(256, 131072, 65536, 200, 0)).kv_split > 8, "a wide band is not cut");
+}
+
 static void test_div_small() {
   for (int n = 1; n <= 32; n++)
     for (int idx = 0; idx < 1024; idx++) CHECK(div_small(idx, recip16(n)) == idx / n, "div_small(%d, %d)", idx, n);
@@ -199,6 +233,7 @@ int main() {
   test_head_dim_class();
   test_dkdv_split();
   test_slice_plans();
+  test_visible_row_keys();
   test_div_small();
   if (failures) printf("%d checks failed\n", failures);
   else printf("index math: all checks passed\n");

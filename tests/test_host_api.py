@@ -106,6 +106,17 @@ def test_null_outputs_and_workspace_sizes():
     p2.mask_bits = None
 
 
+def test_forward_slices_are_cut_from_the_keys_that_rows_see():
+    # room for slices is asked for where a row block walks many keys, whatever the length of the key sequence
+    lib = _capi.load()
+    part = lambda **kw: (lib.acct_fa_fwd_split_workspace_bytes(ctypes.byref(_params(**kw))) - lib.acct_fa_fwd_workspace_bytes(ctypes.byref(_params(**kw))))
+    size = dict(B=1, N=1, Sq=8192, Sk=8192, D=64)
+    assert part(**size) > 0 and part(prev_block_num=32, next_block_num=32, **size) > 0
+    assert part(prev_block_num=1, next_block_num=1, **size) == 0 and part(prev_block_num=2, next_block_num=0, **size) == 0
+    long = dict(B=1, N=1, Sq=256, Sk=65536, D=128)
+    assert part(**long) > 0 and part(row_block_prefix=128, **long) == 0 and part(next_block_num=1, **long) == 0
+
+
 def test_forward_rejects_misaligned_output_and_workspace():
     # O is stored in 16-byte rows and the workspace regions are 256-byte aligned: a misaligned pointer is an error
     # code, not a misaligned vector access (checked before any device is touched)

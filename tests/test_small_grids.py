@@ -30,7 +30,7 @@ def _forward(p, q, workspace_bytes):
     (257, 257, 128, "mask", False), (130, 500, 128, "drop", False), (200, 333, 64, "row_bias", False), (96, 264, 128, "bias", False),
     (128, 400, 160, "none", False), (1, 3000, 128, "none", True), (64, 8197, 40, "none", True), (200, 6000, 128, "mask", True),
     (40, 5000, 64, "drop", True), (72, 4104, 128, "row_bias", True), (70, 4104, 80, "bias", True), (31, 5000, 160, "none", True),
-    (129, 4500, 256, "none", True), (1500, 4000, 128, "prefix", True)])
+    (129, 4500, 256, "none", True), (1500, 4000, 128, "prefix", False), (2600, 4000, 128, "prefix", True), (300, 6000, 64, "band", True), (1500, 2000, 128, "narrow", False)])
 def test_forward_of_small_grids(Sq, Sk, D, side, splits):
     B, N, g = 1, 2, torch.Generator().manual_seed(Sq * 7 + Sk)
     q, k, v = (torch.randn(B, N, S, D, generator=g).half() for S in (Sq, Sk, Sk))
@@ -46,8 +46,13 @@ def test_forward_of_small_grids(Sq, Sk, D, side, splits):
         kw.update(mask_kind=_capi.MASK_DENSE_U8, attn_mask=torch.from_numpy(m).to(DEV))
         okw.update(attn_mask=m)
     if side == "prefix":
-        kw.update(row_block_prefix=512)
-        okw.update(attn_mask=(np.arange(Sk)[None, None, :] >= ((np.arange(Sq) // 512 + 1) * 512)[None, :, None]).astype(np.uint8))
+        prefix = 1280 if splits else 512                 # (the last group of rows sees 3840 or 1536 keys: the slices are cut from those)
+        kw.update(row_block_prefix=prefix)
+        okw.update(attn_mask=(np.arange(Sk)[None, None, :] >= ((np.arange(Sq) // prefix + 1) * prefix)[None, :, None]).astype(np.uint8))
+    if side in ("band", "narrow"):                       # the slices are cut from what a row block sees: less than Sk, and not from 0
+        prev, nxt = (1, 40) if side == "band" else (2, 1)
+        kw.update(prev_block_num=prev, next_block_num=nxt)
+        okw.update(prev_block_num=prev, next_block_num=nxt)
     if side == "drop":
         d = (rng.random((B, N, Sq, Sk)) < 0.8).astype(np.uint8)
         kw.update(drop_mask=torch.from_numpy(d).to(DEV), keep_prob=0.8)
