@@ -19,6 +19,7 @@ ACCT_F16, ACCT_BF16 = 0, 1
 MASK_NONE, MASK_DENSE_U8, MASK_DENSE_F16, MASK_TILE_U8, MASK_CAUSAL, MASK_TILE_F16 = 0, 1, 2, 3, 4, 5
 _TENSOR_MASKS = (MASK_DENSE_U8, MASK_TILE_U8, MASK_DENSE_F16, MASK_TILE_F16)      # the kinds that read a tensor
 DROP_U8, DROP_F16 = 0, 1
+DROP_BITS_ONE_BAND = 0x100
 BLOCK_UNBOUNDED = 65536
 
 ERROR_NAMES = {

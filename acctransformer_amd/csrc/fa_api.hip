@@ -118,6 +118,7 @@ int mask_elem_size(const acct_fa_params* p) { return (p->mask_kind == ACCT_MASK_
 
 // counter-based dropout is on: the keep mask comes from (drop_seed, drop_offset), not from a tensor
 bool philox_on(const acct_fa_params* p) { return p->drop_philox != 0 && !p->drop_mask && p->keep_prob < 1.f; }
+int drop_kind(const acct_fa_params* p) { return p->drop_mask_kind & ~ACCT_DROP_BITS_ONE_BAND; }
 bool dropout_on(const acct_fa_params* p) { return p->drop_mask != nullptr || philox_on(p); }
 uint32_t philox_threshold(float keep_prob) {
   long t = lroundf(256.f * keep_prob);
@@ -156,8 +157,8 @@ int validate(const acct_fa_params* p, bool backward) {
   if (p->mask_stride_b < 0 || (mask_is_dense(p) && p->mask_stride_b != 0 && p->mask_stride_b < (int64_t)p->Sq * p->Sk))
     return fail(ACCT_E_SHAPE, "mask_stride_b must be 0 (broadcast) or >= Sq*Sk");
   if (mask_elem_size(p) == 2 && ((uintptr_t)p->attn_mask & 1)) return fail(ACCT_E_SHAPE, "a 2-byte attn_mask must be 2-byte aligned");
-  if (p->drop_mask_kind != ACCT_DROP_U8 && p->drop_mask_kind != ACCT_DROP_F16) return fail(ACCT_E_PARAM, "unknown drop_mask_kind %d", p->drop_mask_kind);
-  if (p->drop_mask && p->drop_mask_kind == ACCT_DROP_F16 && ((uintptr_t)p->drop_mask & 1)) return fail(ACCT_E_SHAPE, "a 2-byte drop_mask must be 2-byte aligned");
+  if (drop_kind(p) != ACCT_DROP_U8 && drop_kind(p) != ACCT_DROP_F16) return fail(ACCT_E_PARAM, "unknown drop_mask_kind %d", p->drop_mask_kind);
+  if (p->drop_mask && drop_kind(p) == ACCT_DROP_F16 && ((uintptr_t)p->drop_mask & 1)) return fail(ACCT_E_SHAPE, "a 2-byte drop_mask must be 2-byte aligned");
   if (!p->q || !p->k || !p->v) return fail(ACCT_E_NULLPTR, "q, k and v must be non-NULL");
   const int64_t* st[4] = {p->q_stride, p->k_stride, p->v_stride, p->o_stride};
   const void* ptrs[3] = {p->q, p->k, p->v};
@@ -188,7 +189,7 @@ acct::FaArgs make_args(const acct_fa_params* p) {
   a.mask = (mask_is_dense(p) || mask_is_tile(p)) ? (const uint8_t*)p->attn_mask : nullptr;
   a.mask_es = mask_elem_size(p);
   a.drop = p->keep_prob < 1.f || p->drop_mask ? (const uint8_t*)p->drop_mask : nullptr;
-  a.drop_es = p->drop_mask_kind == ACCT_DROP_F16 ? 2 : 1;
+  a.drop_es = drop_kind(p) == ACCT_DROP_F16 ? 2 : 1;
   a.alibi = p->alibi;
   a.B = p->B; a.N = p->N; a.Sq = p->Sq; a.Sk = p->Sk;
   a.hd = p->D;
@@ -228,8 +229,8 @@ acct::FaArgs make_args(const acct_fa_params* p) {
   // the kernels know one dense and one tile kind; the element size travels beside it
   a.mask_kind = mask_is_dense(p) ? (int)acct::kMaskDense : (mask_is_tile(p) ? (int)acct::kMaskTile : p->mask_kind);
   a.row_prefix = p->row_block_prefix;
-  // (a shared buffer of keep bits belongs to one attn_mask and band where there is a dense mask, else to any call)
-  a.drop_visible = !p->drop_bits || mask_is_dense(p);
+  // (a shared buffer of keep bits may be read with another band, unless the caller says that it is not)
+  a.drop_visible = !p->drop_bits || (p->drop_mask_kind & ACCT_DROP_BITS_ONE_BAND);
   return a;
 }
 

@@ -164,8 +164,8 @@ hipError_t launch_mask_tilebits(const FaArgs& a, uint32_t* out, hipStream_t st) 
 }
 
 // Key blocks whose keep bits no attention kernel reads: those that the attention mask's pre-pass classed 'skip', and
-// those that the band, the causal index compare or the row prefix leaves out for every row of the q block.  (Only
-// with `drop_visible`: a buffer of keep bits that the caller shares between calls without a dense mask holds them all.)
+// those that the band, the causal index compare or the row prefix leaves out for every row of the q block.  (Those only
+// with `drop_visible`: calls with another band may share a lent buffer of keep bits, unless the caller rules it out.)
 // `flags`: the class row of the q block, or null.
 ACCT_DEV bool keep_bits_unread(const FaArgs& a, const uint8_t* flags, int qb, int kvb) {
   if (flags && flags[kvb] == kBlkSkip) return true;

@@ -237,6 +237,8 @@ class _FlashAttentionFn(torch.autograd.Function):
         # with dropout, the keep bits the forward packs (or draws) are kept for the backward of this step
         needs_grad = any(ctx.needs_input_grad[:3])
         ctx.drop_bits = _capi.attach_drop_bits(p, q.device) if needs_grad else None
+        if ctx.drop_bits is not None:
+            p.drop_mask_kind |= _capi.DROP_BITS_ONE_BAND     # (the backward runs on these very parameters)
         o, lse = _capi.fa_fwd(p, q)
         _mask_bits_done(p)
         if ctx.drop_bits is not None:

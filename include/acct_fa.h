@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define ACCT_FA_VERSION 108
+#define ACCT_FA_VERSION 109
 
 /* error codes (0 = success) */
 #define ACCT_OK          0
@@ -64,6 +64,9 @@ extern "C" {
 #define ACCT_DROP_F16 1        /* p->dtype [B,N,Sq,Sk] of {0, 1/keep_prob}, the form the reference op takes
                                   (T/flash_attention_impl.py:48-55, T/attention.py:373-395): nonzero = keep; the
                                   scaling comes from keep_prob, which the caller still passes */
+#define ACCT_DROP_BITS_ONE_BAND 0x100   /* or'ed to drop_mask_kind by a caller that lends drop_bits (since version 109): all
+                                  calls that share the buffer have the same attn_mask, mask_kind, prev_block_num,
+                                  next_block_num and row_block_prefix, so bits that none of them reads may be left out */
 
 #define ACCT_BLOCK_UNBOUNDED 65536   /* default prev/next_block_num, L/flash_attention.py:95-96 */
 
@@ -122,9 +125,9 @@ typedef struct acct_fa_params {
      into that buffer and a call with drop_bits_filled != 0 reads what an earlier call left there.  The
      caller sets drop_bits_filled after the first call returns; the bits depend on drop_mask or on
      (drop_seed, drop_offset, keep_prob) and on B, N, Sq, Sk; with a dense attn_mask the bits of the 128x128
-     blocks that the mask hides completely, or that lie outside the band (prev_block_num, next_block_num,
-     row_block_prefix), are left out (no kernel reads them), so the buffer belongs to the calls of one step on
-     one attn_mask and one band. */
+     blocks that the mask hides completely are left out (no kernel reads them), so the buffer belongs to the
+     calls of one step on one attn_mask; with ACCT_DROP_BITS_ONE_BAND those outside the band (prev_block_num,
+     next_block_num, row_block_prefix, the causal compare) are left out as well. */
   void*    drop_bits;
   int32_t  drop_bits_filled;
   int32_t  drop_mask_kind;       /* ACCT_DROP_* (field added in version 104; 0 = the uint8 form) */
@@ -163,7 +166,8 @@ size_t acct_fa_fwd_workspace_bytes(const acct_fa_params* p);
 /* The same plus, where few query rows meet many keys (a launch that would leave most of the chip idle), room for a
  * launch that cuts the key range into slices on workgroups of their own and adds the slices' sums in a second kernel
  * (fixed order: deterministic).  A call with a workspace of this size makes use of it; with a smaller one that holds
- * acct_fa_fwd_workspace_bytes it runs the unsplit launch.  The two differ in the last bits of O and LSE. */
+ * acct_fa_fwd_workspace_bytes it runs the unsplit launch.  The two differ in the last bits of O and LSE.
+ * (Since version 109.) */
 size_t acct_fa_fwd_split_workspace_bytes(const acct_fa_params* p);
 /* Size of the optional drop_bits buffer (0 without dropout): keep bits by query row for the forward and dQ
  * kernels, then by key column for the dK/dV kernel, a quarter of a byte per score in total. */

@@ -117,6 +117,16 @@ def test_forward_slices_are_cut_from_the_keys_that_rows_see():
     assert part(**long) > 0 and part(row_block_prefix=128, **long) == 0 and part(next_block_num=1, **long) == 0
 
 
+def test_the_one_band_flag_joins_a_drop_mask_kind():
+    lib = _capi.load()
+    buf = (ctypes.c_char * 64)()
+    call = lambda kind: lib.acct_fa_fwd(ctypes.byref(_params(drop_mask_kind=kind, keep_prob=0.5)), ctypes.addressof(buf) // 16 * 16 + 16, ctypes.addressof(buf), None, 0, None)
+    for kind in (_capi.DROP_U8, _capi.DROP_F16):
+        assert call(kind) == call(kind | _capi.DROP_BITS_ONE_BAND) == -1          # (known; what is missing is the mask)
+    for kind in (2, 2 | _capi.DROP_BITS_ONE_BAND, 0x200, -1):
+        assert call(kind) == -8
+
+
 def test_forward_rejects_misaligned_output_and_workspace():
     # O is stored in 16-byte rows and the workspace regions are 256-byte aligned: a misaligned pointer is an error
     # code, not a misaligned vector access (checked before any device is touched)

@@ -80,3 +80,24 @@ def test_row_prefix_and_causal_kind_leave_out_the_same_blocks():
                                drop_mask=drop, keep_prob=phx.keep_threshold(keep) / 256.0)
         ok, ratio, mx = orc.tolerance_gate(O, o.float().cpu().numpy())
         assert ok, f"{kw}: worst ratio {ratio:.3f}, max |d| {mx:.3e}"
+
+
+@pytest.mark.parametrize("source", ["seed", "u8"])
+def test_shared_keep_bits_hold_for_another_band(source):
+    """A lent buffer that a call with a narrow band filled serves a call on the same mask with a wider one."""
+    B, N, S, D, keep = 1, 2, 400, 64, 0.7
+    g = torch.Generator().manual_seed(11)
+    q, k, v = (torch.randn(B, N, S, D, generator=g).half().to(DEV) for _ in range(3))
+    kw = dict(scale=D ** -0.5, keep_prob=keep, mask_kind=_capi.MASK_DENSE_U8, attn_mask=torch.from_numpy(_masks("random", B, S, S)).to(DEV))
+    kw.update(dict(drop_seed=77, drop_offset=2) if source == "seed" else
+              dict(drop_mask=(torch.rand(B, N, S, S, generator=g) < keep).to(torch.uint8).to(DEV)))
+    narrow, wide = _capi.make_params(q, k, v, prev_block_num=0, next_block_num=0, **kw), _capi.make_params(q, k, v, **kw)
+    own = _capi.fa_fwd(wide, q)
+    grads = _capi.fa_bwd(wide, q, k, v, own[0], q, own[1])
+    bits = _capi.attach_drop_bits(narrow, DEV)
+    bits.fill_(0xA5)
+    _capi.fa_fwd(narrow, q)
+    wide.drop_bits, wide.drop_bits_filled = narrow.drop_bits, 1
+    shared = _capi.fa_fwd(wide, q)
+    for a, b in zip(own + grads, shared + _capi.fa_bwd(wide, q, k, v, own[0], q, own[1])):
+        assert torch.equal(a, b)
