@@ -133,10 +133,11 @@ ACCT_HD double dkdv_estimate(int B, int N, int Sq, int Sk, int D, bool tri, int 
   if (ngk == 1 && dc <= 64 && n > n_cu) walk *= 0.53 / 0.65;
   double rounds = (double)(((long long)n + n_cu - 1) / n_cu);
   if (tri) {   // below the causal diagonal half of the workgroups' steps are absent, the heaviest start first
-    // (twice the CUs or a multiple of it: a heavy one and a light one each, no round left over.  32 heads, S4096, D64, 512 and
-    // 1024 workgroups: backward 280.3 us with two groups, 292.6 with one)
-    const bool pairs = (long long)n % (2 * n_cu) == 0;
-    rounds = 0.5 * n / n_cu + (pairs ? 0.1 : 0.3);
+    // (on long walks up to twice as many workgroups as CUs end together, the light ones beside the heaviest; shorter ones do
+    // not.  D64, two groups / one group: 32 heads, S4096 (512 and 1024 workgroups) backward 287 / 302 us, S3500 (448 and 896)
+    // 223 / 232, 40 heads, S3000 (480 and 960) 215 / 219; but 80 heads, S1500 (480 and 960) 133 / 128)
+    rounds = 0.5 * n / n_cu + 0.3;
+    if (steps > 80 && split == 1 && n <= 2 * n_cu && rounds > 1.06) rounds = 1.06;
     if (rounds < 1.0) rounds = 1.0;
   } else if (band.on) {   // the workgroups at the ends of the band are shorter than the rest
     const double whole = (double)(((long long)(band.whole * n) + n_cu - 1) / n_cu), r = band.share * n / n_cu + 0.3;
@@ -160,7 +161,7 @@ ACCT_HD DkdvPlan dkdv_plan(int B, int N, int Sq, int Sk, int D, bool tri, size_t
   for (int s = 1; s <= 16 && s <= (Sq + 63) / 64 && (s == 1 || n1 * s <= (tri ? 2.0 : 1.0) * n_cu); s *= 2) {
     const size_t bytes = dkdv_part_bytes(B, N, Sk, D, 1, s);
     const double t = dkdv_estimate(B, N, Sq, Sk, D, tri, 1, s, n_cu, prev_blk, next_blk);
-    if (bytes <= room && t < (banded ? 0.9 : s > 1 ? 0.95 : 0.97) * t_best) { t_best = t; best = {1, s, bytes}; }
+    if (bytes <= room && t < (banded ? 0.9 : s > 1 ? 0.95 : 1.0) * t_best) { t_best = t; best = {1, s, bytes}; }
   }
   return best;
 }

@@ -207,10 +207,10 @@ static void test_visible_row_keys() {
           }
   CHECK(visible_row_keys(8192, 8192, 1, 1, 0) == 384 && visible_row_keys(8192, 8192, 2, 0, 0) == 384, "three key blocks");
   CHECK(visible_row_keys(1000, 9000, 65536, 65536, 512) == 1024, "two groups of rows");
-  // below the diagonal, a heavy and a light unit for each CU and nothing left over: no finer ones; with a remainder: finer
-  CHECK(dkdv_plan(2, 16, 4096, 4096, 64, true, SIZE_MAX).ngk == 2 && dkdv_plan(2, 16, 3000, 3000, 64, true, SIZE_MAX).ngk == 1, "units of a triangle");
-  // two rounds against three of two thirds: too close to call
-  CHECK(dkdv_plan(4, 12, 2048, 2048, 80, false, SIZE_MAX).ngk == 2, "384 units, two rounds or three");
+  // below the diagonal on long walks, up to twice as many units as CUs end together: no finer ones
+  for (int S : {3500, 4096}) CHECK(dkdv_plan(1, 32, S, S, 64, true, SIZE_MAX).ngk == 2, "S%d", S);
+  CHECK(dkdv_plan(1, 32, 3000, 3000, 64, true, SIZE_MAX).ngk == 1 && dkdv_plan(1, 80, 1500, 1500, 64, true, SIZE_MAX).ngk == 1, "finer units");
+  CHECK(dkdv_plan(1, 64, 4096, 4096, 64, true, SIZE_MAX).ngk == 1 && dkdv_plan(1, 16, 2048, 2048, 128, true, SIZE_MAX).q_split == 1, "finer units");
   // the dK/dV units of a band: as few as fill the CUs where the band is wide, finer ones where it is narrow
   CHECK(dkdv_plan(2, 16, 2048, 2048, 128, false, SIZE_MAX, 256, 8, 0).ngk == 2, "256 workgroups of a wide band");
   CHECK(dkdv_plan(3, 16, 1500, 1500, 80, false, SIZE_MAX, 256, 5, 0).ngk == 2, "288 workgroups, those at the end shorter");
