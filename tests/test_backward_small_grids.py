@@ -1,8 +1,9 @@
 """GPU tests of the backward launches that grids below a full round take: dQ workgroups of two key groups, dK/dV
 workgroups of 128 keys (one 32-key group per wave), query ranges cut into slices that a second kernel adds up.  Sizes
 sit on the edges of the 32-, 64- and 128-row units; every launch runs with the workspace it asks for, and where
-it cuts slices with one that is too small for them.  Gate: that of the parity tests (every element within 2e-3 + 1e-3 |oracle|)."""
+it cuts slices with one that is too small for all of them and one without room for any.  Gate: that of the parity tests (every element within 2e-3 + 1e-3 |oracle|)."""
 import ctypes
+import re
 
 import numpy as np
 import pytest
@@ -13,6 +14,14 @@ from oracle import unfused_attention as orc
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+
+
+def _least_bwd_workspace(p):
+    """The smallest workspace that acct_fa_bwd accepts, from the text with which it refuses none."""
+    lib, buf = _capi.load(), (ctypes.c_char * 64)()
+    addr = ctypes.addressof(buf) // 16 * 16 + 16
+    assert lib.acct_fa_bwd(ctypes.byref(p), *([addr] * 6), None, 0, None) == -7
+    return int(re.search(r"need (\d+) bytes", lib.acct_last_error().decode()).group(1))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -54,7 +63,9 @@ def test_backward_of_small_grids(Sq, Sk, D, side, sliced, dtype):
     refs = orc.unfused_bwd(*(t.float().numpy() for t in (q, k, v, dO)), **okw, O_saved=o.float().cpu().numpy())
     first = None
     wide = dtype == torch.bfloat16
-    for size in (most, most - 256 if sliced else most):
+    least = _least_bwd_workspace(p)
+    assert (most - (least + 255) // 256 * 256 > 0) == sliced
+    for size in (most, most - 256, least) if sliced else (most,):      # all slices, fewer or none, none
         grads = _capi.fa_bwd(p, qd, kd, vd, o, dd, lse, workspace_bytes=size)
         for name, ref, got in zip(("dQ", "dK", "dV"), refs, grads):
             ok, ratio, mx = orc.tolerance_gate(ref, got.float().cpu().numpy(), atol=2e-2 if wide else 2e-3, rtol=1e-2 if wide else 1e-3)

@@ -12,6 +12,7 @@ configurations run at full size and are checked on a sample of (batch, head)
 slices plus size-independent properties.
 """
 import ctypes
+import re
 
 import numpy as np
 import pytest
@@ -57,6 +58,14 @@ def _run(q, k, v, dO=None, *, scale, mask_kind=_capi.MASK_NONE, attn_mask=None, 
         grads = _capi.fa_bwd(p, qd, kd, vd, o, dev(dO), lse)
     torch.cuda.synchronize()
     return o, lse, grads
+
+
+def _least_bwd_workspace(p):
+    """The smallest workspace that acct_fa_bwd accepts, from the text with which it refuses none."""
+    lib, buf = _capi.load(), (ctypes.c_char * 64)()
+    addr = ctypes.addressof(buf) // 16 * 16 + 16
+    assert lib.acct_fa_bwd(ctypes.byref(p), *([addr] * 6), None, 0, None) == -7
+    return int(re.search(r"need (\d+) bytes", lib.acct_last_error().decode()).group(1))
 
 
 def _gate(ref, got, atol=ATOL, rtol=RTOL, what=""):
@@ -387,13 +396,17 @@ def test_block_band(prev, nxt):
     _check_all(q, k, v, dO, okw, _run(q, k, v, dO, scale=D ** -0.5, prev=prev, nxt=nxt))
 
 
+DQ64_BLOCKS = 264                                        # 256-row blocks of the tests below: every CU has one
+DQ64_SHAPES = [(256, 64, False), (256, 192, False), (512, 512, True), (768, 320, True), (512, 1024, True), (256, 64, True), (1024, 2048, False)]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("Sq, Sk, causal", [(256, 64, False), (256, 192, False), (512, 512, True), (768, 320, True),
-                                            (512, 1024, True), (256, 64, True), (1024, 2048, False)])
+@pytest.mark.parametrize("Sq, Sk, causal", DQ64_SHAPES)
 def test_dq_kernel_with_64_rows_per_wave(dtype, Sq, Sk, causal):
     # shapes the hand-scheduled dQ kernel takes (head dim 128, 256-row query blocks, 64-key tiles, no side
-    # inputs): one tile, an odd tile count, diagonals that end inside and past the keys, rows past the last key
-    B, N, D = 2, 3, 128
+    # inputs): one tile, an odd tile count, diagonals that end inside and past the keys, rows past the last key.
+    # At least 256 workgroups of 256 rows: fewer heads run on workgroups of key groups instead
+    B, N, D = 4, DQ64_BLOCKS // (4 * (Sq // 256)), 128
     q, dO = (_gen((B, N, Sq, D), s, dtype) for s in (301, 304))
     k, v = (_gen((B, N, Sk, D), s, dtype) for s in (302, 303))
     okw = dict(scale=D ** -0.5)
@@ -402,11 +415,14 @@ def test_dq_kernel_with_64_rows_per_wave(dtype, Sq, Sk, causal):
         okw.update(attn_mask=np.triu(np.ones((1, Sq, Sk), np.uint8), 1))
         kw.update(mask_kind=_capi.MASK_CAUSAL)
     tol = (ATOL, RTOL) if dtype == torch.float16 else (ATOL_BF16, RTOL_BF16)
-    _check_all(q, k, v, dO, okw, _run(q, k, v, dO, scale=D ** -0.5, **kw), *tol)
+    o, lse, g = _run(q, k, v, dO, scale=D ** -0.5, **kw)
+    for b, h in _sample_heads(B, N, n=5, seed=Sq + Sk):
+        sl = (slice(b, b + 1), slice(h, h + 1))
+        _check_all(q[sl], k[sl], v[sl], dO[sl], okw, (o[sl], lse[sl], tuple(t[sl] for t in g)), *tol)
 
 
 def test_dq_kernel_with_64_rows_per_wave_on_bsnd_views():
-    B, N, S, D = 2, 4, 512, 128
+    B, N, S, D = 4, DQ64_BLOCKS // (4 * 2), 512, 128
     store = [_gen((B, S, N, D), s).to(DEV) for s in (311, 312, 313, 314)]
     q, k, v, dO = (t.permute(0, 2, 1, 3) for t in store)
     tri = np.triu(np.ones((1, S, S), np.uint8), 1)
@@ -414,7 +430,9 @@ def test_dq_kernel_with_64_rows_per_wave_on_bsnd_views():
     o, lse = _capi.fa_fwd(p, q)
     grads = _capi.fa_bwd(p, q, k, v, o, dO.contiguous(), lse)
     torch.cuda.synchronize()
-    _check_all(q.cpu(), k.cpu(), v.cpu(), dO.cpu(), dict(scale=D ** -0.5, attn_mask=tri), (o, lse, grads))
+    for b, h in _sample_heads(B, N, n=5, seed=315):
+        sl = (slice(b, b + 1), slice(h, h + 1))
+        _check_all(q[sl].cpu(), k[sl].cpu(), v[sl].cpu(), dO[sl].cpu(), dict(scale=D ** -0.5, attn_mask=tri), (o[sl], lse[sl], tuple(t[sl] for t in grads)))
 
 
 @pytest.mark.parametrize("D", [64, 80])
@@ -872,15 +890,16 @@ def test_dkdv_query_split_against_oracle_and_unsplit_launch(D, Sq, Sk, side):
     o, lse = _capi.fa_fwd(p, qd)
     full = lib.acct_fa_bwd_workspace_bytes(ctypes.byref(p))
     g_split = _capi.fa_bwd(p, qd, kd, vd, o, dO.to(DEV), lse)
-    # the slices' sums are the last part of the workspace, well over 256 bytes: a workspace that is 256 bytes
-    # short cannot hold them, and the launch is not split
-    stats = 2 * ((B * N * Sq * 4 + 255) // 256 * 256)
-    assert full - stats >= (1 << 20), "this shape is expected to split its dK/dV launch"
-    g_plain = _capi.fa_bwd(p, qd, kd, vd, o, dO.to(DEV), lse, workspace_bytes=full - 256)
+    # the slices' sums are the last part of the workspace: the least that is accepted has no room for any
+    least = _least_bwd_workspace(p)
+    assert full - least >= (1 << 20), "this shape is expected to split its dK/dV launch"
+    g_plain = _capi.fa_bwd(p, qd, kd, vd, o, dO.to(DEV), lse, workspace_bytes=least)
+    g_fewer = _capi.fa_bwd(p, qd, kd, vd, o, dO.to(DEV), lse, workspace_bytes=full - 256)      # (fewer slices, or none)
     torch.cuda.synchronize()
-    assert torch.equal(g_split[0], g_plain[0])
+    assert torch.equal(g_split[0], g_plain[0]) and torch.equal(g_split[0], g_fewer[0])
     _check_all(q, k, v, dO, okw, (o, lse, g_split))
     _check_all(q, k, v, dO, okw, (o, lse, g_plain))
+    _check_all(q, k, v, dO, okw, (o, lse, g_fewer))
 
 
 def _random_case(rng):
@@ -1014,6 +1033,37 @@ def test_one_to_fifteen_keys_with_side_inputs(D):
             _gate(dK, grads[1], atol=wide, what=what + " dK")
             _gate(dV, grads[2], atol=wide, what=what + " dV")
             n += 1
+
+
+FULL_GRIDS = [(40, 512, 512, "none"), (40, 500, 500, "dense"), (40, 505, 250, "drop"), (40, 490, 250, "none"), (40, 512, 512, "causal"),
+              (160, 490, 77, "none"), (160, 505, 333, "dense"), (160, 500, 500, "drop"), (256, 300, 333, "dense")]
+FULL_GRID_HEADS = (8, 32)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D, Sq, Sk, side", FULL_GRIDS)
+def test_head_dims_without_bias_variants_on_full_grids(D, Sq, Sk, side, dtype):
+    # head dims 40, 160 and 256 at sizes that fill the chip: the forward without key groups, the dQ kernel without them and
+    # (D 40) the dK/dV kernel with two key groups per wave, on sampled heads
+    B, N = FULL_GRID_HEADS
+    q, dO = (_gen((B, N, Sq, D), s, dtype) for s in (951, 954))
+    k, v = (_gen((B, N, Sk, D), s, dtype) for s in (952, 953))
+    rng = np.random.default_rng(Sk + D)
+    kw, okw = dict(scale=D ** -0.5), dict(scale=D ** -0.5)
+    if side == "causal":
+        kw.update(mask_kind=_capi.MASK_CAUSAL); okw.update(attn_mask=np.triu(np.ones((1, Sq, Sk), np.uint8), 1))
+    if side == "dense":
+        m = (rng.random((1, Sq, Sk)) < 0.3).astype(np.uint8); m[:, :, 0] = 0
+        kw.update(mask_kind=_capi.MASK_DENSE_U8, attn_mask=m); okw.update(attn_mask=m)
+    if side == "drop":
+        kw.update(keep_prob=0.8, drop_seed=9 << 33, drop_offset=D)
+    tol = (ATOL, RTOL) if dtype == torch.float16 else (ATOL_BF16, RTOL_BF16)
+    o, lse, g = _run(q, k, v, dO, **kw)
+    keep = phx.dropout_keep_mask(B, N, Sq, Sk, 9 << 33, D, 0.8) if side == "drop" else None
+    for b, h in _sample_heads(B, N, n=2, seed=Sq):
+        sl = (slice(b, b + 1), slice(h, h + 1))
+        ok1 = dict(okw, drop_mask=keep[sl], keep_prob=phx.keep_threshold(0.8) / 256.0) if side == "drop" else okw
+        _check_all(q[sl], k[sl], v[sl], dO[sl], ok1, (o[sl], lse[sl], tuple(t[sl] for t in g)), *tol, saved_o=True)
 
 
 @pytest.mark.parametrize("block", range(3))

@@ -16,3 +16,24 @@ def test_index_math_host_build(tmp_path):
     sys.stdout.write(res.stdout)
     assert res.returncode == 0, res.stdout[-2000:]
     assert "all checks passed" in res.stdout
+
+
+def _plans(tmp_path, problems):
+    src, exe = os.path.join(ROOT, "tests", "host", "launch_plan.cpp"), str(tmp_path / "launch_plan")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-o", exe, src], check=True)
+    text = "\n".join(" ".join(str(int(x)) for x in p) for p in problems)
+    out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True, timeout=60).stdout
+    return [dict(zip(("kg", "kv_split", "dq_kg", "ngk", "q_split"), map(int, line.split()))) for line in out.splitlines()]
+
+
+def test_the_gpu_tests_of_one_kernel_run_it(tmp_path):
+    """The launch plan decides which kernel a shape reaches: the parity tests written for a kernel are large enough."""
+    import test_gpu_parity as gpu
+    rows = [(4, gpu.DQ64_BLOCKS // (4 * (Sq // 256)), Sq, Sk, 128, causal) for Sq, Sk, causal in gpu.DQ64_SHAPES]
+    for row, plan in zip(rows, _plans(tmp_path, rows)):
+        assert plan["dq_kg"] == 1, (row, plan)
+    rows = [gpu.FULL_GRID_HEADS + (Sq, Sk, D, side == "causal") for D, Sq, Sk, side in gpu.FULL_GRIDS]
+    plans = _plans(tmp_path, rows)
+    for row, plan in zip(rows, plans):
+        assert (plan["kg"], plan["kv_split"], plan["dq_kg"], plan["q_split"]) == (1, 1, 1, 1), (row, plan)
+    assert sum(plan["ngk"] == 2 for row, plan in zip(rows, plans) if row[4] == 40) >= 3, plans
