@@ -314,7 +314,7 @@ def fa_fwd(p, q):
 def fa_bwd(p, q, k, v, o, do, lse, workspace_bytes=None):
     """Run acct_fa_bwd; returns (dQ, dK, dV) laid out like q, k, v.  `workspace_bytes`: the size of the
     workspace to pass instead of acct_fa_bwd_workspace_bytes (a smaller one that still holds the required
-    parts makes the library run the dK/dV kernel without splitting the query range)."""
+    parts makes the library cut the query range of the dK/dV kernel into the slices that fit, or not at all)."""
     lib = load()
     if not q.is_cuda:
         raise RuntimeError("acct_fa_bwd needs device tensors (there is no CPU path)")

@@ -348,7 +348,7 @@ size_t acct_fa_bwd_workspace_bytes(const acct_fa_params* p) {
   if (!p || p->B <= 0 || p->N <= 0 || p->Sq <= 0) return 0;
   if (p->Sk <= 0 || p->D <= 0) return 0;
   // plus room for the per-slice sums of a dK/dV launch that splits the query range (few heads, short key
-  // sequence); a caller that passes less gets the unsplit launch
+  // sequence); a caller that passes less gets a launch with the slices that fit, or without
   return align_up(bwd_min_workspace_bytes(p), 256) + plan_dkdv(p, SIZE_MAX, 256).part_bytes;
 }
 

@@ -591,14 +591,14 @@ __global__ void __launch_bounds__(256) fa_bwd_dkdv_reduce_kernel(const FaArgs a,
 }
 
 // ============================================================================
-// dK/dV kernel: kv-tile owner, 8 waves in 4 pairs.  A pair owns 64 key rows.
+// dK/dV kernel: kv-tile owner, 8 waves in 4 pairs.  A pair owns 32 NGK key rows.
 // Its first wave (V role) keeps the K fragments of those rows in registers,
 // recomputes S = Q K^T and P, hands P (fp16) to its partner through LDS and
 // accumulates dV^T += dO^T P.  The partner (K role) keeps the V fragments,
 // computes dP = dO V^T, forms dS = P*(dP - D) and accumulates dK^T += Q^T dS.
 // Splitting the two accumulators over two waves halves the registers per wave
 // (two waves fit on each SIMD and overlap each other's MFMA and exp/convert
-// phases) while every Q / dO fragment read from LDS still feeds two MFMAs.
+// phases) while every Q / dO fragment read from LDS still feeds NGK MFMAs.
 // ============================================================================
 constexpr int kPark = 6;        // stationary fragments parked in LDS per wave (D = 128)
 constexpr int kParkHot = 4;     // the variant without side inputs has registers for two more fragments
@@ -620,7 +620,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
   constexpr int BNK = 4 * WK;                       // key rows per workgroup
   constexpr int TILEB = 64 * C::PITCH;
   constexpr int STATB = 2 * 64 * 4;                 // -LSE*log2(e) and D of the 64 rows of a tile
-  constexpr int DROPB = DROP ? 2048 : 0;            // keep bits of the tile's 64 rows for the workgroup's 256 keys: [key][2 chunks] words
+  constexpr int DROPB = DROP ? 2048 : 0;            // keep bits of the tile's 64 rows for 256 keys (NGK = 1 reads the first 128): [key][2 chunks] words
   constexpr int STAGEB = 2 * TILEB + STATB + DROPB; // one buffer: Q tile | dO tile | -LSE*log2(e) | D | keep bits
   constexpr int PXB = 2048 * NGK;                   // P of one pair and chunk: 64 lanes x 32 bytes per key group
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -683,7 +683,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
     }
   }
 
-  // stationary B operands: K fragments (V role) or V fragments (K role) of the pair's 64 key rows;
+  // stationary B operands: K fragments (V role) or V fragments (K role) of the pair's key rows;
   // lane holds key row 32 gk + l32, d = 16t + 8g ..
   // The last PARK k-steps of the second key group live in a wave-private LDS slab instead of
   // registers (16 VGPRs at D = 128): that is what lets two waves share a SIMD without spilling.

@@ -127,6 +127,8 @@ def run_other_configs(args, lib, dev, st, stream, g, D, scale, check, only):
         # the same step reads (drop_bits / drop_bits_filled of the C ABI), as the Python operator does; the same
         # for what the pre-pass derives from a mask tensor (mask_bits): once per step, in the forward call
         bits = _capi.attach_drop_bits(pp, dev)
+        if bits is not None:
+            pp.drop_mask_kind |= _capi.DROP_BITS_ONE_BAND
         mbits = _capi.attach_mask_bits(pp, dev)
         nw = max(lib.acct_fa_bwd_workspace_bytes(P(pp)), lib.acct_fa_fwd_workspace_bytes(P(pp)), 256)
         w = torch.empty(nw, dtype=torch.uint8, device=dev)

@@ -187,8 +187,9 @@ int acct_fa_bwd(const acct_fa_params* p, const void* O, const void* dO, const fl
 /* Workspace of the backward, 256-byte aligned.  With few heads and a short key sequence (cross attention on 77
  * keys: a handful of key tiles for 256 CUs) the size includes room for a dK/dV launch that cuts the query range
  * into slices on workgroups of their own and adds the slices' sums in a second kernel (fixed order: still
- * deterministic).  A smaller workspace that still holds everything else is accepted and runs the unsplit launch;
- * the two launches differ in the last bits of dK and dV (another order of summation). */
+ * deterministic).  A smaller workspace that still holds everything else is accepted: the launch then takes as many
+ * slices as there is room for, none if there is room for none.  Launches with different numbers of slices differ in
+ * the last bits of dK and dV (another order of summation). */
 size_t acct_fa_bwd_workspace_bytes(const acct_fa_params* p);
 
 /* The two halves of acct_fa_bwd, for callers that need one side of the gradient
