@@ -638,11 +638,13 @@ __global__ void __launch_bounds__(256) fa_fwd_combine_kernel(const FaArgs a, int
     for (int e = 0; e < 4; e++) o[e] *= al;
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      if (s0 + 4 * u >= a.kv_split) break;                                  // (weight 0 would turn an infinity of V into NaN)
-      const float w = fast_exp2((ml[u][0] - m) * cmul);
+      // (selects on values that are loaded in any case: a branch around each slice serialised the eight loads, 12.2 us
+      // instead of 7 for 256 queries x 131072 keys; a weight of 0 alone would turn an infinity of V into NaN)
+      const bool in = s0 + 4 * u < a.kv_split;
+      const float w = in ? fast_exp2((ml[u][0] - m) * cmul) : 0.f;
       l = __builtin_fmaf(ml[u][1], w, l);
 #pragma unroll
-      for (int e = 0; e < 4; e++) o[e] = __builtin_fmaf(v[u][e], w, o[e]);
+      for (int e = 0; e < 4; e++) o[e] = __builtin_fmaf(in ? v[u][e] : 0.f, w, o[e]);
     }
   }
   if (wave > 0) {
