@@ -260,7 +260,7 @@ ACCT_DEV u32x4 load_once(const uint8_t* p) { return __builtin_nontemporal_load(r
 // is needed) 274.7 -> 185.1 us.  Neighbouring blocks share the lines of the row words and of each mask row's pages:
 // each XCD takes one contiguous eighth of them, and the mask, read once, does not displace anything in the caches:
 // 155.5 us with the first alone, 175.1 with the second alone, 142.3 = 4.2 TB/s with both; S3001, 3 x 8 heads 83.9 ->
-// 82.0, S1024 12.6 -> 11.8.  (The Philox kernel below reads nothing, and an eighth of its blocks each evens out less
+// 82 to 86, S1024 12.6 -> 11.1 to 11.8 over the runs seen.  (The Philox kernel below reads nothing, and an eighth of its blocks each evens out less
 // well: 46.5 -> 48.8 on a padded batch, so it takes them in order.)
 template <int ES>
 __global__ void __launch_bounds__(256) fa_drop_bits_kernel(const FaArgs a, uint32_t* rowbits, uint32_t* colbits) {
