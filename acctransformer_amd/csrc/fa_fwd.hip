@@ -638,8 +638,8 @@ __global__ void __launch_bounds__(256) fa_fwd_combine_kernel(const FaArgs a, int
     l *= al;
 #pragma unroll
     for (int e = 0; e < 4; e++) o[e] *= al;
-    // (eight whole slices need no test: 6.3 us for 256 queries x 131072 keys, 7.3 with it.  Fewer: selects on values that are loaded in any case -- a branch around each slice
-    // serialised the loads, 12.2 us, and a weight of 0 alone would turn an
+    // (eight whole slices need no test: 6.3 us for 256 queries x 131072 keys, 7.3 with it.  Fewer: selects on values that are
+    // loaded in any case -- a branch around each slice serialised the loads, 12.2 us, and a weight of 0 alone would turn an
     // infinity of V into NaN)
     auto add = [&](auto some) {
 #pragma unroll
