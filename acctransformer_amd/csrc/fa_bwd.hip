@@ -40,7 +40,7 @@ ACCT_DEV typename Elem<T>::V8 pack8(const float* x) {
 // KG = 2 (grids that leave CUs idle): the waves form NW / 2 row groups times two key groups, one 32-key chunk of every
 // tile each; the key groups' sums meet in LDS before the epilogue -- twice as many workgroups for the same rows.
 template <int D, int RG> constexpr int dq_merge_at() { return RG * 32 * (SwzCfg<D>::DB * 64 + 16); }   // behind the epilogue's staging
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KG = 1>
+template <typename T, int D, int QG, int NW, int BIAS, bool DROP, bool MASKT, int KG = 1>
 ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
   static_assert(KG == 1 || (KG == 2 && QG == 1 && NW % 2 == 0), "two key groups of one 32-key chunk each");
   constexpr int CW = 2 / KG, WN = 32 * CW;                // 32-key chunks and keys of a tile that one wave works on
@@ -51,7 +51,12 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
   constexpr int BM = 32 * QG * RG;
   constexpr int TILEB = 64 * C::PITCH;
   constexpr int FRING = 4, TRING = 3;                     // fragment reads in flight ahead of their MFMA (row-major / transposed)
-  constexpr bool RINGS = !(BIAS || DROP);                 // (the side-input variants have no registers for the rings)
+  constexpr bool TBIAS = BIAS == kBiasAny, RBIAS = BIAS == kBiasKey;
+  constexpr bool RINGS = !(TBIAS || DROP);                // (the side-input variants have no registers for the rings)
+  // Products ahead of the other wave's vector work, by wave priority, where a tile's products outlast it: 64 heads, 2048 x 2048
+  // causal, D128 121 -> 114 us, 4096 x 4096 429 -> 402, bf16 116 -> 110; D64 113 -> 114, D40 97 -> 100.  (The variants without the
+  // rings have no register left for the order it brings: with dropout eight more spills, 239 -> 320 us.)
+  constexpr bool DQPRIO = D == 128 && RINGS;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   ACCT_LDS char* smem = (ACCT_LDS char*)smem_raw;   // [2 buffers][K tile | V tile]; reused by the epilogue
 
@@ -135,8 +140,8 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
       // (minus p_shift: the recomputed probabilities carry a factor 2^p_shift, see FaArgs)
       lq[gq] = a.lse[(int64_t)bh * a.Sq + row] * kLog2e - a.p_shift;
       if (g == 0 && kg == 0) {
-        a.delta[(int64_t)bh * a.Sq + row] = dl[gq];
-        a.nlse[(int64_t)bh * a.Sq + row] = -lq[gq];        // p_shift - LSE*log2(e): the exp2 offset the dK/dV kernel adds
+        a.delta[(int64_t)bh * a.Sq + row] = -dl[gq];
+        a.nlse[(int64_t)bh * a.Sq + row] = -lq[gq] * a.inv_scale_log2e;
       }
     }
   }
@@ -166,7 +171,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
   const int mb = a.mask_sb ? b : 0;
   const uint8_t* maskp = a.mask ? a.mask + (a.mask_kind == kMaskDense ? (int64_t)mb * a.mask_sb * a.mask_es : 0) : nullptr;
   const T* alibip = BIAS ? (const T*)a.alibi + b * a.al_sb + h * a.al_sh : nullptr;
-  const bool alibi_vec = BIAS && (((uintptr_t)a.alibi & 7) | ((a.al_sb | a.al_sh | a.al_sq) & 3)) == 0;
+  const bool alibi_vec = TBIAS && (((uintptr_t)a.alibi & 7) | ((a.al_sb | a.al_sh | a.al_sq) & 3)) == 0;
 
   TileDma<T, D, 64, NW> kdma, vdma;
   const int cpr = a.hd >> 3;                                // valid 16-byte chunks per row
@@ -174,14 +179,21 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
   vdma.plan(a.v_ss, cpr);
   // bias tiles of this wave's rows are staged through a wave-private LDS region one tile ahead
   ACCT_LDS char* bias_lds = smem + 4 * TILEB + wave * (QG * 4096);
-  const bool bias_staged = BIAS && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh | a.al_sq) & 7)) == 0;
-  const bool row_bias = BIAS && a.al_sq == 0;            // the bias depends on the key only: one 128-byte row per tile
+  const bool bias_staged = RBIAS || (TBIAS && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh | a.al_sq) & 7)) == 0);
+  const bool row_bias = RBIAS || (TBIAS && a.al_sq == 0);           // the bias depends on the key only: one 128-byte row per tile
   auto stage_bias = [&](int jn) {
 #pragma unroll
     for (int gq = 0; gq < QG; gq++) {
       if (row_bias) bias_row_dma<T>(alibip, jn * 64, a.Sk, bias_lds + gq * 4096);
       else bias_tile_dma<T>(alibip, a.al_sq, wq0 + 32 * gq, a.Sq, jn * 64, a.Sk, bias_lds + gq * 4096);
     }
+  };
+  // A key-only bias (kBiasKey) becomes float32 / scale in the wave's region, 128 keys' dwords after the staged row, once
+  // per tile and wave, and is the C operand of the first product from there: nothing per score.
+  auto convert_bias = [&]() {
+    const typename E::V2 v = *reinterpret_cast<const ACCT_LDS typename E::V2*>(bias_lds + lane * 4);
+    const f32x2 f = {(float)v[0] * a.inv_scale, (float)v[1] * a.inv_scale};
+    *reinterpret_cast<ACCT_LDS f32x2*>(bias_lds + 256 + lane * 8) = f;
   };
   // keep bits of this wave's rows and one tile, staged with the tile's DMA (double buffered)
   using DropStage = DropRowStage<DROP, QG, 2>;
@@ -194,6 +206,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
     // A full wait the compiler can see: every load issued so far (Q, dO fragments included) is complete,
     // so it places no vmcnt wait inside the loop -- such a wait would also stall on the next tile's DMA.
     __builtin_amdgcn_s_waitcnt(0);
+    if (RBIAS) convert_bias();
     __syncthreads();
 
     // block classes of a dense mask: 64 blocks at a time into scalar registers
@@ -214,6 +227,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
           tile_dma<T, D, 64, NW>(vp, a.v_ss, (j + 1) * 64, a.Sk, nb + TILEB, a.hd >> 3);
         }
         DropStage::issue(a, bh, wq0, j + 1, lane, drop_lds + (buf ^ 1) * DropStage::BYTES);
+        if (RBIAS && wq0 < a.Sq) stage_bias(j + 1);       // (the staged row was converted before this step)
       }
       const int kv0 = j * 64 + kg * WN;                     // this wave's first key of the tile
       const int kvb = j >> 1;
@@ -251,7 +265,14 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
           f32x16 s[QG], dp[QG];
 #pragma unroll
           for (int gq = 0; gq < QG; gq++) {
-            if (BIAS && bias_staged) {
+            if (RBIAS) {
+#pragma unroll
+              for (int r4 = 0; r4 < 4; r4++) {
+                const f32x4 v = *reinterpret_cast<const ACCT_LDS f32x4*>(bias_lds + 256 + (32 * ct + 8 * r4 + 4 * g) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) s[gq][4 * r4 + e] = v[e];
+              }
+            } else if (TBIAS && bias_staged) {
               // the bias enters as the initial value of the score accumulators (bias / scale, the MFMAs add
               // q.k): nothing per score afterwards, no bias registers alive next to the scores
               typename E::V4 bv[4];
@@ -272,6 +293,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
             // barriers keep the compiler from folding the ring back into read-wait-MFMA.
             constexpr int NF = 2 * C::KS;
             auto faddr = [&](int i) { return ((i & 1) ? vw : kw) + koff(i >> 1) + c * 32 * C::PITCH; };
+            if (DQPRIO) __builtin_amdgcn_s_setprio(1);
             V8 ring[FRING];
 #pragma unroll
             for (int i = 0; i < FRING; i++) ring[i] = lds_read_frag<T>(faddr(i));
@@ -287,6 +309,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
               if (i + FRING < NF) ring[i % FRING] = lds_read_frag<T>(faddr(i + FRING));
             }
             __builtin_amdgcn_sched_barrier(0);
+            if (DQPRIO) __builtin_amdgcn_s_setprio(0);
           } else {
             V8 kf[C::KS], vf[C::KS];
 #pragma unroll
@@ -302,7 +325,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
 #pragma unroll
               for (int gq = 0; gq < QG; gq++) dp[gq] = E::mfma(vf[t], dof[gq][t], dp[gq]);
           }
-          if (BIAS && bias_staged && c == CW - 1) {
+          if (TBIAS && bias_staged && c == CW - 1) {
             // this wave's part of the bias tile has been read and the reads consumed: its LDS region can take the next
             // tile, which has the rest of this step to land (the end-of-step wait covers it)
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -314,7 +337,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
             const int qrow = wq0 + 32 * gq + l32;
             const int qrow_c = min(qrow, a.Sq - 1);
             float ds[16];
-            const bool bias_pending = BIAS && !bias_staged;  // (a staged bias is already inside s)
+            const bool bias_pending = TBIAS && !bias_staged;  // (a staged bias is already inside s)
             if (!edge && !bias_pending && !DROP) {           // interior tile: no side inputs at all
 #pragma unroll
               for (int r = 0; r < 16; r++) {
@@ -337,7 +360,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
               float x[16];
 #pragma unroll
               for (int r = 0; r < 16; r++) x[r] = __builtin_fmaf(s[gq][r], a.scale_log2e, -lq[gq]);
-              if (BIAS && !bias_staged) {                    // a bias the DMA cannot stage (alignment): direct loads
+              if (TBIAS && !bias_staged) {                   // a bias the DMA cannot stage (alignment): direct loads
 #pragma unroll
                 for (int r4 = 0; r4 < 4; r4++) {
                   float bias[4];
@@ -386,6 +409,7 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
           }
         }
         // ---- dQ^T += K^T dS^T : transposed K fragments through a ring of TRING register sets ----
+        if (DQPRIO) __builtin_amdgcn_s_setprio(1);
         if constexpr (RINGS) {
           constexpr int NT = 2 * CW * C::DB;
           auto tread = [&](int i) {
@@ -418,10 +442,12 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
                 for (int gq = 0; gq < QG; gq++) acc[gq][db] = E::mfma(ktf, dsf[gq][c][hh], acc[gq][db]);
               }
         }
-      } else if (BIAS && bias_staged && j < j_hi && wq0 < a.Sq) {
+        if (DQPRIO) __builtin_amdgcn_s_setprio(0);
+      } else if (TBIAS && bias_staged && j < j_hi && wq0 < a.Sq) {
         stage_bias(j + 1);                                  // nothing to read in this step: the region is free
       }
       dma_wait();
+      if (RBIAS && j < j_hi) convert_bias();
       __syncthreads();
     }
   }
@@ -484,9 +510,13 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
 // The variant that knows mask tensors but neither a bias nor dropout carries a second body: a workgroup whose
 // rows see nothing but the causal pattern in a dense mask (block classes: clean before the diagonal, the
 // causal diagonal, skipped after it) runs the code of the variant without side inputs, by index compare.
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KG>
+template <typename T, int D, int QG, int NW, int BIAS, bool DROP, bool MASKT, int KG>
 __global__ void __launch_bounds__(64 * NW) fa_bwd_dq_kernel(const FaArgs a) {
-  if constexpr (MASKT && !BIAS && !DROP) {
+  if constexpr (MASKT && BIAS != kBiasAny && !DROP) {
+    if (BIAS && a.mask_kind != kMaskDense && a.mask_kind != kMaskTile) {
+      fa_bwd_dq_body<T, D, QG, NW, BIAS, false, false, KG>(a);
+      return;
+    }
     if (a.mask_kind == kMaskDense) {
       constexpr int BM = 32 * QG * NW / KG;
       int bh, rank;
@@ -498,7 +528,7 @@ __global__ void __launch_bounds__(64 * NW) fa_bwd_dq_kernel(const FaArgs a) {
       if (dense_lines_are_causal(fl, 1, a.Tc, qb_lo, qb_hi - qb_lo + 1, kvb_lo, kvb_hi, false, a, threadIdx.x & 63)) {
         FaArgs c = a;
         c.mask_kind = kMaskCausal;
-        fa_bwd_dq_body<T, D, QG, NW, false, false, false, KG>(c);
+        fa_bwd_dq_body<T, D, QG, NW, BIAS, false, false, KG>(c);
         return;
       }
     }
@@ -603,18 +633,19 @@ __global__ void __launch_bounds__(256) fa_bwd_dkdv_reduce_kernel(const FaArgs a,
 constexpr int kPark = 6;        // stationary fragments parked in LDS per wave (D = 128)
 constexpr int kParkHot = 4;     // the variant without side inputs has registers for two more fragments
 // stationary fragments parked in LDS per wave: the bias variants give one up for the bias tiles' LDS
-template <int D, bool BIAS, bool MASKT, int NGK>
-constexpr int dkdv_park() { return D == 128 && NGK == 2 ? (BIAS ? kPark - 1 : (MASKT ? kPark : kParkHot)) : 0; }
+template <int D, bool TBIAS, bool MASKT, int NGK>
+constexpr int dkdv_park() { return D == 128 && NGK == 2 ? (TBIAS ? kPark - 1 : (MASKT ? kPark : kParkHot)) : 0; }
 
 // MASKT = false compiles the mask-tensor handling out (no mask, or the causal mask by index compare):
 // the hot variant must not carry that code's register pressure.
 // NGK: key groups of 32 rows per wave.  One where head dims above 128 leave registers for the accumulators of one only,
 // and in grids that two would leave half empty (DkdvPlan).
-template <typename T, int D, bool BIAS, bool DROP, bool MASKT, int NGK>
+template <typename T, int D, int BIAS, bool DROP, bool MASKT, int NGK>
 ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
   using E = Elem<T>;
   using V8 = typename E::V8;
   using C = SwzCfg<D>;
+  constexpr bool TBIAS = BIAS == kBiasAny;           // may be a tile per wave; a key-only bias is a value per lane
   constexpr int NW = 8;
   constexpr int WK = 32 * NGK;                      // key rows per wave pair
   constexpr int BNK = 4 * WK;                       // key rows per workgroup
@@ -668,7 +699,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
     const uint8_t* fl = a.blkflags + ((int64_t)(a.mask_sb ? b : 0) * a.Tr) * a.Tc;
     int b_lo = i_lo >> 1, b_hi = i_hi >> 1;
     // (the bias variants have no register to spare for the key tails: they read such blocks through the bitmaps)
-    const uint8_t* tails = (!BIAS && a.blktail) ? a.blktail + ((int64_t)(a.mask_sb ? b : 0) * a.Tr) * a.Tc : nullptr;
+    const uint8_t* tails = (!TBIAS && a.blktail) ? a.blktail + ((int64_t)(a.mask_sb ? b : 0) * a.Tr) * a.Tc : nullptr;
     if (i_lo <= i_hi && flwin.init_trimmed(fl, a.Tc, 1, kb_lo, kb_hi - kb_lo + 1, min(wkb, kb_hi), b_lo, b_hi, lane, tails)) {
       i_lo = max(i_lo, b_lo * 2);
       i_hi = min(i_hi, b_hi * 2 + 1);
@@ -687,7 +718,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
   // lane holds key row 32 gk + l32, d = 16t + 8g ..
   // The last PARK k-steps of the second key group live in a wave-private LDS slab instead of
   // registers (16 VGPRs at D = 128): that is what lets two waves share a SIMD without spilling.
-  constexpr int PARK = dkdv_park<D, BIAS, MASKT, NGK>();
+  constexpr int PARK = dkdv_park<D, TBIAS, MASKT, NGK>();
   V8 bf[NGK][C::KS];
   ACCT_LDS char* park = pexch + 8 * PXB + wave * (PARK * 1024) + lane * 16;
   // bias tile (32 query rows x the pair's 64 keys) of the V-role wave, staged one chunk ahead by DMA
@@ -753,15 +784,55 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
     }
   };
 
+  // The tiles after the first one are whole (the walk goes down from the last), so what a lane adds to the tile's base is
+  // the same for all of them.  It waits in LDS, where the variants without a bias have 8 KB left: derived anew it cost
+  // every second step some 550 cycles before its first product, and no register is free for it.
+  constexpr bool KEEP_VOFF = D <= 128 && !TBIAS;
+  constexpr int NV = TileDma<T, D, 64, NW>::NV;
+  ACCT_LDS char* voff_lds = pexch + 8 * PXB + 8 * (PARK * 1024) + wave * (NV * 512) + lane * (NV * 8);
+  auto plan_stage = [&]() {
+    TileDma<T, D, 64, NW> qd, dd;
+    qd.plan(a.q_ss, a.hd >> 3);
+    dd.plan(a.o_ss, a.hd >> 3);
+#pragma unroll
+    for (int t = 0; t < NV; t++) {
+      *reinterpret_cast<ACCT_LDS uint32_t*>(voff_lds + 4 * t) = qd.voff[t];
+      *reinterpret_cast<ACCT_LDS uint32_t*>(voff_lds + 4 * (NV + t)) = dd.voff[t];
+    }
+  };
+  auto stage_next = [&](int i, ACCT_LDS char* sb) {  // like stage, for a tile after the first
+    if constexpr (KEEP_VOFF) {
+      typedef uint32_t Voff __attribute__((ext_vector_type(2 * NV)));
+      const Voff vo = *reinterpret_cast<const ACCT_LDS Voff*>(voff_lds);
+      TileDma<T, D, 64, NW> qd, dd;
+      qd.lds0 = dd.lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(wave * TileDma<T, D, 64, NW>::NIW * 1024));
+#pragma unroll
+      for (int t = 0; t < NV; t++) {
+        qd.voff[t] = vo[t];
+        dd.voff[t] = vo[NV + t];
+      }
+      qd.issue(qp, a.q_ss, i * 64, sb);
+      dd.issue(dop, a.o_ss, i * 64, sb + TILEB);
+      if (wave < 2) dma4_row((wave == 0 ? a.nlse : a.delta) + (int64_t)bh * a.Sq + i * 64, lane * 4, sb + 2 * TILEB + wave * 256);
+      if (DROP) {
+        const int idx = wave * 64 + lane, key = min(k0 + (idx >> 1), a.Sk - 1);
+        dma4_row(a.dropcol + ((((int64_t)bh * a.Tr + (i >> 1)) * a.Sk) << 2) + 2 * (i & 1), (key << 4) + ((idx & 1) << 2),
+                 sb + 2 * TILEB + STATB + wave * 256);
+      }
+    } else {
+      stage(i, sb);
+    }
+  };
+
   // A bias with row stride 0 (the reference's ALiBi form [B, N, 1, Sk]) depends on the key only: a lane of this
   // kernel owns a key column, so the bias is one value per lane and key group for the whole query loop
-  // (in units of the raw scores; 0 for the K role, whose accumulators hold dP)
-  const bool row_bias = BIAS && a.al_sq == 0;
+  // (in units of the exp2 argument)
+  const bool row_bias = BIAS == kBiasKey || (TBIAS && a.al_sq == 0);
   float brow[NGK];
 #pragma unroll
   for (int gk = 0; gk < NGK; gk++)
-    brow[gk] = (row_bias && !krole) ? (float)alibip[min(wk0 + 32 * gk + l32, a.Sk - 1)] * a.inv_scale : 0.f;
-  const bool bias_staged = BIAS && !row_bias && !krole && wk0 < a.Sk && (a.Sk & 7) == 0 &&
+    brow[gk] = (row_bias && !krole) ? (float)alibip[min(wk0 + 32 * gk + l32, a.Sk - 1)] * kLog2e : 0.f;
+  const bool bias_staged = TBIAS && !row_bias && !krole && wk0 < a.Sk && (a.Sk & 7) == 0 &&
                            (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh | a.al_sq) & 7)) == 0;
   auto stage_bias = [&](int cn) { bias_tile_dma<T, false>(alibip, a.al_sq, cn * 32, a.Sq, wk0, a.Sk, bias_lds); };
 
@@ -806,12 +877,19 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
     const int ntile = i_hi - i_lo + 1, npos = 2 * ntile;
     auto chunk_at = [&](int pos) { return 2 * (i_hi - (pos >> 1)) + (pos & 1); };
     stage(i_hi, smem);
-    if (BIAS && bias_staged) stage_bias(chunk_at(0));
+    if (KEEP_VOFF) plan_stage();
+    if (TBIAS && bias_staged) stage_bias(chunk_at(0));
     // A full wait the compiler can see: the stationary fragments loaded above are complete, so it places
     // no vmcnt wait inside the loop -- such a wait would also stall on the next tile's DMA.
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
+    // Wave priorities: every wave of a pair begins with its products and the two contend for the SIMD's matrix pipe.  By
+    // default the older (V role) wave wins; with the K role first -- its vector work is the shorter -- and the
+    // accumulating products ahead of the partner's vector work the step is 4 to 6 % shorter at head dim 128 (64 heads,
+    // 2048 x 2048 causal 150 -> 146 us, 4096 x 4096 548 -> 519; bf16 147 -> 140).  One key group per wave has fewer products
+    // to put in order: 96 heads, 1000 x 1000, D64 69 -> 72, D128 119 -> 121; head dim 80 178 -> 180.
+    constexpr bool PRIO = D == 128 && NGK == 2;
     // The K role runs one chunk behind the V role: in step n the V role recomputes P of chunk n,
     // publishes it and accumulates dV; the K role picks up P of chunk n-1.  One barrier per step,
     // nothing is carried across it in registers.
@@ -819,7 +897,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
     (void)c_lo;
     // offsets of the transposed fragments of d block db: kept across the steps where the registers allow
     // (a fifth of the step's vector instructions otherwise), re-derived in every step in the bias + dropout variant
-    constexpr bool KEEP_TOFF = !(BIAS && DROP);
+    constexpr bool KEEP_TOFF = !(TBIAS && DROP);
     int toff2_kept[2] = {0, 0};
     if (KEEP_TOFF) {
       const int trow = 4 * g + ((lane & 15) >> 2);
@@ -827,27 +905,29 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
 #pragma unroll
       for (int db = 0; db < 2; db++) toff2_kept[db] = trow * C::PITCH + swz_off(4 * db + tchunk, C::swz(trow)) + 8 * (lane & 1);
     }
-    constexpr bool KEEP_FOFF = !BIAS;   // the variants without a bias have the registers for the row-major offsets too
+    constexpr bool KEEP_FOFF = !TBIAS;   // the variants without a bias have the registers for the row-major offsets too
     int foff4_kept[4] = {0, 0, 0, 0};
     if (KEEP_FOFF) {
 #pragma unroll
       for (int t = 0; t < 4; t++) foff4_kept[t] = l32 * C::PITCH + swz_off(2 * t + g, C::swz(l32));
     }
     const uint8_t* flcol = (MASKT && a.mask_kind == kMaskDense) ? a.blkflags + (int64_t)mb * a.Tr * a.Tc + wkb : nullptr;
-    if (!flwin_ready) flwin.init_descending(flcol, a.Tc, c_lo >> 2, c_hi >> 2, lane, (!BIAS && flcol && a.blktail) ? a.blktail + (flcol - a.blkflags) : nullptr);
+    if (!flwin_ready) flwin.init_descending(flcol, a.Tc, c_lo >> 2, c_hi >> 2, lane, (!TBIAS && flcol && a.blktail) ? a.blktail + (flcol - a.blkflags) : nullptr);
+    const bool kfirst = PRIO && __builtin_amdgcn_readfirstlane(wave) >= 4;
     for (int n = 0; n <= npos; n++) {
-      if ((n & 1) && (n >> 1) + 1 < ntile) stage(i_hi - ((n >> 1) + 1), smem + ((((n >> 1) + 1) & 1) * STAGEB));
+      if (kfirst) __builtin_amdgcn_s_setprio(1);
+      if ((n & 1) && (n >> 1) + 1 < ntile) stage_next(i_hi - ((n >> 1) + 1), smem + ((((n >> 1) + 1) & 1) * STAGEB));
       const int cpos = __builtin_amdgcn_readfirstlane(krole ? n - 1 : n);   // position of the chunk this wave works on in this step (wave-uniform: scalar)
       if (cpos >= 0 && cpos < npos) {
         const int cidx = chunk_at(cpos);
         const uint32_t fl_cur = flwin.get(cidx >> 2, lane);
-        const uint32_t cls = classify(cidx, fl_cur, (MASKT && !BIAS) ? flwin.tail(cidx >> 2) : 0u);
+        const uint32_t cls = classify(cidx, fl_cur, (MASKT && !TBIAS) ? flwin.tail(cidx >> 2) : 0u);
         const bool act = cls & 1u, apply_mask = cls & 2u, limits = cls & 4u, diag = cls & 8u;
         // keys from key_end on are hidden from every row of the chunk (a key tail): a lane owns a key, so its whole
         // column of P is zeroed after the probabilities are packed (one AND per packed word)
         const int key_end = (cls >> 8) ? wkb * 128 + (int)(cls >> 8) : 0x7fffffff;
         const bool ktail = wk0 + WK > key_end;
-        const bool edge = (BIAS && !bias_staged && !row_bias) || apply_mask || limits;   // (a staged or per-key bias is already inside the scores)
+        const bool edge = (TBIAS && !bias_staged && !row_bias) || apply_mask || limits;   // (a staged or per-key bias is already inside the scores)
         if (act) {
           const int c = cidx & 1, qc0 = cidx * 32;
           // Where the registers do not allow keeping them (see above), the per-lane LDS offsets are
@@ -875,8 +955,32 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
           const ACCT_LDS float* dbuf = lbuf + 64;
           ACCT_LDS char* px = pexch + ((cidx & 1) * 4 + pair) * PXB + ln * 16;
           // rows of this lane's C registers: q = qc0 + 8 (r/4) + 4 g + r%4 ; key = wk0 + 32 gk + l32
+          //
+          // The row statistics go in as the INITIAL value of the accumulators: -LSE / scale for the scores, -D for
+          // dP.  P is then exp2(scale*log2e * S) and dS = P * dP with nothing subtracted per element, and the LDS reads of
+          // the statistics (once per chunk, for both key groups) overlap the fragment reads instead of standing between
+          // the products and the exponentials (a step's timeline showed 1200 cycles there for 450 of vector work).  With dropout
+          // dP is masked first, so D is subtracted afterwards.  With the kept offsets above, dK/dV before / now (us): 96 heads,
+          // 1000 x 1000, D64 72.9 / 69.1; 16, 4096 x 4096, D40 144 / 136, D80 189 / 178; 96, 1000 x 1000, D128 127 / 119.
           f32x16 t0[NGK];                              // S (V role) or dP (K role) of the two key groups
-          if (BIAS && bias_staged) {
+          f32x16 rowc;                                 // their initial value by query row
+          auto read_rowc = [&](const ACCT_LDS float* stat) {
+#pragma unroll
+            for (int r4 = 0; r4 < 4; r4++) {
+              const f32x4 v = *reinterpret_cast<const ACCT_LDS f32x4*>(stat + 32 * c + 8 * r4 + 4 * g);
+#pragma unroll
+              for (int e = 0; e < 4; e++) rowc[4 * r4 + e] = v[e];
+            }
+          };
+          // (mask bits: a row that sees nothing but masked keys has LSE near -10000, which must meet the -10000 of its
+          // keys before a score is added, or the score's low bits are lost)
+          if (krole ? DROP : (MASKT && apply_mask)) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) rowc[r] = 0.f;
+          } else {
+            read_rowc(krole ? dbuf : lbuf);
+          }
+          if (TBIAS && bias_staged) {
             // V role: the bias enters as the initial value of the score accumulators (bias / scale, the MFMAs
             // add q.k): no bias registers alive next to the scores.  Transposed reads of the row-major tile:
             // each hands a lane the four consecutive rows 8i + 4g .. +3 of its key column (a 16-lane group
@@ -888,13 +992,13 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
               for (int i = 0; i < 4; i++) {
                 const typename E::V4 bv = __builtin_bit_cast(typename E::V4, lds_read_tr(bl + i * 8 * 128 + gk * 64));
 #pragma unroll
-                for (int e = 0; e < 4; e++) t0[gk][4 * i + e] = (float)bv[e] * a.inv_scale;
+                for (int e = 0; e < 4; e++) t0[gk][4 * i + e] = __builtin_fmaf((float)bv[e], a.inv_scale, rowc[4 * i + e]);
               }
           } else {
 #pragma unroll
             for (int gk = 0; gk < NGK; gk++)
 #pragma unroll
-              for (int r = 0; r < 16; r++) t0[gk][r] = BIAS ? brow[gk] : 0.f;
+              for (int r = 0; r < 16; r++) t0[gk][r] = rowc[r];
           }
           {
             // software pipeline: the A fragments travel through a ring of ARING register sets (ARING reads in
@@ -919,10 +1023,11 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
               b1 = b1n;
             }
           }
-          if (BIAS && bias_staged) {
+          if (TBIAS && bias_staged) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // bias tile consumed: stage the next chunk's
             if (cpos + 1 < npos) stage_bias(chunk_at(cpos + 1));
           }
+          if (PRIO) __builtin_amdgcn_s_setprio(0);
           uint32_t dcw[NGK] = {};                       // keep bits of the chunk's 32 rows for this lane's two key columns
           if (DROP) {
             const ACCT_LDS uint32_t* dc = (const ACCT_LDS uint32_t*)(qbuf + 2 * TILEB + STATB) + 2 * (pair * WK + l32) + c;
@@ -936,7 +1041,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
               // passes that each keep few values live: + bias/scale (unstaged bias only); - 10000/scale where the mask bit of
               // (row, key) is set; -inf where the key comes after the query (causal) or where the key
               // or the query row does not exist (the probability is exactly 0 either way).
-              if (BIAS && !bias_staged && !row_bias) {      // a bias the DMA cannot stage (alignment): direct loads
+              if (TBIAS && !bias_staged && !row_bias) {      // a bias the DMA cannot stage (alignment): direct loads
                 const int qlast = a.Sq - 1 - qc0;               // last valid row, relative to the chunk
                 const T* brow0 = alibip + (int64_t)qc0 * a.al_sq;
 #pragma unroll
@@ -956,6 +1061,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
                                          ? a.colbits + ((((int64_t)mb * a.Tr + (qc0 >> 7)) * a.Sk) << 2) + ((qc0 >> 5) & 3)
                                          : a.colbits + ((qc0 >> 5) & 3);
                 const uint32_t addbits = __float_as_uint(a.mask_add_raw);
+                read_rowc(lbuf);
 #pragma unroll
                 for (int gk = 0; gk < NGK; gk++) {
                   const int kv_c = min(wk0 + 32 * gk + l32, a.Sk - 1);
@@ -964,7 +1070,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
                   for (int r = 0; r < 16; r++) {
                     // (bit ? -1 : 0) & bits(-10000/scale), added
                     const int32_t sel = (int32_t)(w << (31 - (8 * (r >> 2) + (r & 3)))) >> 31;
-                    t0[gk][r] += __uint_as_float((uint32_t)sel & addbits);
+                    t0[gk][r] += rowc[r] + __uint_as_float((uint32_t)sel & addbits);
                   }
                 }
               }
@@ -983,17 +1089,16 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
               }
             }
 #pragma unroll
-            for (int gk = 0; gk < NGK; gk++) {
-              const int kv_c = min(wk0 + 32 * gk + l32, a.Sk - 1);
+            for (int hh = 0; hh < 2; hh++) {
 #pragma unroll
-              for (int hh = 0; hh < 2; hh++) {
+              for (int gk = 0; gk < NGK; gk++) {
                 float p[8], pd[8];
 #pragma unroll
                 for (int r4 = 0; r4 < 2; r4++) {
-                  const f32x4 lv = *reinterpret_cast<const ACCT_LDS f32x4*>(lbuf + 32 * c + 16 * hh + 8 * r4 + 4 * g);
 #pragma unroll
                   for (int e = 0; e < 4; e++) {
-                    p[4 * r4 + e] = fast_exp2(__builtin_fmaf(t0[gk][8 * hh + 4 * r4 + e], a.scale_log2e, lv[e]));
+                    p[4 * r4 + e] = fast_exp2(BIAS ? __builtin_fmaf(t0[gk][8 * hh + 4 * r4 + e], a.scale_log2e, brow[gk])
+                                                     : t0[gk][8 * hh + 4 * r4 + e] * a.scale_log2e);
                     pd[4 * r4 + e] = p[4 * r4 + e];
                     // dropped: 0; kept: P (the 1 / keep_prob is applied to dV once, at the end)
                     if (DROP) pd[4 * r4 + e] = __uint_as_float(__float_as_uint(p[4 * r4 + e]) & (uint32_t)__builtin_amdgcn_sbfe((int)dcw[gk], 16 * hh + 8 * r4 + e, 1));
@@ -1016,20 +1121,19 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
           } else {
 #pragma unroll
             for (int gk = 0; gk < NGK; gk++) {
-              const int kv_c = min(wk0 + 32 * gk + l32, a.Sk - 1);
 #pragma unroll
               for (int hh = 0; hh < 2; hh++) {
                 const f16x8 ph = *reinterpret_cast<const ACCT_LDS f16x8*>(px + (2 * gk + hh) * 1024);
                 float ds[8];
 #pragma unroll
                 for (int r4 = 0; r4 < 2; r4++) {
-                  const f32x4 dv4 = *reinterpret_cast<const ACCT_LDS f32x4*>(dbuf + 32 * c + 16 * hh + 8 * r4 + 4 * g);
+                  f32x4 nd = {0.f, 0.f, 0.f, 0.f};                     // -D
+                  if (DROP) nd = *reinterpret_cast<const ACCT_LDS f32x4*>(dbuf + 32 * c + 16 * hh + 8 * r4 + 4 * g);
 #pragma unroll
                   for (int e = 0; e < 4; e++) {
-                    float dpv = t0[gk][8 * hh + 4 * r4 + e];
-                    float dpd = dpv - dv4[e];
+                    float dpd = t0[gk][8 * hh + 4 * r4 + e];
                     // dropped: dP = 0; kept: dP / keep_prob, scaled by the FMA that subtracts D
-                    if (DROP) dpd = __builtin_fmaf(__uint_as_float(__float_as_uint(dpv) & (uint32_t)__builtin_amdgcn_sbfe((int)dcw[gk], 16 * hh + 8 * r4 + e, 1)), a.inv_keep, -dv4[e]);
+                    if (DROP) dpd = __builtin_fmaf(__uint_as_float(__float_as_uint(dpd) & (uint32_t)__builtin_amdgcn_sbfe((int)dcw[gk], 16 * hh + 8 * r4 + e, 1)), a.inv_keep, nd[e]);
                     // (an FMA with a zero addend keeps the fp16 -> fp32 conversion inside one mixed-precision instruction)
                     ds[4 * r4 + e] = __builtin_fmaf((float)ph[4 * r4 + e], dpd, 0.0f);
                   }
@@ -1038,6 +1142,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
               }
             }
           }
+          if (PRIO) __builtin_amdgcn_s_setprio(1);
           // dV^T += dO^T P (V role) ; dK^T += Q^T dS (K role): contract over the 32 query rows of the chunk
           const ACCT_LDS char* tb = (krole ? qbuf : dobuf) + c * 32 * C::PITCH;
           {
@@ -1061,10 +1166,11 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
               if (i + BRING < NT) tr[i % BRING] = tread(i + BRING);
             }
           }
-        } else if (BIAS && bias_staged && cpos + 1 < npos) {
+        } else if (TBIAS && bias_staged && cpos + 1 < npos) {
           stage_bias(chunk_at(cpos + 1));               // nothing to read in this step: the region is free
         }
       }
+      if (PRIO) __builtin_amdgcn_s_setprio(0);
       dma_wait();                                     // a tile requested at the top of this step has landed
       __syncthreads();
     }
@@ -1089,9 +1195,13 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
 
 // (two bodies in the variant that knows mask tensors only, as in the dQ kernel: a workgroup whose key blocks
 // see nothing but the causal pattern runs the code of the variant without side inputs)
-template <typename T, int D, bool BIAS, bool DROP, bool MASKT, int NGK>
+template <typename T, int D, int BIAS, bool DROP, bool MASKT, int NGK>
 __global__ void __launch_bounds__(512) fa_bwd_dkdv_kernel(const FaArgs a) {
-  if constexpr (MASKT && !BIAS && !DROP) {
+  if constexpr (MASKT && BIAS != kBiasAny && !DROP) {
+    if (BIAS && a.mask_kind != kMaskDense && a.mask_kind != kMaskTile) {
+      fa_bwd_dkdv_body<T, D, BIAS, false, false, NGK>(a);
+      return;
+    }
     if (a.mask_kind == kMaskDense) {
       constexpr int BNK = 4 * 32 * NGK;
       const int BH = a.B * a.N, n_wg = BH * a.n_tiles;
@@ -1106,7 +1216,7 @@ __global__ void __launch_bounds__(512) fa_bwd_dkdv_kernel(const FaArgs a) {
       if (dense_lines_are_causal(fl, a.Tc, 1, kb_lo, kb_hi - kb_lo + 1, qb_lo, qb_hi, true, a, threadIdx.x & 63)) {
         FaArgs c = a;
         c.mask_kind = kMaskCausal;
-        fa_bwd_dkdv_body<T, D, false, false, false, NGK>(c);
+        fa_bwd_dkdv_body<T, D, BIAS, false, false, NGK>(c);
         return;
       }
     }
@@ -1115,7 +1225,7 @@ __global__ void __launch_bounds__(512) fa_bwd_dkdv_kernel(const FaArgs a) {
 }
 
 // ---- launchers ----------------------------------------------------------------
-template <typename T, int D, bool BIAS, bool DROP, int KG>
+template <typename T, int D, int BIAS, bool DROP, int KG>
 static hipError_t launch_bwd_dq(FaArgs a, hipStream_t st) {
   constexpr int QG = 1, NW = D > 128 ? 4 : 8;            // (wide head dims: one wave per SIMD has the registers)
   constexpr int RG = NW / KG, BM = 32 * QG * RG;
@@ -1133,11 +1243,11 @@ static hipError_t launch_bwd_dq(FaArgs a, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <typename T, int D, bool BIAS, bool DROP, int NGK>
+template <typename T, int D, int BIAS, bool DROP, int NGK>
 static hipError_t launch_bwd_dkdv(FaArgs a, hipStream_t st) {
   using CS = SwzCfg<D>;
   constexpr size_t stageb = 2 * 64 * (size_t)CS::PITCH + 512 + (DROP ? 2048 : 0);
-  constexpr size_t loopb = 2 * stageb + 8 * 2048 * NGK + 8 * (size_t)dkdv_park<D, BIAS, true, NGK>() * 1024 + (BIAS ? 4 * 4096 : 0),
+  constexpr size_t loopb = 2 * stageb + 8 * 2048 * NGK + 8 * (size_t)dkdv_park<D, BIAS == kBiasAny, true, NGK>() * 1024 + (BIAS == kBiasAny ? 4 * 4096 : D <= 128 ? 8 * TileDma<T, D, 64, 8>::NV * 512 : 0),
                    epib = (size_t)8 * 32 * (CS::DB * 64 + 16);
   constexpr size_t smem = loopb > epib ? loopb : epib;
   static_assert(smem <= 160 * 1024, "the workgroup's LDS must fit the CU's 160 KB");
@@ -1157,7 +1267,7 @@ static hipError_t launch_bwd_dkdv(FaArgs a, hipStream_t st) {
   return e;
 }
 
-template <typename T, int D, bool BIAS, bool DROP>
+template <typename T, int D, int BIAS, bool DROP>
 static hipError_t launch_bwd_t(FaArgs a, int stages, hipStream_t st) {
   hipError_t e = hipSuccess;
   if (stages & kStageDq) {
@@ -1193,14 +1303,16 @@ static hipError_t launch_bwd_d(const FaArgs& a, int stages, hipStream_t st) {
   const bool bias = a.alibi != nullptr, drop = a.droprow != nullptr || a.dropcol != nullptr;
 #ifndef ACCT_DEV_BUILD
   if constexpr (SIDE == 2) {
-    if (bias) return drop ? launch_bwd_t<T, D, true, true>(a, stages, st) : launch_bwd_t<T, D, true, false>(a, stages, st);
+    // a bias per key (the reference's ALiBi form) that the DMA can stage has variants of its own, without dropout
+    if (bias && !drop && key_bias_stageable(a)) return launch_bwd_t<T, D, kBiasKey, false>(a, stages, st);
+    if (bias) return drop ? launch_bwd_t<T, D, kBiasAny, true>(a, stages, st) : launch_bwd_t<T, D, kBiasAny, false>(a, stages, st);
   }
   if constexpr (SIDE >= 1) {
-    if (drop && !bias) return launch_bwd_t<T, D, false, true>(a, stages, st);
+    if (drop && !bias) return launch_bwd_t<T, D, kBiasNone, true>(a, stages, st);
   }
 #endif
   if (bias || drop) return hipErrorNotSupported;       // (development build, head dims 40 / 160: plain variants only)
-  return launch_bwd_t<T, D, false, false>(a, stages, st);
+  return launch_bwd_t<T, D, kBiasNone, false>(a, stages, st);
 }
 
 template <typename T>

@@ -160,8 +160,8 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   const bool bias_staged = BIAS && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh | a.al_sq) & 7)) == 0;
   // (the launcher picks 128-key tiles for a bias only when both hold: known at compile time there)
   const bool row_bias = BIAS && (KT == 4 || a.al_sq == 0);   // the bias depends on the key only: one row per tile
-  const bool acc_bias = BIAS && (KT == 4 || (row_bias && bias_staged));
-  const bool scaled = BIAS && !acc_bias;                   // scores are turned into scale*s + bias before the softmax
+  constexpr bool acc_bias = BIAS && KT == 4;
+  constexpr bool scaled = BIAS && !acc_bias;                   // scores are turned into scale*s + bias before the softmax
   const float cmul = scaled ? kLog2e : a.scale_log2e;
   const float madd = scaled ? kMaskFill : a.mask_add_raw;          // the additive -10000 in the units of s
   const float lazy_thr = 8.0f / cmul;                              // 8 octaves, in the units of s
@@ -180,7 +180,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   vdma.plan(a.v_ss, cpr);
   // bias tiles of this wave's rows are staged through a wave-private LDS region one tile ahead
   // (with 128-key tiles only the key-only form is served: two 256-byte rows per wave)
-  constexpr int BIASB = BIAS ? (KT == 4 ? 512 : QG * 4096) : 0;
+  constexpr int BIASB = BIAS ? (KT == 4 ? 1024 : QG * 4096) : 0;
   static_assert(KT == 2 || !BIAS || QG == 1, "128-key tiles with a bias: 32 rows per wave");
   ACCT_LDS char* bias_lds = smem + 4 * TILEB + wave * BIASB;
   // (a key-only bias: rows of consecutive tiles alternate between two 256-byte slots of the region, so the next
@@ -191,6 +191,13 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       if (row_bias) bias_row_dma<T>(alibip, jn * BN, a.Sk, bias_lds + gq * 4096 + (acc_bias ? (jn & 1) * 256 : 0));
       else bias_tile_dma<T>(alibip, a.al_sq, wq0 + 32 * gq, a.Sq, jn * 64, a.Sk, bias_lds + gq * 4096);
     }
+  };
+  // The staged row of a key-only bias becomes float32 / scale behind its two slots, once per tile and wave, and is the C
+  // operand of the first product from there: nothing per score.
+  auto convert_bias = [&](int jn) {
+    const typename E::V2 v = *reinterpret_cast<const ACCT_LDS typename E::V2*>(bias_lds + (jn & 1) * 256 + lane * 4);
+    const f32x2 f = {(float)v[0] * a.inv_scale, (float)v[1] * a.inv_scale};
+    *reinterpret_cast<ACCT_LDS f32x2*>(bias_lds + 512 + lane * 8) = f;
   };
   // keep bits of this wave's rows and one tile, staged with the tile's DMA (double buffered)
   using DropStage = DropRowStage<DROP, QG, KT>;
@@ -240,9 +247,9 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
         for (int c = 0; c < KTW; c++)
 #pragma unroll
           for (int r4 = 0; r4 < 4; r4++) {
-            const typename E::V4 bv = bias_tile_read<T>(bias_lds + gq * 4096 + (j & 1) * 256, 0, 4 * (kg * KTW + c) + r4, g);
+            const f32x4 bv = *reinterpret_cast<const ACCT_LDS f32x4*>(bias_lds + 512 + (32 * (kg * KTW + c) + 8 * r4 + 4 * g) * 4);
 #pragma unroll
-            for (int e = 0; e < 4; e++) s[gq][c][4 * r4 + e] = (float)bv[e] * a.inv_scale;
+            for (int e = 0; e < 4; e++) s[gq][c][4 * r4 + e] = bv[e];
           }
     } else {
 #pragma unroll
@@ -438,6 +445,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     // A full wait the compiler can see: every load issued so far (Q fragments included) is complete, so
     // it places no vmcnt wait inside the loop -- such a wait would also stall on the next tile's DMA.
     __builtin_amdgcn_s_waitcnt(0);
+    if (acc_bias) convert_bias(j_lo);
     __syncthreads();
     for (int j = j_lo; j <= j_hi; j++) {
       const int buf = (j - j_lo) & 1;
@@ -461,6 +469,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
         stage_bias(j + 1);                                  // nothing to read in this step: the region is free
       }
       dma_wait();
+      if (acc_bias && j < j_hi) convert_bias(j + 1);
       __syncthreads();
     }
   }
@@ -577,7 +586,11 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
 // A causal mask given as a tensor then costs one look at the class table per workgroup.
 template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2, int KG = 1>
 __global__ void __launch_bounds__(64 * NW) fa_fwd_kernel(const FaArgs a) {
-  if constexpr (MASKT && !BIAS && !DROP) {
+  if constexpr (MASKT && (!BIAS || KT == 4) && !DROP) {
+    if (BIAS && a.mask_kind != kMaskDense && a.mask_kind != kMaskTile) {
+      fa_fwd_body<T, D, QG, NW, BIAS, false, false, KT, KG>(a);
+      return;
+    }
     if (a.mask_kind == kMaskDense) {
       constexpr int BM = 32 * QG * NW / KG;
       const int BH = a.B * a.N;
@@ -592,7 +605,7 @@ __global__ void __launch_bounds__(64 * NW) fa_fwd_kernel(const FaArgs a) {
       if (dense_lines_are_causal(fl, 1, a.Tc, qb_lo, qb_hi - qb_lo + 1, kvb_lo, kvb_hi, false, a, threadIdx.x & 63)) {
         FaArgs c = a;
         c.mask_kind = kMaskCausal;
-        fa_fwd_body<T, D, QG, NW, false, false, false, KT, KG>(c);
+        fa_fwd_body<T, D, QG, NW, BIAS, false, false, KT, KG>(c);
         return;
       }
     }
@@ -694,7 +707,7 @@ static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   constexpr int QG = 1, RG = NW / KG, BM = 32 * QG * RG;
   a.n_tiles = (a.Sq + BM - 1) / BM;
   const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
-  constexpr size_t biasb = BIAS ? (KT == 4 ? 512 : QG * 4096) : 0;     // per wave, as in the kernel
+  constexpr size_t biasb = BIAS ? (KT == 4 ? 1024 : QG * 4096) : 0;     // per wave, as in the kernel
   constexpr size_t tiles = 4 * 32 * KT * (size_t)C::PITCH + NW * biasb + (size_t)NW * 2 * DropRowStage<DROP, QG, KT>::BYTES,
                    stage = KG > 1 ? fwd_merge_at<D, RG>() + (size_t)(KG - 1) * RG * fwd_merge_slot<D>() : (size_t)NW * 32 * (C::DB * 64 + 16);
   constexpr size_t smem = tiles > stage ? tiles : stage;
@@ -707,7 +720,7 @@ static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   e = hipGetLastError();
   if (e == hipSuccess && a.kv_split > 1) {
     // a full bias is added in natural units, everything else in units of q.k (see the kernel)
-    const bool acc_bias = BIAS && a.al_sq == 0 && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh) & 7)) == 0;
+    const bool acc_bias = BIAS && KT == 4;
     const bool scaled = BIAS && !acc_bias;
     hipLaunchKernelGGL(fa_fwd_combine_kernel<T>, dim3((unsigned)(nblk * RG * 4 * C::DB)), dim3(256), 0, st, a, RG, (int)C::DB,
                        scaled ? kLog2e : a.scale_log2e, scaled ? 1.0f : a.scale, DROP ? a.inv_keep : 1.0f);
@@ -723,8 +736,7 @@ static hipError_t launch_fwd_t(const FaArgs& a, hipStream_t st) {
   // them; a key-only bias that the DMA can stage (the kernel's own test, repeated here) is a 256-byte row and does.
   constexpr bool BIG = NW == 8 && D <= 128;
   if constexpr (BIG && BIAS) {
-    const bool row_staged = a.al_sq == 0 && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh) & 7)) == 0;
-    return row_staged ? launch_fwd_kt<T, D, NW, BIAS, DROP, 4, KG>(a, st) : launch_fwd_kt<T, D, NW, BIAS, DROP, 2, KG>(a, st);
+    return key_bias_stageable(a) ? launch_fwd_kt<T, D, NW, BIAS, DROP, 4, KG>(a, st) : launch_fwd_kt<T, D, NW, BIAS, DROP, 2, KG>(a, st);
   } else {
     return launch_fwd_kt<T, D, NW, BIAS, DROP, BIG ? 4 : 2, KG>(a, st);
   }
