@@ -201,9 +201,7 @@ acct::FaArgs make_args(const acct_fa_params* p) {
   a.mask_sb = mask_is_dense(p) ? p->mask_stride_b : 0;
   a.al_sb = p->alibi_stride_b; a.al_sh = p->alibi_stride_h; a.al_sq = p->alibi_stride_q;
   a.scale = p->scale;
-  // (the floor keeps LSE / scale finite in the backward; below it the scores vanish beside any LSE either way)
-  a.scale_log2e = fmaxf(p->scale * acct::kLog2e, 1e-37f);
-  a.inv_scale_log2e = 1.0f / a.scale_log2e;
+  a.scale_log2e = p->scale * acct::kLog2e;
   a.inv_keep = 1.0f / p->keep_prob;
   if (philox_on(p)) {
     a.philox_k0 = (uint32_t)p->drop_seed;

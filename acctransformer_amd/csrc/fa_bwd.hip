@@ -140,8 +140,8 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
       // (minus p_shift: the recomputed probabilities carry a factor 2^p_shift, see FaArgs)
       lq[gq] = a.lse[(int64_t)bh * a.Sq + row] * kLog2e - a.p_shift;
       if (g == 0 && kg == 0) {
-        a.delta[(int64_t)bh * a.Sq + row] = -dl[gq];
-        a.nlse[(int64_t)bh * a.Sq + row] = -lq[gq] * a.inv_scale_log2e;
+        a.delta[(int64_t)bh * a.Sq + row] = dl[gq];
+        a.nlse[(int64_t)bh * a.Sq + row] = -lq[gq];        // p_shift - LSE*log2(e): the exp2 offset the dK/dV kernel adds
       }
     }
   }
@@ -826,12 +826,12 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
 
   // A bias with row stride 0 (the reference's ALiBi form [B, N, 1, Sk]) depends on the key only: a lane of this
   // kernel owns a key column, so the bias is one value per lane and key group for the whole query loop
-  // (in units of the exp2 argument)
+  // (in units of the raw scores, the initial value of their accumulators; 0 for the K role, whose accumulators hold dP)
   const bool row_bias = BIAS == kBiasKey || (TBIAS && a.al_sq == 0);
   float brow[NGK];
 #pragma unroll
   for (int gk = 0; gk < NGK; gk++)
-    brow[gk] = (row_bias && !krole) ? (float)alibip[min(wk0 + 32 * gk + l32, a.Sk - 1)] * kLog2e : 0.f;
+    brow[gk] = (row_bias && !krole) ? (float)alibip[min(wk0 + 32 * gk + l32, a.Sk - 1)] * a.inv_scale : 0.f;
   const bool bias_staged = TBIAS && !row_bias && !krole && wk0 < a.Sk && (a.Sk & 7) == 0 &&
                            (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh | a.al_sq) & 7)) == 0;
   auto stage_bias = [&](int cn) { bias_tile_dma<T, false>(alibip, a.al_sq, cn * 32, a.Sq, wk0, a.Sk, bias_lds); };
@@ -956,30 +956,17 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
           ACCT_LDS char* px = pexch + ((cidx & 1) * 4 + pair) * PXB + ln * 16;
           // rows of this lane's C registers: q = qc0 + 8 (r/4) + 4 g + r%4 ; key = wk0 + 32 gk + l32
           //
-          // The row statistics go in as the INITIAL value of the accumulators: -LSE / scale for the scores, -D for
-          // dP.  P is then exp2(scale*log2e * S) and dS = P * dP with nothing subtracted per element, and the LDS reads of
-          // the statistics (once per chunk, for both key groups) overlap the fragment reads instead of standing between
-          // the products and the exponentials (a step's timeline showed 1200 cycles there for 450 of vector work).  With dropout
-          // dP is masked first, so D is subtracted afterwards.  With the kept offsets above, dK/dV before / now (us): 96 heads,
-          // 1000 x 1000, D64 72.9 / 69.1; 16, 4096 x 4096, D40 144 / 136, D80 189 / 178; 96, 1000 x 1000, D128 127 / 119.
+          // The row statistics (p_shift - LSE*log2(e) in the V role, D in the K role) are read once per chunk for both key
+          // groups: ahead of the last products where the registers allow (the wait for them else stands between the products
+          // and the exponentials), half a chunk at a time in the other variants.  dK/dV, half chunks / ahead (us): 96 heads,
+          // 1000 x 1000, D64 72.7 / 70.1; 16, 4096 x 4096, D40 144.6 / 141.7, D80 186.3 / 184.1; but 64, 2048 x 2048 causal, D128,
+          // where eleven registers are spilled for it, 150 / 176, and with a bias tile and dropout D64 loses the second
+          // workgroup of a CU.  As initial value of the accumulators (-LSE / scale, -D) they cost nothing per element, another
+          // 2 to 3 %, but every product then rounds the score at the magnitude of LSE: P in float32 was 4.5e-7 off instead of
+          // 2.3e-7 (N(0,1), D128).
+          constexpr bool EARLY = D <= 80 && !TBIAS;
+          f32x4 early[4];                              // rows 8 i + 4 g .. +3 of the chunk
           f32x16 t0[NGK];                              // S (V role) or dP (K role) of the two key groups
-          f32x16 rowc;                                 // their initial value by query row
-          auto read_rowc = [&](const ACCT_LDS float* stat) {
-#pragma unroll
-            for (int r4 = 0; r4 < 4; r4++) {
-              const f32x4 v = *reinterpret_cast<const ACCT_LDS f32x4*>(stat + 32 * c + 8 * r4 + 4 * g);
-#pragma unroll
-              for (int e = 0; e < 4; e++) rowc[4 * r4 + e] = v[e];
-            }
-          };
-          // (mask bits: a row that sees nothing but masked keys has LSE near -10000, which must meet the -10000 of its
-          // keys before a score is added, or the score's low bits are lost)
-          if (krole ? DROP : (MASKT && apply_mask)) {
-#pragma unroll
-            for (int r = 0; r < 16; r++) rowc[r] = 0.f;
-          } else {
-            read_rowc(krole ? dbuf : lbuf);
-          }
           if (TBIAS && bias_staged) {
             // V role: the bias enters as the initial value of the score accumulators (bias / scale, the MFMAs
             // add q.k): no bias registers alive next to the scores.  Transposed reads of the row-major tile:
@@ -992,13 +979,16 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
               for (int i = 0; i < 4; i++) {
                 const typename E::V4 bv = __builtin_bit_cast(typename E::V4, lds_read_tr(bl + i * 8 * 128 + gk * 64));
 #pragma unroll
-                for (int e = 0; e < 4; e++) t0[gk][4 * i + e] = __builtin_fmaf((float)bv[e], a.inv_scale, rowc[4 * i + e]);
+                for (int e = 0; e < 4; e++) t0[gk][4 * i + e] = (float)bv[e] * a.inv_scale;
               }
           } else {
 #pragma unroll
-            for (int gk = 0; gk < NGK; gk++)
+            for (int gk = 0; gk < NGK; gk++) {
+              float first = BIAS ? brow[gk] : 0.f;
+              if (BIAS == kBiasKey) asm volatile("" : "+v"(first));   // (or its 16 copies are kept from step to step: 97 registers spilled at head dim 128)
 #pragma unroll
-              for (int r = 0; r < 16; r++) t0[gk][r] = rowc[r];
+              for (int r = 0; r < 16; r++) t0[gk][r] = first;
+            }
           }
           {
             // software pipeline: the A fragments travel through a ring of ARING register sets (ARING reads in
@@ -1015,6 +1005,10 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
               V8 b1n = b1;
               if (t + 1 < C::KS)
                 b1n = (t + 1 >= C::KS - PARK) ? *reinterpret_cast<const ACCT_LDS V8*>(park + (t + 1 - (C::KS - PARK)) * 1024) : bf[NGK - 1][t + 1];
+              if (EARLY && t == C::KS - 1) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) early[i] = *reinterpret_cast<const ACCT_LDS f32x4*>((krole ? dbuf : lbuf) + 32 * c + 8 * i + 4 * g);
+              }
               __builtin_amdgcn_sched_barrier(0);
               t0[0] = E::mfma(ar[t % ARING], bf[0][t], t0[0]);                              // S[q, key] or dP[q, key]
               if (NGK == 2) t0[NGK - 1] = E::mfma(ar[t % ARING], b1, t0[NGK - 1]);
@@ -1061,7 +1055,6 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
                                          ? a.colbits + ((((int64_t)mb * a.Tr + (qc0 >> 7)) * a.Sk) << 2) + ((qc0 >> 5) & 3)
                                          : a.colbits + ((qc0 >> 5) & 3);
                 const uint32_t addbits = __float_as_uint(a.mask_add_raw);
-                read_rowc(lbuf);
 #pragma unroll
                 for (int gk = 0; gk < NGK; gk++) {
                   const int kv_c = min(wk0 + 32 * gk + l32, a.Sk - 1);
@@ -1070,7 +1063,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
                   for (int r = 0; r < 16; r++) {
                     // (bit ? -1 : 0) & bits(-10000/scale), added
                     const int32_t sel = (int32_t)(w << (31 - (8 * (r >> 2) + (r & 3)))) >> 31;
-                    t0[gk][r] += rowc[r] + __uint_as_float((uint32_t)sel & addbits);
+                    t0[gk][r] += __uint_as_float((uint32_t)sel & addbits);
                   }
                 }
               }
@@ -1090,6 +1083,9 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
             }
 #pragma unroll
             for (int hh = 0; hh < 2; hh++) {
+              f32x4 nl[2];
+#pragma unroll
+              for (int r4 = 0; r4 < 2; r4++) nl[r4] = EARLY ? early[2 * hh + r4] : *reinterpret_cast<const ACCT_LDS f32x4*>(lbuf + 32 * c + 16 * hh + 8 * r4 + 4 * g);
 #pragma unroll
               for (int gk = 0; gk < NGK; gk++) {
                 float p[8], pd[8];
@@ -1097,8 +1093,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
                 for (int r4 = 0; r4 < 2; r4++) {
 #pragma unroll
                   for (int e = 0; e < 4; e++) {
-                    p[4 * r4 + e] = fast_exp2(BIAS ? __builtin_fmaf(t0[gk][8 * hh + 4 * r4 + e], a.scale_log2e, brow[gk])
-                                                     : t0[gk][8 * hh + 4 * r4 + e] * a.scale_log2e);
+                    p[4 * r4 + e] = fast_exp2(__builtin_fmaf(t0[gk][8 * hh + 4 * r4 + e], a.scale_log2e, nl[r4][e]));
                     pd[4 * r4 + e] = p[4 * r4 + e];
                     // dropped: 0; kept: P (the 1 / keep_prob is applied to dV once, at the end)
                     if (DROP) pd[4 * r4 + e] = __uint_as_float(__float_as_uint(p[4 * r4 + e]) & (uint32_t)__builtin_amdgcn_sbfe((int)dcw[gk], 16 * hh + 8 * r4 + e, 1));
@@ -1120,20 +1115,22 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
             }
           } else {
 #pragma unroll
-            for (int gk = 0; gk < NGK; gk++) {
+            for (int hh = 0; hh < 2; hh++) {
+              f32x4 dd[2];
 #pragma unroll
-              for (int hh = 0; hh < 2; hh++) {
+              for (int r4 = 0; r4 < 2; r4++) dd[r4] = EARLY ? early[2 * hh + r4] : *reinterpret_cast<const ACCT_LDS f32x4*>(dbuf + 32 * c + 16 * hh + 8 * r4 + 4 * g);
+#pragma unroll
+              for (int gk = 0; gk < NGK; gk++) {
                 const f16x8 ph = *reinterpret_cast<const ACCT_LDS f16x8*>(px + (2 * gk + hh) * 1024);
                 float ds[8];
 #pragma unroll
                 for (int r4 = 0; r4 < 2; r4++) {
-                  f32x4 nd = {0.f, 0.f, 0.f, 0.f};                     // -D
-                  if (DROP) nd = *reinterpret_cast<const ACCT_LDS f32x4*>(dbuf + 32 * c + 16 * hh + 8 * r4 + 4 * g);
 #pragma unroll
                   for (int e = 0; e < 4; e++) {
-                    float dpd = t0[gk][8 * hh + 4 * r4 + e];
+                    const float dp = t0[gk][8 * hh + 4 * r4 + e];
+                    float dpd = dp - dd[r4][e];
                     // dropped: dP = 0; kept: dP / keep_prob, scaled by the FMA that subtracts D
-                    if (DROP) dpd = __builtin_fmaf(__uint_as_float(__float_as_uint(dpd) & (uint32_t)__builtin_amdgcn_sbfe((int)dcw[gk], 16 * hh + 8 * r4 + e, 1)), a.inv_keep, nd[e]);
+                    if (DROP) dpd = __builtin_fmaf(__uint_as_float(__float_as_uint(dp) & (uint32_t)__builtin_amdgcn_sbfe((int)dcw[gk], 16 * hh + 8 * r4 + e, 1)), a.inv_keep, -dd[r4][e]);
                     // (an FMA with a zero addend keeps the fp16 -> fp32 conversion inside one mixed-precision instruction)
                     ds[4 * r4 + e] = __builtin_fmaf((float)ph[4 * r4 + e], dpd, 0.0f);
                   }

@@ -117,8 +117,8 @@ __global__ void __launch_bounds__(256) fa_bwd_dq64_kernel(const FaArgs a) {
     const float lq = a.lse[(int64_t)bh * a.Sq + row] * kLog2e - a.p_shift;
     nlq[gq] = -lq;
     if (g == 0) {
-      a.delta[(int64_t)bh * a.Sq + row] = -dl[gq];
-      a.nlse[(int64_t)bh * a.Sq + row] = -lq * a.inv_scale_log2e;   // (p_shift - LSE*log2(e)) / scale_log2e: the dK/dV kernel's score accumulators start from it
+      a.delta[(int64_t)bh * a.Sq + row] = dl[gq];
+      a.nlse[(int64_t)bh * a.Sq + row] = -lq;          // p_shift - LSE*log2(e): the exp2 offset the dK/dV kernel adds
     }
   }
 

@@ -107,7 +107,7 @@ struct FaArgs {
   const void* q; const void* k; const void* v;
   void* o; float* lse;                 // fwd outputs / bwd inputs
   const void* dout; void* dq; void* dk; void* dv;                // bwd only
-  float* delta; float* nlse;           // bwd workspace: -D = -rowsum(dO*O) and (p_shift - LSE*log2(e)) / scale_log2e, [B,N,Sq] each
+  float* delta; float* nlse;           // bwd workspace: D = rowsum(dO*O) and p_shift - LSE*log2(e), [B,N,Sq] each
   float* dkdv_part;                    // q_split > 1: per-slice dK / dV sums of the dK/dV kernel, [q_split][workgroup][wave][regs x 64 lanes]
   const uint8_t* mask; const uint8_t* drop; const void* alibi;   // mask / drop: elements of mask_es / drop_es bytes
   const uint8_t* blkflags;             // [MB, Tr, Tc] block classes of a dense mask
@@ -149,16 +149,14 @@ struct FaArgs {
   int kv_split;                        // forward kernel: slices of the key range, each on workgroups of its own (1 = no split)
   int dq_kg;                           // dQ kernel: key groups of the workgroup (dq_key_groups, fa_index_math.hpp)
   int dkdv_ngk;                        // dK/dV kernel: 32-key groups per wave (DkdvPlan, fa_index_math.hpp)
-  float inv_scale_log2e;               // 1 / scale_log2e
   int drop_visible;                    // keep bits: != 0 when those of key blocks outside the band (or past the causal / prefix limit) may be left out
 };
 static_assert(offsetof(FaArgs, fwd_part) > offsetof(FaArgs, philox_thr), "new fields stand behind those of the inner loops");
 
 // The bias a kernel variant is built for: none, any, or one value per key (row stride 0, the reference's ALiBi form) that
-// the DMA can stage.  The last spends nothing per score -- the initial value of the score accumulators (forward, dQ) or the
-// addend of the exponent's FMA (dK/dV) -- has the registers of the variants without a bias and, like them, a second body for
-// the causal pattern.  64 heads, 4096 x 4096, D128, causal mask tensor, against the variants for any bias (us): forward
-// 323 / 301, dQ 500 / 400, dK/dV 596 / 490.
+// the DMA can stage.  The last spends nothing per score -- it is the initial value of the score accumulators -- has the
+// registers of the variants without a bias and, like them, a second body for the causal pattern.  64 heads, 4096 x 4096,
+// D128, causal mask tensor, against the variants for any bias (us): forward 323 / 301, dQ 536 / 400, dK/dV 608 / 503.
 enum : int { kBiasNone = 0, kBiasAny = 1, kBiasKey = 2 };
 inline bool key_bias_stageable(const FaArgs& a) {
   return a.al_sq == 0 && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh) & 7)) == 0;

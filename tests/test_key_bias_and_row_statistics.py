@@ -1,9 +1,10 @@
-"""GPU tests of the kernel variants for a bias that depends on the key only, and of the dK/dV kernel's accumulators that
-start from the row statistics.  Key counts on the edges of the 64- and 128-key tiles, one to several query tiles (the
+"""GPU tests of the kernel variants for a bias that depends on the key only, and of the row statistics in the dK/dV kernel.
+Key counts on the edges of the 64- and 128-key tiles, one to several query tiles (the
 first one staged is ragged, the rest take the kept offsets), head dims with and without padding, grids that take one and
 two key groups per wave; every kind of mask, so that both bodies of the variants run; rows that see nothing but masked keys,
 whose LSE is near -10000; scales far below 1 / sqrt(D).  Reference: the operator in float32 with torch.  Gate: that of the parity tests (every element within
-2e-3 + 1e-3 |reference| in fp16, 2e-2 + 1e-2 |reference| in bf16)."""
+2e-3 + 1e-3 |reference| in fp16, 2e-2 + 1e-2 |reference| in bf16).  Where scores, dP and D are exact in float32 the
+kernel's own rounding is checked: P and dS are what one rounding of their difference to the row's statistic gives."""
 import pytest
 import torch
 
@@ -78,7 +79,7 @@ def test_grids_of_two_key_groups(D, mask, nxt, biased):
 @pytest.mark.parametrize("Sq, Sk, D, mask, scale", [
     (130, 140, 128, "blind rows", None), (300, 200, 64, "blind rows", None), (70, 256, 160, "blind rows", None), (257, 129, 40, "random", None),
     (200, 200, 64, None, 1e-3), (200, 200, 64, None, 1e-20), (200, 200, 128, None, 1e-35)])
-def test_row_statistics_in_the_accumulators(Sq, Sk, D, mask, scale):
+def test_rows_of_masked_keys_and_small_scales(Sq, Sk, D, mask, scale):
     _check(1, 4, Sq, Sk, D, torch.float16, mask, False, scale=scale)
 
 
@@ -95,3 +96,55 @@ def test_key_only_bias_without_a_mask_tensor():
         o, lse = _capi.fa_fwd(p, q)
         outs.append((o, lse) + _capi.fa_bwd(p, q, k, v, o, dO, lse))
     assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+@pytest.mark.parametrize("D", [64, 80, 128])
+@pytest.mark.parametrize("heads", [2, 256])                    # one and two key groups per wave
+@pytest.mark.parametrize("bias", ["none", "key", "full"])
+def test_p_takes_one_rounding_of_score_minus_lse(D, heads, bias):
+    """Scores (and bias / scale) are whole numbers near 16384, exact in float32 in any order, and LSE is close to them: P is
+    exp2 of scale*log2e * S - LSE*log2e, rounded once, and dV with one-hot dO is P in fp16.  The difference of two numbers in
+    the thousands taken in several roundings would move P by up to 1e-4, a quarter of an fp16 spacing, and 6 % of the entries with it;
+    exp2's own last place moves 3e-5 of them.  Gate: 1 %."""
+    g = torch.Generator(device=DEV).manual_seed(D + heads)
+    Sk, scale = 256, 0.125
+    const = 16 * 32 * 32
+    def ints(S):
+        x = torch.randint(-1, 2, (1, heads, S, D), generator=g, device=DEV).half()
+        x[..., D - 16:] = 32
+        return x
+    q, k, v = ints(D), ints(Sk), torch.randn(1, heads, Sk, D, generator=g, device=DEV).half()
+    dO = torch.eye(D, device=DEV).half().expand(1, heads, D, D).contiguous()
+    al = None if bias == "none" else torch.randint(-8, 9, (1, heads, 1 if bias == "key" else D, Sk), generator=g, device=DEV).half() / 4
+    S = q.double() @ k.double().transpose(2, 3) + (al.double() / scale if al is not None else 0)
+    assert float((S - const).abs().max()) < 256
+    lse = (scale * S.amax(3) + torch.rand(1, heads, D, generator=g, device=DEV, dtype=torch.float64)).float()
+    log2e = torch.tensor(1.4426950408889634, dtype=torch.float32, device=DEV)
+    mul, off = (torch.tensor(scale, dtype=torch.float32, device=DEV) * log2e).double(), (lse * log2e).double()
+    want = torch.exp2((S * mul - off[..., None]).float().double()).half()
+    p = _capi.make_params(q, k, v, scale=scale, alibi=al)
+    dv = _capi.fa_bwd(p, q, k, v, torch.zeros_like(q), dO, lse)[2]
+    differ = float((dv.transpose(2, 3) != want).double().mean())
+    assert differ < 0.01, f"{100 * differ:.2f} % of P"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("heads", [2, 256])
+def test_ds_takes_one_rounding_of_dp_minus_d(D, heads, dtype):
+    """dP is a sum of whole numbers, exact in float32 although it passes 2^18 on the way, and D is a fraction: with P = 1
+    (K = 0, LSE = 0) and one-hot Q, dK is dP - D in the element type, to the last bit."""
+    g = torch.Generator(device=DEV).manual_seed(D + heads)
+    Sk = 256
+    eye = torch.eye(D, device=DEV).to(dtype).expand(1, heads, D, D).contiguous()
+    dO = torch.ones(1, heads, D, D, device=DEV)
+    v = torch.randint(-1, 2, (1, heads, Sk, D), generator=g, device=DEV).float()
+    dO[..., :32], v[..., :16], v[..., 16:32] = 128, 128, -128
+    o = torch.zeros(1, heads, D, D, device=DEV)
+    o[..., D - 1] = torch.rand(1, heads, D, generator=g, device=DEV)
+    dO, v, o = dO.to(dtype), v.to(dtype), o.to(dtype)
+    k, lse = torch.zeros_like(v), torch.zeros(1, heads, D, device=DEV)
+    p = _capi.make_params(eye, k, v, scale=1.0)
+    dk = _capi.fa_bwd(p, eye, k, v, o, dO, lse)[1]
+    want = (dO.double() @ v.double().transpose(2, 3) - o[..., D - 1:].double()).transpose(2, 3).to(dtype)
+    assert torch.equal(dk, want), f"{int((dk != want).sum())} of {want.numel()} differ"
