@@ -54,7 +54,8 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
   constexpr bool TBIAS = BIAS == kBiasAny, RBIAS = BIAS == kBiasKey;
   constexpr bool RINGS = !(TBIAS || DROP);                // (the side-input variants have no registers for the rings)
   // Products ahead of the other wave's vector work, by wave priority, where a tile's products outlast it: 64 heads, 2048 x 2048
-  // causal, D128 121 -> 114 us, 4096 x 4096 429 -> 402, bf16 116 -> 110; D64 113 -> 114, D40 97 -> 100.  (The variants without the
+  // causal, D128 121 -> 114 us, 4096 x 4096 429 -> 402, bf16 116 -> 110; D64 113 -> 114, D40 97 -> 100, D80 82.4 -> 83.4 (16 heads,
+  // 4096 x 4096 132.5 -> 134.1), D160 95.9 -> 96.9 (one wave per SIMD).  (The variants without the
   // rings have no register left for the order it brings: with dropout eight more spills, 239 -> 320 us.)
   constexpr bool DQPRIO = D == 128 && RINGS;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -885,10 +886,15 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
     __syncthreads();
 
     // Wave priorities: every wave of a pair begins with its products and the two contend for the SIMD's matrix pipe.  By
-    // default the older (V role) wave wins; with the K role first -- its vector work is the shorter -- and the
-    // accumulating products ahead of the partner's vector work the step is 4 to 6 % shorter at head dim 128 (64 heads,
-    // 2048 x 2048 causal 150 -> 146 us, 4096 x 4096 548 -> 519; bf16 147 -> 140).  One key group per wave has fewer products
-    // to put in order: 96 heads, 1000 x 1000, D64 69 -> 72, D128 119 -> 121; head dim 80 178 -> 180.
+    // default the older (V role) wave wins.  At head dim 128 with two key groups the accumulating products go ahead of the
+    // partner's vector work and the K role, whose vector work is the shorter, goes first.  Without / with (us): 64 heads,
+    // 2048 x 2048 254 / 246, causal 145.6 / 145.1, bf16 139 / 141, key bias 4096 x 4096 504 / 474; 32 heads, 4096 x 4096 causal
+    // with dropout 303 / 300.  The variants for mask tensors leave the V role first: where it applies mask bits its vector
+    // work is the longer part of the step (64 heads, 2048 x 2048, three keys in ten masked: K role first 310, bf16 314, with dropout
+    // 339; V role first 290, 285, 332; no priorities 294, 285, 330; key padding 133 / 134 / 134.5).
+    // Elsewhere priorities gain nothing -- one key group per wave has fewer products to put in order: 96 heads, 1000 x 1000,
+    // D64 67 / 72, D128 119 / 122; head dim 80 177.5 / 178; 160 715 / 713, with dropout 213 / 218; 256 causal 539 / 534, with a
+    // mask tensor 289 / 298.
     constexpr bool PRIO = D == 128 && NGK == 2;
     // The K role runs one chunk behind the V role: in step n the V role recomputes P of chunk n,
     // publishes it and accumulates dV; the K role picks up P of chunk n-1.  One barrier per step,
@@ -913,7 +919,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
     }
     const uint8_t* flcol = (MASKT && a.mask_kind == kMaskDense) ? a.blkflags + (int64_t)mb * a.Tr * a.Tc + wkb : nullptr;
     if (!flwin_ready) flwin.init_descending(flcol, a.Tc, c_lo >> 2, c_hi >> 2, lane, (!TBIAS && flcol && a.blktail) ? a.blktail + (flcol - a.blkflags) : nullptr);
-    const bool kfirst = PRIO && __builtin_amdgcn_readfirstlane(wave) >= 4;
+    const bool kfirst = PRIO && !MASKT && __builtin_amdgcn_readfirstlane(wave) >= 4;
     for (int n = 0; n <= npos; n++) {
       if (kfirst) __builtin_amdgcn_s_setprio(1);
       if ((n & 1) && (n >> 1) + 1 < ntile) stage_next(i_hi - ((n >> 1) + 1), smem + ((((n >> 1) + 1) & 1) * STAGEB));
