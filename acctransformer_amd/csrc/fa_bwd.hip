@@ -780,7 +780,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
       // Read from LDS in the loop, the words cost no wait on the vector-memory counter, which would also wait
       // for the tile DMA in flight.
       const int idx = wave * 64 + lane, key = min(k0 + (idx >> 1), a.Sk - 1);
-      dma4(a.dropcol + ((((int64_t)bh * a.Tr + (i >> 1)) * a.Sk + key) << 2) + 2 * (i & 1) + (idx & 1),
+      dma4(a.dropcol + keep_col_entry(bh, a.Tr, i >> 1, a.Sk, key) + 2 * (i & 1) + (idx & 1),
            sb + 2 * TILEB + STATB + wave * 256);
     }
   };
@@ -816,8 +816,8 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
       dd.issue(dop, a.o_ss, i * 64, sb + TILEB);
       if (wave < 2) dma4_row((wave == 0 ? a.nlse : a.delta) + (int64_t)bh * a.Sq + i * 64, lane * 4, sb + 2 * TILEB + wave * 256);
       if (DROP) {
-        const int idx = wave * 64 + lane, key = min(k0 + (idx >> 1), a.Sk - 1);
-        dma4_row(a.dropcol + ((((int64_t)bh * a.Tr + (i >> 1)) * a.Sk) << 2) + 2 * (i & 1), (key << 4) + ((idx & 1) << 2),
+        const int idx = wave * 64 + lane;
+        dma4_row(a.dropcol + keep_col_entry(bh, a.Tr, i >> 1, a.Sk, k0) + 2 * (i & 1), keep_col_offset(min(k0 + (idx >> 1), a.Sk - 1) - k0, idx & 1),
                  sb + 2 * TILEB + STATB + wave * 256);
       }
     } else {

@@ -68,6 +68,12 @@ ACCT_HD uint32_t recip16(int n) { return (65536u + (uint32_t)n - 1u) / (uint32_t
 // byte offset of logical chunk `lc` in a row whose swz3(row) is `swz`
 ACCT_HD int swz_off(int lc, int swz) { return (lc ^ swz) << 4; }
 
+// The keep bits by key column (FaArgs::dropcol), [B*N, Tr, Sk] entries of four 32-bit words: index of the first word of an
+// entry, and the byte offset of word `w` of the entry `dk` keys after it.  A workgroup addresses the entries of its keys
+// as a 64-bit base for its first one and such an offset per lane, which stays below 4 KB whatever Sk is.
+ACCT_HD int64_t keep_col_entry(int64_t bh, int Tr, int qb, int Sk, int key) { return ((bh * Tr + qb) * Sk + key) * 4; }
+ACCT_HD uint32_t keep_col_offset(int dk, int w) { return (uint32_t)dk * 16u + (uint32_t)w * 4u; }
+
 // The kernels are built for the head dims 40, 64, 80, 128, 160 and 256.  Any other multiple of 8 runs on the next
 // built size of its row layout (128-, 256- or 512-byte LDS rows): the columns past the head dim are never loaded
 // as operands (zero fragments) and never stored.

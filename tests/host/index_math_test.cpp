@@ -226,6 +226,19 @@ static void test_div_small() {
     for (int idx = 0; idx < 1024; idx++) CHECK(div_small(idx, recip16(n)) == idx / n, "div_small(%d, %d)", idx, n);
 }
 
+// a workgroup's base and a lane's 32-bit offset reach the entry of every one of its keys, also where 16 bytes a key pass 4 GB
+static void test_keep_columns() {
+  for (int Sk : {1, 200, 4096, (1 << 28) + 200, 0x7fffff00})
+    for (int k0 : {0, 128, Sk / 256 * 256, (Sk - 1) / 128 * 128})
+      for (int t : {0, 1, 127, 255}) {
+        if (k0 >= Sk) continue;
+        const int dk = t < Sk - 1 - k0 ? t : Sk - 1 - k0, key = k0 + dk;
+        const int64_t want = ((((int64_t)5 * 3 + 2) * Sk + key) * 4 + 1) * 4;          // (head 5, block 2 of 3, word 1)
+        const uint32_t off = keep_col_offset(dk, 1);
+        CHECK(keep_col_entry(5, 3, 2, Sk, k0) * 4 + off == want && off < 4096, "Sk %d k0 %d key %d", Sk, k0, key);
+      }
+}
+
 int main() {
   test_wg_map();
   test_swizzle_rows<64>();
@@ -238,6 +251,7 @@ int main() {
   test_dkdv_split();
   test_slice_plans();
   test_visible_row_keys();
+  test_keep_columns();
   test_div_small();
   if (failures) printf("%d checks failed\n", failures);
   else printf("index math: all checks passed\n");
