@@ -180,8 +180,9 @@ ACCT_DEV void fa_bwd_dq_body(const FaArgs& a) {
   vdma.plan(a.v_ss, cpr);
   // bias tiles of this wave's rows are staged through a wave-private LDS region one tile ahead
   ACCT_LDS char* bias_lds = smem + 4 * TILEB + wave * (QG * 4096);
-  const bool bias_staged = RBIAS || (TBIAS && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh | a.al_sq) & 7)) == 0);
-  const bool row_bias = RBIAS || (TBIAS && a.al_sq == 0);           // the bias depends on the key only: one 128-byte row per tile
+  const bool bias_staged = RBIAS || (TBIAS && bias_stageable(a));
+  // the bias depends on the key only: one 128-byte row per tile (without dropout a staged one has the kBiasKey variants)
+  const bool row_bias = RBIAS || (TBIAS && DROP && a.al_sq == 0);
   auto stage_bias = [&](int jn) {
 #pragma unroll
     for (int gq = 0; gq < QG; gq++) {
@@ -651,9 +652,9 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
   constexpr int WK = 32 * NGK;                      // key rows per wave pair
   constexpr int BNK = 4 * WK;                       // key rows per workgroup
   constexpr int TILEB = 64 * C::PITCH;
-  constexpr int STATB = 2 * 64 * 4;                 // -LSE*log2(e) and D of the 64 rows of a tile
+  constexpr int STATB = 2 * 64 * 4;                 // p_shift - LSE*log2(e) and D of the 64 rows of a tile
   constexpr int DROPB = DROP ? 2048 : 0;            // keep bits of the tile's 64 rows for 256 keys (NGK = 1 reads the first 128): [key][2 chunks] words
-  constexpr int STAGEB = 2 * TILEB + STATB + DROPB; // one buffer: Q tile | dO tile | -LSE*log2(e) | D | keep bits
+  constexpr int STAGEB = 2 * TILEB + STATB + DROPB; // one buffer: Q tile | dO tile | p_shift - LSE*log2(e) | D | keep bits
   constexpr int PXB = 2048 * NGK;                   // P of one pair and chunk: 64 lanes x 32 bytes per key group
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   ACCT_LDS char* smem = (ACCT_LDS char*)smem_raw;   // [2 stage buffers][2 x 4 pair P buffers]
@@ -718,7 +719,8 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
   // stationary B operands: K fragments (V role) or V fragments (K role) of the pair's key rows;
   // lane holds key row 32 gk + l32, d = 16t + 8g ..
   // The last PARK k-steps of the second key group live in a wave-private LDS slab instead of
-  // registers (16 VGPRs at D = 128): that is what lets two waves share a SIMD without spilling.
+  // registers (16 to 24 VGPRs at D = 128): that is what lets two waves share a SIMD without spilling (bias and dropout
+  // together still spill two).
   constexpr int PARK = dkdv_park<D, TBIAS, MASKT, NGK>();
   V8 bf[NGK][C::KS];
   ACCT_LDS char* park = pexch + 8 * PXB + wave * (PARK * 1024) + lane * 16;
@@ -761,8 +763,9 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
   const T* alibip = BIAS ? (const T*)a.alibi + b * a.al_sb + h * a.al_sh : nullptr;
 
   // stage q tile i into buffer `sb`: Q and dO by 16-byte DMA (2 instructions per wave each),
-  // LSE (wave 0) and D (wave 1) by 4-byte DMA; rows past Sq repeat the last row
-  // (addresses are re-derived per call here: this kernel has no registers to spare for a TileDma plan)
+  // p_shift - LSE*log2(e) (wave 0) and D (wave 1) by 4-byte DMA; rows past Sq repeat the last row
+  // (this kernel has no registers to spare for a TileDma plan: the addresses are derived anew here, which the variants
+  // with a tile bias and the wide head dims do for every tile, the others for the first one only: stage_next)
   auto stage = [&](int i, ACCT_LDS char* sb) {
     if ((i + 1) * 64 <= a.Sq) {
       TileDma<T, D, 64, NW>::issue_direct(qp, a.q_ss, i * 64, sb, a.hd >> 3);
@@ -833,8 +836,7 @@ ACCT_DEV void fa_bwd_dkdv_body(const FaArgs& a) {
 #pragma unroll
   for (int gk = 0; gk < NGK; gk++)
     brow[gk] = (row_bias && !krole) ? (float)alibip[min(wk0 + 32 * gk + l32, a.Sk - 1)] * a.inv_scale : 0.f;
-  const bool bias_staged = TBIAS && !row_bias && !krole && wk0 < a.Sk && (a.Sk & 7) == 0 &&
-                           (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh | a.al_sq) & 7)) == 0;
+  const bool bias_staged = TBIAS && !row_bias && !krole && wk0 < a.Sk && bias_stageable(a);
   auto stage_bias = [&](int cn) { bias_tile_dma<T, false>(alibip, a.al_sq, cn * 32, a.Sq, wk0, a.Sk, bias_lds); };
 
   // per-chunk predicates of this pair (chunk = 32 query rows; two per staged tile), as bits of one value

@@ -158,9 +158,11 @@ static_assert(offsetof(FaArgs, fwd_part) > offsetof(FaArgs, philox_thr), "new fi
 // registers of the variants without a bias and, like them, a second body for the causal pattern.  64 heads, 4096 x 4096,
 // D128, causal mask tensor, against the variants for any bias (us): forward 323 / 301, dQ 536 / 400, dK/dV 608 / 503.
 enum : int { kBiasNone = 0, kBiasAny = 1, kBiasKey = 2 };
-inline bool key_bias_stageable(const FaArgs& a) {
-  return a.al_sq == 0 && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh) & 7)) == 0;
+// The DMA brings a bias into LDS in 16-byte chunks of its rows.
+__host__ __device__ __forceinline__ bool bias_stageable(const FaArgs& a) {
+  return (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh | a.al_sq) & 7)) == 0;
 }
+inline bool key_bias_stageable(const FaArgs& a) { return a.al_sq == 0 && bias_stageable(a); }
 
 enum : int { kMaskNone = 0, kMaskDense = 1, kMaskTile = 3, kMaskCausal = 4 };
 enum : uint8_t { kBlkClean = 0, kBlkApply = 1, kBlkSkip = 2, kBlkTriu = 3 };

@@ -156,12 +156,11 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   // bias is added, in which case they become scale*s + bias first (one mixed-precision FMA per score:
   // the fp16 / bf16 bias is an operand as it is).
   // A key-only bias (row stride 0) that the DMA can stage goes in as the INITIAL value of the score accumulators
-  // instead (bias / scale, the MFMAs add q.k): the scores stay in raw units and nothing is spent per score.
-  const bool bias_staged = BIAS && (a.Sk & 7) == 0 && (((uintptr_t)a.alibi & 15) | ((a.al_sb | a.al_sh | a.al_sq) & 7)) == 0;
-  // (the launcher picks 128-key tiles for a bias only when both hold: known at compile time there)
-  const bool row_bias = BIAS && (KT == 4 || a.al_sq == 0);   // the bias depends on the key only: one row per tile
+  // instead (bias / scale, the MFMAs add q.k): the scores stay in raw units and nothing is spent per score.  The launcher
+  // picks 128-key tiles for such a bias and for no other.
   constexpr bool acc_bias = BIAS && KT == 4;
   constexpr bool scaled = BIAS && !acc_bias;                   // scores are turned into scale*s + bias before the softmax
+  const bool bias_staged = acc_bias || (scaled && bias_stageable(a));
   const float cmul = scaled ? kLog2e : a.scale_log2e;
   const float madd = scaled ? kMaskFill : a.mask_add_raw;          // the additive -10000 in the units of s
   const float lazy_thr = 8.0f / cmul;                              // 8 octaves, in the units of s
@@ -188,7 +187,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   auto stage_bias = [&](int jn) {
 #pragma unroll
     for (int gq = 0; gq < QG; gq++) {
-      if (row_bias) bias_row_dma<T>(alibip, jn * BN, a.Sk, bias_lds + gq * 4096 + (acc_bias ? (jn & 1) * 256 : 0));
+      if constexpr (acc_bias) bias_row_dma<T>(alibip, jn * BN, a.Sk, bias_lds + (jn & 1) * 256);
       else bias_tile_dma<T>(alibip, a.al_sq, wq0 + 32 * gq, a.Sq, jn * 64, a.Sk, bias_lds + gq * 4096);
     }
   };
@@ -320,7 +319,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
 #pragma unroll
           for (int c = 0; c < KB; c++)
 #pragma unroll
-            for (int r4 = 0; r4 < 4; r4++) bv[c][r4] = bias_tile_read<T>(bias_lds + gq * 4096, row_bias ? 0 : l32, 4 * (kg * KTW + c) + r4, g);
+            for (int r4 = 0; r4 < 4; r4++) bv[c][r4] = bias_tile_read<T>(bias_lds + gq * 4096, l32, 4 * (kg * KTW + c) + r4, g);
           if (gq == QG - 1) {
             // the tile is in registers: its LDS region can take the next tile, which has the rest of
             // this step to land (the end-of-step wait covers it)
@@ -733,8 +732,9 @@ template <typename T, int D, int NW, int KG, bool BIAS, bool DROP>
 static hipError_t launch_fwd_t(const FaArgs& a, hipStream_t st) {
   // K/V stream in tiles of 128 keys where registers and LDS allow (8 waves, D <= 128): twice the
   // matrix work between two barriers, -2 % (causal) to -6 % (full).  A bias tile per wave does not fit beside
-  // them; a key-only bias that the DMA can stage (the kernel's own test, repeated here) is a 256-byte row and does.
+  // them; a key-only bias that the DMA can stage is a 256-byte row and does.
   constexpr bool BIG = NW == 8 && D <= 128;
+  static_assert(BIG || !BIAS, "the bias variants rest on this choice");
   if constexpr (BIG && BIAS) {
     return key_bias_stageable(a) ? launch_fwd_kt<T, D, NW, BIAS, DROP, 4, KG>(a, st) : launch_fwd_kt<T, D, NW, BIAS, DROP, 2, KG>(a, st);
   } else {
