@@ -37,3 +37,13 @@ def test_the_gpu_tests_of_one_kernel_run_it(tmp_path):
     for row, plan in zip(rows, plans):
         assert (plan["kg"], plan["kv_split"], plan["dq_kg"], plan["q_split"]) == (1, 1, 1, 1), (row, plan)
     assert sum(plan["ngk"] == 2 for row, plan in zip(rows, plans) if row[4] == 40) >= 3, plans
+
+
+def test_the_two_key_group_tests_run_two(tmp_path):
+    """The shapes written for two key groups per wave of the dK/dV kernel get them from the plan."""
+    import test_key_bias_and_row_statistics as gpu
+    rows = [shape + (nxt == 0,) for shape, mask, nxt, biased, keep in gpu.TWO_KEY_GROUPS]
+    for row, plan in zip(rows, _plans(tmp_path, rows)):
+        assert (plan["ngk"], plan["q_split"]) == (2, 1), (row, plan)
+    rows = [(1, heads, D, 256, D, False) for heads, D in ((256, 64), (256, 80), (256, 128), (2, 64), (2, 80), (2, 128))]
+    assert [plan["ngk"] for plan in _plans(tmp_path, rows)] == [2, 2, 2, 1, 1, 1]

@@ -2,7 +2,7 @@
 Key counts on the edges of the 64- and 128-key tiles, one to several query tiles (the
 first one staged is ragged, the rest take the kept offsets), head dims with and without padding, grids that take one and
 two key groups per wave; every kind of mask, so that both bodies of the variants run; rows that see nothing but masked keys,
-whose LSE is near -10000; scales far below 1 / sqrt(D).  Reference: the operator in float32 with torch.  Gate: that of the parity tests (every element within
+whose LSE is near -10000; scales far below 1 / sqrt(D).  Reference: the operator in float64 with torch.  Gate: that of the parity tests (every element within
 2e-3 + 1e-3 |reference| in fp16, 2e-2 + 1e-2 |reference| in bf16).  Where scores, dP and D are exact in float32 the
 kernel's own rounding is checked: P and dS are what one rounding of their difference to the row's statistic gives."""
 import pytest
@@ -32,26 +32,37 @@ def _mask(kind, B, Sq, Sk, g):
     return None
 
 
-def _check(B, N, Sq, Sk, D, dtype, mask, biased, scale=None, nxt=65536):
+def _check(B, N, Sq, Sk, D, dtype, mask, biased, scale=None, nxt=65536, prev=65536, prefix=0, per_batch=False, low=None, keep=1.0):
     g = torch.Generator(device=DEV).manual_seed(Sq * 7 + Sk + D)
     scale = D ** -0.5 if scale is None else scale
     q, k, v, dO = (torch.randn(B, N, S, D, generator=g, device=DEV).to(dtype) for S in (Sq, Sk, Sk, Sq))
     m = _mask(mask, B, Sq, Sk, g)
-    al = torch.randn(1, N, 1, Sk, generator=g, device=DEV).to(dtype) if biased else None
-    qf, kf, vf, df = (t.float() for t in (q, k, v, dO))
+    al = torch.randn(B if per_batch else 1, N, 1, Sk, generator=g, device=DEV).to(dtype) if biased else None
+    if low is not None:
+        al[..., 1::3] = low if low != "lowest" else torch.finfo(dtype).min
+    drop = (torch.rand(B, N, Sq, Sk, generator=g, device=DEV) < keep).to(torch.uint8) if keep < 1 else None
+    qf, kf, vf, df = (t.double() for t in (q, k, v, dO))     # (beside a mask's 10000, float32 rounds a score to 5e-4)
     s = qf @ kf.transpose(2, 3) * scale
-    s = s + al.float() if biased else s
-    s = s - 10000.0 * m[:, None].float() if m is not None else s
-    if nxt == 0:
-        b = torch.arange(Sk, device=DEV)[None, :] // 128 > torch.arange(Sq, device=DEV)[:, None] // 128
-        s = s.masked_fill(b, float("-inf"))
+    s = s + al.double() if biased else s
+    s = s - 10000.0 * m[:, None].double() if m is not None else s
+    i, j = torch.arange(Sq, device=DEV)[:, None], torch.arange(Sk, device=DEV)[None, :]
+    s = s.masked_fill((j // 128 > i // 128 + nxt) | (j // 128 < i // 128 - prev), float("-inf"))
+    if prefix:
+        s = s.masked_fill(j >= (i // prefix + 1) * prefix, float("-inf"))
     x = [t.clone().requires_grad_(True) for t in (q, k, v)]
-    o, lse = get_flash_attention(scale=scale, next_block_num=nxt)(*x, m, None, al)
-    got = (o,) + torch.autograd.grad(o, x, dO)
+    if prefix:                                           # (the C interface only)
+        p = _capi.make_params(q, k, v, scale=scale, alibi=al, prev_block_num=prev, next_block_num=nxt, row_block_prefix=prefix, drop_mask=drop,
+                              keep_prob=keep, mask_kind=_capi.MASK_DENSE_U8 if m is not None else _capi.MASK_NONE, attn_mask=m)
+        o, lse = _capi.fa_fwd(p, q)
+        got = (o,) + _capi.fa_bwd(p, q, k, v, o, dO, lse)
+    else:
+        o, lse = get_flash_attention(scale=scale, prev_block_num=prev, next_block_num=nxt, keep_prob=keep)(*x, m, drop, al)
+        got = (o,) + torch.autograd.grad(o, x, dO)
     P = torch.softmax(s, 3)
+    kept = drop.double() / keep if drop is not None else 1.0
     # (D from the O that the backward is given, as it defines it)
-    dS = P * (df @ vf.transpose(2, 3) - (df * o.detach().float()).sum(3, keepdim=True))
-    want = (P @ vf, dS @ kf * scale, dS.transpose(2, 3) @ qf * scale, P.transpose(2, 3) @ df)
+    dS = P * (df @ vf.transpose(2, 3) * kept - (df * o.detach().double()).sum(3, keepdim=True))
+    want = ((P * kept) @ vf, dS @ kf * scale, dS.transpose(2, 3) @ qf * scale, (P * kept).transpose(2, 3) @ df)
     wide = dtype == torch.bfloat16
     for name, a, b in zip(("O", "dQ", "dK", "dV"), want, got):
         ok, ratio, mx = orc.tolerance_gate(a.detach().cpu().numpy(), b.detach().float().cpu().numpy(), atol=2e-2 if wide else 2e-3, rtol=1e-2 if wide else 1e-3)
@@ -69,11 +80,35 @@ def test_key_only_bias(Sq, Sk, D, mask, nxt, dtype):
     _check(2, 3, Sq, Sk, D, dtype, mask, True, nxt=nxt)
 
 
-@pytest.mark.parametrize("D, mask, nxt, biased", [
-    (128, "causal", 0, True), (128, "padded", 65536, True), (64, "random", 65536, True), (80, None, 65536, True),
-    (128, "causal", 0, False), (128, "padded", 65536, False), (64, None, 65536, False), (80, "causal", 65536, False)])
-def test_grids_of_two_key_groups(D, mask, nxt, biased):
-    _check(2, 64, 584, 512, D, torch.float16, mask, biased, nxt=nxt)
+# (B, N, Sq, Sk, D), mask, next_block_num, key-only bias, keep_prob: tests/test_index_math.py checks that the dK/dV plan gives
+# each two key groups per wave.  (A causal launch of fewer rows has one.)
+TWO_KEY_GROUPS = [
+    ((2, 64, 768, 768, 128), "causal", 0, True, 1.0), ((2, 64, 584, 512, 128), "padded", 65536, True, 1.0), ((2, 64, 584, 512, 64), "random", 65536, True, 1.0),
+    ((2, 64, 584, 512, 80), None, 65536, True, 1.0), ((2, 64, 768, 768, 128), "causal", 0, False, 1.0), ((2, 64, 584, 512, 128), "padded", 65536, False, 1.0),
+    ((2, 64, 584, 512, 64), None, 65536, False, 1.0), ((2, 64, 584, 512, 80), "causal", 65536, False, 1.0), ((2, 64, 584, 512, 128), "random", 65536, False, 1.0),
+    ((2, 64, 584, 456, 128), "padded", 65536, False, 0.8), ((2, 64, 768, 768, 128), "causal", 0, False, 0.8), ((2, 64, 584, 512, 64), "random", 65536, True, 0.8),
+    ((2, 64, 584, 500, 128), None, 65536, True, 0.8)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape, mask, nxt, biased, keep", TWO_KEY_GROUPS)
+def test_grids_of_two_key_groups(shape, mask, nxt, biased, keep, dtype):
+    _check(*shape, dtype, mask, biased, nxt=nxt, keep=keep)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Sq, Sk, D, mask, prev, nxt, prefix, low", [
+    (300, 392, 128, "random", 1, 1, 0, None), (520, 520, 64, "causal", 0, 0, 0, None), (640, 640, 80, None, 65536, 65536, 256, "lowest"),
+    (400, 456, 128, "padded", 65536, 65536, 0, float("-inf")), (385, 264, 128, "blind rows", 2, 65536, 128, "lowest"), (700, 704, 128, "causal", 65536, 0, 0, float("-inf"))])
+def test_key_only_bias_per_batch_entry(Sq, Sk, D, mask, prev, nxt, prefix, low, dtype):
+    """One bias per batch entry and head, in bands, under row prefixes, and with keys that the bias hides."""
+    _check(3, 2, Sq, Sk, D, dtype, mask, True, prev=prev, nxt=nxt, prefix=prefix, per_batch=True, low=low)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D, mask, keep", [(256, "random", 1.0), (256, None, 0.8), (256, "padded", 0.8), (160, "random", 1.0), (160, "random", 0.8)])
+def test_wide_head_dims_over_several_query_tiles(D, mask, keep, dtype):
+    _check(2, 3, 420, 390, D, dtype, mask, False, keep=keep)
 
 
 @pytest.mark.parametrize("Sq, Sk, D, mask, scale", [
