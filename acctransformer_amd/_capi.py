@@ -110,6 +110,33 @@ def load():
     return lib
 
 
+_native = None
+
+
+def native():
+    """The call path in native code (csrc/torch_call.cpp, loaded once).  Raises if it has not been built."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from acctransformer_amd import _native as module
+        except ImportError as e:
+            raise ImportError("acctransformer_amd/_native.so does not load: build it with `make -C acctransformer_amd/csrc` "
+                              "(or `python -c 'import __graft_entry__ as g; g.build()'`)") from e
+        module.setup(AcctError, _params_view)
+        _native = module
+    return _native
+
+
+def _params_view(raw, tensors, entry):
+    """The parameters of a recorded native call, as `make_params` would have left them."""
+    p = AcctFaParams.from_buffer_copy(raw)
+    p._keepalive = tensors
+    if entry is not None:
+        p._mask_bits_entry = entry
+    return p
+
+
 def _check(rc):
     if rc != 0:
         raise AcctError(rc, load().acct_last_error().decode())

@@ -121,19 +121,22 @@ def _classify_mask(attn_mask, Sq, Sk, io_dtype):
 _mask_bits_cache = {}
 
 
+def _mask_bits_hit(mask_tensor, kind, B, Sq, Sk, prev_block_num, next_block_num, row_block_prefix, device):
+    """(what the pre-pass results of `mask_tensor` depend on, the kept record of them or None)."""
+    sig = (kind, B, Sq, Sk, prev_block_num, next_block_num, row_block_prefix, _capi._stream(device), mask_tensor.data_ptr())
+    hit = _mask_bits_cache.get(id(mask_tensor))
+    if hit is not None and hit[0]() is mask_tensor and hit[1] == mask_tensor._version and hit[2] == sig:
+        return sig, hit
+    return sig, None
+
+
 def _attach_mask_bits(p, mask_tensor, device):
     """Points `p` at the pre-pass results of `mask_tensor` (the tensor handed to the library): a filled buffer
     from an earlier call, or a fresh one that `_mask_bits_done(p)` marks as filled once a call has run."""
-    if p.mask_kind not in (_capi.MASK_DENSE_U8, _capi.MASK_DENSE_F16, _capi.MASK_TILE_U8, _capi.MASK_TILE_F16):
+    if p.mask_kind not in _capi._TENSOR_MASKS:
         return
-    stream = _capi._stream(device)
-    sig = (p.mask_kind, p.B, p.Sq, p.Sk, p.prev_block_num, p.next_block_num, p.row_block_prefix, stream,
-           mask_tensor.data_ptr())
-    key = id(mask_tensor)
-    hit = _mask_bits_cache.get(key)
-    if hit is not None and hit[0]() is mask_tensor and hit[1] == mask_tensor._version and hit[2] == sig:
-        entry = hit
-    else:
+    sig, entry = _mask_bits_hit(mask_tensor, p.mask_kind, p.B, p.Sq, p.Sk, p.prev_block_num, p.next_block_num, p.row_block_prefix, device)
+    if entry is None:
         buf = _capi.attach_mask_bits(p, device)
         if buf is None:
             return
@@ -141,7 +144,7 @@ def _attach_mask_bits(p, mask_tensor, device):
             for k_ in [k_ for k_, v_ in _mask_bits_cache.items() if v_[0]() is None]:
                 del _mask_bits_cache[k_]
         entry = (weakref.ref(mask_tensor), mask_tensor._version, sig, buf, [False])
-        _mask_bits_cache[key] = entry
+        _mask_bits_cache[id(mask_tensor)] = entry
     p.mask_bits = entry[3].data_ptr()
     p.mask_bits_filled = 1 if entry[4][0] else 0
     p._keepalive.append(entry[3])
@@ -209,22 +212,65 @@ def _rows_contiguous(t):
     return t if t.stride(-1) == 1 else t.contiguous()
 
 
-def _nothing_to_record(*tensors):
-    """No gradient, tangent, transform or trace can want to know of this call: plain tensors, none of which -- side inputs
-    included -- asks for a gradient in this mode, outside vmap / jvp / grad transforms, forward-mode levels and
-    compilation.  The forward then runs without an autograd function around it, whose bookkeeping costs a small call
-    half of its host time."""
+_UNRECORDED, _RECORDED, _UNUSUAL = 0, 1, 2
+
+
+def _call_kind(q, k, v, *side):
+    """_UNRECORDED: no gradient, tangent, transform or trace can want to know of this call -- plain tensors, none of which
+    (side inputs included) asks for a gradient in this mode, outside vmap / jvp / grad transforms, forward-mode levels and
+    compilation; it runs without an autograd function around it.  _RECORDED: the same, but q, k or v ask for a gradient.
+    _UNUSUAL: everything else, which the Python autograd function takes."""
     if (torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0 or torch.compiler.is_compiling()
             or torch._C._get_tracing_state() is not None):
-        return False
+        return _UNUSUAL
     record = torch.is_grad_enabled()
-    for t in tensors:
+    for t in side:
         if type(t) in _PLAIN:
             if record and t.requires_grad:
-                return False
+                return _UNUSUAL
         elif t is not None and not _is_seed_pair(t):
-            return False
-    return True
+            return _UNUSUAL
+    if not (type(q) in _PLAIN and type(k) in _PLAIN and type(v) in _PLAIN):
+        return _UNUSUAL
+    return _RECORDED if record and (q.requires_grad or k.requires_grad or v.requires_grad) else _UNRECORDED
+
+
+def _native_call(kind_of_call, q, k, v, attn_mask, dropout_mask, alibi_mask, prev_block_num, next_block_num, scale, keep_prob,
+                 row_block_prefix):
+    """A call that is not _UNUSUAL in native code (csrc/torch_call.cpp): (O, LSE) with their graph, or None where the
+    Python path has to look at the call (other devices; shapes and dtypes that it refuses in its own words)."""
+    if not (q.is_cuda and k.is_cuda and v.is_cuda and q.dim() == 4 and k.dim() == 4 and v.dim() == 4):
+        return None
+    kind, mask, entry, bits, filled = _capi.MASK_NONE, None, None, None, False
+    if attn_mask is not None:
+        Sq, Sk = q.shape[2], k.shape[2]
+        kind, mask = _classify_mask(attn_mask, Sq, Sk, q.dtype)
+        if mask is None:                                  # (DETECT_CAUSAL_MASKS found the causal pattern)
+            return None
+        if not mask.is_cuda:
+            return None
+        _, entry = _mask_bits_hit(mask, kind, q.shape[0], Sq, Sk, min(prev_block_num, _capi.BLOCK_UNBOUNDED),
+                                  min(next_block_num, _capi.BLOCK_UNBOUNDED), row_block_prefix, q.device)
+        if entry is None:
+            if not (q.stride(3) == 1 and k.stride(3) == 1 and v.stride(3) == 1):
+                return None
+            p = _capi.make_params(q, k, v, scale=scale, prev_block_num=prev_block_num, next_block_num=next_block_num, mask_kind=kind,
+                                  attn_mask=mask, row_block_prefix=row_block_prefix)
+            _attach_mask_bits(p, mask, q.device)
+            entry = p._mask_bits_entry
+        bits, filled = entry[3], entry[4][0]
+    drop, keep, philox, seed, offset = None, 1.0, False, 0, 0
+    if dropout_mask is not None:
+        drop, keep, pair = _prepare_dropout(dropout_mask, keep_prob, q.dtype)
+        if pair is not None:
+            philox, seed, offset = True, pair[0] & 0xFFFFFFFFFFFFFFFF, pair[1] & 0xFFFFFFFF
+    if alibi_mask is not None and alibi_mask.dtype != q.dtype:
+        alibi_mask = alibi_mask.to(q.dtype)
+    out = _capi.native().forward(kind_of_call == _RECORDED, q, k, v, kind, mask, bits, filled, entry, drop, seed, offset, philox, alibi_mask,
+                                 prev_block_num, next_block_num, scale, keep, row_block_prefix)
+    if entry is not None and out is not None:
+        entry[4][0] = True
+    return out
 
 
 class _FlashAttentionFn(torch.autograd.Function):
@@ -286,9 +332,18 @@ def get_flash_attention(prev_block_num=65536, next_block_num=65536, tiling_stgy_
     alibi_mask=None) -> (output [B,N,Sq,D] in q's dtype, rowsum fp32 [B,N,Sq]),
     differentiable in query, key and value."""
     _check_strategy(tiling_stgy_name)
+    # (plain numbers cannot change between two calls; whatever else stands for one is read anew by the Python path)
+    plain_numbers = (type(scale) in (int, float) and type(keep_prob) in (int, float, type(None)) and type(prev_block_num) is int
+                     and type(next_block_num) is int and type(row_block_prefix) is int)
 
     def fa_forward(query, key, value, attn_mask=None, dropout_mask=None, alibi_mask=None):
-        if _nothing_to_record(query, key, value, attn_mask, dropout_mask, alibi_mask):
+        kind = _call_kind(query, key, value, attn_mask, dropout_mask, alibi_mask)
+        if plain_numbers and kind != _UNUSUAL:
+            out = _native_call(kind, query, key, value, attn_mask, dropout_mask, alibi_mask, prev_block_num, next_block_num, scale,
+                               keep_prob, row_block_prefix)
+            if out is not None:
+                return out
+        if kind == _UNRECORDED:
             q, k, v = _rows_contiguous(query), _rows_contiguous(key), _rows_contiguous(value)
             p = _build_params(q, k, v, attn_mask, dropout_mask, alibi_mask, prev_block_num, next_block_num, scale, keep_prob,
                               row_block_prefix)

@@ -21,6 +21,7 @@ from __future__ import annotations
 import torch
 
 from acctransformer_amd import _capi
+from acctransformer_amd.flash_attention.ops.flash_attention.flash_attention_impl import _UNUSUAL, _call_kind
 
 __all__ = ["flash_attention_tik"]
 
@@ -33,8 +34,11 @@ def flash_attention_tik(q, k, v, y=None, kernel_name="flash_attention_tik"):
         raise TypeError("q, k and v must be float16")  # op_info_cfg/ai_core/ascend310p: float16 only
     q4, k4, v4 = (t.unsqueeze(0) if t.dim() == 3 else t for t in (q, k, v))
     q4, k4, v4 = (t if t.stride(-1) == 1 else t.contiguous() for t in (q4, k4, v4))
-    p = _capi.make_params(q4, k4, v4, scale=1.0)
-    o, _ = _capi.fa_fwd(p, q4)
+    out = None
+    if q4.is_cuda and _call_kind(q4, k4, v4) != _UNUSUAL:
+        out = _capi.native().forward(False, q4, k4, v4, _capi.MASK_NONE, None, None, False, None, None, 0, 0, False, None,
+                                     _capi.BLOCK_UNBOUNDED, _capi.BLOCK_UNBOUNDED, 1.0, 1.0, 0)
+    o, _ = out or _capi.fa_fwd(_capi.make_params(q4, k4, v4, scale=1.0), q4)
     o = o.reshape(out_shape)
     if y is not None:
         y.copy_(o)
