@@ -280,6 +280,13 @@ acct::FwdPlan plan_forward(const acct_fa_params* p, bool can_split, int n_cu) {
   const int row_keys = acct::visible_row_keys(p->Sq, p->Sk, p->prev_block_num, p->next_block_num, p->row_block_prefix);
   return acct::fwd_plan(p->B, p->N, p->Sq, p->Sk, p->D, p->alibi || dropout_on(p), is_tri(p), can_split, n_cu, row_keys, ends_at_query(p));
 }
+// One query row per head without side inputs has a kernel of its own (fa_fwd_row.hip): the keys it sees, 0 for other calls.
+int row_keys(const acct_fa_params* p) {
+  if (p->Sq != 1 || p->mask_kind != ACCT_MASK_NONE || p->alibi || dropout_on(p)) return 0;
+  // (32-bit arithmetic in the kernel: a lane's offset within a load is up to 7 rows, batches times parts stay below 2^31)
+  if (p->k_stride[2] >= 1 << 26 || p->v_stride[2] >= 1 << 26 || p->Sk > 1 << 29) return 0;
+  return acct::visible_row_keys(1, p->Sk, p->prev_block_num, p->next_block_num, p->row_block_prefix);
+}
 acct::DkdvPlan plan_dkdv(const acct_fa_params* p, size_t room, int n_cu) {
   return acct::dkdv_plan(p->B, p->N, p->Sq, p->Sk, p->D, is_tri(p), room, n_cu, p->prev_block_num, p->mask_kind == ACCT_MASK_CAUSAL ? 0 : p->next_block_num);
 }
@@ -323,7 +330,8 @@ size_t acct_fa_fwd_workspace_bytes(const acct_fa_params* p) {
 
 size_t acct_fa_fwd_split_workspace_bytes(const acct_fa_params* p) {
   if (!p || p->B <= 0 || p->N <= 0 || p->Sq <= 0 || p->Sk <= 0 || p->D <= 0) return 0;
-  const size_t part = plan_forward(p, true, 256).part_bytes;
+  const int row = row_keys(p);
+  const size_t part = row ? acct::row_plan(p->B, p->N, row, p->D, true).part_bytes : plan_forward(p, true, 256).part_bytes;
   const size_t need = acct_fa_fwd_workspace_bytes(p);
   return part ? align_up(need, 256) + part : need;
 }
@@ -384,8 +392,18 @@ int acct_fa_fwd(const acct_fa_params* p, void* O, float* LSE, void* workspace, s
       if (e != hipSuccess) return fail(ACCT_E_LAUNCH, "dropout bitmap kernel: %s", hipGetErrorString(e));
     }
   }
-  acct::FwdPlan plan = plan_forward(p, true, n_cu);
   const size_t part_at = align_up(need, 256);
+  if (const int row = row_keys(p)) {
+    acct::RowPlan plan = acct::row_plan(p->B, p->N, row, p->D, true);
+    if (plan.parts > 1 && (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < part_at + plan.part_bytes))
+      plan = acct::row_plan(p->B, p->N, row, p->D, false);
+    a.kv_split = plan.parts;
+    if (plan.parts > 1) a.fwd_part = (float*)((char*)workspace + part_at);
+    const hipError_t e = p->dtype == ACCT_F16 ? acct::launch_fwd_row_elem<acct::f16>(a, row, st) : acct::launch_fwd_row_elem<acct::bf16>(a, row, st);
+    if (e != hipSuccess) return fail(ACCT_E_LAUNCH, "forward kernel: %s", hipGetErrorString(e));
+    return ACCT_OK;
+  }
+  acct::FwdPlan plan = plan_forward(p, true, n_cu);
   if (plan.kv_split > 1 && (!workspace || ((uintptr_t)workspace & 255) || workspace_bytes < part_at + plan.part_bytes))
     plan = plan_forward(p, false, n_cu);              // no room for the slices' sums
   a.kv_split = plan.kv_split;

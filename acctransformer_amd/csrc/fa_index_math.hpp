@@ -244,6 +244,34 @@ ACCT_HD FwdPlan fwd_plan(int B, int N, int Sq, int Sk, int D, bool side, bool tr
   return {kg, split, fwd_part_bytes(B, N, Sq, D, kg, split)};
 }
 
+// The forward with one query row per head (fa_fwd_row.hip): parts of the key range per head, each a workgroup of its own,
+// which a second kernel adds up (1: none).  A workgroup alone takes 1.1 us per batch of 64 KB of K and V, a little more the more
+// others there are, those that share a CU 1.8; all of them together 1 us per 6.6 MB; 95 of them start per us; the second kernel
+// takes 3.4 us and more.
+// One part / the parts taken (us; bf16): 8 heads, 512 keys, D128 7.3 / 7.3 (4 parts 7.9); 8, 8192, D128 75 / 13.7 (16); 64, 2048,
+// D64 13.7 / 12.1 (2); 96, 8192, D128 88 / 65 (2); 256, 8192, D128 157 / 157 (2 parts 160); 512, 128, D64 6.8 / 6.8 (2 13.4).
+struct RowPlan { int parts; size_t part_bytes; };
+ACCT_HD int row_batch(int D) { return D <= 64 ? 256 : D <= 128 ? 128 : 64; }             // keys
+ACCT_HD size_t row_part_bytes(int B, int N, int D, int parts) {
+  return parts > 1 ? (size_t)parts * (size_t)B * N * (D + 2) * sizeof(float) : 0;
+}
+ACCT_HD RowPlan row_plan(int B, int N, int keys, int D, bool can_split) {
+  const double heads = (double)B * N, stream = heads * keys * D * 4 / 6.6e6;
+  const int batches = (keys + row_batch(D) - 1) / row_batch(D);
+  int best = 1;
+  double t_best = 0;
+  for (int parts = 1; parts <= 256 && parts <= batches && (parts == 1 || can_split); parts *= 2) {
+    const double n = heads * parts, walk = (double)((batches + parts - 1) / parts);
+    double t = walk * (1.12 + 0.002 * (n < 256 ? n : 256));
+    if (n > 256) t = walk * 1.82 * (double)(((long long)n + 255) / 256);                 // several workgroups share some CUs
+    if (stream > t) t = stream;
+    if (n / 95 > t) t = n / 95;
+    if (parts > 1) t += 3.4 + 0.02 * parts;
+    if (parts == 1 || t < t_best) { t_best = t; best = parts; }
+  }
+  return {best, row_part_bytes(B, N, D, best)};
+}
+
 // Key groups of the dQ kernel (fa_bwd.hip): 2 where 256-row workgroups would leave CUs idle.  A workgroup of half the
 // rows takes 0.6 to 0.75 of the time, so it pays in one round only: 8 heads, S3728, D128 causal 175 -> 112 us; 16 heads,
 // 1024 x 1024, D128 with dropout 47.9 -> 33.4; 24 heads, S2424, D128 causal 116 -> 90; but 80 heads, 2000 x 2000 272 / 277

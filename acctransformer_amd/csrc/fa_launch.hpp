@@ -26,6 +26,10 @@ inline hipError_t allow_dynamic_lds(const void* kern, size_t bytes) {
 // a.alibi / a.droprow, the key-range split from a.kv_split / a.fwd_part
 template <typename T> hipError_t launch_fwd_elem(const FaArgs& a, int D, int kg, hipStream_t st);
 
+// forward with one query row per head, the keys 0 .. key_end - 1 and no side inputs (fa_fwd_row.hip); a.kv_split / a.fwd_part:
+// parts of the key range (RowPlan, fa_index_math.hpp)
+template <typename T> hipError_t launch_fwd_row_elem(const FaArgs& a, int key_end, hipStream_t st);
+
 // backward: delta pre-pass, dK/dV kernel (kv-tile owner) and dQ kernel (q-tile owner)
 enum : int { kStageDq = 1, kStageDkDv = 2 };
 template <typename T> hipError_t launch_bwd_elem(const FaArgs& a, int D, int stages, hipStream_t st);
