@@ -24,23 +24,23 @@
 
 namespace acct {
 
-// LDS of the key-group merge: behind the output staging of the RG row groups, one slot per wave of the key groups
-// 1 .. KG - 1 (accumulators as they sit in the registers, then running max and sum)
-template <int D, int RG> constexpr int fwd_merge_at() { return RG * 32 * (SwzCfg<D>::DB * 64 + 16); }
-template <int D> constexpr int fwd_merge_slot() { return SwzCfg<D>::DB * 4096 + 512; }
+// LDS of the key-group merge: the accumulators are cut into 4 DB pieces of 8 columns, of which every key group finishes
+// 4 DB / KG; a wave leaves the pieces of the other groups here, then its running max and sum.
+template <int D, int KG> constexpr int fwd_merge_pieces() { return 4 * SwzCfg<D>::DB / KG; }
+template <int D, int NW, int KG> constexpr int fwd_merge_stats() { return NW * (KG - 1) * fwd_merge_pieces<D, KG>() * 1024; }
 
 // KG > 1 (small grids): the waves of a workgroup form NW / KG row groups times KG key groups.  A wave then works on
 // its key group's share of every tile only, with softmax statistics of its own, and the key groups of a row group
 // are merged through LDS before the epilogue -- KG times as many workgroups for the same rows, every wave busy.
 template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2, int KG = 1>
 ACCT_DEV void fa_fwd_body(const FaArgs& a) {
-  static_assert(KT == 2 || KT == 4, "key tiles are 64 or 128 rows (with a bias, 128 rows take the key-only form of it only)");
+  static_assert(KT == 2 || KT == 4 || (KT == 8 && !BIAS && !DROP), "key tiles are 64, 128 or 256 rows (with a bias, 128 rows take the key-only form of it only)");
   static_assert(KG == 1 || (QG == 1 && KT % KG == 0 && NW % KG == 0), "key groups own whole 32-key chunks");
+  static_assert(KT / KG <= 4, "a wave's keys of a tile lie in one 128-key block");
   constexpr int BN = 32 * KT;                       // key rows per tile
   constexpr int KTW = KT / KG, WN = 32 * KTW;       // 32-key chunks and keys of a tile that one wave works on
   constexpr int RG = NW / KG;                       // row groups
   constexpr int FRING = 4, VRING = 3;   // fragment reads in flight ahead of their MFMA (K row-major / V transposed)
-  constexpr int TPB = 128 / BN;                     // tiles per 128-column block
   using E = Elem<T>;
   using V8 = typename E::V8;
   using C = SwzCfg<D>;
@@ -74,7 +74,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   // ---- visible kv tiles of this block (128-block band; causal and row-prefix clip the top) ----
   const int qb_lo = q0 / 128, qb_hi = (q_end - 1) / 128;
   const int kvb_lo = max(0, qb_lo - a.prev_blk), kvb_hi = min(a.Tc - 1, qb_hi + a.next_blk);
-  int j_lo = kvb_lo * TPB, j_hi = min(kvb_hi * TPB + TPB - 1, (a.Sk - 1) / BN);
+  int j_lo = kvb_lo * 128 / BN, j_hi = min(kvb_hi * 128 + 127, a.Sk - 1) / BN;
   const bool causal = a.mask_kind == kMaskCausal;
   if (causal) j_hi = min(j_hi, (q_end - 1) / BN);
   if (a.row_prefix) j_hi = min(j_hi, (((q_end - 1) / a.row_prefix + 1) * a.row_prefix - 1) / BN);
@@ -86,16 +86,17 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     // not streamed at all (key padding: the padded tail of every sequence).  With at most 64 blocks in the
     // band, one round trip to memory yields both the trimmed range and the wave's class window.
     const uint8_t* fl = a.blkflags + ((int64_t)(a.mask_sb ? b : 0) * a.Tr) * a.Tc;
-    int b_lo = j_lo / TPB, b_hi = j_hi / TPB;
+    int b_lo = j_lo * BN / 128, b_hi = min((j_hi * BN + BN - 1) / 128, a.Tc - 1);
     const uint8_t* tails = a.blktail ? a.blktail + ((int64_t)(a.mask_sb ? b : 0) * a.Tr) * a.Tc : nullptr;
     if (j_lo <= j_hi && flwin.init_trimmed(fl, 1, a.Tc, qb_lo, qb_hi - qb_lo + 1, min(wqb, qb_hi), b_lo, b_hi, lane, tails)) {
-      j_lo = max(j_lo, b_lo * TPB);
-      j_hi = min(j_hi, b_hi * TPB + TPB - 1);
+      j_lo = max(j_lo, b_lo * 128 / BN);
+      j_hi = min(j_hi, (b_hi * 128 + 127) >> __builtin_ctz(BN));    // (b_hi is -1 when nothing is left)
       flwin_ready = true;
     } else {
       auto dead = [&](int j) {
-        for (int qb = qb_lo; qb <= qb_hi; qb++)
-          if (fl[(int64_t)qb * a.Tc + j / TPB] != kBlkSkip) return false;
+        for (int kb = j * BN / 128; kb <= min((j * BN + BN - 1) / 128, a.Tc - 1); kb++)
+          for (int qb = qb_lo; qb <= qb_hi; qb++)
+            if (fl[(int64_t)qb * a.Tc + kb] != kBlkSkip) return false;
         return true;
       };
       trim_dead_tiles(j_lo, j_hi, lane, dead);
@@ -107,6 +108,21 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     j_hi = lo + (int)((int64_t)n * (slice + 1) / a.kv_split) - 1;
   }
   const int wkv_limit = a.row_prefix ? (wq0 / a.row_prefix + 1) * a.row_prefix : 0x7fffffff;   // keys past it are absent
+
+  // ---- the first tile is requested ahead of everything that can be done meanwhile ----
+  TileDma<T, D, BN, NW> kdma, vdma;
+  const int cpr = a.hd >> 3;                                // valid 16-byte chunks per row
+  kdma.plan(a.k_ss, cpr);
+  vdma.plan(a.v_ss, cpr);
+  // stage key rows [j BN, (j+1) BN) of K or V into an LDS tile
+  auto stage_tile = [&](const TileDma<T, D, BN, NW>& dma, const T* base, int64_t ss, int j, ACCT_LDS char* dst) {
+    if ((j + 1) * BN <= a.Sk) dma.issue(base, ss, j * BN, dst);
+    else tile_dma<T, D, BN, NW>(base, ss, j * BN, a.Sk, dst, cpr);   // ragged last tile: clamped rows
+  };
+  if (j_lo <= j_hi) {
+    stage_tile(kdma, kp, a.k_ss, j_lo, smem);
+    stage_tile(vdma, vp, a.v_ss, j_lo, smem + TILEB);
+  }
 
   // ---- Q fragments (B operand of K Q^T): lane holds row l32, d = 16t + 8g .. +7 ----
   V8 qf[QG][C::KS];
@@ -173,10 +189,6 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   const bool mask_dense = a.mask_kind == kMaskDense;
   const bool alibi_vec = BIAS && (((uintptr_t)a.alibi & 7) | ((a.al_sb | a.al_sh | a.al_sq) & 3)) == 0;
 
-  TileDma<T, D, BN, NW> kdma, vdma;
-  const int cpr = a.hd >> 3;                                // valid 16-byte chunks per row
-  kdma.plan(a.k_ss, cpr);
-  vdma.plan(a.v_ss, cpr);
   // bias tiles of this wave's rows are staged through a wave-private LDS region one tile ahead
   // (with 128-key tiles only the key-only form is served: two 256-byte rows per wave)
   constexpr int BIASB = BIAS ? (KT == 4 ? 1024 : QG * 4096) : 0;
@@ -204,12 +216,12 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   // ---- the phases of a tile step: classification, S^T = K Q^T, online softmax, O^T += V^T P^T ----
   const uint8_t* flrow = (MASKT && a.mask_kind == kMaskDense) ? a.blkflags + ((int64_t)mb * a.Tr + wqb) * a.Tc : nullptr;
   if (!flwin_ready && j_lo <= j_hi)
-    flwin.init(flrow, 1, j_lo / TPB, j_hi / TPB, lane, (flrow && a.blktail) ? a.blktail + (flrow - a.blkflags) : nullptr);
+    flwin.init(flrow, 1, j_lo * BN / 128, min((j_hi * BN + BN - 1) / 128, a.Tc - 1), lane, (flrow && a.blktail) ? a.blktail + (flrow - a.blkflags) : nullptr);
   enum : uint32_t { kAct = 1u, kApply = 2u, kDiag = 4u, kTailShift = 8u };   // bits 8..15: key tail of the tile's block (0: none)
   // what this wave does with tile j (tiles must be asked for in ascending order)
   auto classify = [&](int j) -> uint32_t {
-    const uint32_t fl_cur = flwin.get(j / TPB, lane);
-    const int kv0 = j * BN + kg * WN, kvb = j / TPB;
+    const int kv0 = j * BN + kg * WN, kvb = kv0 / 128;
+    const uint32_t fl_cur = flwin.get(kvb, lane);
     bool act = (kvb - a.next_blk <= wqb) && (wqb <= kvb + a.prev_blk) && (wq0 < a.Sq);
     if (causal) act = act && (kv0 <= wq_end - 1);
     act = act && (kv0 < wkv_limit);
@@ -230,11 +242,6 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       apply_mask = wqb == kvb;
     }
     return (act ? kAct : 0u) | (apply_mask ? kApply : 0u) | (diag ? kDiag : 0u) | (tail << kTailShift);
-  };
-  // stage key rows [j BN, (j+1) BN) of K or V into an LDS tile
-  auto stage_tile = [&](const TileDma<T, D, BN, NW>& dma, const T* base, int64_t ss, int j, ACCT_LDS char* dst) {
-    if ((j + 1) * BN <= a.Sk) dma.issue(base, ss, j * BN, dst);
-    else tile_dma<T, D, BN, NW>(base, ss, j * BN, a.Sk, dst, cpr);   // ragged last tile: clamped rows
   };
   // S^T = K Q^T : s[gq][c] is the 32(kv) x 32(q) tile of kv chunk c
   auto gemm_s = [&](const ACCT_LDS char* kbuf, int j, f32x16 (&s)[QG][KTW]) {
@@ -305,7 +312,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     const int kv0 = j * BN + kg * WN;
     const bool apply_mask = MASKT && (info & kApply), diag = info & kDiag;
     const int tail = MASKT ? (int)((info >> kTailShift) & 0xffu) : 0;
-    const int last_key = tail ? min(a.Sk, (j / TPB) * 128 + tail) - 1 : a.Sk - 1;     // last key that exists and is not behind a key tail
+    const int last_key = tail ? min(a.Sk, kv0 / 128 * 128 + tail) - 1 : a.Sk - 1;     // last key that exists and is not behind a key tail
     // element (gq, c, r): q = wq0 + 32 gq + l32 ; kv = kv0 + 32 c + 8 (r/4) + 4 g + r%4
     const bool edge = apply_mask || (diag && (kv0 + WN - 1 > wq0)) || (kv0 + WN - 1 > last_key);
 #pragma unroll
@@ -437,8 +444,6 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   };
 
   if (j_lo <= j_hi) {
-    tile_dma<T, D, BN, NW>(kp, a.k_ss, j_lo * BN, a.Sk, smem, cpr);
-    tile_dma<T, D, BN, NW>(vp, a.v_ss, j_lo * BN, a.Sk, smem + TILEB, cpr);
     if (BIAS && bias_staged && wq0 < a.Sq) stage_bias(j_lo);
     DropStage::issue(a, bh, wq0, j_lo, lane, drop_lds);
     // A full wait the compiler can see: every load issued so far (Q fragments included) is complete, so
@@ -473,51 +478,91 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     }
   }
 
-  // ---- key groups: the waves of group 0 take in the sums of the others ----
+  // ---- key groups: each finishes its share of the columns from the sums of all.  (One group merging and storing all of
+  // them while the others idled: 3900 cycles from the last tile on, of a workgroup that walked four tiles in 8000, D64, kg 4;
+  // shared 2400.) ----
   if constexpr (KG > 1) {
-    ACCT_LDS char* mg = smem + fwd_merge_at<D, RG>();
-    if (kg > 0) {
-      ACCT_LDS char* slot = mg + ((kg - 1) * RG + rg) * fwd_merge_slot<D>();
+    constexpr int PC = fwd_merge_pieces<D, KG>();
+    static_assert(PC * KG == 4 * C::DB, "every key group finishes the same number of pieces");
+    // pieces of key group `own` that key group `from` holds
+    auto slot = [&](int own, int from) {
+      return smem + ((rg * KG + own) * (KG - 1) + from - (from > own ? 1 : 0)) * (PC * 1024) + lane * 16;
+    };
+    ACCT_LDS char* stats = smem + fwd_merge_stats<D, NW, KG>() + rg * (KG * 512) + lane * 8;
+    auto piece = [&](int i) -> f32x4 {
+      return {o[0][i / 4][4 * (i % 4)], o[0][i / 4][4 * (i % 4) + 1], o[0][i / 4][4 * (i % 4) + 2], o[0][i / 4][4 * (i % 4) + 3]};
+    };
 #pragma unroll
-      for (int db = 0; db < C::DB; db++)
+    for (int k = 0; k < KG; k++)
+      if (k != kg) {
 #pragma unroll
-        for (int r4 = 0; r4 < 4; r4++) {
-          const f32x4 v = {o[0][db][4 * r4], o[0][db][4 * r4 + 1], o[0][db][4 * r4 + 2], o[0][db][4 * r4 + 3]};
-          *reinterpret_cast<ACCT_LDS f32x4*>(slot + (4 * db + r4) * 1024 + lane * 16) = v;
-        }
-      const f32x2 ml = {m[0], lsum[0]};
-      *reinterpret_cast<ACCT_LDS f32x2*>(slot + C::DB * 4096 + lane * 8) = ml;
-    }
+        for (int i = 0; i < PC; i++) *reinterpret_cast<ACCT_LDS f32x4*>(slot(k, kg) + i * 1024) = piece(k * PC + i);
+      }
+    const f32x2 mine = {m[0], lsum[0]};
+    *reinterpret_cast<ACCT_LDS f32x2*>(stats + kg * 512) = mine;
     __syncthreads();
-    if (kg > 0) return;
-    f32x2 ml[KG - 1];
-    float mm = m[0];
+    f32x2 ml[KG];
+    float w[KG], mm = -1e30f, l = 0.f;
 #pragma unroll
-    for (int k = 0; k < KG - 1; k++) {
-      ml[k] = *reinterpret_cast<const ACCT_LDS f32x2*>(mg + (k * RG + rg) * fwd_merge_slot<D>() + C::DB * 4096 + lane * 8);
+    for (int k = 0; k < KG; k++) {
+      ml[k] = *reinterpret_cast<const ACCT_LDS f32x2*>(stats + k * 512);
       mm = fmaxf(mm, ml[k][0]);
     }
-    const float w0 = fast_exp2((m[0] - mm) * cmul);
-    m[0] = mm;
-    lsum[0] *= w0;
 #pragma unroll
-    for (int db = 0; db < C::DB; db++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) o[0][db][r] *= w0;
-#pragma unroll
-    for (int k = 0; k < KG - 1; k++) {
-      const ACCT_LDS char* slot = mg + (k * RG + rg) * fwd_merge_slot<D>();
-      const float w = fast_exp2((ml[k][0] - mm) * cmul);
-      lsum[0] = __builtin_fmaf(ml[k][1], w, lsum[0]);
-#pragma unroll
-      for (int db = 0; db < C::DB; db++)
-#pragma unroll
-        for (int r4 = 0; r4 < 4; r4++) {
-          const f32x4 v = *reinterpret_cast<const ACCT_LDS f32x4*>(slot + (4 * db + r4) * 1024 + lane * 16);
-#pragma unroll
-          for (int e = 0; e < 4; e++) o[0][db][4 * r4 + e] = __builtin_fmaf(v[e], w, o[0][db][4 * r4 + e]);
-        }
+    for (int k = 0; k < KG; k++) {
+      w[k] = fast_exp2((ml[k][0] - mm) * cmul);
+      l = k == 0 ? ml[0][1] * w[0] : __builtin_fmaf(ml[k][1], w[k], l);
     }
+    l = pair_sum(l);
+    f32x4 acc[PC];
+#pragma unroll
+    for (int own = 0; own < KG; own++)
+      if (own == kg) {
+#pragma unroll
+        for (int i = 0; i < PC; i++)
+#pragma unroll
+          for (int k = 0; k < KG; k++) {                     // (in the order of the keys, whoever adds)
+            const f32x4 v = k == own ? piece(own * PC + i) : *reinterpret_cast<const ACCT_LDS f32x4*>(slot(own, k) + i * 1024);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[i][e] = k == 0 ? v[e] * w[0] : __builtin_fmaf(v[e], w[k], acc[i][e]);
+          }
+      }
+    if (wq0 >= a.Sq) return;
+    if (a.kv_split > 1) {                                    // sums and statistics of a key slice (as below)
+      const int64_t idx = ((int64_t)slice * n_wg + wg) * RG + rg, n_idx = (int64_t)a.kv_split * n_wg * RG;
+      float* part = a.fwd_part + idx * (C::DB * 1024) + kg * (PC * 256) + lane * 4;
+#pragma unroll
+      for (int i = 0; i < PC; i++) *reinterpret_cast<f32x4*>(part + i * 256) = acc[i];
+      const f32x2 msl = {mm, l};
+      if (kg == 0 && g == 0) *reinterpret_cast<f32x2*>(a.fwd_part + n_idx * (C::DB * 1024) + (idx * 32 + l32) * 2) = msl;
+      return;
+    }
+    const int row = wq0 + l32, nch = a.hd >> 3;
+    const float inv = l > 0.f ? (DROP ? a.inv_keep : 1.0f) / l : 0.f;
+    if (row >= a.Sq) return;
+    if (kg == 0 && g == 0) a.lse[(int64_t)bh * a.Sq + row] = l > 0.f ? mm * (scaled ? 1.0f : a.scale) + __logf(l) : -INFINITY;
+    T* orow = (T*)a.o + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_ss;
+    // lanes l and l + 32 hold half a 16-byte chunk of two pieces each: they exchange halves and store one whole chunk each
+#pragma unroll
+    for (int i = 0; i < PC; i += 2) {
+      uint32_t t[2][2];
+#pragma unroll
+      for (int x = 0; x < 2 && i + x < PC; x++) {
+        t[x][0] = __builtin_bit_cast(uint32_t, E::cvt2(acc[i + x][0] * inv, acc[i + x][1] * inv));
+        t[x][1] = __builtin_bit_cast(uint32_t, E::cvt2(acc[i + x][2] * inv, acc[i + x][3] * inv));
+      }
+      if (i + 1 < PC) {
+        const u32x2 lo = __builtin_amdgcn_permlane32_swap(t[0][0], t[1][0], false, false), hi = __builtin_amdgcn_permlane32_swap(t[0][1], t[1][1], false, false);
+        const u32x4 v = {lo[0], hi[0], lo[1], hi[1]};
+        const int ch = kg * PC + i + g;
+        if (ch < nch) *reinterpret_cast<u32x4*>(orow + ch * 8) = v;
+      } else {
+        const u32x2 v = {t[0][0], t[0][1]};
+        const int ch = kg * PC + i;
+        if (ch < nch) *reinterpret_cast<u32x2*>(orow + ch * 8 + 4 * g) = v;
+      }
+    }
+    return;
   }
   // ---- key slices: sums and statistics go to the workspace, fa_fwd_combine_kernel adds the slices up ----
   if (a.kv_split > 1) {
@@ -708,7 +753,7 @@ static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
   constexpr size_t biasb = BIAS ? (KT == 4 ? 1024 : QG * 4096) : 0;     // per wave, as in the kernel
   constexpr size_t tiles = 4 * 32 * KT * (size_t)C::PITCH + NW * biasb + (size_t)NW * 2 * DropRowStage<DROP, QG, KT>::BYTES,
-                   stage = KG > 1 ? fwd_merge_at<D, RG>() + (size_t)(KG - 1) * RG * fwd_merge_slot<D>() : (size_t)NW * 32 * (C::DB * 64 + 16);
+                   stage = KG > 1 ? fwd_merge_stats<D, NW, KG>() + (size_t)NW * 512 : (size_t)NW * 32 * (C::DB * 64 + 16);
   constexpr size_t smem = tiles > stage ? tiles : stage;
   static_assert(smem <= 160 * 1024, "the workgroup's LDS must fit the CU's 160 KB");
   auto kern = mask_t ? fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, true, KT, KG> : fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, BIAS || DROP, KT, KG>;
@@ -735,6 +780,12 @@ static hipError_t launch_fwd_t(const FaArgs& a, hipStream_t st) {
   // them; a key-only bias that the DMA can stage is a 256-byte row and does.
   constexpr bool BIG = NW == 8 && D <= 128;
   static_assert(BIG || !BIAS, "the bias variants rest on this choice");
+  // Four key groups leave a wave 32 keys of a 128-key tile: a step of latencies.  Rows of 128 bytes leave room for 256-key
+  // tiles, one workgroup to a CU (forward, 128 / 256 keys, us: 4 heads, 512 x 512, D64 7.4 / 6.9; 1024 x 1024 10.6 / 9.6; but
+  // 20 heads, 1024 x 1024 causal, 320 workgroups 12.2 / 12.7).
+  if constexpr (KG == 4 && D <= 64) {
+    if (a.Sk > 128 && (long long)a.B * a.N * ((a.Sq + 63) / 64) <= 256) return launch_fwd_kt<T, D, NW, BIAS, DROP, 8, KG>(a, st);
+  }
   if constexpr (BIG && BIAS) {
     return key_bias_stageable(a) ? launch_fwd_kt<T, D, NW, BIAS, DROP, 4, KG>(a, st) : launch_fwd_kt<T, D, NW, BIAS, DROP, 2, KG>(a, st);
   } else {
