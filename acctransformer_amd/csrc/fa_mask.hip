@@ -240,11 +240,6 @@ ACCT_DEV void transpose_16x16(uint32_t (&x)[8]) {
   transpose_bytes8(x);
 }
 
-// workgroup id -> block span: the ids that one XCD gets (id % 8) take consecutive spans
-ACCT_DEV int xcd_span(int id, int n) {
-  const int per = n / 8, rem = n % 8, xcd = id & 7;
-  return xcd * per + min(xcd, rem) + (id >> 3);
-}
 // sixteen bytes at any address that nothing reads again
 typedef u32x4 u32x4_any __attribute__((aligned(1)));
 ACCT_DEV u32x4 load_once(const uint8_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p)); }

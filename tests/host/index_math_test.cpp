@@ -221,6 +221,32 @@ static void test_visible_row_keys() {
   CHECK(fwd_plan(1, 1, 256, 131072, 128, false, false, true, 256, visible_row_keys(256, 131072, 65536, 200, 0)).kv_split > 8, "a wide band is not cut");
 }
 
+// every (slice, workgroup) once, and the row tiles of a head and slice next to each other on one XCD (but where its share ends)
+static void test_split_map() {
+  for (int BH : {1, 3, 8, 40, 64, 100, 128})
+    for (int n_tiles : {1, 2, 3, 5})
+      for (int split : {2, 3, 7, 16, 128}) {
+        if (BH == 128 && n_tiles > 1) continue;                                        // (such a launch is not cut)
+        const int n = BH * n_tiles * split;
+        std::vector<int> seen(n, -1);
+        int apart = 0;
+        for (int id = 0; id < n; id++) {
+          int slice = -1, wg = -1;
+          split_map(id, BH, n_tiles, split, slice, wg);
+          const bool in = slice >= 0 && slice < split && wg >= 0 && wg < BH * n_tiles;
+          CHECK(in, "BH %d tiles %d split %d id %d: slice %d wg %d", BH, n_tiles, split, id, slice, wg);
+          if (!in) continue;
+          CHECK(seen[slice * BH * n_tiles + wg] < 0, "BH %d tiles %d split %d id %d: twice", BH, n_tiles, split, id);
+          seen[slice * BH * n_tiles + wg] = id;
+        }
+        for (int slice = 0; slice < split && n_tiles > 1; slice++)
+          for (int bh = 0; bh < BH; bh++)
+            for (int t = 1; t < n_tiles; t++)
+              if (seen[slice * BH * n_tiles + t * BH + bh] != seen[slice * BH * n_tiles + (t - 1) * BH + bh] + 8) apart++;
+        CHECK(apart <= 8, "BH %d tiles %d split %d: %d neighbours apart", BH, n_tiles, split, apart);
+      }
+}
+
 static void test_div_small() {
   for (int n = 1; n <= 32; n++)
     for (int idx = 0; idx < 1024; idx++) CHECK(div_small(idx, recip16(n)) == idx / n, "div_small(%d, %d)", idx, n);
@@ -252,6 +278,7 @@ int main() {
   test_slice_plans();
   test_visible_row_keys();
   test_keep_columns();
+  test_split_map();
   test_div_small();
   if (failures) printf("%d checks failed\n", failures);
   else printf("index math: all checks passed\n");
