@@ -40,6 +40,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   constexpr int BN = 32 * KT;                       // key rows per tile
   constexpr int KTW = KT / KG, WN = 32 * KTW;       // 32-key chunks and keys of a tile that one wave works on
   constexpr int RG = NW / KG;                       // row groups
+  constexpr bool PIPE = !BIAS && !DROP && !MASKT && QG == 1 && KG == 1 && NW == 8 && KT == 4 && D <= 64;
   constexpr int FRING = 4, VRING = 3;   // fragment reads in flight ahead of their MFMA (K row-major / V transposed)
   using E = Elem<T>;
   using V8 = typename E::V8;
@@ -440,7 +441,144 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     }
   };
 
-  if (j_lo <= j_hi) {
+  if constexpr (PIPE) {
+    // ---- tile loop, pipelined: step j issues O^T += V(j-1)^T P(j-1)^T and S(j+1)^T = K(j+1) Q^T with the softmax of tile j
+    // between their MFMAs.  The eight waves start a step together, so in the plain loop below the two of a SIMD are in their
+    // matrix phases at the same time and then both in the softmax.  Needs two tiles of scores and the packed P in registers:
+    // up to head dim 64 (with 64-key tiles head dims 80 and 128 lose 3 % to the plain loop).  Forward, us, plain / pipelined:
+    // 16 heads, 4096 x 4096, D40 73.4 / 71.1; D64 81.0 / 78.8; 32 heads, 2048 x 2048 causal, D64 39.6 / 38.4 ----
+    // this wave's own tiles
+    const int key_end = min(min(causal ? wq_end : a.Sk, wkv_limit), a.Sk) - kg * WN;
+    const int w_lo = max(j_lo, max(0, wqb - a.prev_blk) * 128 / BN);
+    const int w_hi = wq0 < a.Sq && key_end > 0 ? min(min(j_hi, (min(a.Tc - 1, wqb + a.next_blk) * 128 + 127) / BN), (key_end - 1) / BN) : -1;
+    constexpr int NPV = 2 * KTW * C::DB, NQK = KTW * C::KS, NM = NPV + NQK, NE = 16 * KTW;
+    // buffers of step j: it reads those of the other parity and fills its own
+    int par = 0;                                             // byte offset of step j's own buffers
+    const T *kfill = kp + (int64_t)(j_lo + 2) * BN * a.k_ss, *vfill = vp + (int64_t)j_lo * BN * a.v_ss;   // what step j requests
+    const int64_t kstep = BN * a.k_ss, vstep = BN * a.v_ss;
+    auto fill = [&](int j) {
+      if (j + 2 <= j_hi) {
+        if ((j + 3) * BN <= a.Sk) kdma.issue(kfill, a.k_ss, 0, smem + par);
+        else tile_dma<T, D, BN, NW>(kp, a.k_ss, (j + 2) * BN, a.Sk, smem + par, cpr);     // ragged last tile: clamped rows
+      }
+      if (j > j_lo && j <= j_hi) {                           // (that of the first tile is under way)
+        if ((j + 1) * BN <= a.Sk) vdma.issue(vfill, a.v_ss, 0, smem + par + TILEB);
+        else tile_dma<T, D, BN, NW>(vp, a.v_ss, j * BN, a.Sk, smem + par + TILEB, cpr);
+      }
+      kfill += kstep;
+      vfill += vstep;
+    };
+    auto publish = [&] {
+      par ^= 2 * TILEB;
+      dma_wait();
+      __syncthreads();
+    };
+    auto fused = [&](int j, f32x16 (&s)[1][KTW], f32x16 (&sn)[1][KTW], V8 (&pf)[1][KTW][2]) {
+      const ACCT_LDS char* kbuf = smem + (par ^ (2 * TILEB));
+      const ACCT_LDS char* vbuf = kbuf + TILEB;
+      const int kv0 = j * BN;
+      if ((causal && kv0 + WN - 1 > wq0) || kv0 + WN > a.Sk) {
+        int vis = a.Sk - 1 - kv0 - 4 * g;                    // (as in softmax)
+        if (causal) vis = min(vis, wq0 + l32 - kv0 - 4 * g);
+        const float ninf = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < NE; e++) s[0][e / 16][e & 15] = select_if_gt(s[0][e / 16][e & 15], 8 * ((e & 15) >> 2) + (e & 3), vis - 32 * (e / 16), ninf);
+      }
+#pragma unroll
+      for (int c = 0; c < KTW; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) sn[0][c][r] = 0.f;
+      constexpr int RING = 4;
+      auto fread = [&](int i) {
+        if (i < NPV) {
+          const ACCT_LDS char* vaddr = vbuf + voff[i % C::DB] + 16 * (i / C::DB) * C::PITCH;
+          return join_tr<T>(lds_read_tr(vaddr), lds_read_tr(vaddr + C::tr_hi(i % C::DB)));
+        }
+        return lds_read_frag<T>(kbuf + koff((i - NPV) % C::KS) + ((i - NPV) / C::KS) * 32 * C::PITCH);
+      };
+      V8 ring[RING];
+      uint32_t pn[NE / 2];
+#pragma unroll
+      for (int i = 0; i < RING; i++) ring[i] = fread(i);
+      // vector work in the order it depends on itself, dealt out over the MFMAs by its cycles
+      constexpr int CM = 2, CS = 24, CE = 7, CT = NE / 2 * CM + CS + NE * CE;
+      float mx = s[0][0][0], mx1 = s[0][0][2], mc = 0.f, alpha = 1.f, rs = 0.f, p[2];
+#pragma unroll
+      for (int i = 0; i < NM; i++) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (i < NPV) o[0][i % C::DB] = E::mfma(ring[i % RING], pf[0][(i / C::DB) >> 1][(i / C::DB) & 1], o[0][i % C::DB]);
+        else sn[0][(i - NPV) / C::KS] = E::mfma(ring[i % RING], qf[0][(i - NPV) % C::KS], sn[0][(i - NPV) / C::KS]);
+        if (i + RING < NM) ring[i % RING] = fread(i + RING);
+        if (i == 1) fill(j);                                 // (behind the first fragment reads, whose latency it covers)
+#pragma unroll
+        for (int k = 0; k < NE / 2; k++)
+          if (k * CM * NM / CT == i) {
+            float& m2 = k & 1 ? mx1 : mx;                    // (two chains: a dependent maximum waits 8 cycles, issues in 4)
+            m2 = fmaxf(fmaxf(m2, s[0][k / 8][2 * (k & 7)]), s[0][k / 8][2 * (k & 7) + 1]);
+          }
+        if (NE / 2 * CM * NM / CT == i) {
+          mx = pair_max(fmaxf(mx, mx1));
+          const bool grow = mx > m[0] + lazy_thr;
+          const float m_new = grow ? mx : m[0];
+          alpha = grow ? fast_exp2((m[0] - m_new) * cmul) : 1.0f;
+          mc = m_new * cmul;
+          m[0] = m_new;
+        }
+#pragma unroll
+        for (int e = 0; e < NE; e++)
+          if ((NE / 2 * CM + CS + e * CE) * NM / CT == i) {
+            p[e & 1] = fast_exp2(__builtin_fmaf(s[0][e / 16][e & 15], cmul, -mc));
+            rs += p[e & 1];
+            if (e & 1) {
+              // (pinned here: the compiler would move all of it behind the barrier, to where the next step uses it)
+              pn[e / 2] = __builtin_bit_cast(uint32_t, E::cvt2(p[0], p[1]));
+              asm volatile("" : "+v"(pn[e / 2]), "+v"(rs));
+            }
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      lsum[0] = lsum[0] * alpha + rs;
+#pragma unroll
+      for (int c = 0; c < KTW; c++)
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) {
+          const u32x4 t = {pn[8 * c + 4 * hh], pn[8 * c + 4 * hh + 1], pn[8 * c + 4 * hh + 2], pn[8 * c + 4 * hh + 3]};
+          pf[0][c][hh] = __builtin_bit_cast(V8, t);
+        }
+      if (__any(alpha != 1.0f)) {
+#pragma unroll
+        for (int db = 0; db < C::DB; db++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) o[0][db][r] *= alpha;
+      }
+    };
+    f32x16 s0[1][KTW], s1[1][KTW];
+    V8 pf[1][KTW][2];
+    auto step = [&](int j) {
+      const ACCT_LDS char* buf = smem + (par ^ (2 * TILEB)) + kg * (WN * C::PITCH);
+      fill(j);
+      if (j > w_lo && j - 1 <= w_hi) gemm_pv(buf + TILEB, pf);
+      if (j >= w_lo && j <= w_hi) softmax(j, 0, kAct | (causal ? kDiag : 0u), s0, pf);
+      if (j + 1 >= w_lo && j + 1 <= w_hi) gemm_s(buf, j + 1, s0);
+      publish();
+    };
+    if (j_lo <= j_hi) {
+      if (j_lo < j_hi) stage_tile(kdma, kp, a.k_ss, j_lo + 1, smem + 2 * TILEB);
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      if (j_lo == w_lo && j_lo <= w_hi) gemm_s(smem + kg * (WN * C::PITCH), j_lo, s0);
+      __syncthreads();
+      int j = j_lo;
+      for (; j <= min(w_lo, j_hi + 1); j++) step(j);
+      for (; j + 1 < w_hi; j += 2) {
+        fused(j, s0, s1, pf);
+        publish();
+        fused(j + 1, s1, s0, pf);
+        publish();
+      }
+      for (; j <= j_hi + 1; j++) step(j);
+    }
+  } else if (j_lo <= j_hi) {
     if (BIAS && bias_staged && wq0 < a.Sq) stage_bias(j_lo);
     DropStage::issue(a, bh, wq0, j_lo, lane, drop_lds);
     // A full wait the compiler can see: every load issued so far (Q fragments included) is complete, so

@@ -14,6 +14,19 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
+def forward(q, k, v, kw):
+    qd = q.to(DEV)
+    p = _capi.make_params(qd, k.to(DEV), v.to(DEV), **kw)
+    lib = _capi.load()
+    o, lse = torch.empty_like(qd), torch.empty(qd.shape[:3], dtype=torch.float32, device=DEV)
+    p.o_stride = _capi._bhs_strides(o)
+    size = lib.acct_fa_fwd_workspace_bytes(ctypes.byref(p))
+    ws = torch.empty(max(size, 256), dtype=torch.uint8, device=DEV)
+    rc = lib.acct_fa_fwd(ctypes.byref(p), o.data_ptr(), lse.data_ptr(), ws.data_ptr(), size, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, lib.acct_last_error().decode()
+    return o, lse
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B, N, Sq, Sk, D, side", [
     (1, 2, 64, 128, 64, "none"), (1, 2, 65, 129, 64, "none"), (1, 2, 1, 192, 40, "none"), (1, 2, 63, 193, 48, "causal"),
@@ -47,15 +60,7 @@ def test_forward_of_key_groups(B, N, Sq, Sk, D, side, dtype):
     if m is not None:
         kw.update(mask_kind=_capi.MASK_DENSE_U8, attn_mask=torch.from_numpy(m).to(DEV))
         okw.update(attn_mask=m)
-    qd = q.to(DEV)
-    p = _capi.make_params(qd, k.to(DEV), v.to(DEV), **kw)
-    lib = _capi.load()
-    o, lse = torch.empty_like(qd), torch.empty(qd.shape[:3], dtype=torch.float32, device=DEV)
-    p.o_stride = _capi._bhs_strides(o)
-    size = lib.acct_fa_fwd_workspace_bytes(ctypes.byref(p))
-    ws = torch.empty(max(size, 256), dtype=torch.uint8, device=DEV)
-    rc = lib.acct_fa_fwd(ctypes.byref(p), o.data_ptr(), lse.data_ptr(), ws.data_ptr(), size, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-    assert rc == 0, lib.acct_last_error().decode()
+    o, lse = forward(q, k, v, kw)
     O, L = orc.unfused_fwd(q.float().numpy(), k.float().numpy(), v.float().numpy(), **okw)
     tol = dict(atol=2e-3, rtol=1e-3) if dtype == torch.float16 else dict(atol=2e-2, rtol=1e-2)
     ok, ratio, mx = orc.tolerance_gate(O, o.float().cpu().numpy(), **tol)
