@@ -55,7 +55,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   const int rg = KG > 1 ? wave % RG : wave, kg = KG > 1 ? wave / RG : 0;
   const int BH = a.B * a.N, n_wg = BH * a.n_tiles;
   int wg = blockIdx.x, slice = 0;                           // kv_split > 1: the grid holds every query tile once per key slice
-  if (a.kv_split > 1) split_map(blockIdx.x, BH, a.n_tiles, a.kv_split, slice, wg);
+  if (a.kv_split > 1) split_map(blockIdx.x, BH, a.n_tiles, a.kv_split, split_shares(BH, a.Sk, a.hd), slice, wg);
   int bh, rank;
   wg_map(wg, BH, a.n_tiles, bh, rank);
   const int qt = a.n_tiles - 1 - rank;                      // heaviest (latest) causal tiles first
@@ -774,7 +774,7 @@ __global__ void __launch_bounds__(64 * NW) fa_fwd_kernel(const FaArgs a) {
       constexpr int BM = 32 * QG * NW / KG;
       const int BH = a.B * a.N;
       int wg = blockIdx.x, slice;
-      if (a.kv_split > 1) split_map(blockIdx.x, BH, a.n_tiles, a.kv_split, slice, wg);
+      if (a.kv_split > 1) split_map(blockIdx.x, BH, a.n_tiles, a.kv_split, split_shares(BH, a.Sk, a.hd), slice, wg);
       int bh, rank;
       wg_map(wg, BH, a.n_tiles, bh, rank);
       const int q0 = (a.n_tiles - 1 - rank) * BM, q_end = min(q0 + BM, a.Sq);

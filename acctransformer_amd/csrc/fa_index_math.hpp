@@ -41,9 +41,12 @@ ACCT_HD int xcd_span(int id, int n) {
 // and slice read the same keys: they follow each other on one XCD, whose L2 then fetches them once (in the plain order, slice
 // by slice, they sit on different XCDs).  Forward, us: 1 head, 256 queries x 131072 keys, D128 34.5 -> 32.9; 3 heads, 300 x 60000
 // 51.4 -> 45.1; 5 heads, 400 x 30000 55.8 -> 49.3.  (Above 64 heads in wg_map's other order a split launch has one row tile per head.)
-ACCT_HD void split_map(int id, int BH, int n_tiles, int split, int& slice, int& wg) {
+// Below 64 MB of K and V the plain order is as fast or faster: 2 heads, 512 x 16000 25.1 / 27.0 (shared); 8, 512 x 8192 33.7 / 34.3;
+// 8, 256 x 12000 28.4 / 28.9.
+ACCT_HD bool split_shares(int BH, int Sk, int D) { return (long long)BH * Sk * D >= 16000000; }
+ACCT_HD void split_map(int id, int BH, int n_tiles, int split, bool share, int& slice, int& wg) {
   const int n_wg = BH * n_tiles;
-  if (n_tiles == 1 || (BH > 64 && (BH & 63) == 0)) {
+  if (!share || n_tiles == 1 || (BH > 64 && (BH & 63) == 0)) {
     slice = id / n_wg;
     wg = id - slice * n_wg;
     return;

@@ -232,7 +232,7 @@ static void test_split_map() {
         int apart = 0;
         for (int id = 0; id < n; id++) {
           int slice = -1, wg = -1;
-          split_map(id, BH, n_tiles, split, slice, wg);
+          split_map(id, BH, n_tiles, split, true, slice, wg);
           const bool in = slice >= 0 && slice < split && wg >= 0 && wg < BH * n_tiles;
           CHECK(in, "BH %d tiles %d split %d id %d: slice %d wg %d", BH, n_tiles, split, id, slice, wg);
           if (!in) continue;
