@@ -338,8 +338,22 @@ def fa_fwd(p, q):
     return o, lse
 
 
+def _apart(t):
+    """`t`, or a copy of it where elements may share memory (an expanded operand): its gradient has the same layout and
+    needs a place of its own for every element.  (Rows that overlap are left to the library, which refuses them.)"""
+    room = 1
+    if t.shape[2] > 1 and t.stride(2) < t.shape[3]:
+        return t
+    for stride, size in sorted(zip(t.stride(), t.shape)):
+        if size > 1:
+            if stride < room:
+                return t.contiguous()
+            room += stride * (size - 1)
+    return t
+
+
 def fa_bwd(p, q, k, v, o, do, lse, workspace_bytes=None):
-    """Run acct_fa_bwd; returns (dQ, dK, dV) laid out like q, k, v.  `workspace_bytes`: the size of the
+    """Run acct_fa_bwd; returns (dQ, dK, dV) laid out like q, k, v, those of expanded operands contiguous.  `workspace_bytes`: the size of the
     workspace to pass instead of acct_fa_bwd_workspace_bytes (a smaller one that still holds the required
     parts makes the library cut the query range of the dK/dV kernel into the slices that fit, or not at all)."""
     lib = load()
@@ -351,6 +365,12 @@ def fa_bwd(p, q, k, v, o, do, lse, workspace_bytes=None):
         tmp.copy_(do)
         do = tmp
     p.o_stride = _bhs_strides(o)
+    own = [_apart(t) for t in (q, k, v)]
+    if any(a is not b for a, b in zip(own, (q, k, v))):
+        q, k, v = own
+        p = AcctFaParams.from_buffer_copy(p)
+        p.q, p.k, p.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
+        p.q_stride, p.k_stride, p.v_stride = _bhs_strides(q), _bhs_strides(k), _bhs_strides(v)
     gdt = torch.float32 if p.grad_f32 else q.dtype       # (grad_f32: the reference's registered output type)
     dq = torch.empty_strided(q.size(), q.stride(), dtype=gdt, device=q.device)
     dk = torch.empty_strided(k.size(), k.stride(), dtype=gdt, device=k.device)

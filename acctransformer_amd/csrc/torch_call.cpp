@@ -17,6 +17,8 @@
 #include <c10/core/SafePyObject.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
+#include <array>
 #include <mutex>
 #include <optional>
 
@@ -61,6 +63,21 @@ Tensor bytes_like(const Tensor& like, size_t n) {
   return n ? at::empty({(int64_t)n}, like.options().dtype(at::kByte)) : Tensor();
 }
 
+// `t`, or a copy of it where elements may share memory (an expanded operand): its gradient has the same layout and needs a
+// place of its own for every element.
+Tensor apart(Tensor t) {
+  std::array<std::pair<int64_t, int64_t>, 4> dims;
+  for (int i = 0; i < 4; i++) dims[i] = {t.stride(i), t.size(i)};
+  std::sort(dims.begin(), dims.end());
+  int64_t room = 1;
+  for (const auto& [stride, size] : dims) {
+    if (size <= 1) continue;
+    if (stride < room) return t.contiguous();
+    room += stride * (size - 1);
+  }
+  return t;
+}
+
 struct FlashAttentionBackward : public torch::autograd::Node {
   Problem problem;
   std::optional<c10::SafePyObject> entry;      // the operator's record of the mask_bits buffer, for `params`
@@ -73,9 +90,11 @@ struct FlashAttentionBackward : public torch::autograd::Node {
   }
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
-    const Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), o = o_.unpack(shared_from_this()), lse = lse_.unpack();
+    Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack();
+    const Tensor o = o_.unpack(shared_from_this()), lse = lse_.unpack();
     c10::DeviceGuard device(q.device());
     at::AutoDispatchBelowADInplaceOrView below;
+    q = apart(q); k = apart(k); v = apart(v);
     Tensor dout = grads[0];
     if (!dout.defined()) dout = at::zeros_like(o);
     if (dout.strides() != o.strides()) {       // the kernels read dO with O's strides

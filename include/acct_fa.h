@@ -180,7 +180,9 @@ size_t acct_fa_mask_bits_bytes(const acct_fa_params* p);
  * T/flash_attention_bwd.py:436-477 (the bprop of T/flash_attention_impl.py:117-124
  * casts its fp32 results to fp16; here dQ,dK,dV are written in p->dtype directly,
  * accumulated in fp32 registers).  O and dO use p->o_stride; dQ,dK,dV use the
- * strides of q,k,v.  Deterministic: no atomics. */
+ * strides of q,k,v, so operands whose heads or batches share memory (a stride
+ * of 0) have to be copied first: their gradients would be written over each
+ * other.  Deterministic: no atomics. */
 int acct_fa_bwd(const acct_fa_params* p, const void* O, const void* dO, const float* LSE,
                 void* dQ, void* dK, void* dV,
                 void* workspace, size_t workspace_bytes, void* stream);

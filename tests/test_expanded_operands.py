@@ -1,0 +1,58 @@
+"""Operands that share memory between heads or batches (`k.expand(...)`): their gradients are those of materialised copies."""
+import pytest
+import torch
+
+from acctransformer_amd import _capi
+from acctransformer_amd.flash_attention.ops.flash_attention import flash_attention_impl as impl
+from acctransformer_amd.flash_attention.ops.flash_attention.flash_attention_impl import get_flash_attention
+
+DEV = "cuda:0"
+B, N, SQ, SK, D = 2, 3, 130, 200, 64
+
+
+def test_which_operands_are_copied():
+    t = torch.zeros(B, N, 8, 16)
+    for own in (t, t.transpose(1, 2), t[:, 1:2].expand(B, 1, 8, 16), t[:, :, ::2], torch.zeros(1, 1, 8, 16).expand(1, 1, 8, 16)):
+        assert _capi._apart(own) is own
+    for shared in (t[:, :1].expand(B, N, 8, 16), t[:1].expand(B, N, 8, 16), t.as_strided((B, N, 4, 16), (N * 8 * 16, 32, 16, 1))):
+        copy = _capi._apart(shared)
+        assert copy is not shared and copy.is_contiguous() and torch.equal(copy, shared)
+    rows = t[:, :, :1].expand(B, N, 8, 16)                    # (refused by the library)
+    assert _capi._apart(rows) is rows
+
+
+def _leaf(shape, seed):
+    return torch.randn(*shape, generator=torch.Generator(device=DEV).manual_seed(seed), device=DEV).half().requires_grad_()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("form", ["heads", "batches", "query", "windows"])
+def test_gradients_of_expanded_operands(form, native, monkeypatch):
+    if not native:
+        monkeypatch.setattr(impl, "_native_call", lambda *a: None)
+    op = get_flash_attention(scale=0.125)
+    do = _leaf((B, N, SQ, D), 9).detach()
+    kv = (B, 1, SK, D) if form == "heads" else (1, N, SK, D) if form == "batches" else (B, N, SK, D)
+    leaves = [_leaf((B, 1, SQ, D) if form == "query" else (B, N, SQ, D), 1), _leaf(kv, 2), _leaf(kv, 3)]
+
+    def operands(copied):
+        q, k, v = leaves
+        if form == "windows":                                 # heads are overlapping windows of one longer sequence
+            k, v = (t.as_strided((B, N, 100, D), (N * SK * D, 50 * D, D, 1)) for t in (k, v))
+        else:
+            q, k, v = q.expand(B, N, SQ, D), k.expand(B, N, SK, D), v.expand(B, N, SK, D)
+        return [t.contiguous() for t in (q, k, v)] if copied else [q, k, v]
+
+    o, _ = op(*operands(False))
+    got = torch.autograd.grad(o, leaves, do)
+    ref, _ = op(*operands(True))
+    want = torch.autograd.grad(ref, leaves, do)
+    assert torch.equal(o, ref)
+    for a, b in zip(got, want):                               # the same kernels on the same values, and autograd's own sums
+        assert torch.equal(a, b)
+    q, k, v = operands(False)
+    o, lse = op(q, k, v)
+    bprop = op.bprop(q, k, v, None, None, None, (o, lse), (do,))[:3]
+    want = op.bprop(*operands(True), None, None, None, (o, lse), (do,))[:3]
+    assert all(torch.equal(a, b) for a, b in zip(bprop, want))
