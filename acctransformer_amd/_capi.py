@@ -22,6 +22,7 @@ DROP_U8, DROP_F16 = 0, 1
 DROP_BITS_ONE_BAND = 0x100
 BLOCK_UNBOUNDED = 65536
 
+ACCT_E_SHAPE = -2
 ERROR_NAMES = {
     0: "ACCT_OK", -1: "ACCT_E_NULLPTR", -2: "ACCT_E_SHAPE", -3: "ACCT_E_DTYPE", -4: "ACCT_E_HEADDIM",
     -5: "ACCT_E_ARCH", -6: "ACCT_E_LAUNCH", -7: "ACCT_E_WORKSPACE", -8: "ACCT_E_PARAM",
@@ -150,6 +151,10 @@ def _bhs_strides(t):
     """(batch, head, row) element strides of a [B,N,S,D] tensor whose last dim is contiguous."""
     if t.stride(3) != 1 and t.size(3) != 1:
         raise ValueError("last dimension must be contiguous")
+    if not any(t.stride()[:3]):                            # one row for all (to the library, three zeros are a contiguous tensor)
+        if t.size(2) > 1:
+            raise AcctError(ACCT_E_SHAPE, "row stride smaller than D")
+        return (ctypes.c_int64 * 3)(0, 0, t.size(3))
     return (ctypes.c_int64 * 3)(t.stride(0), t.stride(1), t.stride(2))
 
 

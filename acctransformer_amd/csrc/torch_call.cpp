@@ -43,6 +43,7 @@ void set_error(int rc) {
 
 void take_strides(const Tensor& t, int64_t (&s)[3]) {
   for (int i = 0; i < 3; i++) s[i] = t.stride(i);
+  if (!s[0] && !s[1] && !s[2]) s[2] = t.size(3);       // one row for all (to the library, three zeros are a contiguous tensor)
 }
 
 // One call: its parameters without addresses, and the tensors beside q, k, v that they go with.
@@ -196,6 +197,8 @@ bool describe(Problem& c, const Tensor& q, const Tensor& k, const Tensor& v) {
   const int64_t B = q.size(0), N = q.size(1), Sq = q.size(2), D = q.size(3), Sk = k.size(2);
   for (int64_t x : {B, N, Sq, Sk, D})
     if (x > INT32_MAX) return false;
+  for (const Tensor* t : {&q, &k, &v})
+    if (t->size(2) > 1 && t->stride(0) == 0 && t->stride(1) == 0 && t->stride(2) == 0) return false;    // (refused there)
   if (k.size(0) != B || k.size(1) != N || k.size(3) != D || v.sizes() != k.sizes()) return false;
   const Tensor* all[] = {&q, &k, &v, &c.mask, &c.drop, &c.alibi, &c.mask_bits};
   for (const Tensor* t : all)

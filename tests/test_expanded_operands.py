@@ -21,6 +21,28 @@ def test_which_operands_are_copied():
     assert _capi._apart(rows) is rows
 
 
+def test_one_row_for_all_is_not_a_contiguous_tensor():
+    t = torch.zeros(B, N, 8, 16, dtype=torch.float16)
+    row = torch.zeros(16, dtype=torch.float16)
+    for operands in ((row.expand(B, N, 8, 16), t, t), (t, row.expand(B, N, 8, 16), t), (t, t, row.expand(B, N, 8, 16))):
+        with pytest.raises(_capi.AcctError, match="row stride"):
+            _capi.make_params(*operands, scale=1.0)
+    one = row.as_strided((B, N, 1, 16), (0, 0, 0, 1))         # (a single row per head is accepted)
+    assert list(_capi.make_params(one, t, t, scale=1.0).q_stride) == [0, 0, 16]
+
+
+@pytest.mark.gpu
+def test_one_row_for_all_on_the_gpu():
+    op = get_flash_attention(scale=0.125)
+    q, row = _leaf((B, N, SQ, D), 1), _leaf((D,), 2)
+    with pytest.raises(_capi.AcctError, match="row stride"):
+        op(q, row.expand(B, N, SK, D), row.expand(B, N, SK, D))
+    k = _leaf((B, N, SK, D), 3)
+    with torch.no_grad():
+        one = row.as_strided((B, N, 1, D), (0, 0, 0, 1))
+        assert torch.equal(op(one, k, k)[0], op(one.contiguous(), k, k)[0])
+
+
 def _leaf(shape, seed):
     return torch.randn(*shape, generator=torch.Generator(device=DEV).manual_seed(seed), device=DEV).half().requires_grad_()
 
