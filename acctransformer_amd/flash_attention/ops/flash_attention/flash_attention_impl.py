@@ -257,7 +257,9 @@ def _native_call(kind_of_call, q, k, v, attn_mask, dropout_mask, alibi_mask, pre
             p = _capi.make_params(q, k, v, scale=scale, prev_block_num=prev_block_num, next_block_num=next_block_num, mask_kind=kind,
                                   attn_mask=mask, row_block_prefix=row_block_prefix)
             _attach_mask_bits(p, mask, q.device)
-            entry = p._mask_bits_entry
+            entry = getattr(p, "_mask_bits_entry", None)
+            if entry is None:                             # (an extent of 0: nothing to derive, and the call is refused there)
+                return None
         bits, filled = entry[3], entry[4][0]
     drop, keep, philox, seed, offset = None, 1.0, False, 0, 0
     if dropout_mask is not None:

@@ -107,6 +107,15 @@ def test_native_call_refuses_as_before():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("record", [True, False])
+@pytest.mark.parametrize("B, N, Sq, Sk", [(0, 2, 64, 64), (2, 0, 64, 64), (2, 2, 0, 64), (2, 2, 64, 0)])
+def test_extents_of_zero_with_a_mask_are_refused_in_the_librarys_words(B, N, Sq, Sk, record):
+    q, k, v = (torch.zeros(B, N, S, 64, dtype=torch.float16, device=DEV, requires_grad=record) for S in (Sq, Sk, Sk))
+    with pytest.raises(_capi.AcctError, match="ACCT_E_SHAPE"):
+        get_flash_attention(scale=0.125)(q, k, v, torch.zeros(1, Sq, Sk, dtype=torch.uint8, device=DEV))
+
+
+@pytest.mark.gpu
 def test_native_call_on_another_stream_and_in_the_inference_operator():
     q, k, v, do, *_ = _inputs("plain")
     op = get_flash_attention(scale=1.0)
