@@ -20,7 +20,6 @@
 #include <algorithm>
 #include <array>
 #include <mutex>
-#include <optional>
 
 #include "../../include/acct_fa.h"
 
@@ -81,13 +80,25 @@ Tensor apart(Tensor t) {
 
 struct FlashAttentionBackward : public torch::autograd::Node {
   Problem problem;
-  std::optional<c10::SafePyObject> entry;      // the operator's record of the mask_bits buffer, for `params`
+  std::shared_ptr<c10::SafePyObject> entry;    // the operator's record of the mask_bits buffer, for `params`
   torch::autograd::SavedVariable q_, k_, v_, o_, lse_;
 
   std::string name() const override { return "_FlashAttentionFnBackward"; }
+  // what a reader on another thread sees while a backward ends (called with the interpreter lock, waits without it)
+  std::pair<Problem, std::shared_ptr<c10::SafePyObject>> record() {
+    pybind11::gil_scoped_release free_python;
+    std::lock_guard<std::mutex> lock(mutex_);
+    return {problem, entry};
+  }
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
     for (auto* s : {&q_, &k_, &v_, &o_, &lse_}) s->reset_data();
+    // (no backward can follow, and whoever still holds an output would hold the keep bits of its dropout with it)
+    problem = Problem{problem.p};
+    acct_fa_params& p = problem.p;
+    p.q = p.k = p.v = p.attn_mask = p.drop_mask = p.alibi = nullptr;
+    p.mask_bits = p.drop_bits = nullptr;
+    entry.reset();
   }
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -129,8 +140,7 @@ FlashAttentionBackward* node_of(PyObject* self) {
 
 PyObject* get_params(PyObject* self, void*) {
   HANDLE_TH_ERRORS
-  FlashAttentionBackward* n = node_of(self);
-  const Problem& c = n->problem;
+  const auto [c, entry] = node_of(self)->record();
   const Tensor* kept[] = {&c.mask, &c.drop, &c.alibi, &c.mask_bits, &c.drop_bits};
   THPObjectPtr tensors(PyList_New(0));
   if (!tensors) return nullptr;
@@ -141,14 +151,14 @@ PyObject* get_params(PyObject* self, void*) {
     }
   THPObjectPtr raw(PyBytes_FromStringAndSize(reinterpret_cast<const char*>(&c.p), sizeof(c.p)));
   if (!raw) return nullptr;
-  PyObject* e = n->entry ? n->entry->ptr(getPyInterpreter()) : Py_None;
+  PyObject* e = entry ? entry->ptr(getPyInterpreter()) : Py_None;
   return PyObject_CallFunctionObjArgs(g_params_view, raw.get(), tensors.get(), e, nullptr);
   END_HANDLE_TH_ERRORS
 }
 
 PyObject* get_drop_bits(PyObject* self, void*) {
   HANDLE_TH_ERRORS
-  const Tensor& t = node_of(self)->problem.drop_bits;
+  const Tensor t = node_of(self)->record().first.drop_bits;
   if (!t.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(t);
   END_HANDLE_TH_ERRORS
@@ -322,7 +332,7 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   if (node && a[7] != Py_None) {
     Py_INCREF(a[7]);
-    node->entry.emplace(a[7], getPyInterpreter());
+    node->entry = std::make_shared<c10::SafePyObject>(a[7], getPyInterpreter());
   }
   THPObjectPtr out(PyTuple_New(2));
   if (!out) return nullptr;

@@ -116,6 +116,24 @@ def test_extents_of_zero_with_a_mask_are_refused_in_the_librarys_words(B, N, Sq,
 
 
 @pytest.mark.gpu
+def test_a_backward_gives_back_the_keep_bits():
+    q, k, v, do, *_ = _inputs("plain")
+    op = get_flash_attention(scale=0.125, keep_prob=0.9)
+    o, _ = op(q, k, v, torch.zeros(1, 200, 264, dtype=torch.uint8, device=DEV), (3, 4))
+    bits = o.grad_fn.drop_bits
+    size, at = bits.numel(), bits.data_ptr()
+    assert at == o.grad_fn.params.drop_bits and o.grad_fn.params.mask_bits
+    del bits
+    torch.autograd.grad(o, q, do, retain_graph=True)
+    assert o.grad_fn.drop_bits.data_ptr() == at               # (a second backward may follow)
+    before = torch.cuda.memory_allocated()
+    dq, = torch.autograd.grad(o, q, do)
+    assert torch.cuda.memory_allocated() <= before + dq.numel() * 2 - size
+    p = o.grad_fn.params
+    assert o.grad_fn.drop_bits is None and not p.drop_bits and not p.mask_bits and not p.q and p.Sq == 200 and p.drop_bits_filled
+
+
+@pytest.mark.gpu
 def test_native_call_on_another_stream_and_in_the_inference_operator():
     q, k, v, do, *_ = _inputs("plain")
     op = get_flash_attention(scale=1.0)
