@@ -115,16 +115,19 @@ _native = None
 
 
 def native():
-    """The call path in native code (csrc/torch_call.cpp, loaded once).  Raises if it has not been built."""
+    """The call path in native code (csrc/torch_call.cpp, loaded once), over the library that `load` loaded.  Raises if it has
+    not been built."""
     global _native
     if _native is None:
-        load()
+        lib = load()
         try:
             from acctransformer_amd import _native as module
         except ImportError as e:
             raise ImportError("acctransformer_amd/_native.so does not load: build it with `make -C acctransformer_amd/csrc` "
                               "(or `python -c 'import __graft_entry__ as g; g.build()'`)") from e
-        module.setup(AcctError, _params_view)
+        entries = (lib.acct_fa_fwd, lib.acct_fa_bwd, lib.acct_fa_fwd_split_workspace_bytes, lib.acct_fa_bwd_workspace_bytes,
+                   lib.acct_fa_drop_bits_bytes, lib.acct_last_error)
+        module.setup(AcctError, _params_view, *(ctypes.cast(f, ctypes.c_void_p).value for f in entries))
         _native = module
     return _native
 

@@ -27,6 +27,15 @@ namespace {
 
 using at::Tensor;
 
+// the library's entry points, as the Python binding loaded them (one library in the process, whichever file it came from)
+struct Library {
+  decltype(&acct_fa_fwd) fwd;
+  decltype(&acct_fa_bwd) bwd;
+  decltype(&acct_fa_fwd_split_workspace_bytes) fwd_workspace_bytes;
+  decltype(&acct_fa_bwd_workspace_bytes) bwd_workspace_bytes;
+  decltype(&acct_fa_drop_bits_bytes) drop_bits_bytes;
+  decltype(&acct_last_error) last_error;
+} g_lib;
 PyObject* g_error = nullptr;         // AcctError
 PyObject* g_params_view = nullptr;   // (bytes of acct_fa_params, tensors, mask_bits entry) -> AcctFaParams
 
@@ -34,7 +43,7 @@ void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device
 
 // runs with the interpreter lock held
 void set_error(int rc) {
-  PyObject* e = PyObject_CallFunction(g_error, "is", rc, acct_last_error());
+  PyObject* e = PyObject_CallFunction(g_error, "is", rc, g_lib.last_error());
   if (!e) return;
   PyErr_SetObject(g_error, e);
   Py_DECREF(e);
@@ -119,10 +128,10 @@ struct FlashAttentionBackward : public torch::autograd::Node {
     take_strides(o, c.p.o_stride);
     Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = at::empty_strided(k.sizes(), k.strides(), k.options()),
            dv = at::empty_strided(v.sizes(), v.strides(), v.options());
-    const size_t n = acct_fa_bwd_workspace_bytes(&c.p);
+    const size_t n = g_lib.bwd_workspace_bytes(&c.p);
     const Tensor ws = bytes_like(q, n);
-    const int rc = acct_fa_bwd(&c.p, o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                               n ? ws.data_ptr() : nullptr, n, stream_of(q));
+    const int rc = g_lib.bwd(&c.p, o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                             n ? ws.data_ptr() : nullptr, n, stream_of(q));
     if (rc != ACCT_OK) {
       pybind11::gil_scoped_acquire lock_python;
       set_error(rc);
@@ -302,15 +311,15 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         take_strides(o, p.o_stride);
         if (record) {
           // with dropout, the keep bits the forward packs (or draws) are kept for the backward of this step
-          c.drop_bits = bytes_like(q, acct_fa_drop_bits_bytes(&p));
+          c.drop_bits = bytes_like(q, g_lib.drop_bits_bytes(&p));
           if (c.drop_bits.defined()) {
             p.drop_bits = c.drop_bits.data_ptr();
             p.drop_mask_kind |= ACCT_DROP_BITS_ONE_BAND;     // (the backward runs on these very parameters)
           }
         }
-        const size_t bytes = acct_fa_fwd_split_workspace_bytes(&p);
+        const size_t bytes = g_lib.fwd_workspace_bytes(&p);
         const Tensor ws = bytes_like(q, bytes);
-        rc = acct_fa_fwd(&p, o.data_ptr(), lse.data_ptr<float>(), bytes ? ws.data_ptr() : nullptr, bytes, stream_of(q));
+        rc = g_lib.fwd(&p, o.data_ptr(), lse.data_ptr<float>(), bytes ? ws.data_ptr() : nullptr, bytes, stream_of(q));
       }
     }
     if (known && rc == ACCT_OK && record) {
@@ -346,16 +355,26 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// setup(AcctError, view of the parameters)
+// setup(AcctError, view of the parameters, address of each entry point in the order of `Library`)
 PyObject* setup(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 2) {
-    PyErr_SetString(PyExc_TypeError, "setup takes 2 arguments");
+  HANDLE_TH_ERRORS
+  if (n != 8) {
+    PyErr_SetString(PyExc_TypeError, "setup takes 8 arguments");
     return nullptr;
   }
+  void* at[6];
+  for (int i = 0; i < 6; i++) {
+    at[i] = PyLong_AsVoidPtr(a[2 + i]);
+    if (PyErr_Occurred()) return nullptr;
+  }
+  auto take = [](auto& f, void* p) { f = reinterpret_cast<std::decay_t<decltype(f)>>(p); };
+  take(g_lib.fwd, at[0]); take(g_lib.bwd, at[1]); take(g_lib.fwd_workspace_bytes, at[2]);
+  take(g_lib.bwd_workspace_bytes, at[3]); take(g_lib.drop_bits_bytes, at[4]); take(g_lib.last_error, at[5]);
   Py_INCREF(a[0]); Py_INCREF(a[1]);
   g_error = a[0];
   g_params_view = a[1];
   Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef g_methods[] = {{"forward", (PyCFunction)(void (*)())forward, METH_FASTCALL, "one call of the operator"},

@@ -1,5 +1,10 @@
 """The operator's native call (csrc/torch_call.cpp) against the Python autograd function that takes the unusual calls: the same
 outputs, gradients, refusals and graph."""
+import os
+import shutil
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -9,6 +14,7 @@ from acctransformer_amd.flash_attention.ops.flash_attention.flash_attention_impl
 from acctransformer_amd.infer.flash_attention.tik.flash_attention_tik import flash_attention_tik
 
 DEV = "cuda:0"
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def test_what_the_native_call_leaves_to_python():
@@ -19,6 +25,19 @@ def test_what_the_native_call_leaves_to_python():
     assert _capi.native().forward(False, None, t(), t(), *rest) is None
     with pytest.raises(TypeError):
         _capi.native().forward(False, t(), t(), t())
+
+
+def test_the_native_call_uses_the_library_that_was_loaded(tmp_path):
+    other = shutil.copy(_capi.lib_path(), tmp_path / "other.so")
+    run = subprocess.run([sys.executable, "-c", f"""
+from acctransformer_amd import _capi
+_capi._LIB_PATH = {str(other)!r}
+_capi.native()
+maps = open('/proc/self/maps').read()
+assert {str(other)!r} in maps and '_native.so' in maps and 'libacct_fa.so' not in maps
+print('one library')
+"""], capture_output=True, text=True, cwd=ROOT, timeout=300)
+    assert run.stdout.strip() == "one library", run.stderr
 
 
 def _inputs(form):
