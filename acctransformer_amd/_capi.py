@@ -123,7 +123,7 @@ def native():
         try:
             from acctransformer_amd import _native as module
         except ImportError as e:
-            raise ImportError("acctransformer_amd/_native.so does not load: build it with `make -C acctransformer_amd/csrc` "
+            raise ImportError(f"acctransformer_amd/_native.so does not load ({e}): build it with `make -C acctransformer_amd/csrc` "
                               "(or `python -c 'import __graft_entry__ as g; g.build()'`)") from e
         entries = (lib.acct_fa_fwd, lib.acct_fa_bwd, lib.acct_fa_fwd_split_workspace_bytes, lib.acct_fa_bwd_workspace_bytes,
                    lib.acct_fa_drop_bits_bytes, lib.acct_last_error)

@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <array>
+#include <cstring>
 #include <mutex>
 
 #include "../../include/acct_fa.h"
@@ -385,6 +386,14 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, g_methods
 }  // namespace
 
 PyMODINIT_FUNC PyInit__native() {
+  // torch's classes are compiled in: another version has other layouts, which a symbol that still resolves does not show
+  THPObjectPtr torch(PyImport_ImportModule("torch"));
+  THPObjectPtr version(torch ? PyObject_GetAttrString(torch.get(), "__version__") : nullptr);
+  if (!version) return nullptr;
+  THPObjectPtr text(PyObject_Str(version.get()));
+  const char* now = text ? PyUnicode_AsUTF8(text.get()) : nullptr;
+  if (!now) return nullptr;
+  if (strcmp(now, ACCT_TORCH)) return PyErr_Format(PyExc_ImportError, "built for torch %s, this is torch %s", ACCT_TORCH, now);
   torch::autograd::_initFunctionPyTypeObject(g_node_type, "acctransformer_amd._FlashAttentionFnBackward", g_node_properties, nullptr);
   torch::autograd::registerCppFunction(typeid(FlashAttentionBackward), &g_node_type);
   return PyModule_Create(&g_module);

@@ -40,6 +40,32 @@ print('one library')
     assert run.stdout.strip() == "one library", run.stderr
 
 
+def test_a_module_of_another_torch_does_not_load():
+    run = subprocess.run([sys.executable, "-c", """
+import torch
+torch.__version__ = '0.0.0'
+from acctransformer_amd import _capi
+try:
+    _capi.native()
+except ImportError as e:
+    print(e)
+"""], capture_output=True, text=True, cwd=ROOT, timeout=300)
+    assert "this is torch 0.0.0" in run.stdout and "make -C" in run.stdout, run.stderr
+
+
+@pytest.mark.parametrize("torch_there", [True, False])
+def test_the_c_abi_builds_without_torch(torch_there, tmp_path):
+    python = sys.executable
+    if not torch_there:
+        python = str(tmp_path / "python")                   # an interpreter without installed packages
+        (tmp_path / "python").write_text(f"#!/bin/sh\nexec {sys.executable} -S \"$@\"\n")
+        os.chmod(python, 0o755)
+    run = subprocess.run(["make", "-n", "-B", "-C", "acctransformer_amd/csrc", f"PYTHON={python}"], capture_output=True, text=True, cwd=ROOT,
+                         timeout=300)
+    assert run.returncode == 0 and "libacct_fa.so" in run.stdout and "libacct_fa_ms.so" in run.stdout, run.stderr
+    assert ("torch_call.cpp" in run.stdout) == torch_there and ("no torch" in run.stdout) != torch_there
+
+
 def _inputs(form):
     g = torch.Generator(device=DEV).manual_seed(5)
     B, N, Sq, Sk, D = 2, 3, 200, 264, 64
