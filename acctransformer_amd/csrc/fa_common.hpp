@@ -413,11 +413,12 @@ ACCT_DEV void load_bias4(const T* row, int kv, int limit, bool vec_ok, float out
 #define ACCT_GLB __attribute__((address_space(1)))
 
 // Stage rows [row0, row0 + ROWS) of a row-major global matrix into a swizzled LDS
-// tile with NW waves.  Rows past nrows repeat the last valid row (finite data whose
-// contribution is zeroed by the caller's masking), slots past the `cpr` valid 16-byte
+// tile with NW waves.  Rows past nrows repeat the last valid row, for callers that remove
+// their scores by a select; with ZERO they are zeros (V of the forward: they are multiplied by a
+// probability of 0, which would turn an infinity in the last row into NaN).  Slots past the `cpr` valid 16-byte
 // chunks of a row (head dim / 8) repeat the last valid chunk.
 // `wv` < 0: the NW waves are the workgroup's first NW; else the calling wave's index among the NW.
-template <typename T, int D, int ROWS, int NW>
+template <typename T, int D, int ROWS, int NW, bool ZERO = false>
 ACCT_DEV void tile_dma(const T* base, int64_t row_stride, int row0, int nrows, ACCT_LDS char* buf, int cpr, int wv = -1) {
   using C = SwzCfg<D>;
   constexpr int NI = ROWS / C::RPI;
@@ -431,6 +432,10 @@ ACCT_DEV void tile_dma(const T* base, int64_t row_stride, int row0, int nrows, A
     const int r = inst * C::RPI + lane / C::CH;
     const int lc = min((lane % C::CH) ^ C::swz(r), cpr - 1);
     const int grow = min(row0 + r, nrows - 1);
+    if (ZERO && row0 + r >= nrows) {
+      *reinterpret_cast<ACCT_LDS u32x4*>(buf + inst * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+      continue;
+    }
     const T* src = base + (int64_t)grow * row_stride + lc * 8;
     // Issued as inline assembly on purpose: the compiler then does not order every later LDS read
     // behind these loads (it cannot tell the two tile buffers apart), which would serialise the

@@ -112,14 +112,18 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   const int cpr = a.hd >> 3;                                // valid 16-byte chunks per row
   kdma.plan(a.k_ss, cpr);
   vdma.plan(a.v_ss, cpr);
-  // stage key rows [j BN, (j+1) BN) of K or V into an LDS tile
-  auto stage_tile = [&](const TileDma<T, D, BN, NW>& dma, const T* base, int64_t ss, int j, ACCT_LDS char* dst) {
-    if ((j + 1) * BN <= a.Sk) dma.issue(base, ss, j * BN, dst);
-    else tile_dma<T, D, BN, NW>(base, ss, j * BN, a.Sk, dst, cpr);   // ragged last tile: clamped rows
+  // stage key rows [j BN, (j+1) BN) into an LDS tile
+  auto stage_k = [&](int j, ACCT_LDS char* dst) {
+    if ((j + 1) * BN <= a.Sk) kdma.issue(kp, a.k_ss, j * BN, dst);
+    else tile_dma<T, D, BN, NW>(kp, a.k_ss, j * BN, a.Sk, dst, cpr);         // ragged last tile: clamped rows
+  };
+  auto stage_v = [&](int j, ACCT_LDS char* dst) {
+    if ((j + 1) * BN <= a.Sk) vdma.issue(vp, a.v_ss, j * BN, dst);
+    else tile_dma<T, D, BN, NW, true>(vp, a.v_ss, j * BN, a.Sk, dst, cpr);   // and zeros
   };
   if (j_lo <= j_hi) {
-    stage_tile(kdma, kp, a.k_ss, j_lo, smem);
-    stage_tile(vdma, vp, a.v_ss, j_lo, smem + TILEB);
+    stage_k(j_lo, smem);
+    stage_v(j_lo, smem + TILEB);
   }
 
   // ---- Q fragments (B operand of K Q^T): lane holds row l32, d = 16t + 8g .. +7 ----
@@ -463,7 +467,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       }
       if (j > j_lo && j <= j_hi) {                           // (that of the first tile is under way)
         if ((j + 1) * BN <= a.Sk) vdma.issue(vfill, a.v_ss, 0, smem + par + TILEB);
-        else tile_dma<T, D, BN, NW>(vp, a.v_ss, j * BN, a.Sk, smem + par + TILEB, cpr);
+        else tile_dma<T, D, BN, NW, true>(vp, a.v_ss, j * BN, a.Sk, smem + par + TILEB, cpr);
       }
       kfill += kstep;
       vfill += vstep;
@@ -563,7 +567,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       publish();
     };
     if (j_lo <= j_hi) {
-      if (j_lo < j_hi) stage_tile(kdma, kp, a.k_ss, j_lo + 1, smem + 2 * TILEB);
+      if (j_lo < j_hi) stage_k(j_lo + 1, smem + 2 * TILEB);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
       if (j_lo == w_lo && j_lo <= w_hi) gemm_s(smem + kg * (WN * C::PITCH), j_lo, s0);
@@ -592,8 +596,8 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       ACCT_LDS char* vbuf = kbuf + TILEB;
       if (j < j_hi) {                                       // next tile streams into the other buffer meanwhile
         ACCT_LDS char* nb = smem + (buf ^ 1) * 2 * TILEB;
-        stage_tile(kdma, kp, a.k_ss, j + 1, nb);
-        stage_tile(vdma, vp, a.v_ss, j + 1, nb + TILEB);
+        stage_k(j + 1, nb);
+        stage_v(j + 1, nb + TILEB);
         DropStage::issue(a, bh, wq0, j + 1, lane, drop_lds + (buf ^ 1) * DropStage::BYTES);
         if (BIAS && acc_bias && wq0 < a.Sq) stage_bias(j + 1);
       }
