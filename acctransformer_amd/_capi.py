@@ -346,10 +346,16 @@ def fa_fwd(p, q):
     return o, lse
 
 
+_ROW_STRIDE_END = 34087040           # (of a backward, in elements)
+
+
 def _apart(t):
     """`t`, or a copy of it where elements may share memory (an expanded operand): its gradient has the same layout and
-    needs a place of its own for every element.  (Rows that overlap are left to the library, which refuses them.)"""
+    needs a place of its own for every element.  A copy also where rows are further apart than the library takes.
+    (Rows that overlap are left to it, and refused.)"""
     room = 1
+    if t.stride(2) >= _ROW_STRIDE_END:
+        return t.contiguous()
     if t.shape[2] > 1 and t.stride(2) < t.shape[3]:
         return t
     for stride, size in sorted(zip(t.stride(), t.shape)):
@@ -367,6 +373,8 @@ def fa_bwd(p, q, k, v, o, do, lse, workspace_bytes=None):
     lib = load()
     if not q.is_cuda:
         raise RuntimeError("acct_fa_bwd needs device tensors (there is no CPU path)")
+    if o.stride(2) >= _ROW_STRIDE_END:
+        o = o.contiguous()
     if do.stride() != o.stride():
         # the kernels read dO with O's strides: copy the values into a buffer laid out like O
         tmp = torch.empty_strided(o.size(), o.stride(), dtype=o.dtype, device=o.device)

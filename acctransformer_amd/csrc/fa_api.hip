@@ -139,7 +139,6 @@ int validate(const acct_fa_params* p, bool backward) {
   }
   if (p->D > 256) return fail(ACCT_E_HEADDIM, "head_dim too large, reduce head_dim and try again. (D=%d > 256)", p->D);
   if (p->D % 8 != 0) return fail(ACCT_E_HEADDIM, "head_dim %d is not a multiple of 8", p->D);
-  (void)backward;
   // bias variants are built for the head-dim classes 64, 80 and 128 (dropout: every head dim)
   if ((p->D == 40 || p->D > 128) && p->alibi)
     return fail(ACCT_E_HEADDIM, "head_dim %d is built without the bias variants", p->D);
@@ -167,6 +166,9 @@ int validate(const acct_fa_params* p, bool backward) {
     for (int j = 0; j < 3; j++)
       if (st[i][j] < 0 || st[i][j] % 8 != 0) return fail(ACCT_E_SHAPE, "strides must be non-negative multiples of 8 elements");
     if (st[i][2] < p->D) return fail(ACCT_E_SHAPE, "row stride smaller than D");
+    const int rows = i == 0 || i == 3 ? p->Sq : p->Sk;
+    if (backward && st[i][2] >= acct::kBwdRowStrideEnd && rows >= 64)
+      return fail(ACCT_E_SHAPE, "row strides of a backward must stay below %lld elements, got %lld", (long long)acct::kBwdRowStrideEnd, (long long)st[i][2]);
   }
   for (int i = 0; i < 3; i++)
     if ((uintptr_t)ptrs[i] & 15) return fail(ACCT_E_SHAPE, "q, k and v must be 16-byte aligned");

@@ -56,6 +56,12 @@ ACCT_HD void split_map(int id, int BH, int n_tiles, int split, bool share, int& 
   wg = rank * BH + (pair - slice * BH);
 }
 
+// A tile of `rows` rows of 2-byte elements is addressed by a base and 32-bit byte offsets: whether the last row's fit (a row
+// has up to 256 elements).
+ACCT_HD bool tile_offsets_fit(int64_t row_stride, int rows) { return row_stride * (rows - 1) <= 0x7fffffffll - 256; }
+// Row strides of a backward end here (its tiles have 64 rows; in whole chunks of 8 elements).
+constexpr int64_t kBwdRowStrideEnd = 34087040;
+
 // ---- swizzle of the LDS tiles that the direct-to-LDS loads fill ----
 // Row pitch is a power of two (no padding, as the DMA writes 64 consecutive 16-byte
 // slots per wave instruction); the 16-byte chunk c of row r lives in slot c ^ swz(r).

@@ -74,8 +74,10 @@ Tensor bytes_like(const Tensor& like, size_t n) {
 }
 
 // `t`, or a copy of it where elements may share memory (an expanded operand): its gradient has the same layout and needs a
-// place of its own for every element.
+// place of its own for every element.  A copy also where rows are further apart than the library's backward takes.
+constexpr int64_t kRowStrideEnd = 34087040;
 Tensor apart(Tensor t) {
+  if (t.stride(2) >= kRowStrideEnd) return t.contiguous();
   std::array<std::pair<int64_t, int64_t>, 4> dims;
   for (int i = 0; i < 4; i++) dims[i] = {t.stride(i), t.size(i)};
   std::sort(dims.begin(), dims.end());
@@ -113,10 +115,12 @@ struct FlashAttentionBackward : public torch::autograd::Node {
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack();
-    const Tensor o = o_.unpack(shared_from_this()), lse = lse_.unpack();
+    Tensor o = o_.unpack(shared_from_this());
+    const Tensor lse = lse_.unpack();
     c10::DeviceGuard device(q.device());
     at::AutoDispatchBelowADInplaceOrView below;
     q = apart(q); k = apart(k); v = apart(v);
+    if (o.stride(2) >= kRowStrideEnd) o = o.contiguous();
     Tensor dout = grads[0];
     if (!dout.defined()) dout = at::zeros_like(o);
     if (dout.strides() != o.strides()) {       // the kernels read dO with O's strides

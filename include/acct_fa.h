@@ -182,7 +182,8 @@ size_t acct_fa_mask_bits_bytes(const acct_fa_params* p);
  * accumulated in fp32 registers).  O and dO use p->o_stride; dQ,dK,dV use the
  * strides of q,k,v, so operands whose heads or batches share memory (a stride
  * of 0) have to be copied first: their gradients would be written over each
- * other.  Deterministic: no atomics. */
+ * other.  Rows must be less than 34087040 elements apart (from 64 rows on;
+ * ACCT_E_SHAPE).  Deterministic: no atomics. */
 int acct_fa_bwd(const acct_fa_params* p, const void* O, const void* dO, const float* LSE,
                 void* dQ, void* dK, void* dV,
                 void* workspace, size_t workspace_bytes, void* stream);

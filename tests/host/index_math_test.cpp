@@ -247,6 +247,18 @@ static void test_split_map() {
       }
 }
 
+// the largest offset of a tile, as TileDma keeps it: (r * stride + 8 chunk) * 2 bytes in 32 bits
+static void test_tile_offsets() {
+  for (int rows : {64, 128, 256})
+    for (int64_t stride : {int64_t(64), int64_t(1) << 23, int64_t(9) << 20, int64_t(1) << 24, (int64_t(1) << 24) + (1 << 20), kBwdRowStrideEnd - 8, kBwdRowStrideEnd,
+                           int64_t(35) << 20, int64_t(1) << 31, int64_t(1) << 40}) {
+      const int64_t most = ((rows - 1) * stride + 256) * 2;
+      CHECK(tile_offsets_fit(stride, rows) == (most <= 0xffffffffll), "%d rows, stride %lld", rows, (long long)stride);
+    }
+  CHECK(tile_offsets_fit(kBwdRowStrideEnd - 8, 64) && !tile_offsets_fit(kBwdRowStrideEnd, 64), "where the backward's strides end");
+  CHECK(!tile_offsets_fit(int64_t(9) << 20, 256) && tile_offsets_fit(int64_t(9) << 20, 128), "256-key tiles reach half as far");
+}
+
 static void test_div_small() {
   for (int n = 1; n <= 32; n++)
     for (int idx = 0; idx < 1024; idx++) CHECK(div_small(idx, recip16(n)) == idx / n, "div_small(%d, %d)", idx, n);
@@ -279,6 +291,7 @@ int main() {
   test_visible_row_keys();
   test_keep_columns();
   test_split_map();
+  test_tile_offsets();
   test_div_small();
   if (failures) printf("%d checks failed\n", failures);
   else printf("index math: all checks passed\n");

@@ -1,4 +1,5 @@
-"""Operands that share memory between heads or batches (`k.expand(...)`): their gradients are those of materialised copies."""
+"""Operands in unusual memory.  Heads or batches that share it (`k.expand(...)`): their gradients are those of materialised
+copies.  Rows so far apart that 32-bit offsets within a tile do not reach: results are those of contiguous copies."""
 import pytest
 import torch
 
@@ -78,3 +79,37 @@ def test_gradients_of_expanded_operands(form, native, monkeypatch):
     bprop = op.bprop(q, k, v, None, None, None, (o, lse), (do,))[:3]
     want = op.bprop(*operands(True), None, None, None, (o, lse), (do,))[:3]
     assert all(torch.equal(a, b) for a, b in zip(bprop, want))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B, N, Sq, Sk, D", [(1, 2, 64, 300, 64), (1, 2, 64, 300, 128), (16, 16, 256, 260, 64), (16, 16, 256, 260, 128), (1, 2, 64, 200, 160), (2, 3, 1, 300, 64)])
+@pytest.mark.parametrize("stride", [9 << 20, 17 << 20, 35 << 20])
+def test_forward_with_rows_far_apart(B, N, Sq, Sk, D, stride):
+    g = torch.Generator(device=DEV).manual_seed(D)
+    q, k, v = (torch.randn(B, N, S, D, generator=g, device=DEV).half() for S in (Sq, Sk, Sk))
+    at = (2 * N * D, 2 * D, stride, 1)
+    memory = torch.empty((Sk - 1) * stride + 2 * B * N * D, dtype=torch.float16, device=DEV)
+    kw, vw = memory.as_strided(k.shape, at), memory.as_strided(v.shape, at, D)
+    kw.copy_(k)
+    vw.copy_(v)
+    op = get_flash_attention(scale=0.125)
+    for a, b in ((kw, v), (k, vw), (kw, vw)):
+        assert all(torch.equal(x, y) for x, y in zip(op(q, a, b), op(q, k, v)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("which", [0, 1, 2])
+@pytest.mark.parametrize("stride", [_capi._ROW_STRIDE_END - 8, _capi._ROW_STRIDE_END])
+def test_gradients_with_rows_far_apart(stride, which, native, monkeypatch):
+    if not native:
+        monkeypatch.setattr(impl, "_native_call", lambda *a: None)
+    op = get_flash_attention(scale=0.125)
+    close = [_leaf((1, 2, 130, D), s) for s in (1, 2, 3)]
+    wide = [t.detach() for t in close]
+    memory = torch.empty(129 * stride + 2 * D, dtype=torch.float16, device=DEV)
+    wide[which] = memory.as_strided((1, 2, 130, D), (2 * D, D, stride, 1)).copy_(wide[which])
+    wide = [t.requires_grad_() for t in wide]
+    do = _leaf((1, 2, 130, D), 4).detach()
+    for a, b in zip(torch.autograd.grad(op(*wide)[0], wide, do), torch.autograd.grad(op(*close)[0], close, do)):
+        assert torch.equal(a, b)

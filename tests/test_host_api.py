@@ -77,6 +77,18 @@ def test_validation_error_codes(over, code):
     assert rc == code
 
 
+def test_row_strides_that_the_backward_cannot_address():
+    lib, buf = _capi.load(), (ctypes.c_char * 64)()
+    for name in ("q_stride", "k_stride", "v_stride", "o_stride"):
+        p = _params(**{name: (ctypes.c_int64 * 3)(128, 128, _capi._ROW_STRIDE_END)})
+        assert lib.acct_fa_bwd(ctypes.byref(p), *([ctypes.addressof(buf)] * 6), None, 0, None) == -2
+        assert "row strides" in lib.acct_last_error().decode()
+        rc = lib.acct_fa_fwd(ctypes.byref(p), ctypes.addressof(buf), ctypes.addressof(buf), None, 0, None)
+        assert rc == -5                                       # (the forward takes them: no device is what ends it here)
+    for p in (_params(k_stride=(ctypes.c_int64 * 3)(128, 128, _capi._ROW_STRIDE_END - 8)), _params(k_stride=(ctypes.c_int64 * 3)(128, 128, _capi._ROW_STRIDE_END), Sk=63)):
+        assert lib.acct_fa_bwd(ctypes.byref(p), *([ctypes.addressof(buf)] * 6), None, 0, None) == -7
+
+
 def test_null_outputs_and_workspace_sizes():
     lib = _capi.load()
     p = _params()
