@@ -32,7 +32,7 @@ template <int D, int NW, int KG> constexpr int fwd_merge_stats() { return NW * (
 // KG > 1 (small grids): the waves of a workgroup form NW / KG row groups times KG key groups.  A wave then works on
 // its key group's share of every tile only, with softmax statistics of its own, and the key groups of a row group
 // are merged through LDS before the epilogue -- KG times as many workgroups for the same rows, every wave busy.
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2, int KG = 1>
+template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2, int KG = 1, bool PIPE = false>
 ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   static_assert(KT == 2 || KT == 4 || (KT == 8 && !BIAS && !DROP), "key tiles are 64, 128 or 256 rows (with a bias, 128 rows take the key-only form of it only)");
   static_assert(KG == 1 || (QG == 1 && KT % KG == 0 && NW % KG == 0), "key groups own whole 32-key chunks");
@@ -40,7 +40,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   constexpr int BN = 32 * KT;                       // key rows per tile
   constexpr int KTW = KT / KG, WN = 32 * KTW;       // 32-key chunks and keys of a tile that one wave works on
   constexpr int RG = NW / KG;                       // row groups
-  constexpr bool PIPE = !BIAS && !DROP && !MASKT && QG == 1 && KG == 1 && NW == 8 && KT == 4 && D <= 64;
+  static_assert(!PIPE || (!BIAS && !DROP && !MASKT && QG == 1 && KG == 1 && NW == 8 && KT == 4 && D <= 64), "the pipelined loop has no side inputs");
   constexpr int FRING = 4, VRING = 3;   // fragment reads in flight ahead of their MFMA (K row-major / V transposed)
   using E = Elem<T>;
   using V8 = typename E::V8;
@@ -451,8 +451,8 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     // ---- tile loop, pipelined: step j issues O^T += V(j-1)^T P(j-1)^T and S(j+1)^T = K(j+1) Q^T with the softmax of tile j
     // between their MFMAs.  The eight waves start a step together, so in the plain loop below the two of a SIMD are in their
     // matrix phases at the same time and then both in the softmax.  Needs two tiles of scores and the packed P in registers:
-    // up to head dim 64 (with 64-key tiles head dims 80 and 128 lose 3 % to the plain loop).  Forward, us, plain / pipelined:
-    // 16 heads, 4096 x 4096, D40 73.4 / 71.1; D64 81.0 / 78.8; 32 heads, 2048 x 2048 causal, D64 39.6 / 38.4 ----
+    // up to head dim 64 (with 64-key tiles head dims 80 and 128 lose 3 % to the plain loop).  For long walks: pipelined_pays,
+    // which has both sides' times ----
     // this wave's own tiles
     const int key_end = min(min(causal ? wq_end : a.Sk, wkv_limit), a.Sk) - kg * WN;
     const int w_lo = max(j_lo, max(0, wqb - a.prev_blk) * 128 / BN);
@@ -769,7 +769,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
 // rows see nothing but the causal pattern in a dense mask (block classes: clean before the diagonal, the
 // causal diagonal, skipped after it) runs the code of the variant without side inputs, by index compare.
 // A causal mask given as a tensor then costs one look at the class table per workgroup.
-template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2, int KG = 1>
+template <typename T, int D, int QG, int NW, bool BIAS, bool DROP, bool MASKT, int KT = 2, int KG = 1, bool PIPE = false>
 __global__ void __launch_bounds__(64 * NW) fa_fwd_kernel(const FaArgs a) {
   if constexpr (MASKT && (!BIAS || KT == 4) && !DROP) {
     if (BIAS && a.mask_kind != kMaskDense && a.mask_kind != kMaskTile) {
@@ -790,12 +790,12 @@ __global__ void __launch_bounds__(64 * NW) fa_fwd_kernel(const FaArgs a) {
       if (dense_lines_are_causal(fl, 1, a.Tc, qb_lo, qb_hi - qb_lo + 1, kvb_lo, kvb_hi, false, a, threadIdx.x & 63)) {
         FaArgs c = a;
         c.mask_kind = kMaskCausal;
-        fa_fwd_body<T, D, QG, NW, BIAS, false, false, KT, KG>(c);
+        fa_fwd_body<T, D, QG, NW, BIAS, false, false, KT, KG, PIPE>(c);
         return;
       }
     }
   }
-  fa_fwd_body<T, D, QG, NW, BIAS, DROP, MASKT, KT, KG>(a);
+  fa_fwd_body<T, D, QG, NW, BIAS, DROP, MASKT, KT, KG, PIPE && !MASKT>(a);
 }
 
 // Second half of a forward launch whose key range was cut into a.kv_split slices: O = sum_s w_s O_s / sum_s w_s l_s
@@ -886,7 +886,7 @@ __global__ void __launch_bounds__(256) fa_fwd_combine_kernel(const FaArgs a, int
   if (dr == 0 && g == 0) a.lse[(int64_t)bh * a.Sq + row] = l > 0.f ? mm * mnat + __logf(l) : -INFINITY;
 }
 
-template <typename T, int D, int NW, bool BIAS, bool DROP, int KT, int KG>
+template <typename T, int D, int NW, bool BIAS, bool DROP, int KT, int KG, bool PIPE = false>
 static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   using C = SwzCfg<D>;
   constexpr int QG = 1, RG = NW / KG, BM = 32 * QG * RG;
@@ -897,7 +897,7 @@ static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
                    stage = KG > 1 ? fwd_merge_stats<D, NW, KG>() + (size_t)NW * 512 : (size_t)NW * 32 * (C::DB * 64 + 16);
   constexpr size_t smem = tiles > stage ? tiles : stage;
   static_assert(smem <= 160 * 1024, "the workgroup's LDS must fit the CU's 160 KB");
-  auto kern = mask_t ? fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, true, KT, KG> : fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, BIAS || DROP, KT, KG>;
+  auto kern = mask_t ? fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, true, KT, KG, PIPE> : fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, BIAS || DROP, KT, KG, PIPE>;
   hipError_t e = allow_dynamic_lds((const void*)kern, smem);
   if (e != hipSuccess) return e;
   const long long nblk = (long long)a.n_tiles * a.B * a.N;
@@ -926,6 +926,11 @@ static hipError_t launch_fwd_t(const FaArgs& a, hipStream_t st) {
   // 20 heads, 1024 x 1024 causal, 320 workgroups 12.2 / 12.7).
   if constexpr (KG == 4 && D <= 64) {
     if (a.Sk > 128 && (long long)a.B * a.N * ((a.Sq + 63) / 64) <= 256) return launch_fwd_kt<T, D, NW, BIAS, DROP, 8, KG>(a, st);
+  }
+  // (with a mask tensor the loop runs where a workgroup sees the causal pattern in it)
+  if constexpr (BIG && KG == 1 && D <= 64 && !BIAS && !DROP) {
+    const int seen = visible_row_keys(a.Sq, a.Sk, a.prev_blk, a.next_blk, a.row_prefix);
+    if (pipelined_pays(a.Sq, seen, a.mask_kind != kMaskNone || a.next_blk == 0 || a.row_prefix)) return launch_fwd_kt<T, D, NW, false, false, 4, 1, true>(a, st);
   }
   if constexpr (BIG && BIAS) {
     return key_bias_stageable(a) ? launch_fwd_kt<T, D, NW, BIAS, DROP, 4, KG>(a, st) : launch_fwd_kt<T, D, NW, BIAS, DROP, 2, KG>(a, st);

@@ -213,6 +213,19 @@ ACCT_HD int visible_row_keys(int Sq, int Sk, int prev_blk, int next_blk, int row
   return keys < Sk ? (int)keys : Sk;
 }
 
+// Keys that a row sees on average.  `one_sided`: what it sees ends with the row (causal, a band that ends at the query's block,
+// a row prefix).
+ACCT_HD long long mean_row_keys(int Sq, int row_keys, bool one_sided) {
+  if (!one_sided) return row_keys;
+  return row_keys >= Sq ? ((long long)Sq + 1) / 2 : row_keys - (long long)row_keys * row_keys / (2ll * Sq);
+}
+// The forward's pipelined tile loop (fa_fwd.hip, head dims up to 64) takes 3 to 6 % off a tile's step, but the first scores and the
+// last product have nothing beside them: about one step, with its wait and barrier, more per workgroup.  Forward, us, plain /
+// pipelined: 256 heads, 2048 x 128 keys, D64 48 / 56; x 512 102 / 109; x 768 141 / 144; x 1024 178 / 179; x 1536 258 / 255; x 3000
+// 506 / 478; x 8192 1295 / 1243; D40 39 / 46; 92 / 93; 125 / 128; 160 / 162; 235 / 226; 460 / 427; 1172 / 1127.  16 heads, 4096 rows are alike.
+// Causal: 256 heads, S1024, D40 52.9 / 54.7; S1536 108 / 109; S2048 176 / 173; S4096 640 / 623; 32 heads, S2048 35.6 / 33.5.
+ACCT_HD bool pipelined_pays(int Sq, int row_keys, bool one_sided) { return mean_row_keys(Sq, row_keys, one_sided) >= 1024; }
+
 // How the forward kernel cuts its work.  kg: key groups of the workgroup (fa_fwd.hip; 256 / kg query rows per
 // workgroup).  kv_split: slices of the key range on workgroups of their own, which a second kernel adds up (1: none).
 //

@@ -247,6 +247,22 @@ static void test_split_map() {
       }
 }
 
+// the mean of what the rows see, against a count
+static void test_pipelined_walks() {
+  for (int Sq : {1, 100, 256, 1000, 3000})
+    for (int Sk : {1, 77, 1024, 5000}) {
+      long long all = 0;
+      for (int i = 0; i < Sq; i++) all += i + 1 < Sk ? i + 1 : Sk;
+      const double mean = (double)all / Sq;
+      const long long got = mean_row_keys(Sq, Sk, true);
+      CHECK(got >= mean - 2 && got <= mean + 2, "Sq %d Sk %d: %lld, %.1f", Sq, Sk, got, mean);
+      CHECK(mean_row_keys(Sq, Sk, false) == Sk, "all rows see all keys");
+    }
+  CHECK(!pipelined_pays(4096, 1023, false) && pipelined_pays(256, 1024, false), "short and long walks");
+  CHECK(!pipelined_pays(2046, 2046, true) && pipelined_pays(2048, 2048, true) && !pipelined_pays(256, 8192, true), "causal walks");
+  CHECK(!pipelined_pays(8192, visible_row_keys(8192, 8192, 3, 3, 0), false) && pipelined_pays(8192, visible_row_keys(8192, 8192, 4, 4, 0), false), "bands");
+}
+
 // the largest offset of a tile, as TileDma keeps it: (r * stride + 8 chunk) * 2 bytes in 32 bits
 static void test_tile_offsets() {
   for (int rows : {64, 128, 256})
@@ -292,6 +308,7 @@ int main() {
   test_keep_columns();
   test_split_map();
   test_tile_offsets();
+  test_pipelined_walks();
   test_div_small();
   if (failures) printf("%d checks failed\n", failures);
   else printf("index math: all checks passed\n");

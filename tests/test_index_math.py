@@ -23,7 +23,7 @@ def _plans(tmp_path, problems):
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-o", exe, src], check=True)
     text = "\n".join(" ".join(str(int(x)) for x in p) for p in problems)
     out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True, timeout=60).stdout
-    return [dict(zip(("kg", "kv_split", "dq_kg", "ngk", "q_split"), map(int, line.split()))) for line in out.splitlines()]
+    return [dict(zip(("kg", "kv_split", "dq_kg", "ngk", "q_split", "pipelined"), map(int, line.split()))) for line in out.splitlines()]
 
 
 def test_the_gpu_tests_of_one_kernel_run_it(tmp_path):
@@ -47,3 +47,12 @@ def test_the_two_key_group_tests_run_two(tmp_path):
         assert (plan["ngk"], plan["q_split"]) == (2, 1), (row, plan)
     rows = [(1, heads, D, 256, D, False) for heads, D in ((256, 64), (256, 80), (256, 128), (2, 64), (2, 80), (2, 128))]
     assert [plan["ngk"] for plan in _plans(tmp_path, rows)] == [2, 2, 2, 1, 1, 1]
+
+
+def test_the_gpu_tests_of_the_pipelined_forward_run_it(tmp_path):
+    import test_pipelined_forward as gpu
+    cases = [(c, long) for long, some in ((0, gpu.SHORT), (1, gpu.LONG)) for c in some if c[3] in ("none", "causal", "causal tensor")]
+    for tri in (0, 1):                                        # (a mask tensor is planned as if it hid nothing)
+        some = [(c, long) for (c, long) in cases if (c[3] == "causal") == tri]
+        for ((Sq, Sk, D, side), long), plan in zip(some, _plans(tmp_path, [gpu.heads(c[0]) + c[:3] + (tri,) for c, _ in some])):
+            assert (plan["kg"], plan["kv_split"], plan["pipelined"]) == (1, 1, long), (Sq, Sk, D, side, plan)
