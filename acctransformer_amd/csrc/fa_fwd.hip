@@ -479,17 +479,10 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       dma_wait();
       __syncthreads();
     };
+    // (a tile before the wave's last: all of its keys exist, and under the causal mask they come before the wave's first row)
     auto fused = [&](int j, f32x16 (&s)[1][KTW], f32x16 (&sn)[1][KTW], V8 (&pf)[1][KTW][2]) {
       const ACCT_LDS char* kbuf = smem + (par ^ (2 * TILEB));
       const ACCT_LDS char* vbuf = kbuf + TILEB;
-      const int kv0 = j * BN;
-      if ((causal && kv0 + WN - 1 > wq0) || kv0 + WN > a.Sk) {
-        int vis = a.Sk - 1 - kv0 - 4 * g;                    // (as in softmax)
-        if (causal) vis = min(vis, wq0 + l32 - kv0 - 4 * g);
-        const float ninf = -INFINITY;
-#pragma unroll
-        for (int e = 0; e < NE; e++) s[0][e / 16][e & 15] = select_if_gt(s[0][e / 16][e & 15], 8 * ((e & 15) >> 2) + (e & 3), vis - 32 * (e / 16), ninf);
-      }
 #pragma unroll
       for (int c = 0; c < KTW; c++)
 #pragma unroll
