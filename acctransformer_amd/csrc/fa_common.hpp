@@ -150,6 +150,7 @@ struct FaArgs {
   int dq_kg;                           // dQ kernel: key groups of the workgroup (dq_key_groups, fa_index_math.hpp)
   int dkdv_ngk;                        // dK/dV kernel: 32-key groups per wave (DkdvPlan, fa_index_math.hpp)
   int drop_visible;                    // keep bits: != 0 when those of key blocks outside the band (or past the causal / prefix limit) may be left out
+  int sk_plan;                         // forward kernel: keys up to which whole tiles are staged by plan: Sk, or 0 where rows are too far apart for that
 };
 static_assert(offsetof(FaArgs, fwd_part) > offsetof(FaArgs, philox_thr), "new fields stand behind those of the inner loops");
 
@@ -433,7 +434,9 @@ ACCT_DEV void tile_dma(const T* base, int64_t row_stride, int row0, int nrows, A
     const int lc = min((lane % C::CH) ^ C::swz(r), cpr - 1);
     const int grow = min(row0 + r, nrows - 1);
     if (ZERO && row0 + r >= nrows) {
-      *reinterpret_cast<ACCT_LDS u32x4*>(buf + inst * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+      uint32_t z = 0;
+      asm volatile("" : "+v"(z));                 // (made here: four registers of zeros would live through the caller's loop)
+      *reinterpret_cast<ACCT_LDS u32x4*>(buf + inst * 1024 + lane * 16) = u32x4{z, z, z, z};
       continue;
     }
     const T* src = base + (int64_t)grow * row_stride + lc * 8;

@@ -112,15 +112,13 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   const int cpr = a.hd >> 3;                                // valid 16-byte chunks per row
   kdma.plan(a.k_ss, cpr);
   vdma.plan(a.v_ss, cpr);
-  // stage key rows [j BN, (j+1) BN) into an LDS tile (keys before `k_whole` / `v_whole` by plan; rows that are too far apart for
-  // its 32-bit offsets never)
-  const int k_whole = tile_offsets_fit(a.k_ss, BN) ? a.Sk : 0, v_whole = tile_offsets_fit(a.v_ss, BN) ? a.Sk : 0;
+  // stage key rows [j BN, (j+1) BN) into an LDS tile (whole tiles by plan)
   auto stage_k = [&](int j, ACCT_LDS char* dst) {
-    if ((j + 1) * BN <= k_whole) kdma.issue(kp, a.k_ss, j * BN, dst);
+    if ((j + 1) * BN <= a.sk_plan) kdma.issue(kp, a.k_ss, j * BN, dst);
     else tile_dma<T, D, BN, NW>(kp, a.k_ss, j * BN, a.Sk, dst, cpr);         // ragged last tile: clamped rows
   };
   auto stage_v = [&](int j, ACCT_LDS char* dst) {
-    if ((j + 1) * BN <= v_whole) vdma.issue(vp, a.v_ss, j * BN, dst);
+    if ((j + 1) * BN <= a.sk_plan) vdma.issue(vp, a.v_ss, j * BN, dst);
     else tile_dma<T, D, BN, NW, true>(vp, a.v_ss, j * BN, a.Sk, dst, cpr);   // and zeros
   };
   if (j_lo <= j_hi) {
@@ -464,11 +462,11 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     const int64_t kstep = BN * a.k_ss, vstep = BN * a.v_ss;
     auto fill = [&](int j) {
       if (j + 2 <= j_hi) {
-        if ((j + 3) * BN <= k_whole) kdma.issue(kfill, a.k_ss, 0, smem + par);
+        if ((j + 3) * BN <= a.sk_plan) kdma.issue(kfill, a.k_ss, 0, smem + par);
         else tile_dma<T, D, BN, NW>(kp, a.k_ss, (j + 2) * BN, a.Sk, smem + par, cpr);     // ragged last tile: clamped rows
       }
       if (j > j_lo && j <= j_hi) {                           // (that of the first tile is under way)
-        if ((j + 1) * BN <= v_whole) vdma.issue(vfill, a.v_ss, 0, smem + par + TILEB);
+        if ((j + 1) * BN <= a.sk_plan) vdma.issue(vfill, a.v_ss, 0, smem + par + TILEB);
         else tile_dma<T, D, BN, NW, true>(vp, a.v_ss, j * BN, a.Sk, smem + par + TILEB, cpr);
       }
       kfill += kstep;
@@ -884,6 +882,7 @@ static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   using C = SwzCfg<D>;
   constexpr int QG = 1, RG = NW / KG, BM = 32 * QG * RG;
   a.n_tiles = (a.Sq + BM - 1) / BM;
+  a.sk_plan = tile_offsets_fit(a.k_ss, 32 * KT) && tile_offsets_fit(a.v_ss, 32 * KT) ? a.Sk : 0;
   const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
   constexpr size_t biasb = BIAS ? (KT == 4 ? 1024 : QG * 4096) : 0;     // per wave, as in the kernel
   constexpr size_t tiles = 4 * 32 * KT * (size_t)C::PITCH + NW * biasb + (size_t)NW * 2 * DropRowStage<DROP, QG, KT>::BYTES,
