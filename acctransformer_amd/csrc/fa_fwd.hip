@@ -913,15 +913,13 @@ static hipError_t launch_fwd_t(const FaArgs& a, hipStream_t st) {
   // them; a key-only bias that the DMA can stage is a 256-byte row and does.
   constexpr bool BIG = NW == 8 && D <= 128;
   static_assert(BIG || !BIAS, "the bias variants rest on this choice");
-  // Four key groups leave a wave 32 keys of a 128-key tile: a step of latencies.  Rows of 128 bytes leave room for 256-key
-  // tiles, one workgroup to a CU (forward, 128 / 256 keys, us: 4 heads, 512 x 512, D64 7.4 / 6.9; 1024 x 1024 10.6 / 9.6; but
-  // 20 heads, 1024 x 1024 causal, 320 workgroups 12.2 / 12.7).
+  int seen = visible_row_keys(a.Sq, a.Sk, a.prev_blk, a.next_blk, a.row_prefix);
   if constexpr (KG == 4 && D <= 64) {
-    if (a.Sk > 128 && (long long)a.B * a.N * ((a.Sq + 63) / 64) <= 256) return launch_fwd_kt<T, D, NW, BIAS, DROP, 8, KG>(a, st);
+    if (a.mask_kind == kMaskCausal && a.Sq < seen) seen = a.Sq;
+    if (long_tiles_pay(a.B * a.N, a.Sq, a.Sk, a.hd, seen, a.prev_blk < (a.Sq - 1) / 128)) return launch_fwd_kt<T, D, NW, BIAS, DROP, 8, KG>(a, st);
   }
   // (with a mask tensor the loop runs where a workgroup sees the causal pattern in it)
   if constexpr (BIG && KG == 1 && D <= 64 && !BIAS && !DROP) {
-    const int seen = visible_row_keys(a.Sq, a.Sk, a.prev_blk, a.next_blk, a.row_prefix);
     if (pipelined_pays(a.Sq, seen, a.mask_kind != kMaskNone || a.next_blk == 0 || a.row_prefix)) return launch_fwd_kt<T, D, NW, false, false, 4, 1, true>(a, st);
   }
   if constexpr (BIG && BIAS) {

@@ -226,6 +226,20 @@ ACCT_HD long long mean_row_keys(int Sq, int row_keys, bool one_sided) {
 // Causal: 256 heads, S1024, D40 52.9 / 54.7; S1536 108 / 109; S2048 176 / 173; S4096 640 / 623; 32 heads, S2048 35.6 / 33.5.
 ACCT_HD bool pipelined_pays(int Sq, int row_keys, bool one_sided) { return mean_row_keys(Sq, row_keys, one_sided) >= 1024; }
 
+// Four key groups leave a wave 32 keys of a 128-key tile: a step of latencies.  At head dims up to 64 LDS has room for 256-key
+// tiles, one workgroup to a CU, and a step of those takes 1.65 times as long.  They pay where the longest walk has that much fewer
+// of them: forward, 128 / 256 keys, us, D64, 4 heads, 512 queries x 129 keys 5.9 / 5.6; 257 (3 and 2 tiles) 6.7 / 7.0; 384 6.5 / 6.9; 512
+// 7.3 / 6.7; 600 (5 and 3) 8.5 / 8.4; 768 9.0 / 8.1; 1000 11.0 / 10.0; 64 x 512 causal (1 and 1) 4.7 / 5.2; a band of two blocks (2 and 2,
+// where it starts within a tile) 5.7 / 6.2.  Not where every workgroup has keys of its own from memory: 250 heads, 64 x 500 (32 MB
+// of K and V, what the eight L2s hold) 8.5 / 8.2; x 600 10.3 / 11.1; x 1024 13.7 / 14.3 (D40, 41 MB: 11.0 / 10.3).  Nor in more than one
+// round: 20 heads, 1024 x 1024 causal, 320 workgroups 12.2 / 12.7.
+// `seen`: keys of the longest walk; `moving`: walks that start at any block.
+ACCT_HD bool long_tiles_pay(int BH, int Sq, int Sk, int D, int seen, bool moving) {
+  const int n128 = (seen + 127) / 128, n256 = moving ? n128 / 2 + 1 : (n128 + 1) / 2;
+  const bool own_keys = Sq <= 64 && D > 40 && (long long)BH * Sk * D > (8 << 20);
+  return (long long)BH * ((Sq + 63) / 64) <= 256 && !own_keys && 20 * n128 > 33 * n256;
+}
+
 // How the forward kernel cuts its work.  kg: key groups of the workgroup (fa_fwd.hip; 256 / kg query rows per
 // workgroup).  kv_split: slices of the key range on workgroups of their own, which a second kernel adds up (1: none).
 //

@@ -3,6 +3,7 @@
 // prints one line per failed check and exits with the number of failures.
 // Test tier modelled on the reference's helper-level unit tests
 // (tests/train/flash_attention/ut/test_split_core_strategy.py, test_tensor_transformat.py).
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <set>
@@ -263,6 +264,21 @@ static void test_pipelined_walks() {
   CHECK(!pipelined_pays(8192, visible_row_keys(8192, 8192, 3, 3, 0), false) && pipelined_pays(8192, visible_row_keys(8192, 8192, 4, 4, 0), false), "bands");
 }
 
+// 256-key tiles of small grids: as many tiles of either length as the longest walk touches, wherever it starts
+static void test_long_tiles() {
+  for (int seen = 1; seen <= 3000; seen += seen % 128 == 0 || seen % 128 == 127 ? 1 : 126)
+    for (int moving = 0; moving < 2; moving++) {
+      int most = 0;                                        // of the 256-key tiles that hold `blocks` blocks from any one on
+      const int blocks = (seen + 127) / 128;
+      for (int first = 0; first < (moving ? 2 : 1); first++) most = std::max(most, (first + blocks - 1) / 2 + 1);
+      CHECK(long_tiles_pay(4, 512, 4096, 64, seen, moving) == (blocks > 1.65 * most), "%d keys, moving %d", seen, moving);
+    }
+  for (int Sk : {129, 256, 400, 512, 600, 2000}) CHECK(long_tiles_pay(16, 512, Sk, 64, Sk, false), "Sk %d", Sk);
+  for (int Sk : {1, 128, 257, 384}) CHECK(!long_tiles_pay(16, 512, Sk, 64, Sk, false), "Sk %d", Sk);
+  CHECK(!long_tiles_pay(257, 64, 500, 40, 500, false) && long_tiles_pay(256, 64, 500, 40, 500, false), "one round");
+  CHECK(!long_tiles_pay(250, 64, 600, 64, 600, false) && long_tiles_pay(250, 64, 512, 64, 512, false) && long_tiles_pay(250, 64, 1024, 40, 1024, false), "keys from memory");
+}
+
 // the largest offset of a tile, as TileDma keeps it: (r * stride + 8 chunk) * 2 bytes in 32 bits
 static void test_tile_offsets() {
   for (int rows : {64, 128, 256})
@@ -309,6 +325,7 @@ int main() {
   test_split_map();
   test_tile_offsets();
   test_pipelined_walks();
+  test_long_tiles();
   test_div_small();
   if (failures) printf("%d checks failed\n", failures);
   else printf("index math: all checks passed\n");

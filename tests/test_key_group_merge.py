@@ -34,6 +34,9 @@ def forward(q, k, v, kw):
     (1, 2, 511, 513, 40, "padded"), (1, 2, 700, 700, 64, "mixed"), (1, 2, 640, 640, 64, "band"), (1, 2, 640, 641, 56, "late band"),
     (1, 2, 896, 896, 64, "prefix"), (1, 1, 130, 9000, 64, "mixed"),      # (more than 64 blocks: the class window moves)
     (2, 10, 1024, 300, 64, "causal"),                                   # 320 workgroups: 128-key tiles again
+    # walks of as many 128-key tiles as 256-key ones do not pay for (above: 257 to 384 keys, bands of two blocks), and some that do
+    (1, 2, 400, 450, 48, "causal"), (2, 2, 512, 512, 64, "causal"), (1, 3, 200, 450, 64, "padded"), (2, 2, 520, 512, 64, "padded"),
+    (1, 2, 1100, 1100, 64, "wide band"), (1, 2, 1100, 1101, 56, "wide late band"), (1, 2, 900, 1290, 40, "wide band"),
     (1, 2, 100, 300, 80, "none"), (1, 2, 100, 300, 128, "padded"),      # four groups, 3 and 4 pieces
     (4, 10, 500, 200, 64, "none"), (4, 10, 500, 200, 80, "none"), (4, 10, 500, 200, 128, "mixed"), (2, 10, 500, 200, 160, "none")])   # two groups
 def test_forward_of_key_groups(B, N, Sq, Sk, D, side, dtype):
@@ -50,8 +53,9 @@ def test_forward_of_key_groups(B, N, Sq, Sk, D, side, dtype):
         m[:, :, 128:256] = 1
         m[:, : Sq // 2, 256:384] = 0
         m[:, :, 0] = 0
-    elif side in ("band", "late band"):                   # a first block in the upper half of a tile, and ends in the lower half
-        prev, nxt = (1, 0) if side == "band" else (0, 1)
+    elif "band" in side:                                  # a first block in the upper half of a tile, and ends in the lower half
+        width = 4 if "wide" in side else 1
+        prev, nxt = (0, width) if "late" in side else (width, 0)
         kw.update(prev_block_num=prev, next_block_num=nxt)
         okw.update(prev_block_num=prev, next_block_num=nxt)
     elif side == "prefix":
