@@ -5,12 +5,14 @@
 //
 // Bound by reading K and V once.  The tile kernel of fa_fwd.hip stages them through LDS in steps with a barrier and fills
 // one row of 64 of its matrix tiles.  Here 16-byte chunks of the rows go from memory straight into registers, past the
-// caches (nothing is read twice), 16 loads per wave in flight, and stay there: a row of K or V is spread over the CH lanes of a
+// caches where nothing is read twice, 16 loads per wave in flight, and stay there: a row of K or V is spread over the CH lanes of a
 // group, a wave holds 64 / CH rows per load, and every group keeps softmax statistics and sums of its own, in float32
 // from the score to the sum (the probabilities are not rounded to the element type).  The groups meet at the end.
 // Tile kernel / this one (us, bfloat16, caches read from memory): 256 heads, 3000 keys, D128 71.5 / 59.9 (6.6 TB/s); 384, 2000
 // 85.8 / 62.8; 64, 1000, D64 13.0 / 8.6; 8, 8192, D128 18.0 / 13.6; 1, 131072 27.6 / 20.7; 64, 128, D64 5.1 / 5.2.  Error of O against 64
 // bits 2.3e-3 / 1.7e-3 (bfloat16), 2.9e-4 / 2.1e-4 (float16): what is left is the rounding of O.
+#include <type_traits>
+
 #include "fa_common.hpp"
 #include "fa_launch.hpp"
 
@@ -59,8 +61,18 @@ ACCT_DEV float over_lanes(float x, F f) {
   else return x;
 }
 
-// CH: 16-byte chunk slots per row (8, 16, 32 for head dims up to 64, 128, 256)
-template <typename T, int CH>
+// Whether workgroups of different heads or batches read the same lines of an operand: it is expanded over them, or heads lie
+// beside each other in a row and do not end with a line of 128 bytes.  The loads then leave the lines in the caches.  Past the
+// caches / through them (us, bfloat16): one K and V for all 32 heads, 16 batches, 8000 keys, D64 113 / 52 (tile kernel 85); 8
+// batches, 3000, D128 37.7 / 22.8 (34.2); one for all batches, 4 x 64 heads, 8000, D128 86.7 / 59.9 (85.6); [B, S, N, D], 32 heads,
+// 20000, D40 36.3 / 25.2 (47.1); 256, 4000, D80 80.1 / 77.1 (77.0).  Where nothing is shared, through them is slower: 256 heads, 3000,
+// D128 61.0 / 67.6; 512, 8000, D64 164 / 177.
+inline bool lines_are_shared(int extent, int64_t stride, int64_t row_stride, int hd) {
+  return extent > 1 && stride < row_stride && (stride < hd || stride % 64 != 0);
+}
+
+// CH: 16-byte chunk slots per row (8, 16, 32 for head dims up to 64, 128, 256); KEEP: the loads leave their lines in the caches
+template <typename T, int CH, bool KEEP>
 __global__ void __launch_bounds__(64 * kRowWaves) fa_fwd_row_kernel(const FaArgs a, int key_end) {
   using E = Elem<T>;
   using V8 = typename E::V8;
@@ -87,21 +99,25 @@ __global__ void __launch_bounds__(64 * kRowWaves) fa_fwd_row_kernel(const FaArgs
 #pragma unroll
   for (int e = 0; e < 8; e++) o[e] = 0.f;
 
+  auto fetch = [](const void* p) {
+    if constexpr (KEEP) return *reinterpret_cast<const V8*>(p);
+    else return __builtin_nontemporal_load(reinterpret_cast<const V8*>(p));
+  };
   auto load = [&](V8 (&kf)[U], V8 (&vf)[U], int batch) {
     const int row = batch * STEP + wave * (R * U);           // wave-uniform: a row's address is a scalar, the lane's part of it 32 bits
     if ((batch + 1) * STEP <= k_hi) {
 #pragma unroll
       for (int u = 0; u < U; u++)
-        kf[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>((const char*)(kp + (int64_t)(row + R * u) * a.k_ss) + koff));
+        kf[u] = fetch((const char*)(kp + (int64_t)(row + R * u) * a.k_ss) + koff);
 #pragma unroll
       for (int u = 0; u < U; u++)
-        vf[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>((const char*)(vp + (int64_t)(row + R * u) * a.v_ss) + voff));
+        vf[u] = fetch((const char*)(vp + (int64_t)(row + R * u) * a.v_ss) + voff);
     } else {                                                 // rows past the last key repeat it
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const int64_t r = min(row + R * u + lrow, k_hi - 1);
-        kf[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(kp + r * a.k_ss + cc * 8));
-        vf[u] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(vp + r * a.v_ss + cc * 8));
+        kf[u] = fetch(kp + r * a.k_ss + cc * 8);
+        vf[u] = fetch(vp + r * a.v_ss + cc * 8);
       }
     }
   };
@@ -234,7 +250,13 @@ template <typename T>
 hipError_t launch_fwd_row_elem(const FaArgs& a, int key_end, hipStream_t st) {
   const int ch = a.hd <= 64 ? 8 : a.hd <= 128 ? 16 : 32;
   const unsigned heads = (unsigned)(a.B * a.N);
-  auto kern = ch == 8 ? fa_fwd_row_kernel<T, 8> : ch == 16 ? fa_fwd_row_kernel<T, 16> : fa_fwd_row_kernel<T, 32>;
+  const bool keep = lines_are_shared(a.N, a.k_sh, a.k_ss, a.hd) || lines_are_shared(a.B, a.k_sb, a.k_ss, a.hd) ||
+                    lines_are_shared(a.N, a.v_sh, a.v_ss, a.hd) || lines_are_shared(a.B, a.v_sb, a.v_ss, a.hd);
+  auto pick = [&](auto k) {
+    constexpr bool KEEP = decltype(k)::value;
+    return ch == 8 ? fa_fwd_row_kernel<T, 8, KEEP> : ch == 16 ? fa_fwd_row_kernel<T, 16, KEEP> : fa_fwd_row_kernel<T, 32, KEEP>;
+  };
+  auto kern = keep ? pick(std::true_type{}) : pick(std::false_type{});
   hipLaunchKernelGGL(kern, dim3(heads * (a.kv_split > 1 ? a.kv_split : 1)), dim3(64 * kRowWaves), 0, st, a, key_end);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && a.kv_split > 1) {

@@ -56,6 +56,20 @@ def test_one_row_against_64_bits(B, N, Sk, D, parts, dtype):
     _check(*_call(q2, k2, v2)[:2], q2, k2, v2)
 
 
+@pytest.mark.parametrize("Sk, D", [(127, 64), (1000, 40), (3001, 128), (700, 256)])
+def test_one_row_of_shared_keys(Sk, D):
+    """Keys and values that heads or batches share, and heads beside each other in a row: the same bits as from copies."""
+    g = torch.Generator(device=DEV).manual_seed(Sk)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)
+    B, N, q = 3, 4, r(3, 4, 1, D)
+    for k, v in ((r(B, 1, Sk, D).expand(B, N, Sk, D), r(B, 1, Sk, D).expand(B, N, Sk, D)), (r(1, N, Sk, D).expand(B, N, Sk, D), r(B, N, Sk, D)),
+                 (r(B, N, Sk, D), r(1, 1, Sk, D).expand(B, N, Sk, D)), (r(B, Sk, N, D).transpose(1, 2), r(B, Sk, N, D).transpose(1, 2))):
+        o, lse, _ = _call(q, k, v)
+        _check(o, lse, q, k, v)
+        want, want_lse, _ = _call(q, k.contiguous(), v.contiguous())
+        assert torch.equal(o, want) and torch.equal(lse, want_lse)
+
+
 @pytest.mark.parametrize("seen, band", [(128, dict(next_block_num=0)), (384, dict(next_block_num=2)), (256, dict(row_block_prefix=256)), (500, dict(prev_block_num=0))])
 def test_one_row_sees_its_band(seen, band):
     g = torch.Generator(device=DEV).manual_seed(3)
