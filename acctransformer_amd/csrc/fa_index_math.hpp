@@ -38,12 +38,17 @@ ACCT_HD int xcd_span(int id, int n) {
 }
 
 // Workgroup id of a forward launch over `split` key slices -> slice and the id that wg_map takes.  The row tiles of one head
-// and slice read the same keys: they follow each other on one XCD, whose L2 then fetches them once (in the plain order, slice
-// by slice, they sit on different XCDs).  Forward, us: 1 head, 256 queries x 131072 keys, D128 34.5 -> 32.9; 3 heads, 300 x 60000
-// 51.4 -> 45.1; 5 heads, 400 x 30000 55.8 -> 49.3.  (Above 64 heads in wg_map's other order a split launch has one row tile per head.)
-// Below 64 MB of K and V the plain order is as fast or faster: 2 heads, 512 x 16000 25.1 / 27.0 (shared); 8, 512 x 8192 33.7 / 34.3;
-// 8, 256 x 12000 28.4 / 28.9.
-ACCT_HD bool split_shares(int BH, int Sk, int D) { return (long long)BH * Sk * D >= 16000000; }
+// and slice read the same keys.  `share`: they follow each other on one XCD, whose L2 then fetches them once; in the plain order,
+// slice by slice, they sit on different XCDs.  (Above 64 heads in wg_map's other order a split launch has one row tile per head.)
+//
+// In the plain order a head's tiles sit on one XCD anyway where the heads are a multiple of 8: nothing to gain there (1.00 to
+// 1.04 of the plain time).  Otherwise sharing pays once K and V no longer fit the eight L2s (32 MB, less what else passes
+// through).  Time shared / plain, 1 to 7 heads (4 heads, whose tiles sit on two XCDs, gain half), 256 / 512 / 1024 queries; a
+// pass that finds K and V in the caches: 5 million elements of K D64 1.09 / 1.04 / 0.98, D128 1.06 / 1.01 / 0.96; 6: 1.06 / 1.01 / 0.99,
+// 1.03 / 0.95 / 0.95; 7: 1.00 / 0.97 / 0.97, 0.97 / 0.95 / 0.95; 9: 0.98 / 0.97 / 0.96, 0.96 / 0.95 / 0.94; 16: 0.97 / 0.94 / 0.93, 0.95 /
+// 0.92 / 0.92; 32: 0.96 / 0.93 / 0.93, 0.94 / 0.91 / 0.92; from memory 0.91 to 1.04, 0.97 on average.  1 head, 256 x 131072, D128 34.5 / 32.9 us;
+// 2, 500 x 100000, D64 45.9 / 43.2; 5, 400 x 30000, D128 55.8 / 49.3.
+ACCT_HD bool split_shares(int BH, int Sk, int D) { return BH % 8 != 0 && (long long)BH * Sk * D >= 7000000; }
 ACCT_HD void split_map(int id, int BH, int n_tiles, int split, bool share, int& slice, int& wg) {
   const int n_wg = BH * n_tiles;
   if (!share || n_tiles == 1 || (BH > 64 && (BH & 63) == 0)) {

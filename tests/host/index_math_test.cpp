@@ -222,30 +222,38 @@ static void test_visible_row_keys() {
   CHECK(fwd_plan(1, 1, 256, 131072, 128, false, false, true, 256, visible_row_keys(256, 131072, 65536, 200, 0)).kv_split > 8, "a wide band is not cut");
 }
 
-// every (slice, workgroup) once, and the row tiles of a head and slice next to each other on one XCD (but where its share ends)
+// every (slice, workgroup) once; shared: the row tiles of a head and slice next to each other on one XCD (but where its share
+// ends); plain: on one XCD where the heads are a multiple of 8, which is why such launches do not share
 static void test_split_map() {
-  for (int BH : {1, 3, 8, 40, 64, 100, 128})
-    for (int n_tiles : {1, 2, 3, 5})
-      for (int split : {2, 3, 7, 16, 128}) {
-        if (BH == 128 && n_tiles > 1) continue;                                        // (such a launch is not cut)
-        const int n = BH * n_tiles * split;
-        std::vector<int> seen(n, -1);
-        int apart = 0;
-        for (int id = 0; id < n; id++) {
-          int slice = -1, wg = -1;
-          split_map(id, BH, n_tiles, split, true, slice, wg);
-          const bool in = slice >= 0 && slice < split && wg >= 0 && wg < BH * n_tiles;
-          CHECK(in, "BH %d tiles %d split %d id %d: slice %d wg %d", BH, n_tiles, split, id, slice, wg);
-          if (!in) continue;
-          CHECK(seen[slice * BH * n_tiles + wg] < 0, "BH %d tiles %d split %d id %d: twice", BH, n_tiles, split, id);
-          seen[slice * BH * n_tiles + wg] = id;
+  for (bool share : {true, false})
+    for (int BH : {1, 3, 8, 40, 64, 100, 128})
+      for (int n_tiles : {1, 2, 3, 5})
+        for (int split : {2, 3, 7, 16, 128}) {
+          if (BH == 128 && n_tiles > 1) continue;                                        // (such a launch is not cut)
+          const int n = BH * n_tiles * split;
+          std::vector<int> seen(n, -1);
+          int apart = 0, other_xcd = 0;
+          for (int id = 0; id < n; id++) {
+            int slice = -1, wg = -1;
+            split_map(id, BH, n_tiles, split, share, slice, wg);
+            const bool in = slice >= 0 && slice < split && wg >= 0 && wg < BH * n_tiles;
+            CHECK(in, "BH %d tiles %d split %d id %d: slice %d wg %d", BH, n_tiles, split, id, slice, wg);
+            if (!in) continue;
+            CHECK(seen[slice * BH * n_tiles + wg] < 0, "BH %d tiles %d split %d id %d: twice", BH, n_tiles, split, id);
+            seen[slice * BH * n_tiles + wg] = id;
+          }
+          for (int slice = 0; slice < split && n_tiles > 1; slice++)
+            for (int bh = 0; bh < BH; bh++)
+              for (int t = 1; t < n_tiles; t++) {
+                const int id = seen[slice * BH * n_tiles + t * BH + bh], before = seen[slice * BH * n_tiles + (t - 1) * BH + bh];
+                apart += id != before + 8;
+                other_xcd += id % 8 != before % 8;
+              }
+          if (share) CHECK(apart <= 8, "BH %d tiles %d split %d: %d neighbours apart", BH, n_tiles, split, apart);
+          else CHECK((other_xcd == 0) == (BH % 8 == 0 || n_tiles == 1), "BH %d tiles %d split %d: %d on other XCDs", BH, n_tiles, split, other_xcd);
         }
-        for (int slice = 0; slice < split && n_tiles > 1; slice++)
-          for (int bh = 0; bh < BH; bh++)
-            for (int t = 1; t < n_tiles; t++)
-              if (seen[slice * BH * n_tiles + t * BH + bh] != seen[slice * BH * n_tiles + (t - 1) * BH + bh] + 8) apart++;
-        CHECK(apart <= 8, "BH %d tiles %d split %d: %d neighbours apart", BH, n_tiles, split, apart);
-      }
+  CHECK(split_shares(1, 131072, 128) && split_shares(2, 100000, 64) && split_shares(1, 110000, 64) && split_shares(12, 9200, 64), "more than the L2s hold");
+  CHECK(!split_shares(1, 109000, 64) && !split_shares(3, 16000, 128) && !split_shares(8, 131072, 128) && !split_shares(64, 8192, 128), "nothing to gain");
 }
 
 // the mean of what the rows see, against a count
