@@ -11,6 +11,7 @@
 #include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/dynamo/compiled_autograd.h>
 #include <torch/csrc/PyInterpreter.h>
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
@@ -60,6 +61,8 @@ struct Problem {
   acct_fa_params p{};
   Tensor mask, drop, alibi, mask_bits, drop_bits;
 
+  std::array<Tensor*, 5> tensors() { return {&mask, &drop, &alibi, &mask_bits, &drop_bits}; }
+  std::array<const Tensor*, 5> tensors() const { return {&mask, &drop, &alibi, &mask_bits, &drop_bits}; }
   void point(const Tensor& q, const Tensor& k, const Tensor& v) {
     auto at = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
     p.q = q.data_ptr(); p.k = k.data_ptr(); p.v = v.data_ptr();
@@ -73,21 +76,22 @@ Tensor bytes_like(const Tensor& like, size_t n) {
   return n ? at::empty({(int64_t)n}, like.options().dtype(at::kByte)) : Tensor();
 }
 
-// `t`, or a copy of it where elements may share memory (an expanded operand): its gradient has the same layout and needs a
+// Makes `t` a copy of it where elements may share memory (an expanded operand): its gradient has the same layout and needs a
 // place of its own for every element.  A copy also where rows are further apart than the library's backward takes.
 constexpr int64_t kRowStrideEnd = 34087040;
-Tensor apart(Tensor t) {
-  if (t.stride(2) >= kRowStrideEnd) return t.contiguous();
+void take_apart(Tensor& t) {
+  bool apart = t.stride(2) < kRowStrideEnd;
+  if (apart && t.is_non_overlapping_and_dense()) return;
   std::array<std::pair<int64_t, int64_t>, 4> dims;
   for (int i = 0; i < 4; i++) dims[i] = {t.stride(i), t.size(i)};
   std::sort(dims.begin(), dims.end());
   int64_t room = 1;
   for (const auto& [stride, size] : dims) {
     if (size <= 1) continue;
-    if (stride < room) return t.contiguous();
+    apart = apart && stride >= room;
     room += stride * (size - 1);
   }
-  return t;
+  if (!apart) t = t.contiguous();
 }
 
 struct FlashAttentionBackward : public torch::autograd::Node {
@@ -114,22 +118,64 @@ struct FlashAttentionBackward : public torch::autograd::Node {
   }
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
-    Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack();
-    Tensor o = o_.unpack(shared_from_this());
-    const Tensor lse = lse_.unpack();
+    return backward(problem, q_.unpack(), k_.unpack(), v_.unpack(), o_.unpack(shared_from_this()), lse_.unpack(), grads[0]);
+  }
+  // Compiled autograd records the backward as a call of `compiled`, with the tensors and (as one more of them) the parameters
+  // as its arguments.
+  void compiled_args(torch::dynamo::autograd::CompiledNodeArgs& args) const override {
+    for (const auto* s : {&q_, &k_, &v_, &lse_}) args.collect(*s, false);
+    args.collect(o_, true);
+    params_ = at::empty({(int64_t)sizeof(acct_fa_params)}, at::kByte);
+    std::memcpy(params_.data_ptr(), &problem.p, sizeof(acct_fa_params));
+    args.collect(params_);
+    for (const Tensor* t : problem.tensors()) args.collect(*t);
+  }
+  torch::autograd::variable_list apply_with_saved(const torch::autograd::variable_list& grads,
+                                                  torch::dynamo::autograd::SwapSavedVariables& saved) override {
+    using namespace torch::dynamo::autograd;
+    for (auto* s : {&q_, &k_, &v_, &lse_, &o_}) saved.before(*s);
+    saved.before(params_);
+    for (Tensor* t : problem.tensors()) saved.before(*t);
+    PackedArgs args;
+    for (const Tensor& t : {q_.unpack(), k_.unpack(), v_.unpack(), o_.unpack(shared_from_this()), lse_.unpack(), params_}) args.pack(t);
+    for (Tensor* t : problem.tensors()) args.pack(t->defined() ? *t : params_);      // (absent: null in the parameters, and not looked at)
+    const auto& compiler = getPyCompilerInterface();
+    const std::string fn = compiler->bind_function(saved.get_py_compiler(), name(), compiled,
+                                                   std::vector<at::TypePtr>(11, at::TensorType::get()), true, false);
+    auto metadata = IValuePacker<std::vector<std::optional<torch::autograd::InputMetadata>>>::pack(get_input_metadata(next_edges()));
+    auto out = compiler->call_function(saved.get_py_compiler(), "apply_functional", fn, grads, args.vec(), metadata);
+    for (auto* s : {&q_, &k_, &v_, &lse_, &o_}) saved.after(*s);
+    saved.after(params_);
+    for (Tensor* t : problem.tensors()) saved.after(*t);
+    return out;
+  }
+
+ private:
+  mutable Tensor params_;
+
+  static torch::autograd::variable_list compiled(const torch::autograd::variable_list& grads, const std::vector<c10::IValue>& a) {
+    Problem c;
+    const Tensor params = a[5].toTensor();
+    std::memcpy(&c.p, params.data_ptr(), sizeof(c.p));
+    const void* there[] = {c.p.attn_mask, c.p.drop_mask, c.p.alibi, c.p.mask_bits, c.p.drop_bits};
+    auto side = c.tensors();
+    for (int i = 0; i < 5; i++)
+      if (there[i]) *side[i] = a[6 + i].toTensor();
+    return backward(c, a[0].toTensor(), a[1].toTensor(), a[2].toTensor(), a[3].toTensor(), a[4].toTensor(), grads[0]);
+  }
+
+  static torch::autograd::variable_list backward(Problem c, Tensor q, Tensor k, Tensor v, Tensor o, const Tensor& lse, Tensor dout) {
     c10::DeviceGuard device(q.device());
     at::AutoDispatchBelowADInplaceOrView below;
-    q = apart(q); k = apart(k); v = apart(v);
+    take_apart(q); take_apart(k); take_apart(v);
     if (o.stride(2) >= kRowStrideEnd) o = o.contiguous();
-    Tensor dout = grads[0];
     if (!dout.defined()) dout = at::zeros_like(o);
     if (dout.strides() != o.strides()) {       // the kernels read dO with O's strides
       Tensor t = at::empty_strided(o.sizes(), o.strides(), o.options());
       t.copy_(dout);
       dout = t;
     }
-    Problem c = problem;                       // (a backward may run twice, and on other copies of the saved tensors)
-    c.point(q, k, v);
+    c.point(q, k, v);                          // (a backward may run twice, and on other copies of the saved tensors)
     take_strides(o, c.p.o_stride);
     Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = at::empty_strided(k.sizes(), k.strides(), k.options()),
            dv = at::empty_strided(v.sizes(), v.strides(), v.options());
@@ -155,10 +201,9 @@ FlashAttentionBackward* node_of(PyObject* self) {
 PyObject* get_params(PyObject* self, void*) {
   HANDLE_TH_ERRORS
   const auto [c, entry] = node_of(self)->record();
-  const Tensor* kept[] = {&c.mask, &c.drop, &c.alibi, &c.mask_bits, &c.drop_bits};
   THPObjectPtr tensors(PyList_New(0));
   if (!tensors) return nullptr;
-  for (const Tensor* t : kept)
+  for (const Tensor* t : c.tensors())
     if (t->defined()) {
       THPObjectPtr w(THPVariable_Wrap(*t));
       if (!w || PyList_Append(tensors.get(), w.get())) return nullptr;

@@ -179,6 +179,30 @@ def test_a_backward_gives_back_the_keep_bits():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("backend", ["eager", "aot_eager"])
+@pytest.mark.parametrize("form", ["plain", "bsnd", "mask u8", "seed", "bias", "one gradient"])
+def test_compiled_autograd(form, backend):
+    """The backward as a call in a compiled graph, twice (the second time with other tensors, and another dropout seed)."""
+    from torch._dynamo import compiled_autograd
+    q, k, v, do, mask, drop, alibi = _inputs(form)
+    op = get_flash_attention(scale=0.125, keep_prob=0.9)
+    wanted = [t for t in (q, k, v) if t.requires_grad]
+    torch._dynamo.reset()
+    for step in range(2):
+        if drop is not None:
+            drop = (drop[0], drop[1] + step)
+        with torch.no_grad():
+            q.mul_(1 + step)
+        want = torch.autograd.grad(op(q * 1, k, v, mask, drop, alibi)[0], wanted, do)
+        o, _ = op(q * 1, k, v, mask, drop, alibi)
+        for t in wanted:
+            t.grad = None
+        with compiled_autograd._enable(torch.compile(backend=backend)):
+            o.backward(do)
+        assert all(torch.equal(a, t.grad) for a, t in zip(want, wanted))
+
+
+@pytest.mark.gpu
 def test_native_call_on_another_stream_and_in_the_inference_operator():
     q, k, v, do, *_ = _inputs("plain")
     op = get_flash_attention(scale=1.0)
