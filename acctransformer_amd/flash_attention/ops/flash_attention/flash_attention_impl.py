@@ -30,6 +30,7 @@ Differences from the reference that a caller can see:
 """
 from __future__ import annotations
 
+import sys
 import weakref
 
 import torch
@@ -275,6 +276,21 @@ def _native_call(kind_of_call, q, k, v, attn_mask, dropout_mask, alibi_mask, pre
     return out
 
 
+_untraced_bwd = None
+
+
+def _untraced_backward():
+    """`_capi.fa_bwd` as compiled autograd calls and does not trace it: of a trace through its ctypes calls, the gradients held
+    nothing.  (Asked for in the forward: the backward may be traced itself.)"""
+    global _untraced_bwd
+    dynamo = sys.modules.get("torch._dynamo")
+    if dynamo is None or not hasattr(dynamo, "disable"):
+        return _capi.fa_bwd
+    if _untraced_bwd is None:
+        _untraced_bwd = dynamo.disable(_capi.fa_bwd)
+    return _untraced_bwd
+
+
 class _FlashAttentionFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, attn_mask, dropout_mask, alibi_mask, prev_block_num, next_block_num, scale, keep_prob,
@@ -293,6 +309,7 @@ class _FlashAttentionFn(torch.autograd.Function):
             p.drop_bits_filled = 1
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.params = p
+        ctx.fa_bwd = _untraced_backward()
         ctx.mark_non_differentiable(lse)
         ctx.set_materialize_grads(False)              # (no tensor of zeros for lse, which has no gradient)
         return o, lse
@@ -302,7 +319,7 @@ class _FlashAttentionFn(torch.autograd.Function):
         q, k, v, o, lse = ctx.saved_tensors
         if do is None:
             do = torch.zeros_like(o)
-        dq, dk, dv = _capi.fa_bwd(ctx.params, q, k, v, o, do, lse)
+        dq, dk, dv = ctx.fa_bwd(ctx.params, q, k, v, o, do, lse)
         return dq, dk, dv, None, None, None, None, None, None, None, None
 
 

@@ -179,11 +179,14 @@ def test_a_backward_gives_back_the_keep_bits():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
 @pytest.mark.parametrize("backend", ["eager", "aot_eager"])
 @pytest.mark.parametrize("form", ["plain", "bsnd", "mask u8", "seed", "bias", "one gradient"])
-def test_compiled_autograd(form, backend):
+def test_compiled_autograd(form, backend, native, monkeypatch):
     """The backward as a call in a compiled graph, twice (the second time with other tensors, and another dropout seed)."""
     from torch._dynamo import compiled_autograd
+    if not native:
+        monkeypatch.setattr(impl, "_native_call", lambda *a: None)
     q, k, v, do, mask, drop, alibi = _inputs(form)
     op = get_flash_attention(scale=0.125, keep_prob=0.9)
     wanted = [t for t in (q, k, v) if t.requires_grad]
@@ -200,6 +203,17 @@ def test_compiled_autograd(form, backend):
         with compiled_autograd._enable(torch.compile(backend=backend)):
             o.backward(do)
         assert all(torch.equal(a, t.grad) for a, t in zip(want, wanted))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("backend", ["eager", "aot_eager"])
+def test_compiled_forward(backend):
+    q, k, v, do, mask, _, alibi = _inputs("bias")
+    op = get_flash_attention(scale=0.125)
+    torch._dynamo.reset()
+    want, got = ((o, *torch.autograd.grad(o, (q, k, v), do)) for o in (op(q * 1, k, v, mask, None, alibi)[0],
+                                                                       torch.compile(lambda: op(q * 1, k, v, mask, None, alibi)[0], backend=backend)()))
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
 
 
 @pytest.mark.gpu
