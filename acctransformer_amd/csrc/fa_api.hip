@@ -267,8 +267,6 @@ size_t dropcol_bytes(const acct_fa_params* p) {
 
 // key blocks after the query's block are left out, row by row (a row prefix of a few large blocks leaves out less, and in
 // steps: 4 row blocks, 16 heads, S3584, D64 59.8 us with 224 forward workgroups, 61.0 with 448)
-// (not a band that leaves out the blocks far before the query's too: its workgroups are equally long.  32 heads, S2048, D128,
-// 8 blocks back: backward 130.7 us as equal workgroups, 143.6 as a triangle)
 bool ends_at_query(const acct_fa_params* p) {
   return (p->mask_kind == ACCT_MASK_CAUSAL || p->next_block_num == 0) && 8 * (int64_t)p->row_block_prefix <= p->Sq;
 }

@@ -151,6 +151,7 @@ struct FaArgs {
   int dkdv_ngk;                        // dK/dV kernel: 32-key groups per wave (DkdvPlan, fa_index_math.hpp)
   int drop_visible;                    // keep bits: != 0 when those of key blocks outside the band (or past the causal / prefix limit) may be left out
   int sk_plan;                         // forward kernel: keys up to which whole tiles are staged by plan: Sk, or 0 where rows are too far apart for that
+  int kv_share;                        // forward kernel, key slices: their order (split_shares, fa_index_math.hpp)
 };
 static_assert(offsetof(FaArgs, fwd_part) > offsetof(FaArgs, philox_thr), "new fields stand behind those of the inner loops");
 

@@ -55,7 +55,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   const int rg = KG > 1 ? wave % RG : wave, kg = KG > 1 ? wave / RG : 0;
   const int BH = a.B * a.N, n_wg = BH * a.n_tiles;
   int wg = blockIdx.x, slice = 0;                           // kv_split > 1: the grid holds every query tile once per key slice
-  if (a.kv_split > 1) split_map(blockIdx.x, BH, a.n_tiles, a.kv_split, split_shares(BH, a.Sk, a.hd), slice, wg);
+  if (a.kv_split > 1) split_map(blockIdx.x, BH, a.n_tiles, a.kv_split, a.kv_share, slice, wg);
   int bh, rank;
   wg_map(wg, BH, a.n_tiles, bh, rank);
   const int qt = a.n_tiles - 1 - rank;                      // heaviest (latest) causal tiles first
@@ -771,7 +771,7 @@ __global__ void __launch_bounds__(64 * NW) fa_fwd_kernel(const FaArgs a) {
       constexpr int BM = 32 * QG * NW / KG;
       const int BH = a.B * a.N;
       int wg = blockIdx.x, slice;
-      if (a.kv_split > 1) split_map(blockIdx.x, BH, a.n_tiles, a.kv_split, split_shares(BH, a.Sk, a.hd), slice, wg);
+      if (a.kv_split > 1) split_map(blockIdx.x, BH, a.n_tiles, a.kv_split, a.kv_share, slice, wg);
       int bh, rank;
       wg_map(wg, BH, a.n_tiles, bh, rank);
       const int q0 = (a.n_tiles - 1 - rank) * BM, q_end = min(q0 + BM, a.Sq);
@@ -883,6 +883,7 @@ static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   constexpr int QG = 1, RG = NW / KG, BM = 32 * QG * RG;
   a.n_tiles = (a.Sq + BM - 1) / BM;
   a.sk_plan = tile_offsets_fit(a.k_ss, 32 * KT) && tile_offsets_fit(a.v_ss, 32 * KT) ? a.Sk : 0;
+  a.kv_share = split_shares(a.B * a.N, a.Sk, a.hd);
   const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
   constexpr size_t biasb = BIAS ? (KT == 4 ? 1024 : QG * 4096) : 0;     // per wave, as in the kernel
   constexpr size_t tiles = 4 * 32 * KT * (size_t)C::PITCH + NW * biasb + (size_t)NW * 2 * DropRowStage<DROP, QG, KT>::BYTES,
