@@ -152,6 +152,7 @@ struct FaArgs {
   int drop_visible;                    // keep bits: != 0 when those of key blocks outside the band (or past the causal / prefix limit) may be left out
   int sk_plan;                         // forward kernel: keys up to which whole tiles are staged by plan: Sk, or 0 where rows are too far apart for that
   int kv_share;                        // forward kernel, key slices: their order (split_shares, fa_index_math.hpp)
+  int merge_alone;                     // forward kernel, two key groups: the first one merges and stores alone
 };
 static_assert(offsetof(FaArgs, fwd_part) > offsetof(FaArgs, philox_thr), "new fields stand behind those of the inner loops");
 
@@ -420,6 +421,7 @@ ACCT_DEV void load_bias4(const T* row, int kv, int limit, bool vec_ok, float out
 // probability of 0, which would turn an infinity in the last row into NaN).  Slots past the `cpr` valid 16-byte
 // chunks of a row (head dim / 8) repeat the last valid chunk.
 // `wv` < 0: the NW waves are the workgroup's first NW; else the calling wave's index among the NW.
+static __device__ const u32x4 g_zero_chunk = {0, 0, 0, 0};        // (a select of addresses: stores of zeros to LDS instead cost 1 to 4 % of a short call)
 template <typename T, int D, int ROWS, int NW, bool ZERO = false>
 ACCT_DEV void tile_dma(const T* base, int64_t row_stride, int row0, int nrows, ACCT_LDS char* buf, int cpr, int wv = -1) {
   using C = SwzCfg<D>;
@@ -434,13 +436,8 @@ ACCT_DEV void tile_dma(const T* base, int64_t row_stride, int row0, int nrows, A
     const int r = inst * C::RPI + lane / C::CH;
     const int lc = min((lane % C::CH) ^ C::swz(r), cpr - 1);
     const int grow = min(row0 + r, nrows - 1);
-    if (ZERO && row0 + r >= nrows) {
-      uint32_t z = 0;
-      asm volatile("" : "+v"(z));                 // (made here: four registers of zeros would live through the caller's loop)
-      *reinterpret_cast<ACCT_LDS u32x4*>(buf + inst * 1024 + lane * 16) = u32x4{z, z, z, z};
-      continue;
-    }
     const T* src = base + (int64_t)grow * row_stride + lc * 8;
+    if (ZERO && row0 + r >= nrows) src = (const T*)&g_zero_chunk;
     // Issued as inline assembly on purpose: the compiler then does not order every later LDS read
     // behind these loads (it cannot tell the two tile buffers apart), which would serialise the
     // prefetch of the next tile with the work on the current one.  dma_wait() + the workgroup

@@ -29,6 +29,9 @@ namespace acct {
 template <int D, int KG> constexpr int fwd_merge_pieces() { return 4 * SwzCfg<D>::DB / KG; }
 template <int D, int NW, int KG> constexpr int fwd_merge_stats() { return NW * (KG - 1) * fwd_merge_pieces<D, KG>() * 1024; }
 
+// Two key groups at head dims up to 64, launches of more than one round: the first group merges alone (see there).
+template <int D, int KG> constexpr bool fwd_merge_alone() { return KG == 2 && D <= 64; }
+
 // KG > 1 (small grids): the waves of a workgroup form NW / KG row groups times KG key groups.  A wave then works on
 // its key group's share of every tile only, with softmax statistics of its own, and the key groups of a row group
 // are merged through LDS before the epilogue -- KG times as many workgroups for the same rows, every wave busy.
@@ -612,8 +615,37 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
 
   // ---- key groups: each finishes its share of the columns from the sums of all.  (One group merging and storing all of
   // them while the others idled: 3900 cycles from the last tile on, of a workgroup that walked four tiles in 8000, D64, kg 4;
-  // shared 2400.) ----
-  if constexpr (KG > 1) {
+  // shared 2400.)  Not in a launch of several rounds at head dims up to 64: there the others are better gone, as three waves
+  // fit a SIMD and the next workgroup starts beside the first group's merge.  Forward, shared / alone (us): 1024 heads,
+  // 300 x 77, key padding, D40 71.6 / 65.2, D64 73.7 / 66.9; dropout 58.9 / 53.2, 66.9 / 59.2; 384 heads, 300 x 300 padded 35.6 / 32.9,
+  // 39.7 / 36.9; 24 heads, 3000 x 500 28.9 / 27.8, 29.1 / 27.5; without side inputs level.  The sums and their order are the same. ----
+  bool merged = false;
+  if constexpr (fwd_merge_alone<D, KG>()) if (a.merge_alone) {
+    merged = true;
+    ACCT_LDS char* slot = smem + RG * 32 * (C::DB * 64 + 16) + rg * (C::DB * 4096 + 512) + lane * 16;
+    ACCT_LDS char* stat = slot + C::DB * 4096 - lane * 8;
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < 4 * C::DB; i++) {
+        const f32x4 v = {o[0][i / 4][4 * (i % 4)], o[0][i / 4][4 * (i % 4) + 1], o[0][i / 4][4 * (i % 4) + 2], o[0][i / 4][4 * (i % 4) + 3]};
+        *reinterpret_cast<ACCT_LDS f32x4*>(slot + i * 1024) = v;
+      }
+      *reinterpret_cast<ACCT_LDS f32x2*>(stat) = f32x2{m[0], lsum[0]};
+    }
+    __syncthreads();
+    if (kg > 0) return;
+    const f32x2 ml = *reinterpret_cast<const ACCT_LDS f32x2*>(stat);
+    const float mm = fmaxf(m[0], ml[0]), w0 = fast_exp2((m[0] - mm) * cmul), w1 = fast_exp2((ml[0] - mm) * cmul);
+    m[0] = mm;
+    lsum[0] = __builtin_fmaf(ml[1], w1, lsum[0] * w0);
+#pragma unroll
+    for (int i = 0; i < 4 * C::DB; i++) {
+      const f32x4 v = *reinterpret_cast<const ACCT_LDS f32x4*>(slot + i * 1024);
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[0][i / 4][4 * (i % 4) + e] = __builtin_fmaf(v[e], w1, o[0][i / 4][4 * (i % 4) + e] * w0);
+    }
+  }
+  if constexpr (KG > 1) if (!merged) {
     constexpr int PC = fwd_merge_pieces<D, KG>();
     static_assert(PC * KG == 4 * C::DB, "every key group finishes the same number of pieces");
     // pieces of key group `own` that key group `from` holds
@@ -884,10 +916,12 @@ static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   a.n_tiles = (a.Sq + BM - 1) / BM;
   a.sk_plan = tile_offsets_fit(a.k_ss, 32 * KT) && tile_offsets_fit(a.v_ss, 32 * KT) ? a.Sk : 0;
   a.kv_share = split_shares(a.B * a.N, a.Sk, a.hd);
+  a.merge_alone = fwd_merge_alone<D, KG>() && a.kv_split <= 1 && (long long)a.n_tiles * a.B * a.N > 256;
   const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
   constexpr size_t biasb = BIAS ? (KT == 4 ? 1024 : QG * 4096) : 0;     // per wave, as in the kernel
   constexpr size_t tiles = 4 * 32 * KT * (size_t)C::PITCH + NW * biasb + (size_t)NW * 2 * DropRowStage<DROP, QG, KT>::BYTES,
                    stage = KG > 1 ? fwd_merge_stats<D, NW, KG>() + (size_t)NW * 512 : (size_t)NW * 32 * (C::DB * 64 + 16);
+  static_assert(!fwd_merge_alone<D, KG>() || (size_t)RG * (32 * (C::DB * 64 + 16) + C::DB * 4096 + 512) <= tiles, "the tiles' LDS holds the lone merge");
   constexpr size_t smem = tiles > stage ? tiles : stage;
   static_assert(smem <= 160 * 1024, "the workgroup's LDS must fit the CU's 160 KB");
   auto kern = mask_t ? fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, true, KT, KG, PIPE> : fa_fwd_kernel<T, D, QG, NW, BIAS, DROP, BIAS || DROP, KT, KG, PIPE>;
