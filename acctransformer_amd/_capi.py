@@ -346,7 +346,8 @@ def fa_fwd(p, q):
     return o, lse
 
 
-_ROW_STRIDE_END = 34087040           # (of a backward, in elements)
+# Row strides (in elements) from which the library may refuse an operand of 64 rows and more.
+FWD_ROW_STRIDE_END, _ROW_STRIDE_END = 16909320, 34087040             # (of a forward, of a backward)
 
 
 def _apart(t):

@@ -409,6 +409,8 @@ int acct_fa_fwd(const acct_fa_params* p, void* O, float* LSE, void* workspace, s
   a.kv_split = plan.kv_split;
   if (plan.kv_split > 1) a.fwd_part = (float*)((char*)workspace + part_at);
   hipError_t e = p->dtype == ACCT_F16 ? acct::launch_fwd_elem<acct::f16>(a, p->D, plan.kg, st) : acct::launch_fwd_elem<acct::bf16>(a, p->D, plan.kg, st);
+  if (e == hipErrorInvalidPitchValue)
+    return fail(ACCT_E_SHAPE, "rows of k or v are too far apart: %lld and %lld elements", (long long)a.k_ss, (long long)a.v_ss);
   if (e != hipSuccess) return fail(ACCT_E_LAUNCH, "forward kernel: %s", hipGetErrorString(e));
   return ACCT_OK;
 }

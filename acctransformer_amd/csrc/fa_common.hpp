@@ -150,7 +150,6 @@ struct FaArgs {
   int dq_kg;                           // dQ kernel: key groups of the workgroup (dq_key_groups, fa_index_math.hpp)
   int dkdv_ngk;                        // dK/dV kernel: 32-key groups per wave (DkdvPlan, fa_index_math.hpp)
   int drop_visible;                    // keep bits: != 0 when those of key blocks outside the band (or past the causal / prefix limit) may be left out
-  int sk_plan;                         // forward kernel: keys up to which whole tiles are staged by plan: Sk, or 0 where rows are too far apart for that
   int kv_share;                        // forward kernel, key slices: their order (split_shares, fa_index_math.hpp)
   int merge_alone;                     // forward kernel, two key groups: the first one merges and stores alone
 };

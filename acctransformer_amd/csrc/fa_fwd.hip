@@ -117,11 +117,11 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   vdma.plan(a.v_ss, cpr);
   // stage key rows [j BN, (j+1) BN) into an LDS tile (whole tiles by plan)
   auto stage_k = [&](int j, ACCT_LDS char* dst) {
-    if ((j + 1) * BN <= a.sk_plan) kdma.issue(kp, a.k_ss, j * BN, dst);
+    if ((j + 1) * BN <= a.Sk) kdma.issue(kp, a.k_ss, j * BN, dst);
     else tile_dma<T, D, BN, NW>(kp, a.k_ss, j * BN, a.Sk, dst, cpr);         // ragged last tile: clamped rows
   };
   auto stage_v = [&](int j, ACCT_LDS char* dst) {
-    if ((j + 1) * BN <= a.sk_plan) vdma.issue(vp, a.v_ss, j * BN, dst);
+    if ((j + 1) * BN <= a.Sk) vdma.issue(vp, a.v_ss, j * BN, dst);
     else tile_dma<T, D, BN, NW, true>(vp, a.v_ss, j * BN, a.Sk, dst, cpr);   // and zeros
   };
   if (j_lo <= j_hi) {
@@ -465,11 +465,11 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     const int64_t kstep = BN * a.k_ss, vstep = BN * a.v_ss;
     auto fill = [&](int j) {
       if (j + 2 <= j_hi) {
-        if ((j + 3) * BN <= a.sk_plan) kdma.issue(kfill, a.k_ss, 0, smem + par);
+        if ((j + 3) * BN <= a.Sk) kdma.issue(kfill, a.k_ss, 0, smem + par);
         else tile_dma<T, D, BN, NW>(kp, a.k_ss, (j + 2) * BN, a.Sk, smem + par, cpr);     // ragged last tile: clamped rows
       }
       if (j > j_lo && j <= j_hi) {                           // (that of the first tile is under way)
-        if ((j + 1) * BN <= a.sk_plan) vdma.issue(vfill, a.v_ss, 0, smem + par + TILEB);
+        if ((j + 1) * BN <= a.Sk) vdma.issue(vfill, a.v_ss, 0, smem + par + TILEB);
         else tile_dma<T, D, BN, NW, true>(vp, a.v_ss, j * BN, a.Sk, smem + par + TILEB, cpr);
       }
       kfill += kstep;
@@ -914,7 +914,7 @@ static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   using C = SwzCfg<D>;
   constexpr int QG = 1, RG = NW / KG, BM = 32 * QG * RG;
   a.n_tiles = (a.Sq + BM - 1) / BM;
-  a.sk_plan = tile_offsets_fit(a.k_ss, 32 * KT) && tile_offsets_fit(a.v_ss, 32 * KT) ? a.Sk : 0;
+  if (a.Sk >= 32 * KT && !(tile_offsets_fit(a.k_ss, 32 * KT) && tile_offsets_fit(a.v_ss, 32 * KT))) return hipErrorInvalidPitchValue;
   a.kv_share = split_shares(a.B * a.N, a.Sk, a.hd);
   a.merge_alone = fwd_merge_alone<D, KG>() && a.kv_split <= 1 && (long long)a.n_tiles * a.B * a.N > 256;
   const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
@@ -951,7 +951,9 @@ static hipError_t launch_fwd_t(const FaArgs& a, hipStream_t st) {
   int seen = visible_row_keys(a.Sq, a.Sk, a.prev_blk, a.next_blk, a.row_prefix);
   if constexpr (KG == 4 && D <= 64) {
     if (a.mask_kind == kMaskCausal && a.Sq < seen) seen = a.Sq;
-    if (long_tiles_pay(a.B * a.N, a.Sq, a.Sk, a.hd, seen, a.prev_blk < (a.Sq - 1) / 128)) return launch_fwd_kt<T, D, NW, BIAS, DROP, 8, KG>(a, st);
+    if (tile_offsets_fit(a.k_ss, 256) && tile_offsets_fit(a.v_ss, 256) &&
+        long_tiles_pay(a.B * a.N, a.Sq, a.Sk, a.hd, seen, a.prev_blk < (a.Sq - 1) / 128))
+      return launch_fwd_kt<T, D, NW, BIAS, DROP, 8, KG>(a, st);
   }
   // (with a mask tensor the loop runs where a workgroup sees the causal pattern in it)
   if constexpr (BIG && KG == 1 && D <= 64 && !BIAS && !DROP) {

@@ -62,7 +62,7 @@ ACCT_HD void split_map(int id, int BH, int n_tiles, int split, bool share, int& 
 }
 
 // A tile of `rows` rows of 2-byte elements is addressed by a base and 32-bit byte offsets: whether the last row's fit (a row
-// has up to 256 elements).
+// has up to 256 elements).  Launchers refuse what does not: a test in the kernels cost the triangle layer's forward 0.6 %.
 ACCT_HD bool tile_offsets_fit(int64_t row_stride, int rows) { return row_stride * (rows - 1) <= 0x7fffffffll - 256; }
 // Row strides of a backward end here (its tiles have 64 rows; in whole chunks of 8 elements).
 constexpr int64_t kBwdRowStrideEnd = 34087040;

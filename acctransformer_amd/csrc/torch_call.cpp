@@ -78,7 +78,7 @@ Tensor bytes_like(const Tensor& like, size_t n) {
 
 // Makes `t` a copy of it where elements may share memory (an expanded operand): its gradient has the same layout and needs a
 // place of its own for every element.  A copy also where rows are further apart than the library's backward takes.
-constexpr int64_t kRowStrideEnd = 34087040;
+constexpr int64_t kRowStrideEnd = 34087040, kFwdRowStrideEnd = 16909320;
 void take_apart(Tensor& t) {
   bool apart = t.stride(2) < kRowStrideEnd;
   if (apart && t.is_non_overlapping_and_dense()) return;
@@ -351,7 +351,7 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     {
       c10::DeviceGuard device(q.device());
       at::AutoDispatchBelowADInplaceOrView below;
-      auto rows = [](Tensor& t) { if (t.stride(3) != 1) t = t.contiguous(); };
+      auto rows = [](Tensor& t) { if (t.stride(3) != 1 || (t.stride(2) >= kFwdRowStrideEnd && t.size(2) >= 64)) t = t.contiguous(); };
       rows(q); rows(k); rows(v);
       known = describe(c, q, k, v) && (q.stride(3) == 1 || q.size(3) == 1);
       if (known) {

@@ -210,7 +210,8 @@ def _build_params(q, k, v, attn_mask, dropout_mask, alibi_mask, prev_block_num, 
 
 
 def _rows_contiguous(t):
-    return t if t.stride(-1) == 1 else t.contiguous()
+    """`t`, or a copy of it where a row is not contiguous or rows are further apart than the library takes."""
+    return t if t.stride(-1) == 1 and (t.dim() < 2 or t.stride(-2) < _capi.FWD_ROW_STRIDE_END or t.shape[-2] < 64) else t.contiguous()
 
 
 _UNRECORDED, _RECORDED, _UNUSUAL = 0, 1, 2
@@ -253,7 +254,7 @@ def _native_call(kind_of_call, q, k, v, attn_mask, dropout_mask, alibi_mask, pre
         _, entry = _mask_bits_hit(mask, kind, q.shape[0], Sq, Sk, min(prev_block_num, _capi.BLOCK_UNBOUNDED),
                                   min(next_block_num, _capi.BLOCK_UNBOUNDED), row_block_prefix, q.device)
         if entry is None:
-            if not (q.stride(3) == 1 and k.stride(3) == 1 and v.stride(3) == 1):
+            if not all(_rows_contiguous(t) is t for t in (q, k, v)):
                 return None
             p = _capi.make_params(q, k, v, scale=scale, prev_block_num=prev_block_num, next_block_num=next_block_num, mask_kind=kind,
                                   attn_mask=mask, row_block_prefix=row_block_prefix)

@@ -21,7 +21,7 @@ from __future__ import annotations
 import torch
 
 from acctransformer_amd import _capi
-from acctransformer_amd.flash_attention.ops.flash_attention.flash_attention_impl import _UNUSUAL, _call_kind
+from acctransformer_amd.flash_attention.ops.flash_attention.flash_attention_impl import _UNUSUAL, _call_kind, _rows_contiguous
 
 __all__ = ["flash_attention_tik"]
 
@@ -33,7 +33,7 @@ def flash_attention_tik(q, k, v, y=None, kernel_name="flash_attention_tik"):
     if q.dtype != torch.float16 or k.dtype != q.dtype or v.dtype != q.dtype:
         raise TypeError("q, k and v must be float16")  # op_info_cfg/ai_core/ascend310p: float16 only
     q4, k4, v4 = (t.unsqueeze(0) if t.dim() == 3 else t for t in (q, k, v))
-    q4, k4, v4 = (t if t.stride(-1) == 1 else t.contiguous() for t in (q4, k4, v4))
+    q4, k4, v4 = (_rows_contiguous(t) for t in (q4, k4, v4))
     out = None
     if q4.is_cuda and _call_kind(q4, k4, v4) != _UNUSUAL:
         out = _capi.native().forward(False, q4, k4, v4, _capi.MASK_NONE, None, None, False, None, None, 0, 0, False, None,

@@ -159,7 +159,10 @@ typedef struct acct_fa_params {
  * (outputs `output` and `rowsum`, T/flash_attention_impl.py:129-154).
  * O is [B,N,Sq,D] in p->dtype with p->o_stride; LSE is fp32 [B,N,Sq] contiguous
  * (L = m + ln l, T/flash_attention_fwd.py:302-306).  `workspace` must hold
- * acct_fa_fwd_workspace_bytes(p) bytes (0 unless mask_kind == DENSE_U8 or dropout is on). */
+ * acct_fa_fwd_workspace_bytes(p) bytes (0 unless mask_kind == DENSE_U8 or dropout is on).
+ * Rows of k and v must be less than 16909320 elements apart (34087040 at head
+ * dims above 128 and with a bias; ACCT_E_SHAPE), unless there is one query row
+ * or there are fewer of them than a tile has. */
 int acct_fa_fwd(const acct_fa_params* p, void* O, float* LSE,
                 void* workspace, size_t workspace_bytes, void* stream);
 size_t acct_fa_fwd_workspace_bytes(const acct_fa_params* p);

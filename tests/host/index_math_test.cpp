@@ -296,6 +296,7 @@ static void test_tile_offsets() {
       CHECK(tile_offsets_fit(stride, rows) == (most <= 0xffffffffll), "%d rows, stride %lld", rows, (long long)stride);
     }
   CHECK(tile_offsets_fit(kBwdRowStrideEnd - 8, 64) && !tile_offsets_fit(kBwdRowStrideEnd, 64), "where the backward's strides end");
+  CHECK(tile_offsets_fit(16909312, 128) && !tile_offsets_fit(16909320, 128), "where the forward's strides end");
   CHECK(!tile_offsets_fit(int64_t(9) << 20, 256) && tile_offsets_fit(int64_t(9) << 20, 128), "256-key tiles reach half as far");
 }
 
