@@ -152,6 +152,7 @@ struct FaArgs {
   int drop_visible;                    // keep bits: != 0 when those of key blocks outside the band (or past the causal / prefix limit) may be left out
   int kv_share;                        // forward kernel, key slices: their order (split_shares, fa_index_math.hpp)
   int merge_alone;                     // forward kernel, two key groups: the first one merges and stores alone
+  int first_late;                      // forward kernel: the first tile is requested behind the Q fragments (first_tile_late, fa_index_math.hpp)
 };
 static_assert(offsetof(FaArgs, fwd_part) > offsetof(FaArgs, philox_thr), "new fields stand behind those of the inner loops");
 

@@ -110,7 +110,7 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
   }
   const int wkv_limit = a.row_prefix ? (wq0 / a.row_prefix + 1) * a.row_prefix : 0x7fffffff;   // keys past it are absent
 
-  // ---- the first tile is requested ahead of everything that can be done meanwhile ----
+  // ---- the first tile is requested ahead of everything that can be done meanwhile (but see first_tile_late) ----
   TileDma<T, D, BN, NW> kdma, vdma;
   const int cpr = a.hd >> 3;                                // valid 16-byte chunks per row
   kdma.plan(a.k_ss, cpr);
@@ -125,7 +125,8 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
     if (__builtin_expect((j + 1) * BN <= a.Sk, 1)) vdma.issue(vp, a.v_ss, j * BN, dst);
     else tile_dma<T, D, BN, NW, true>(vp, a.v_ss, j * BN, a.Sk, dst, cpr);   // and zeros
   };
-  if (j_lo <= j_hi) {
+  const bool late = KG <= 2 && !PIPE && D >= 64 && D <= 128 && a.first_late;
+  if (j_lo <= j_hi && !late) {
     stage_k(j_lo, smem);
     stage_v(j_lo, smem + TILEB);
   }
@@ -580,6 +581,10 @@ ACCT_DEV void fa_fwd_body(const FaArgs& a) {
       for (; j <= j_hi + 1; j++) step(j);
     }
   } else if (j_lo <= j_hi) {
+    if (late) {
+      stage_k(j_lo, smem);
+      stage_v(j_lo, smem + TILEB);
+    }
     if (BIAS && bias_staged && wq0 < a.Sq) stage_bias(j_lo);
     DropStage::issue(a, bh, wq0, j_lo, lane, drop_lds);
     // A full wait the compiler can see: every load issued so far (Q fragments included) is complete, so
@@ -918,6 +923,7 @@ static hipError_t launch_fwd_kt(FaArgs a, hipStream_t st) {
   if (a.Sk >= 32 * KT && !(tile_offsets_fit(a.k_ss, 32 * KT) && tile_offsets_fit(a.v_ss, 32 * KT))) return hipErrorInvalidPitchValue;
   a.kv_share = split_shares(a.B * a.N, a.Sk, a.hd);
   a.merge_alone = fwd_merge_alone<D, KG>() && a.kv_split <= 1 && (long long)a.n_tiles * a.B * a.N > 256;
+  a.first_late = first_tile_late(a.B * a.N, a.n_tiles, visible_row_keys(a.Sq, a.Sk, a.prev_blk, a.next_blk, a.row_prefix), 32 * KT);
   const bool mask_t = BIAS || DROP || a.mask_kind == kMaskDense || a.mask_kind == kMaskTile;
   constexpr size_t biasb = BIAS ? (KT == 4 ? 1024 : QG * 4096) : 0;     // per wave, as in the kernel
   constexpr size_t tiles = 4 * 32 * KT * (size_t)C::PITCH + NW * biasb + (size_t)NW * 2 * DropRowStage<DROP, QG, KT>::BYTES,

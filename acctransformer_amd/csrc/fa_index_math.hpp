@@ -245,6 +245,14 @@ ACCT_HD bool long_tiles_pay(int BH, int Sq, int Sk, int D, int seen, bool moving
   return (long long)BH * ((Sq + 63) / 64) <= 256 && !own_keys && 20 * n128 > 33 * n256;
 }
 
+// Whether the forward requests its first tile behind the Q fragments and not ahead of them: launches of more than one round
+// whose workgroups walk a single tile and have a head's rows to themselves (nothing is left to do meanwhile, and Q waits behind
+// K and V).  Forward, us, ahead / behind, 1024 heads: 77 x 77, D128 31.5 / 29.1; 128 x 128 39.5 / 37.2; 256 x 128 48.7 / 47.2; with
+// dropout 53.4 / 49.4; D80 128 x 128 26.5 / 25.3; D64 18.0 / 16.8, dropout 26.2 / 23.8.  Where the row tiles of a head share its
+// keys it is the other way round: 1024 x 77, D128 174 / 188; D80 124 / 134.  (Head dims 40, 160 and 256: level or 1 to 3 % slower.)
+// `seen`: keys that a workgroup's rows see.
+ACCT_HD bool first_tile_late(int BH, int n_tiles, int seen, int tile_keys) { return n_tiles == 1 && BH > 256 && seen <= tile_keys; }
+
 // How the forward kernel cuts its work.  kg: key groups of the workgroup (fa_fwd.hip; 256 / kg query rows per
 // workgroup).  kv_split: slices of the key range on workgroups of their own, which a second kernel adds up (1: none).
 //

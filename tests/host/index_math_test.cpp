@@ -269,6 +269,7 @@ static void test_pipelined_walks() {
     }
   CHECK(!pipelined_pays(4096, 1023, false) && pipelined_pays(256, 1024, false), "short and long walks");
   CHECK(!pipelined_pays(2046, 2046, true) && pipelined_pays(2048, 2048, true) && !pipelined_pays(256, 8192, true), "causal walks");
+  CHECK(first_tile_late(257, 1, 128, 128) && !first_tile_late(256, 1, 128, 128) && !first_tile_late(512, 2, 128, 128) && !first_tile_late(512, 1, 129, 128), "one tile");
   CHECK(!pipelined_pays(8192, visible_row_keys(8192, 8192, 3, 3, 0), false) && pipelined_pays(8192, visible_row_keys(8192, 8192, 4, 4, 0), false), "bands");
 }
 

@@ -58,9 +58,12 @@ def test_the_gpu_tests_of_the_pipelined_forward_run_it(tmp_path):
             assert (plan["kg"], plan["kv_split"], plan["pipelined"]) == (1, 1, long), (Sq, Sk, D, side, plan)
 
 
-def test_the_gpu_tests_of_the_lone_merge_run_it(tmp_path):
-    from test_key_group_merge import LONE_MERGES
+def test_the_gpu_tests_of_launches_of_several_rounds_run_them(tmp_path):
+    from test_key_group_merge import LATE_TILES, LONE_MERGES
     for whole in (True, False):
         rows = [(B if whole else B // parts, N, Sq, Sk, D, 0) for B, N, Sq, Sk, D, parts in LONE_MERGES]
         for (B, N, Sq, Sk, D, _), plan in zip(rows, _plans(tmp_path, rows)):
             assert plan["kg"] == 2 and (B * N * ((Sq + 127) // 128) > 256) == whole, (B, N, Sq, Sk, D, plan)
+        rows = [(B if whole else B // parts, N, Sq, Sk, D, 0) for B, N, Sq, Sk, D, parts in LATE_TILES]
+        for (B, N, Sq, Sk, D, _), plan in zip(rows, _plans(tmp_path, rows)):
+            assert plan["kg"] == 1 and Sq <= 256 and Sk <= 128 and (B * N > 256) == whole, (B, N, Sq, Sk, D, plan)

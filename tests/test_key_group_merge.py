@@ -73,14 +73,15 @@ def test_forward_of_key_groups(B, N, Sq, Sk, D, side, dtype):
     assert np.max(np.abs(L - lse.cpu().numpy())) < 1e-4 * max(1.0, np.abs(L).max() / 10)
 
 
+# a launch of more than one round and parts that fit into one: two key groups, whose merge the first one does alone there, or one
+# group, whose first tile comes behind the Q fragments there
 LONE_MERGES = [(20, 16, 77, 77, 64, 2), (20, 16, 77, 200, 40, 2), (33, 8, 130, 129, 64, 3), (22, 6, 300, 65, 56, 2)]
+LATE_TILES = [(32, 16, 200, 77, 64, 2), (32, 16, 200, 100, 80, 2), (32, 16, 200, 128, 128, 2)]
 
 
 @pytest.mark.parametrize("side", ["none", "mask", "dropout", "key bias", "bias"])
-@pytest.mark.parametrize("B, N, Sq, Sk, D, parts", LONE_MERGES)
-def test_one_group_merging_alone_gives_the_same_bits(B, N, Sq, Sk, D, parts, side):
-    """A launch of more than one round leaves the merge of its two key groups to the first; each part of it fits into one round,
-    where the groups share it."""
+@pytest.mark.parametrize("B, N, Sq, Sk, D, parts", LONE_MERGES + LATE_TILES)
+def test_launches_of_several_rounds_give_the_bits_of_their_parts(B, N, Sq, Sk, D, parts, side):
     if D == 40 and "bias" in side:
         pytest.skip("not built")
     g = torch.Generator(device=DEV).manual_seed(Sq + Sk)
